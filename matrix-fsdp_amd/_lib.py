@@ -41,6 +41,21 @@ class CopyRun(Structure):
     ]
 
 
+class MuonJob(Structure):
+    """``mfsdp_muon_job``."""
+
+    _fields_ = [
+        ("param", c_void_p),
+        ("grad", c_void_p),
+        ("momentum_buf", c_void_p),
+        ("rows", c_int64),
+        ("cols", c_int64),
+        ("lr", c_double),
+        ("weight_decay", c_double),
+        ("adjusted_lr", c_double),
+    ]
+
+
 # name -> (restype, argtypes); every symbol include/mfsdp_hip.h declares
 SIGNATURES = {
     "mfsdp_last_error": (c_char_p, []),
@@ -87,6 +102,11 @@ SIGNATURES = {
         c_int,
         [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_double, c_double, c_double, c_int,
          c_float, c_float, c_float, c_int, c_float, c_double, c_int, c_void_p, c_int64, c_void_p],
+    ),
+    "mfsdp_muon_many_workspace_bytes": (c_int64, [c_int64, POINTER(c_int64), POINTER(c_int64)]),
+    "mfsdp_muon_step_many": (
+        c_int,
+        [c_int64, POINTER(MuonJob), c_int, c_double, c_int, c_float, c_float, c_float, c_int, c_float, c_void_p, c_int64, c_void_p],
     ),
     "mfsdp_set_muon_tuning": (None, [c_int, c_int, c_int, c_int, c_int]),
     "mfsdp_gemm_nt_bf16": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int64, c_void_p]),

@@ -5,39 +5,48 @@
 //     A  = X X^T                    P = Q = X          (symmetric: lower-triangle tiles, mirrored store)
 //     B  = b A + c A A = b A + c A A^T   P = Q = A     (symmetric)
 //     X' = a X + B X                P = B, Q = X^T     (writes X' and X'^T)
-// Every product is rounded to bf16, as the reference's bf16 addmm / mm do.  Buffers are zero-padded to
-// multiples of 256 so the GEMM needs no edge handling; zero rows and columns stay zero through the iteration.
+// Every product is rounded to bf16, as the reference's bf16 addmm / mm do.  Buffers are padded to multiples of 256 so
+// the GEMM needs no edge handling; what a product reads beyond a matrix's sides along K is zero.
+//
+// A step's matrices do not depend on each other: up to 32 of them go through every stage as ONE launch (momentum, norm,
+// scale + transpose, three products per iteration), so that small matrices fill the machine together and a step costs
+// 3 + 3 x steps launches instead of that many per matrix.
 #include "mfsdp_common.h"
 #include "muon_elementwise.h"
 #include "muon_gemm.h"
 
 #include <algorithm>
 #include <cmath>
+#include <utility>
+#include <vector>
 
 namespace mfsdp {
 namespace {
 
 constexpr int64_t kPad = 256;
 constexpr int64_t kAlign = 256;  // byte alignment of every workspace region
+constexpr int kTileK = 64;       // K of every product is rounded up to this: the operands are zero up to there
 
 int64_t round_up(int64_t v, int64_t to) { return (v + to - 1) / to * to; }
 
-struct Workspace {
+// One matrix in the workspace.  Leading dimensions are padded to multiples of 256, so that tiles of every variant stay
+// inside the buffers; only the part up to the next multiples of 64 is ever read as an operand's K or defined at all.
+struct Matrix {
+  int rows, cols;          // of the parameter
   int m, n, mp, np;        // short / long side and their padded sizes
   bool tall;               // rows > cols: the iteration runs on the transpose
   uint16_t* X[2];          // mp x np
   uint16_t* XT[2];         // np x mp
   uint16_t* A;             // mp x mp
   uint16_t* B;             // mp x mp
-  uint16_t* xraw;          // rows x cols unscaled bf16 update (aliases X[1])
-  float* partials;
-  float* scalars;
-  GemmScratch gemm;        // fp32 partial tiles of K-split GEMM pieces
   int64_t bytes;
+  uint16_t* xraw() const { return X[1]; }  // rows x cols unscaled bf16 update
 };
 
-bool plan_workspace(int64_t rows, int64_t cols, void* base, Workspace* w) {
+bool plan_matrix(int64_t rows, int64_t cols, char* base, Matrix* w) {
   if (rows <= 0 || cols <= 0 || rows > (1 << 30) || cols > (1 << 30)) return false;
+  w->rows = static_cast<int>(rows);
+  w->cols = static_cast<int>(cols);
   w->tall = rows > cols;
   w->m = static_cast<int>(std::min(rows, cols));
   w->n = static_cast<int>(std::max(rows, cols));
@@ -45,105 +54,197 @@ bool plan_workspace(int64_t rows, int64_t cols, void* base, Workspace* w) {
   w->np = static_cast<int>(round_up(w->n, kPad));
   const int64_t x_bytes = round_up(static_cast<int64_t>(w->mp) * w->np * 2, kAlign);
   const int64_t a_bytes = round_up(static_cast<int64_t>(w->mp) * w->mp * 2, kAlign);
-  char* p = static_cast<char*>(base);
   int64_t off = 0;
-  auto take = [&](int64_t bytes) { char* r = p ? p + off : nullptr; off += bytes; return r; };
-  w->X[0] = reinterpret_cast<uint16_t*>(take(x_bytes));
-  w->X[1] = reinterpret_cast<uint16_t*>(take(x_bytes));
-  w->XT[0] = reinterpret_cast<uint16_t*>(take(x_bytes));
-  w->XT[1] = reinterpret_cast<uint16_t*>(take(x_bytes));
-  w->A = reinterpret_cast<uint16_t*>(take(a_bytes));
-  w->B = reinterpret_cast<uint16_t*>(take(a_bytes));
-  w->scalars = reinterpret_cast<float*>(take(kAlign));
-  w->gemm.partials = take(kGemmPartialsBytes);
-  w->gemm.partials_bytes = kGemmPartialsBytes;
-  // the sums of squares of the momentum kernel are consumed by the norm before the first product runs
-  static_assert(kMuonMaxPartials * 4 <= kGemmPartialsBytes, "the partial sums borrow the products' scratch");
-  w->partials = reinterpret_cast<float*>(w->gemm.partials);
-  w->xraw = w->X[1];
+  auto take = [&](int64_t bytes) { char* r = base ? base + off : nullptr; off += bytes; return reinterpret_cast<uint16_t*>(r); };
+  w->X[0] = take(x_bytes);
+  w->X[1] = take(x_bytes);
+  w->XT[0] = take(x_bytes);
+  w->XT[1] = take(x_bytes);
+  w->A = take(a_bytes);
+  w->B = take(a_bytes);
   w->bytes = off;
   return true;
 }
 
-// Newton-Schulz on the update already sitting in w.xraw (rows x cols bf16) with per-block sums of squares in
-// w.partials.  Leaves O in param layout at *ortho with leading dimension *ldo.
-// The parameter update of the step, handed to the last product (see GemmNtArgs::update_param).
-struct ParamUpdate {
-  void* param = nullptr;
-  int dtype = MFSDP_F32;
-  float decay = 1.0f, neg_lr = 0.0f;
+// Behind the matrices of a launch: their norms and the scratch of the products.
+constexpr int64_t kSharedBytes = kAlign + kGemmPartialsBytes;
+static_assert(kMaxMuonGroup <= kMaxGemmGroup && kMaxMuonGroup * sizeof(float) <= kAlign, "a group travels through both kinds of launch");
+// the sums of squares of the momentum kernel are consumed by the norm before the first product runs
+static_assert(static_cast<int64_t>(kMaxMuonGroup) * kMuonMaxPartials * 4 <= kGemmPartialsBytes, "the partial sums borrow the products' scratch");
+
+// Most workspace a group is given beyond what its largest matrix needs anyway: three 15360 x 5120 matrices.  Matrices
+// that large fill the machine on their own, more of them side by side only cost memory.
+constexpr int64_t kGroupBytes = 2304ll << 20;
+
+// A group of matrices that go through every stage of the update together, one launch per stage.
+struct Group {
+  int n = 0;
+  Matrix w[kMaxMuonGroup];
+  void* param[kMaxMuonGroup];
+  float decay[kMaxMuonGroup], neg_lr[kMaxMuonGroup];
+  MuonMatrices elementwise;
+  GemmScratch scratch;
 };
 
-// With `update` and at least one step the last product writes the parameter itself and *ortho stays null.
-int run_newton_schulz(const Workspace& w, int rows, int cols, int n_partials, float a, float b, float c, int steps,
-                      float eps, bool shared, const ParamUpdate* update, const uint16_t** ortho, int* ldo, hipStream_t stream) {
-  if (int rc = muon_norm(w.partials, n_partials, eps, w.scalars, stream)) return rc;
-  // the input is rows x cols; the iteration wants the short side first
-  uint16_t* same = w.tall ? w.XT[0] : w.X[0];   // rows_pad x cols_pad
-  uint16_t* trans = w.tall ? w.X[0] : w.XT[0];  // cols_pad x rows_pad
-  const int rows_pad = w.tall ? w.np : w.mp;
-  const int cols_pad = w.tall ? w.mp : w.np;
-  if (int rc = muon_scale_transpose(w.xraw, rows, cols, w.scalars, same, trans, rows_pad, cols_pad, stream)) return rc;
+void finish_group(Group* g, char* shared) {
+  g->elementwise.n = g->n;
+  g->elementwise.norms = reinterpret_cast<float*>(shared);
+  g->scratch.partials = shared + kAlign;
+  g->scratch.partials_bytes = kGemmPartialsBytes;
+  float* partials = static_cast<float*>(g->scratch.partials);
+  for (int i = 0; i < g->n; ++i) {
+    const Matrix& w = g->w[i];
+    MuonMatrix& m = g->elementwise.m[i];
+    m.xraw = w.xraw();
+    // the input is rows x cols; the iteration wants the short side first
+    m.same = w.tall ? w.XT[0] : w.X[0];
+    m.trans = w.tall ? w.X[0] : w.XT[0];
+    m.ld_same = w.tall ? w.mp : w.np;
+    m.ld_trans = w.tall ? w.np : w.mp;
+    m.rows = w.rows;
+    m.cols = w.cols;
+    m.n_partials = muon_momentum_partials(static_cast<int64_t>(w.rows) * w.cols);
+    m.partials = partials;
+    partials += m.n_partials;
+  }
+}
+
+// Newton-Schulz on the updates already sitting in xraw with their partial sums of squares.  With `update_dtype` >= 0 and
+// at least one step the last product writes the parameters themselves; otherwise O is left in X[steps & 1] (wide) or
+// XT[steps & 1] (tall).
+int run_newton_schulz(const Group& group, float a, float b, float c, int steps, float eps, bool shared, int update_dtype, hipStream_t stream) {
+  if (int rc = muon_norm(group.elementwise, eps, stream)) return rc;
+  if (int rc = muon_scale_transpose(group.elementwise, stream)) return rc;
+  GemmGroup g;
+  g.n = group.n;
+  GemmPlan gram, poly, update;  // made in the first iteration
   for (int s = 0; s < steps; ++s) {
     const int cur = s & 1, nxt = cur ^ 1;
-    GemmNtArgs g{};
-    g.P = w.X[cur]; g.Q = w.X[cur]; g.D = nullptr; g.C = w.A; g.CT = nullptr;
-    g.M = w.mp; g.N = w.mp; g.K = w.np;
-    g.ldp = w.np; g.ldq = w.np; g.ldd = 0; g.ldc = w.mp; g.ldct = 0;
     g.alpha = 1.0f; g.beta = 0.0f; g.symmetric = 1; g.shared = shared;
-    if (int rc = gemm_nt_bf16(g, w.gemm, stream)) return rc;
+    for (int i = 0; i < group.n; ++i) {
+      const Matrix& w = group.w[i];
+      GemmProblem& p = g.problem[i] = GemmProblem{};
+      p.P = w.X[cur]; p.Q = w.X[cur]; p.C = w.A;
+      p.M = w.m; p.N = w.m; p.K = static_cast<int>(round_up(w.n, kTileK));
+      p.ldp = w.np; p.ldq = w.np; p.ldc = w.mp;
+    }
+    if (s == 0) gram = gemm_plan(g, group.scratch);
+    if (int rc = gemm_nt_bf16(g, gram, group.scratch, stream)) return rc;
     if (c == 0.0f) {
       // addmm with alpha = 0 leaves beta * A (the product is not formed at all, torch/optim/_muon.py:61 with a
       // quadratic polynomial); the GEMM's D path needs alpha != 0 (it adds (beta / alpha) D to the accumulators)
-      if (int rc = muon_scale_bf16(w.B, w.A, static_cast<int64_t>(w.mp) * w.mp, b, stream)) return rc;
+      for (int i = 0; i < group.n; ++i)
+        if (int rc = muon_scale_bf16(group.w[i].B, group.w[i].A, static_cast<int64_t>(group.w[i].mp) * group.w[i].mp, b, stream)) return rc;
     } else {
-      g = GemmNtArgs{};
-      g.P = w.A; g.Q = w.A; g.D = w.A; g.C = w.B; g.CT = nullptr;
-      g.d_transposed_is_q = 1;  // A is symmetric
-      g.M = w.mp; g.N = w.mp; g.K = w.mp;
-      g.ldp = w.mp; g.ldq = w.mp; g.ldd = w.mp; g.ldc = w.mp; g.ldct = 0;
-      g.alpha = c; g.beta = b; g.symmetric = 1; g.shared = shared;
-      if (int rc = gemm_nt_bf16(g, w.gemm, stream)) return rc;
+      g.alpha = c; g.beta = b;
+      for (int i = 0; i < group.n; ++i) {
+        const Matrix& w = group.w[i];
+        GemmProblem& p = g.problem[i] = GemmProblem{};
+        p.P = w.A; p.Q = w.A; p.D = w.A; p.C = w.B;  // A is symmetric: D^T is Q
+        p.M = w.m; p.N = w.m; p.K = static_cast<int>(round_up(w.m, kTileK));
+        p.ldp = w.mp; p.ldq = w.mp; p.ldd = w.mp; p.ldc = w.mp;
+      }
+      if (s == 0) poly = gemm_plan(g, group.scratch);
+      if (int rc = gemm_nt_bf16(g, poly, group.scratch, stream)) return rc;
     }
-    g = GemmNtArgs{};
-    g.P = w.B; g.Q = w.XT[cur]; g.D = w.X[cur]; g.C = w.X[nxt]; g.CT = w.XT[nxt];
-    g.d_transposed_is_q = 1;  // Q = X^T
-    g.M = w.mp; g.N = w.np; g.K = w.mp;
-    g.ldp = w.mp; g.ldq = w.mp; g.ldd = w.np; g.ldc = w.np; g.ldct = w.mp;
-    g.alpha = 1.0f; g.beta = a; g.symmetric = 0;
-    if (s + 1 == steps) {  // the last step only has to leave O in the parameter's orientation
-      if (w.tall) g.skip_c = 1;
-      else g.CT = nullptr;
-      if (update != nullptr) {  // ... or take it straight into the parameter: O is never stored
-        g.update_param = update->param;
-        g.update_dtype = update->dtype;
-        g.update_rows = rows;
-        g.update_cols = cols;
-        g.update_transposed = w.tall ? 1 : 0;
-        g.update_decay = update->decay;
-        g.update_neg_lr = update->neg_lr;
+    g.alpha = 1.0f; g.beta = a; g.symmetric = 0; g.shared = 0;
+    for (int i = 0; i < group.n; ++i) {
+      const Matrix& w = group.w[i];
+      GemmProblem& p = g.problem[i] = GemmProblem{};
+      p.P = w.B; p.Q = w.XT[cur]; p.D = w.X[cur]; p.C = w.X[nxt]; p.CT = w.XT[nxt];  // Q = X^T
+      p.M = w.m; p.N = w.n; p.K = static_cast<int>(round_up(w.m, kTileK));
+      p.ldp = w.mp; p.ldq = w.mp; p.ldd = w.np; p.ldc = w.np; p.ldct = w.mp;
+      if (s + 1 == steps) {  // the last step only has to leave O in the parameter's orientation
+        if (w.tall) p.flags |= kGemmSkipC;
+        else p.CT = nullptr;
+        if (update_dtype >= 0) {  // ... or take it straight into the parameter: O is never stored
+          g.update_dtype = update_dtype;
+          p.update_param = group.param[i];
+          p.update_decay = group.decay[i];
+          p.update_neg_lr = group.neg_lr[i];
+          if (w.tall) p.flags |= kGemmUpdateTransposed;
+        }
       }
     }
-    if (int rc = gemm_nt_bf16(g, w.gemm, stream)) return rc;
+    if (s == 0) update = gemm_plan(g, group.scratch);
+    if (int rc = gemm_nt_bf16(g, update, group.scratch, stream)) return rc;
   }
-  const int fin = steps & 1;
-  *ortho = (update != nullptr && steps > 0) ? nullptr : (w.tall ? w.XT[fin] : w.X[fin]);
-  *ldo = w.tall ? w.mp : w.np;
   return MFSDP_OK;
 }
 
-int check_common(int64_t rows, int64_t cols, float a, float b, float c, int steps, const void* workspace, int64_t workspace_bytes, Workspace* w) {
-  // everything that can be refused is refused here, before the first kernel is enqueued (a step must not be left half applied)
+const uint16_t* result_of(const Matrix& w, int steps) { return w.tall ? w.XT[steps & 1] : w.X[steps & 1]; }
+
+// everything that can be refused is refused before the first kernel is enqueued (a step must not be left half applied)
+int check_iteration(float a, float b, float c, int steps) {
   if (!std::isfinite(a) || !std::isfinite(b) || !std::isfinite(c) || (c != 0.0f && !std::isfinite(b / c)))
     return fail(MFSDP_ERR_INVALID, "Newton-Schulz coefficients must be finite (and b / c representable), got (%g, %g, %g)", a, b, c);
   if (steps < 0 || steps >= 100) return fail(MFSDP_ERR_INVALID, "Number of steps must be less than 100 for computational efficiency");
-  if (!plan_workspace(rows, cols, const_cast<void*>(workspace), w))
+  return MFSDP_OK;
+}
+
+int check_matrix(int64_t rows, int64_t cols, Matrix* w) {
+  if (!plan_matrix(rows, cols, nullptr, w))
     return fail(MFSDP_ERR_INVALID, "Input tensor gradient must be a 2D matrix with positive sizes, got %lld x %lld",
                 static_cast<long long>(rows), static_cast<long long>(cols));
-  if (workspace == nullptr || workspace_bytes < w->bytes)
-    return fail(MFSDP_ERR_INVALID, "workspace of %lld bytes needed, got %lld", static_cast<long long>(w->bytes),
-                static_cast<long long>(workspace_bytes));
+  return MFSDP_OK;
+}
+
+int check_workspace(const void* workspace, int64_t have, int64_t need) {
+  if (workspace == nullptr || have < need)
+    return fail(MFSDP_ERR_INVALID, "workspace of %lld bytes needed, got %lld", static_cast<long long>(need), static_cast<long long>(have));
   if (reinterpret_cast<uintptr_t>(workspace) % kAlign) return fail(MFSDP_ERR_INVALID, "workspace must be %lld-byte aligned", static_cast<long long>(kAlign));
+  return MFSDP_OK;
+}
+
+// What the matrices of one step have in common.
+struct StepArgs {
+  int dtype;
+  double momentum;
+  int nesterov;
+  float a, b, c;
+  int steps;
+  float eps;
+  bool shared;
+};
+
+int check_step(const StepArgs& s) {
+  if (int rc = check_iteration(s.a, s.b, s.c, s.steps)) return rc;
+  if (s.dtype != MFSDP_F32 && s.dtype != MFSDP_BF16) return fail(MFSDP_ERR_INVALID, "dtype must be f32 or bf16");
+  if (!(s.momentum >= 0.0)) return fail(MFSDP_ERR_INVALID, "momentum should be >= 0 but is: %g", s.momentum);
+  return MFSDP_OK;
+}
+
+int check_tensors(const void* param, const void* grad, const void* buf, int dtype, double lr, double weight_decay) {
+  if (!param || !grad || !buf) return fail(MFSDP_ERR_INVALID, "null tensor pointer");
+  const uintptr_t elem = dtype == MFSDP_F32 ? 4 : 2;
+  if ((reinterpret_cast<uintptr_t>(param) | reinterpret_cast<uintptr_t>(grad) | reinterpret_cast<uintptr_t>(buf)) % elem)
+    return fail(MFSDP_ERR_INVALID, "tensor pointers must be aligned to their elements");
+  if (!(lr >= 0.0)) return fail(MFSDP_ERR_INVALID, "Learning rate should be >= 0 but is: %g", lr);
+  if (!(weight_decay >= 0.0)) return fail(MFSDP_ERR_INVALID, "weight decay should be >= 0 but is: %g", weight_decay);
+  return MFSDP_OK;
+}
+
+// the host scalars are doubles, as in Python: 1 - lr * wd and -adjusted_lr are rounded to fp32 once, where the tensor
+// operation takes them
+void add_to_group(Group* g, const Matrix& w, void* param, const void* grad, void* buf, double lr, double weight_decay, double adjusted_lr) {
+  g->w[g->n] = w;
+  g->param[g->n] = param;
+  g->decay[g->n] = static_cast<float>(1.0 - lr * weight_decay);
+  g->neg_lr[g->n] = static_cast<float>(-adjusted_lr);
+  g->elementwise.m[g->n].grad = grad;
+  g->elementwise.m[g->n].buf = buf;
+  ++g->n;
+}
+
+int run_step(Group* g, char* shared, const StepArgs& s, hipStream_t stream) {
+  finish_group(g, shared);
+  if (int rc = muon_momentum(g->elementwise, s.dtype, s.momentum, s.nesterov, true, stream)) return rc;
+  if (int rc = run_newton_schulz(*g, s.a, s.b, s.c, s.steps, s.eps, s.shared, s.dtype, stream)) return rc;
+  if (s.steps > 0) return MFSDP_OK;  // the last product has updated the parameters
+  for (int i = 0; i < g->n; ++i) {
+    const Matrix& w = g->w[i];
+    if (int rc = muon_apply(g->param[i], s.dtype, result_of(w, 0), w.rows, w.cols, w.tall ? w.mp : w.np, g->decay[i], g->neg_lr[i], stream)) return rc;
+  }
   return MFSDP_OK;
 }
 
@@ -153,64 +254,72 @@ int check_common(int64_t rows, int64_t cols, float a, float b, float c, int step
 using namespace mfsdp;
 
 extern "C" int64_t mfsdp_muon_workspace_bytes(int64_t rows, int64_t cols) {
-  Workspace w;
-  return plan_workspace(rows, cols, nullptr, &w) ? w.bytes : 0;
+  Matrix w;
+  return plan_matrix(rows, cols, nullptr, &w) ? w.bytes + kSharedBytes : 0;
+}
+
+extern "C" int64_t mfsdp_muon_many_workspace_bytes(int64_t n, const int64_t* rows, const int64_t* cols) {
+  if (n <= 0 || rows == nullptr || cols == nullptr) return 0;
+  int64_t sum = 0, largest = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    Matrix w;
+    if (!plan_matrix(rows[i], cols[i], nullptr, &w)) return 0;
+    sum += w.bytes;
+    largest = std::max(largest, w.bytes);
+  }
+  return std::max(largest, std::min(sum, kGroupBytes)) + kSharedBytes;
 }
 
 extern "C" int64_t mfsdp_muon_executed_flops(int64_t rows, int64_t cols, int steps, int flags) {
-  Workspace w;
-  if (steps < 0 || !plan_workspace(rows, cols, nullptr, &w)) return 0;
-  GemmNtArgs gram{}, poly{}, update{};
-  gram.M = gram.N = w.mp; gram.K = w.np; gram.symmetric = 1;
-  poly.M = poly.N = poly.K = w.mp; poly.symmetric = 1;
+  Matrix w;
+  if (steps < 0 || !plan_matrix(rows, cols, nullptr, &w)) return 0;
+  GemmGroup gram, poly, update;
+  gram.n = poly.n = update.n = 1;
+  gram.symmetric = poly.symmetric = 1;
   gram.shared = poly.shared = (flags & MFSDP_MUON_SHARED_MACHINE) != 0;
-  update.M = w.mp; update.N = w.np; update.K = w.mp;
+  gram.problem[0] = poly.problem[0] = update.problem[0] = GemmProblem{};
+  auto size = [](GemmProblem& p, int64_t m, int64_t n, int64_t k) { p.M = static_cast<int>(m); p.N = static_cast<int>(n); p.K = static_cast<int>(round_up(k, kTileK)); };
+  size(gram.problem[0], w.m, w.m, w.n);
+  size(poly.problem[0], w.m, w.m, w.m);
+  size(update.problem[0], w.m, w.n, w.m);
   return steps * (gemm_nt_executed_flops(gram) + gemm_nt_executed_flops(poly) + gemm_nt_executed_flops(update));
 }
 
 extern "C" int mfsdp_newton_schulz(const void* update, int update_dtype, int64_t rows, int64_t cols, float a, float b, float c,
                                    int steps, float eps, void* out_bf16, void* workspace, int64_t workspace_bytes, void* stream) {
-  Workspace w;
-  if (int rc = check_common(rows, cols, a, b, c, steps, workspace, workspace_bytes, &w)) return rc;
+  Group g;
+  if (int rc = check_iteration(a, b, c, steps)) return rc;
+  if (int rc = check_matrix(rows, cols, &g.w[0])) return rc;
+  if (int rc = check_workspace(workspace, workspace_bytes, g.w[0].bytes + kSharedBytes)) return rc;
   if (update_dtype != MFSDP_F32 && update_dtype != MFSDP_BF16) return fail(MFSDP_ERR_INVALID, "update dtype must be f32 or bf16");
   if (!update || !out_bf16) return fail(MFSDP_ERR_INVALID, "null tensor pointer");
+  if (reinterpret_cast<uintptr_t>(update) % (update_dtype == MFSDP_F32 ? 4 : 2)) return fail(MFSDP_ERR_INVALID, "update must be aligned to its elements");
   hipStream_t s = as_stream(stream);
-  int n_partials = 0;
-  if (int rc = muon_momentum(update, nullptr, update_dtype, rows * cols, 0.0, 0, false, w.xraw, w.partials, &n_partials, s)) return rc;
-  const uint16_t* ortho = nullptr;
-  int ldo = 0;
-  if (int rc = run_newton_schulz(w, static_cast<int>(rows), static_cast<int>(cols), n_partials, a, b, c, steps, eps, false, nullptr, &ortho, &ldo, s)) return rc;
-  return muon_extract(out_bf16, ortho, static_cast<int>(rows), static_cast<int>(cols), ldo, s);
+  char* base = static_cast<char*>(workspace);
+  Matrix w;
+  plan_matrix(rows, cols, base, &w);
+  add_to_group(&g, w, nullptr, update, nullptr, 0.0, 0.0, 0.0);
+  finish_group(&g, base + w.bytes);
+  if (int rc = muon_momentum(g.elementwise, update_dtype, 0.0, 0, false, s)) return rc;
+  if (int rc = run_newton_schulz(g, a, b, c, steps, eps, false, -1, s)) return rc;
+  return muon_extract(out_bf16, result_of(w, steps), w.rows, w.cols, w.tall ? w.mp : w.np, s);
 }
 
 extern "C" int mfsdp_muon_step_ex(void* param, const void* grad, void* momentum_buf, int dtype, int64_t rows, int64_t cols, double lr,
                                   double weight_decay, double momentum, int nesterov, float a, float b, float c, int steps, float eps,
                                   double adjusted_lr, int flags, void* workspace, int64_t workspace_bytes, void* stream) {
-  Workspace w;
-  if (int rc = check_common(rows, cols, a, b, c, steps, workspace, workspace_bytes, &w)) return rc;
-  if (dtype != MFSDP_F32 && dtype != MFSDP_BF16) return fail(MFSDP_ERR_INVALID, "dtype must be f32 or bf16");
-  if (!param || !grad || !momentum_buf) return fail(MFSDP_ERR_INVALID, "null tensor pointer");
-  if (!(lr >= 0.0)) return fail(MFSDP_ERR_INVALID, "Learning rate should be >= 0 but is: %g", lr);
-  if (!(momentum >= 0.0)) return fail(MFSDP_ERR_INVALID, "momentum should be >= 0 but is: %g", momentum);
-  if (!(weight_decay >= 0.0)) return fail(MFSDP_ERR_INVALID, "weight decay should be >= 0 but is: %g", weight_decay);
+  const StepArgs s{dtype, momentum, nesterov, a, b, c, steps, eps, (flags & MFSDP_MUON_SHARED_MACHINE) != 0};
+  Matrix w;
+  if (int rc = check_step(s)) return rc;
+  if (int rc = check_matrix(rows, cols, &w)) return rc;
+  if (int rc = check_workspace(workspace, workspace_bytes, w.bytes + kSharedBytes)) return rc;
+  if (int rc = check_tensors(param, grad, momentum_buf, dtype, lr, weight_decay)) return rc;
   if (flags & ~MFSDP_MUON_SHARED_MACHINE) return fail(MFSDP_ERR_INVALID, "unknown flags 0x%x", flags);
-  hipStream_t s = as_stream(stream);
-  int n_partials = 0;
-  if (int rc = muon_momentum(grad, momentum_buf, dtype, rows * cols, momentum, nesterov, true, w.xraw, w.partials, &n_partials, s)) return rc;
-  const uint16_t* ortho = nullptr;
-  int ldo = 0;
-  // the host scalars are doubles, as in Python: 1 - lr * wd and -adjusted_lr are rounded to fp32 once, where the
-  // tensor operation takes them
-  ParamUpdate update;
-  update.param = param;
-  update.dtype = dtype;
-  update.decay = static_cast<float>(1.0 - lr * weight_decay);
-  update.neg_lr = static_cast<float>(-adjusted_lr);
-  if (int rc = run_newton_schulz(w, static_cast<int>(rows), static_cast<int>(cols), n_partials, a, b, c, steps, eps,
-                                 (flags & MFSDP_MUON_SHARED_MACHINE) != 0, &update, &ortho, &ldo, s))
-    return rc;
-  if (ortho == nullptr) return MFSDP_OK;  // the last product has updated the parameter
-  return muon_apply(param, dtype, ortho, static_cast<int>(rows), static_cast<int>(cols), ldo, update.decay, update.neg_lr, s);
+  char* base = static_cast<char*>(workspace);
+  plan_matrix(rows, cols, base, &w);
+  Group g;
+  add_to_group(&g, w, param, grad, momentum_buf, lr, weight_decay, adjusted_lr);
+  return run_step(&g, base + w.bytes, s, as_stream(stream));
 }
 
 extern "C" int mfsdp_muon_step(void* param, const void* grad, void* momentum_buf, int dtype, int64_t rows, int64_t cols, double lr,
@@ -220,16 +329,53 @@ extern "C" int mfsdp_muon_step(void* param, const void* grad, void* momentum_buf
                             adjusted_lr, 0, workspace, workspace_bytes, stream);
 }
 
+extern "C" int mfsdp_muon_step_many(int64_t n, const mfsdp_muon_job* jobs, int dtype, double momentum, int nesterov, float a, float b,
+                                    float c, int steps, float eps, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (n < 0 || (n > 0 && jobs == nullptr)) return fail(MFSDP_ERR_INVALID, "jobs is null or n negative");
+  if (n == 0) return MFSDP_OK;
+  const StepArgs s{dtype, momentum, nesterov, a, b, c, steps, eps, false};
+  if (int rc = check_step(s)) return rc;
+  std::vector<std::pair<int64_t, int64_t>> order;  // (bytes, job): the largest first, so that a group holds matrices of like size
+  int64_t largest = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    Matrix w;
+    if (int rc = check_matrix(jobs[i].rows, jobs[i].cols, &w)) return rc;
+    if (int rc = check_tensors(jobs[i].param, jobs[i].grad, jobs[i].momentum_buf, dtype, jobs[i].lr, jobs[i].weight_decay)) return rc;
+    order.emplace_back(w.bytes, i);
+    largest = std::max(largest, w.bytes);
+  }
+  if (int rc = check_workspace(workspace, workspace_bytes, largest + kSharedBytes)) return rc;
+  std::stable_sort(order.begin(), order.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+  char* base = static_cast<char*>(workspace);
+  const int64_t room = workspace_bytes - kSharedBytes;
+  for (size_t next = 0; next < order.size();) {
+    Group g;
+    int64_t used = 0;
+    while (next < order.size() && g.n < kMaxMuonGroup && used + order[next].first <= room) {
+      const mfsdp_muon_job& job = jobs[order[next].second];
+      Matrix w;
+      plan_matrix(job.rows, job.cols, base + used, &w);
+      add_to_group(&g, w, job.param, job.grad, job.momentum_buf, job.lr, job.weight_decay, job.adjusted_lr);
+      used += w.bytes;
+      ++next;
+    }
+    if (int rc = run_step(&g, base + used, s, as_stream(stream))) return rc;
+  }
+  return MFSDP_OK;
+}
+
 extern "C" int mfsdp_gemm_nt_bf16(const void* p, const void* q, void* c, int m, int n, int k, void* partials, int64_t partials_bytes, void* stream) {
-  GemmNtArgs g{};
-  g.P = p; g.Q = q; g.C = c;
-  g.M = m; g.N = n; g.K = k;
-  g.ldp = k; g.ldq = k; g.ldc = n;
-  g.alpha = 1.0f;
+  if (m % 256 || n % 256) return fail(MFSDP_ERR_INVALID, "mfsdp_gemm_nt_bf16: M=%d and N=%d must be multiples of 256", m, n);
+  GemmGroup g;
+  g.n = 1;
+  GemmProblem& a = g.problem[0] = GemmProblem{};
+  a.P = p; a.Q = q; a.C = c;
+  a.M = m; a.N = n; a.K = k;
+  a.ldp = k; a.ldq = k; a.ldc = n;
   GemmScratch scratch;
   scratch.partials = partials;
   scratch.partials_bytes = partials ? partials_bytes : 0;
-  return gemm_nt_bf16(g, scratch, as_stream(stream));
+  return gemm_nt_bf16(g, gemm_plan(g, scratch), scratch, as_stream(stream));
 }
 
 extern "C" void mfsdp_set_muon_tuning(int general_variant, int symmetric_variant, int group_m, int split_remainder,

@@ -1,4 +1,4 @@
-// Element-wise stages of the Muon update (see muon_elementwise.hip).  Internal to libmfsdp_hip.
+// Element-wise stages of the Muon update: momentum, norm, scale + transpose, parameter update.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -7,23 +7,49 @@
 
 namespace mfsdp {
 
-constexpr int kMuonMaxPartials = 1 << 18;  // workgroups of the momentum kernel = partial sums of squares (1 MiB of fp32)
+constexpr int kMuonMaxPartials = 1 << 18;  // upper bound on the workgroups of a matrix in the momentum kernel (one partial sum each)
+constexpr int kMaxMuonGroup = 32;          // matrices one launch carries by value in its kernel arguments
 
-// xraw <- bf16(u), partials <- per-block sums of bf16(u)^2, where u is the momentum/Nesterov update
-// (with_momentum; buf updated in place) or grad itself.  dtype: MFSDP_F32 / MFSDP_BF16 of grad and buf.
-int muon_momentum(const void* grad, void* buf, int dtype, int64_t numel, double momentum, int nesterov, bool with_momentum,
-                  void* xraw, float* partials, int* n_partials, hipStream_t stream);
-// scalars[0] <- max(bf16(sqrt(sum partials)), bf16(eps))
-int muon_norm(const float* partials, int n_partials, float eps, float* scalars, hipStream_t stream);
-// same[rows_pad x cols_pad] <- bf16(xraw / scalars[0]) zero-padded; trans[cols_pad x rows_pad] <- its transpose
-int muon_scale_transpose(const void* xraw, int rows, int cols, const float* scalars, void* same, void* trans, int rows_pad,
-                         int cols_pad, hipStream_t stream);
-// param <- round(round(param*decay) + neg_lr*ortho), ortho bf16 with leading dimension ldo
+// One matrix of a launch.  `same` / `trans` receive the scaled update and its transpose: rows x cols with ld_same, cols x
+// rows with ld_trans, both zero up to the next multiples of 64.
+struct MuonMatrix {
+  const void* grad;
+  void* buf;         // momentum buffer
+  uint16_t* xraw;    // rows x cols unscaled bf16 update
+  uint16_t* same;
+  uint16_t* trans;
+  float* partials;   // sums of squares, one per workgroup of the momentum kernel
+  int n_partials;
+  int rows, cols;
+  int ld_same, ld_trans;
+};
+
+struct MuonMatrices {
+  int n = 0;
+  float* norms = nullptr;  // one per matrix
+  MuonMatrix m[kMaxMuonGroup];
+};
+
+// Workgroups (and partial sums) of a matrix of `numel` elements in muon_momentum.
+int muon_momentum_partials(int64_t numel);
+
+// buf <- lerp(buf, g, 1-mu); xraw <- bf16(nesterov ? lerp(g, buf, mu) : buf); partial sums of squares of every matrix
+// (without momentum: xraw <- bf16(g)).
+int muon_momentum(const MuonMatrices& g, int dtype, double momentum, int nesterov, bool with_momentum, hipStream_t stream);
+
+// norms[i] = max(bf16(sqrt(sum of matrix i's partials)), bf16(eps)).
+int muon_norm(const MuonMatrices& g, float eps, hipStream_t stream);
+
+// same[r][c] = bf16(x[r][c] / norm), trans[c][r] = same[r][c].
+int muon_scale_transpose(const MuonMatrices& g, hipStream_t stream);
+
+// p <- p*decay - adj_lr * O (torch/optim/_muon.py:313-315).
 int muon_apply(void* param, int dtype, const void* ortho, int rows, int cols, int ldo, float decay, float neg_lr,
                hipStream_t stream);
-// out <- bf16(scale * in) over numel contiguous bf16 (whole 16-byte groups)
-int muon_scale_bf16(void* out, const void* in, int64_t numel, float scale, hipStream_t stream);
-// out[rows x cols] contiguous bf16 <- ortho (leading dimension ldo)
+
 int muon_extract(void* out, const void* ortho, int rows, int cols, int ldo, hipStream_t stream);
+
+// out <- bf16(scale * in), numel a multiple of 8 and both pointers 16-byte aligned.
+int muon_scale_bf16(void* out, const void* in, int64_t numel, float scale, hipStream_t stream);
 
 }  // namespace mfsdp

@@ -96,22 +96,25 @@ __device__ __forceinline__ float momentum_one(float g, float b_old, float moment
   return xf * xf;
 }
 
-template <bool NT, typename V>
-__device__ __forceinline__ V ld(const V* p) {
-  if constexpr (NT) return __builtin_nontemporal_load(p);
-  else return *p;
-}
-template <bool NT, typename V>
-__device__ __forceinline__ void st(V* p, V v) {
-  if constexpr (NT) __builtin_nontemporal_store(v, p);
-  else *p = v;
-}
+// Four elements as one access.  Parameters, gradients and momentum buffers are views of flat shards that start at any
+// element: the accesses are aligned to an element only (global memory takes that at full vector width).
 template <typename T>
 struct QuadOf;
 template <>
-struct QuadOf<float> { typedef f32x4 type; };
+struct QuadOf<float> {
+  typedef f32x4 type;
+  typedef f32x4 any __attribute__((aligned(4)));
+  static __device__ __forceinline__ type load(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const any*>(p)); }
+  static __device__ __forceinline__ void store(float* p, type v) { __builtin_nontemporal_store(v, reinterpret_cast<any*>(p)); }
+};
 template <>
-struct QuadOf<uint16_t> { typedef u32x2 type; };
+struct QuadOf<uint16_t> {
+  typedef u32x2 type;
+  typedef u32x2 any __attribute__((aligned(2)));
+  static __device__ __forceinline__ type load(const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const any*>(p)); }
+  static __device__ __forceinline__ type load_cached(const uint16_t* p) { return *reinterpret_cast<const any*>(p); }
+  static __device__ __forceinline__ void store(uint16_t* p, type v) { __builtin_nontemporal_store(v, reinterpret_cast<any*>(p)); }
+};
 template <typename T>
 __device__ __forceinline__ float quad_elem(const typename QuadOf<T>::type& q, int e) {
   if constexpr (sizeof(T) == 4) return q[e];
@@ -130,27 +133,49 @@ __device__ __forceinline__ typename QuadOf<T>::type quad_pack(const float (&v)[4
 constexpr int kMomentumThreads = 64;  // one wavefront per workgroup
 constexpr int kMomentumQuads = 2;     // groups of four elements per thread, all of their loads issued before the first use
 
-// n_quads groups of four elements are processed with 128-bit (fp32) / 64-bit (bf16) accesses, the rest one by one.
+struct GroupArgs {
+  int begin[kMaxMuonGroup + 1];  // first workgroup of a matrix; entries past n repeat the end
+  MuonMatrices g;
+};
+static_assert(sizeof(GroupArgs) <= 4000, "kernel arguments are limited to 4 KiB");
+
+// The matrix whose workgroups hold `block`: the whole table is one scalar load, then compares (a search by dependent
+// loads would wait out a memory latency at every step).
+__device__ __forceinline__ int matrix_of(const GroupArgs& a, int block) {
+  if (a.g.n == 1) return 0;
+  int p = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxMuonGroup; ++i) p += block >= a.begin[i] ? 1 : 0;
+  return p < a.g.n ? p : a.g.n - 1;
+}
+
+// Groups of four elements are processed with 128-bit (fp32) / 64-bit (bf16) accesses, the rest one by one.
 // One small workgroup per 512 elements rather than a persistent grid (the grid-stride loop only runs when the grid
 // is capped): workgroups are dispatched in order, so the ones in flight sweep neighbouring addresses of the four
 // streams, and every byte but the bf16 update (read again by the next kernel) is touched once and bypasses the caches.
 // 12288 x 4096 fp32: 113-118 us against 147 us for 2048 persistent workgroups of 256 threads.
-template <typename T, bool MOMENTUM, bool NTX>
+template <typename T, bool MOMENTUM>
 __global__ void __launch_bounds__(kMomentumThreads)
-momentum_kernel(const T* __restrict__ grad, T* __restrict__ buf, uint16_t* __restrict__ xraw, float* __restrict__ partials,
-                int64_t numel, int64_t n_quads, float momentum, float one_minus_momentum, int nesterov) {
-  typedef typename QuadOf<T>::type Q;
+momentum_kernel(GroupArgs args, float momentum, float one_minus_momentum, int nesterov) {
+  typedef QuadOf<T> Q;
   constexpr int U = kMomentumQuads;
+  const int index = matrix_of(args, blockIdx.x);
+  const MuonMatrix& m = args.g.m[index];
+  const int block = blockIdx.x - args.begin[index];
+  const T* __restrict__ grad = static_cast<const T*>(m.grad);
+  T* __restrict__ buf = static_cast<T*>(m.buf);
+  uint16_t* __restrict__ xraw = m.xraw;
+  const int64_t numel = static_cast<int64_t>(m.rows) * m.cols, n_quads = numel / 4;
   float sumsq = 0.0f;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kMomentumThreads;
-  for (int64_t base = static_cast<int64_t>(blockIdx.x) * kMomentumThreads * U + threadIdx.x; base < n_quads; base += stride * U) {
-    Q g[U], b[U];
+  const int64_t stride = static_cast<int64_t>(m.n_partials) * kMomentumThreads;
+  for (int64_t base = static_cast<int64_t>(block) * kMomentumThreads * U + threadIdx.x; base < n_quads; base += stride * U) {
+    typename Q::type g[U], b[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t v = base + u * kMomentumThreads;
       if (v < n_quads) {
-        g[u] = ld<true>(reinterpret_cast<const Q*>(grad) + v);
-        if constexpr (MOMENTUM) b[u] = ld<true>(reinterpret_cast<const Q*>(buf) + v);
+        g[u] = Q::load(grad + 4 * v);
+        if constexpr (MOMENTUM) b[u] = Q::load(buf + 4 * v);
       }
     }
 #pragma unroll
@@ -163,14 +188,16 @@ momentum_kernel(const T* __restrict__ grad, T* __restrict__ buf, uint16_t* __res
         for (int e = 0; e < 4; ++e)
           sumsq += momentum_one<T, MOMENTUM>(quad_elem<T>(g[u], e), MOMENTUM ? quad_elem<T>(b[u], e) : 0.0f, momentum, one_minus_momentum,
                                              nesterov, &bn[e], &xb[e]);
-        if constexpr (MOMENTUM) st<true>(reinterpret_cast<Q*>(buf) + v, quad_pack<T>(bn));
+        if constexpr (MOMENTUM) Q::store(buf + 4 * v, quad_pack<T>(bn));
+        // the bf16 update is stored through the caches: the next kernel reads it (non-temporal stores of it, and of the
+        // scaled matrices behind it, were measured no faster in the step)
         const u32x2 packed = {static_cast<uint32_t>(xb[0]) | (static_cast<uint32_t>(xb[1]) << 16),
                               static_cast<uint32_t>(xb[2]) | (static_cast<uint32_t>(xb[3]) << 16)};
-        st<NTX>(reinterpret_cast<u32x2*>(xraw) + v, packed);
+        reinterpret_cast<u32x2*>(xraw)[v] = packed;
       }
     }
   }
-  for (int64_t i = n_quads * 4 + static_cast<int64_t>(blockIdx.x) * kMomentumThreads + threadIdx.x; i < numel; i += stride) {
+  for (int64_t i = n_quads * 4 + static_cast<int64_t>(block) * kMomentumThreads + threadIdx.x; i < numel; i += stride) {
     float bn = 0.0f;
     uint16_t xb;
     sumsq += momentum_one<T, MOMENTUM>(Elem<T>::load(grad, i), MOMENTUM ? Elem<T>::load(buf, i) : 0.0f, momentum, one_minus_momentum,
@@ -180,14 +207,16 @@ momentum_kernel(const T* __restrict__ grad, T* __restrict__ buf, uint16_t* __res
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) sumsq += __shfl_down(sumsq, off, 64);
-  if (threadIdx.x == 0) partials[blockIdx.x] = sumsq;
+  if (threadIdx.x == 0) m.partials[block] = sumsq;
 }
 
 constexpr int kNormThreads = 1024;
 
-// scalars[0] = max(bf16(sqrt(sum partials)), bf16(eps)); one workgroup, the sum in double and in a fixed order
+// norms[i] = max(bf16(sqrt(sum partials)), bf16(eps)); one workgroup per matrix, the sum in double and in a fixed order
 __global__ void __launch_bounds__(kNormThreads)
-norm_kernel(const float* __restrict__ partials, int n_partials, float eps, float* __restrict__ scalars) {
+norm_kernel(MuonMatrices args, float eps) {
+  const float* __restrict__ partials = args.m[blockIdx.x].partials;
+  const int n_partials = args.m[blockIdx.x].n_partials;
   __shared__ double lds[kNormThreads];
   double s = 0.0;
   const int n_vec = n_partials / 4;
@@ -215,28 +244,34 @@ norm_kernel(const float* __restrict__ partials, int n_partials, float eps, float
   if (threadIdx.x == 0) {
     const float norm = bf16_to_f32(f32_to_bf16(sqrtf(static_cast<float>(lds[0]))));
     const float floor_ = bf16_to_f32(f32_to_bf16(eps));
-    scalars[0] = norm > floor_ ? norm : floor_;
+    args.norms[blockIdx.x] = norm > floor_ ? norm : floor_;
   }
 }
 
-// 64 x 64 tile of the zero-padded outputs per block:
-//   same [r][c]  = bf16(x[r][c] / norm)   (rows_pad x cols_pad, ld = cols_pad)
-//   trans[c][r]  = same[r][c]             (cols_pad x rows_pad, ld = rows_pad)
+// 64 x 64 tile of the outputs per block:
+//   same [r][c]  = bf16(x[r][c] / norm)   (ld_same)
+//   trans[c][r]  = same[r][c]             (ld_trans)
 // with x = 0 outside rows x cols.  Every thread handles groups of four consecutive elements: 64-bit stores on
-// both outputs (the padded buffers are 256-element aligned); the input is read 64 bits at a time when quads is set.
+// both outputs (their rows are 256-element aligned), 64-bit loads that need element alignment only.
 __global__ void __launch_bounds__(kThreads)
-scale_transpose_kernel(const uint16_t* __restrict__ xraw, int rows, int cols, int quads, const float* __restrict__ scalars,
-                       uint16_t* __restrict__ same, uint16_t* __restrict__ trans, int rows_pad, int cols_pad) {
+scale_transpose_kernel(GroupArgs args) {
   __shared__ uint16_t tile[64][68];
-  const float norm = scalars[0];
-  const int r0 = blockIdx.y * 64, c0 = blockIdx.x * 64;
+  const int index = matrix_of(args, blockIdx.x);
+  const MuonMatrix& m = args.g.m[index];
+  const int block = blockIdx.x - args.begin[index];
+  const int rows = m.rows, cols = m.cols, tile_cols = (cols + 63) / 64;
+  const float norm = args.g.norms[index];
+  const uint16_t* __restrict__ xraw = m.xraw;
+  uint16_t* __restrict__ same = m.same;
+  uint16_t* __restrict__ trans = m.trans;
+  const int r0 = block / tile_cols * 64, c0 = block % tile_cols * 64;
   for (int e = threadIdx.x; e < 64 * 16; e += kThreads) {
     const int lr = e >> 4, lc = (e & 15) * 4;
     const int r = r0 + lr, c = c0 + lc;
     uint16_t raw[4] = {0, 0, 0, 0};
     if (r < rows) {
-      if (quads && c + 3 < cols) {
-        const u32x2 q = *reinterpret_cast<const u32x2*>(xraw + static_cast<int64_t>(r) * cols + c);
+      if (c + 3 < cols) {
+        const u32x2 q = QuadOf<uint16_t>::load_cached(xraw + static_cast<int64_t>(r) * cols + c);
         raw[0] = static_cast<uint16_t>(q.x); raw[1] = static_cast<uint16_t>(q.x >> 16);
         raw[2] = static_cast<uint16_t>(q.y); raw[3] = static_cast<uint16_t>(q.y >> 16);
       } else {
@@ -253,14 +288,14 @@ scale_transpose_kernel(const uint16_t* __restrict__ xraw, int rows, int cols, in
     }
     const u32x2 packed = {static_cast<uint32_t>(v[0]) | (static_cast<uint32_t>(v[1]) << 16),
                           static_cast<uint32_t>(v[2]) | (static_cast<uint32_t>(v[3]) << 16)};
-    *reinterpret_cast<u32x2*>(same + static_cast<int64_t>(r) * cols_pad + c) = packed;
+    *reinterpret_cast<u32x2*>(same + static_cast<int64_t>(r) * m.ld_same + c) = packed;
   }
   __syncthreads();
   for (int e = threadIdx.x; e < 64 * 16; e += kThreads) {
     const int lc = e >> 4, lr = (e & 15) * 4;  // a row of trans = a column of the tile, four rows of the tile at a time
     const u32x2 packed = {static_cast<uint32_t>(tile[lr][lc]) | (static_cast<uint32_t>(tile[lr + 1][lc]) << 16),
                           static_cast<uint32_t>(tile[lr + 2][lc]) | (static_cast<uint32_t>(tile[lr + 3][lc]) << 16)};
-    *reinterpret_cast<u32x2*>(trans + static_cast<int64_t>(c0 + lc) * rows_pad + r0 + lr) = packed;
+    *reinterpret_cast<u32x2*>(trans + static_cast<int64_t>(c0 + lc) * m.ld_trans + r0 + lr) = packed;
   }
 }
 
@@ -309,33 +344,35 @@ scale_bf16_kernel(const u32x4* __restrict__ in, u32x4* __restrict__ out, int64_t
   }
 }
 
-int partial_blocks(int64_t numel, int64_t n_quads) {
-  // one workgroup per kMomentumQuads * 64 groups of four, or per 64 of the elements left over (everything, when the
-  // tensors are not aligned for vector accesses)
-  const int64_t work = std::max<int64_t>((n_quads + kMomentumQuads - 1) / kMomentumQuads, numel - n_quads * 4);
-  const int64_t want = (work + kMomentumThreads - 1) / kMomentumThreads;
+}  // namespace
+
+int muon_momentum_partials(int64_t numel) {
+  // one workgroup per kMomentumQuads * 64 groups of four
+  const int64_t want = (numel / 4 + kMomentumQuads * kMomentumThreads - 1) / (kMomentumQuads * kMomentumThreads);
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(want, kMuonMaxPartials)));
 }
 
+namespace {
+template <typename Blocks>
+int fill_group(GroupArgs* args, const MuonMatrices& g, Blocks&& blocks_of) {
+  args->g = g;
+  int blocks = 0;
+  for (int i = 0; i <= kMaxMuonGroup; ++i) {
+    args->begin[i] = blocks;
+    if (i < g.n) blocks += blocks_of(g.m[i]);
+  }
+  return blocks;
+}
 }  // namespace
 
-int muon_momentum(const void* grad, void* buf, int dtype, int64_t numel, double momentum, int nesterov, bool with_momentum,
-                  void* xraw, float* partials, int* n_partials, hipStream_t stream) {
+int muon_momentum(const MuonMatrices& g, int dtype, double momentum, int nesterov, bool with_momentum, hipStream_t stream) {
   // the scalars torch hands to lerp_ are the Python doubles 1 - momentum and momentum, rounded to fp32 by the kernel
   const float one_minus = static_cast<float>(1.0 - momentum);
   const float weight = static_cast<float>(momentum);
-  auto x = static_cast<uint16_t*>(xraw);
-  const uintptr_t need = dtype == MFSDP_F32 ? 16 : 8;  // alignment of a group of four elements
-  const bool aligned = reinterpret_cast<uintptr_t>(grad) % need == 0 && (!with_momentum || reinterpret_cast<uintptr_t>(buf) % need == 0) &&
-                       reinterpret_cast<uintptr_t>(xraw) % 8 == 0;
-  const int64_t n_quads = aligned ? numel / 4 : 0;
-  const int blocks = partial_blocks(numel, n_quads);
-  *n_partials = blocks;
-  // the bf16 update is stored through the caches: the next kernel reads it (non-temporal stores of it, and of the scaled
-  // matrices behind it, were measured no faster in the step)
-#define MFSDP_MOMENTUM(T_, MOM_)                                                                                                  \
-  hipLaunchKernelGGL((momentum_kernel<T_, MOM_, false>), dim3(blocks), dim3(kMomentumThreads), 0, stream, static_cast<const T_*>(grad), \
-                     static_cast<T_*>(buf), x, partials, numel, n_quads, weight, one_minus, nesterov)
+  GroupArgs args;
+  const dim3 grid(fill_group(&args, g, [](const MuonMatrix& m) { return m.n_partials; }));
+#define MFSDP_MOMENTUM(T_, MOM_) \
+  hipLaunchKernelGGL((momentum_kernel<T_, MOM_>), grid, dim3(kMomentumThreads), 0, stream, args, weight, one_minus, nesterov)
   if (dtype == MFSDP_F32) {
     if (with_momentum) MFSDP_MOMENTUM(float, true); else MFSDP_MOMENTUM(float, false);
   } else {
@@ -346,18 +383,16 @@ int muon_momentum(const void* grad, void* buf, int dtype, int64_t numel, double 
   return MFSDP_OK;
 }
 
-int muon_norm(const float* partials, int n_partials, float eps, float* scalars, hipStream_t stream) {
-  hipLaunchKernelGGL(norm_kernel, dim3(1), dim3(kNormThreads), 0, stream, partials, n_partials, eps, scalars);
+int muon_norm(const MuonMatrices& g, float eps, hipStream_t stream) {
+  hipLaunchKernelGGL(norm_kernel, dim3(g.n), dim3(kNormThreads), 0, stream, g, eps);
   MFSDP_CHECK_LAUNCH("norm_kernel");
   return MFSDP_OK;
 }
 
-int muon_scale_transpose(const void* xraw, int rows, int cols, const float* scalars, void* same, void* trans, int rows_pad,
-                         int cols_pad, hipStream_t stream) {
-  const dim3 grid(cols_pad / 64, rows_pad / 64);
-  const int quads = (cols % 4 == 0 && reinterpret_cast<uintptr_t>(xraw) % 8 == 0) ? 1 : 0;
-  hipLaunchKernelGGL(scale_transpose_kernel, grid, dim3(kThreads), 0, stream, static_cast<const uint16_t*>(xraw), rows, cols, quads,
-                     scalars, static_cast<uint16_t*>(same), static_cast<uint16_t*>(trans), rows_pad, cols_pad);
+int muon_scale_transpose(const MuonMatrices& g, hipStream_t stream) {
+  GroupArgs args;
+  const dim3 grid(fill_group(&args, g, [](const MuonMatrix& m) { return ((m.rows + 63) / 64) * ((m.cols + 63) / 64); }));
+  hipLaunchKernelGGL(scale_transpose_kernel, grid, dim3(kThreads), 0, stream, args);
   MFSDP_CHECK_LAUNCH("scale_transpose_kernel");
   return MFSDP_OK;
 }

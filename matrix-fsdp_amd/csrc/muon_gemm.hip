@@ -10,12 +10,19 @@
 // next ones stream from HBM straight into LDS (buffer_load ... lds, no register round trip) while the
 // current one feeds the MFMAs.
 //
-// Tile scheduling.  Tiles are handed to workgroups so that the groups sharing an XCD (block ids
-// congruent mod 8) work on neighbouring tiles and reuse that XCD's L2, whatever the tile count.  When the tile count is not a
-// multiple of the number of resident workgroups, the tiles of the last, partial round are split along
-// K into pieces that fill the machine once more for a fraction of a tile's time; each piece leaves an
-// fp32 partial tile in a workspace and a small fix-up kernel sums the pieces in split order and runs
-// the epilogue (the kernel boundary is the only synchronisation: no fences, no spinning).
+// Several problems in one launch.  A launch carries up to 32 products by value in its kernel arguments: small matrices
+// fill the machine together and pay for one launch (24 matrices of 1536 x 1024: 1.24 ms for the whole Muon step against
+// 6.15 ms with a launch per matrix, stage and fix-up on three streams; two of 512 x 256: 0.16 against 0.37 ms).
+//
+// Tile order.  In every round of resident workgroups an XCD (block ids congruent mod 8) gets one contiguous eighth of the
+// round's tiles and so reuses its L2, while the machine as a whole works on one nearly square block of tiles: the update
+// products of 15360 x 5120 and 5120 x 13824 take 1209 us, against 1260 us when every XCD walks through its own contiguous
+// eighth of a matrix's tiles and 1484 us when it walks through its eighth of both matrices' tiles.
+//
+// K pieces.  When the tile count is not a multiple of the number of resident workgroups, tiles of the last, partial round
+// may be split along K into pieces that fill the machine; each piece leaves an fp32 partial tile in a workspace and a
+// small fix-up kernel sums the pieces in split order and runs the epilogue (the kernel boundary is the only
+// synchronisation: no fences, no spinning).
 #include "muon_gemm.h"
 
 #include "mfsdp_common.h"
@@ -24,6 +31,7 @@
 #include <mutex>
 #include <type_traits>
 #include <utility>
+#include <vector>
 
 namespace mfsdp {
 namespace {
@@ -32,6 +40,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+// 16 bytes of a parameter, aligned to one element (global memory takes any alignment at full vector width)
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
 
 constexpr int kXcds = 8;
 constexpr int kSlabK = 64;  // K granularity of the schedule (operands are padded to it); a slab is BK <= 64 wide
@@ -45,12 +56,14 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 __device__ __forceinline__ float bf16_bits_to_float(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
 
 // param[prow][pcol .. pcol + count - 1] <- round(param * decay) + neg_lr * o for the first `count` bf16 values o of `eight`
-// (those inside the parameter's update_rows x update_cols); a.update_vectors says that whole groups of eight may use
-// 16-byte accesses.
-__device__ __forceinline__ void update_param8(const GemmNtArgs& a, int prow, int pcol, const u32x4& eight, int count = 8) {
-  if (prow >= a.update_rows || pcol >= a.update_cols) return;
-  const int n = a.update_cols - pcol < count ? a.update_cols - pcol : count;
-  const int64_t at = static_cast<int64_t>(prow) * a.update_cols + pcol;
+// (those inside the parameter).  Whole groups use 16-byte accesses aligned to an element only: rows of any length and
+// parameters that start anywhere in a shard go the same way.
+__device__ __forceinline__ void update_param8(const GemmProblem& a, int dtype, int prow, int pcol, const u32x4& eight, int count = 8) {
+  const bool transposed = (a.flags & kGemmUpdateTransposed) != 0;
+  const int update_rows = transposed ? a.N : a.M, update_cols = transposed ? a.M : a.N;
+  if (prow >= update_rows || pcol >= update_cols) return;
+  const int n = update_cols - pcol < count ? update_cols - pcol : count;
+  const int64_t at = static_cast<int64_t>(prow) * update_cols + pcol;
   float o[8];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
@@ -58,17 +71,17 @@ __device__ __forceinline__ void update_param8(const GemmNtArgs& a, int prow, int
     o[2 * e + 1] = __uint_as_float(eight[e] & 0xffff0000u);
   }
   const float decay = a.update_decay, neg_lr = a.update_neg_lr;
-  if (a.update_dtype == MFSDP_F32) {
+  if (dtype == MFSDP_F32) {
     float* p = static_cast<float*>(a.update_param) + at;
-    if (n == 8 && a.update_vectors) {
-      f32x4 lo = reinterpret_cast<const f32x4*>(p)[0], hi = reinterpret_cast<const f32x4*>(p)[1];
+    if (n == 8) {
+      f32x4 lo = reinterpret_cast<const f32x4_a4*>(p)[0], hi = reinterpret_cast<const f32x4_a4*>(p)[1];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         lo[e] = lo[e] * decay + neg_lr * o[e];
         hi[e] = hi[e] * decay + neg_lr * o[4 + e];
       }
-      reinterpret_cast<f32x4*>(p)[0] = lo;
-      reinterpret_cast<f32x4*>(p)[1] = hi;
+      reinterpret_cast<f32x4_a4*>(p)[0] = lo;
+      reinterpret_cast<f32x4_a4*>(p)[1] = hi;
     } else {
       for (int e = 0; e < n; ++e) p[e] = p[e] * decay + neg_lr * o[e];
     }
@@ -78,25 +91,45 @@ __device__ __forceinline__ void update_param8(const GemmNtArgs& a, int prow, int
       const float scaled = bf16_bits_to_float(__builtin_bit_cast(uint16_t, static_cast<__bf16>(bf16_bits_to_float(old) * decay)));
       return __builtin_bit_cast(uint16_t, static_cast<__bf16>(scaled + neg_lr * ov));
     };
-    if (n == 8 && a.update_vectors) {
-      u32x4 v = *reinterpret_cast<const u32x4*>(p);
+    if (n == 8) {
+      u32x4 v = *reinterpret_cast<const u32x4_a2*>(p);
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         v[e] = static_cast<uint32_t>(one(static_cast<uint16_t>(v[e]), o[2 * e])) | (static_cast<uint32_t>(one(static_cast<uint16_t>(v[e] >> 16), o[2 * e + 1])) << 16);
-      *reinterpret_cast<u32x4*>(p) = v;
+      *reinterpret_cast<u32x4_a2*>(p) = v;
     } else {
       for (int e = 0; e < n; ++e) p[e] = one(p[e], o[e]);
     }
   }
 }
 
-struct Schedule {
-  int tiles_m, tiles_n;
-  int full_tiles;   // tiles computed whole, one per workgroup (block ids [0, full_tiles))
-  int splits;       // K pieces per remaining tile (block ids from full_tiles on); 1 when nothing remains
-  float* partials;  // [remaining tiles][splits][BM][BN] fp32
-  int group_m;      // tile rows per group of the general products' tile order
+// Kernel argument: the problems of a launch and which workgroup does what.  Block ids [0, tile_begin[n]) compute one
+// whole tile each, problem after problem (longest K first); behind them come the K pieces of the split tiles.
+struct LaunchArgs {
+  int tile_begin[kMaxGemmGroup + 1];   // first whole-tile block of a problem; entries past n repeat the end
+  int piece_begin[kMaxGemmGroup + 1];  // first piece block
+  int split_begin[kMaxGemmGroup + 1];  // first split tile (the fix-up kernel's order)
+  int class_begin[kMaxGemmGroup + 1];  // first whole-tile block of a class: neighbouring problems with the same K
+  int n;
+  int symmetric;
+  int group_m;      // tile rows per block of the general products' tile order
+  int round_tiles;  // resident workgroups, a multiple of 8
+  int update_dtype;
+  float alpha, beta;
+  float* partials;  // fp32 BM x BN tiles, problem p's from partial_base on: [its split tiles][splits]
+  GemmProblem problem[kMaxGemmGroup];
 };
+static_assert(sizeof(LaunchArgs) <= 4096, "kernel arguments are limited to 4 KiB");
+
+// The problem whose range of `begin` holds `block` (one scalar load of the whole table, then compares: a search by
+// dependent loads would wait out the memory latency at every step).
+__device__ __forceinline__ int problem_of(const int (&begin)[kMaxGemmGroup + 1], int n, int block) {
+  if (n == 1) return 0;  // fewer classes than problems: their entries past the last repeat the end, too
+  int p = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxGemmGroup; ++i) p += block >= begin[i] ? 1 : 0;
+  return p < n ? p : n - 1;
+}
 
 // logical tile index -> (tm, tn)
 __device__ __forceinline__ void tile_coords(int group_m, int logical, int tiles_m, int tiles_n, bool symmetric, int* tm, int* tn) {
@@ -109,20 +142,27 @@ __device__ __forceinline__ void tile_coords(int group_m, int logical, int tiles_
     *tn = logical - i * (i + 1) / 2;
     return;
   }
-  // group_m tile rows at a time, walking down the rows before moving to the next tile column
-  const int per_group = group_m * tiles_n;
-  const int group = logical / per_group;
-  const int first_m = group * group_m;
-  const int rows = min(group_m, tiles_m - first_m);
-  const int in_group = logical - group * per_group;
-  *tm = first_m + in_group % rows;
-  *tn = in_group / rows;
+  // Columns of kSuper tiles, walked down all rows in blocks of group_m x kSuper / 2 tiles: what the whole machine works on
+  // at a time is then nearly square (16 x 16 tiles where a round has 256), and so is what one XCD works on.
+  constexpr int kSuper = 16;
+  const int per_super = kSuper * tiles_m;
+  const int super = logical / per_super;
+  const int first_n = super * kSuper, cols = min(kSuper, tiles_n - first_n);
+  int in = logical - super * per_super;
+  const int band = in / (group_m * cols);  // group_m rows of this super column
+  const int first_m = band * group_m, rows = min(group_m, tiles_m - first_m);
+  in -= band * group_m * cols;
+  const int half = (cols + 1) / 2;
+  const int second = in >= rows * half ? 1 : 0;
+  in -= second * rows * half;
+  *tm = first_m + in % rows;
+  *tn = first_n + second * half + in / rows;
 }
 
 // OCC workgroups are meant to share a CU: the register budget per wave is set for OCC * WM * WN / 4 waves per SIMD.
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, int OCC>
 __global__ void __launch_bounds__(WM * WN * 64, (OCC * WM * WN + 3) / 4)
-gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
+gemm_nt_kernel(LaunchArgs args) {
   constexpr int kThreads = WM * WN * 64;
   constexpr int kWaves = WM * WN;
   constexpr int kWaveM = BM / WM;     // rows of C per wave
@@ -143,28 +183,41 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   __bf16* smem = reinterpret_cast<__bf16*>(smem_raw);
 
-  // ---- which tile, which K range
+  // ---- which problem, which tile, which K range
   const int block = blockIdx.x;
-  const bool whole = block < sched.full_tiles;
+  const bool whole = block < args.tile_begin[kMaxGemmGroup];
+  int index = block;
+  if (whole) {
+    // Workgroup ids congruent mod 8 run on one XCD: in every round of resident workgroups an XCD gets one contiguous eighth
+    // of the round's tiles (the first tiles % 8 XCDs one tile more), so that the workgroups sharing an L2 work on
+    // neighbouring tiles -- of one matrix, or on a few whole matrices where a class holds many small ones -- while the
+    // machine as a whole walks through one matrix after the other.  Classes one by one: every XCD gets its share of the
+    // long and of the short tiles.
+    const int c = problem_of(args.class_begin, args.n, block);
+    const int round = (block - args.class_begin[c]) / args.round_tiles;
+    const int first = args.class_begin[c] + round * args.round_tiles, tiles = min(args.round_tiles, args.class_begin[c + 1] - first);
+    const int i = block - first, xcd = i % kXcds, each = tiles / kXcds, extra = tiles % kXcds;
+    index = first + xcd * each + (xcd < extra ? xcd : extra) + i / kXcds;
+  }
+  const int problem = whole ? problem_of(args.tile_begin, args.n, index) : problem_of(args.piece_begin, args.n, index);
+  const GemmProblem& a = args.problem[problem];
+  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
   int logical, split = 0, piece_tile = 0;
   if (whole) {
-    // workgroup ids congruent mod 8 run on one XCD: hand each XCD one contiguous eighth of the tile order (the first
-    // full_tiles % 8 of them one tile more), so that the workgroups sharing an L2 work on neighbouring tiles
-    const int xcd = block % kXcds, each = sched.full_tiles / kXcds, extra = sched.full_tiles % kXcds;
-    logical = xcd * each + (xcd < extra ? xcd : extra) + block / kXcds;
+    logical = index - args.tile_begin[problem];
   } else {
-    const int piece = block - sched.full_tiles;
-    piece_tile = piece / sched.splits;
-    split = piece - piece_tile * sched.splits;
-    logical = sched.full_tiles + piece_tile;
+    const int piece = index - args.piece_begin[problem];
+    piece_tile = piece / a.splits;
+    split = piece - piece_tile * a.splits;
+    logical = args.tile_begin[problem + 1] - args.tile_begin[problem] + piece_tile;
   }
   int tm, tn;
-  tile_coords(sched.group_m, logical, sched.tiles_m, sched.tiles_n, a.symmetric != 0, &tm, &tn);
+  tile_coords(args.group_m, logical, tiles_m, tiles_n, args.symmetric != 0, &tm, &tn);
   const int row0 = tm * BM;
   const int col0 = tn * BN;
   const int k_slabs_total = a.K / BK;
-  const int ks_begin = whole ? 0 : static_cast<int>(static_cast<int64_t>(k_slabs_total) * split / sched.splits);
-  const int ks_end = whole ? k_slabs_total : static_cast<int>(static_cast<int64_t>(k_slabs_total) * (split + 1) / sched.splits);
+  const int ks_begin = whole ? 0 : static_cast<int>(static_cast<int64_t>(k_slabs_total) * split / a.splits);
+  const int ks_end = whole ? k_slabs_total : static_cast<int>(static_cast<int64_t>(k_slabs_total) * (split + 1) / a.splits);
 
   // Every tile walks its K range from its first slab on: the tiles of an XCD that share a panel then share its slabs in
   // L2 (walks that start at different slabs were measured 3 to 37 % slower).
@@ -224,13 +277,6 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
   // Accumulator register r of lane l holds C[4*(l/16) + r][l%16] of its 16x16 tile.
   const int lcol = wave_n * kWaveN + (lane & 15);
   const int lrow = wave_m * kWaveM + (lane >> 4) * 4;
-  // A whole tile whose D operand is also at hand transposed starts from it instead of adding it at the end:
-  // acc = (beta / alpha) D, so that alpha * acc is alpha P Q^T + beta D with one rounding, as before.  The four
-  // registers of an MFMA tile are four consecutive rows of one column, i.e. four consecutive elements (8 bytes) of a
-  // row of D^T, which come straight from global memory in the accumulator's layout and go out with the first slabs.
-  // (A D tile fetched behind the main loop has to be staged through LDS, since its rows do not match the accumulator
-  // layout, and picked up with 2-byte LDS reads: 5 of the 121 microseconds of a 256x256 tile with K = 4096.  The
-  // fetch itself stays what it is wherever it sits: every CU wants its 128 KiB at the same moment.)
   // A whole tile takes its D operand on the way: D^T is the Q operand itself in both products that have one (X^T in
   // the update product, the symmetric A in A A), and K spans the rows of C there, so the Q slabs with k in
   // [row0, row0 + BM) hold D[k - row0][0 .. BN) of this tile as they pass through LDS.  The waves pick their values
@@ -239,7 +285,7 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
   // cost a 256 x 256 tile with K = 4096 11 of its 121 microseconds: every CU wants its 128 KiB from HBM at the same
   // moment, and the tile has to be staged through LDS because its rows do not match the accumulator layout.)
   const bool d_in_slabs = whole && a.D != nullptr;
-  const float d_scale = d_in_slabs ? a.beta / a.alpha : 0.0f;
+  const float d_scale = d_in_slabs ? args.beta / args.alpha : 0.0f;
   f32x4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -349,14 +395,16 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
   };
   // D values out of a Q slab (see d_in_slabs above).  Slab q of the BM / BK slabs that hold the tile's D rows carries
   // the rows of kTilesPerSlab MFMA tile rows of the waves with wave_m == q / kSlabsPerWave; a lane's four rows of one
-  // column are four consecutive k of one slab row: one 64-bit LDS read per MFMA tile, in three batches at the starts
-  // of the slab's first three half steps (the values wait in registers for half a step, and all reads are back before
-  // the barrier that releases the stage).
+  // column are four consecutive k of one slab row: one 64-bit LDS read per MFMA tile, in two batches that are read at the
+  // start of a half step and added at its end, so that every tile row gets its D between its two MFMAs of the slab.
+  // Every tile variant therefore adds in the same order: the bits of a result do not depend on the tile it was computed
+  // in (only on whether its K walk was cut into pieces).
   constexpr int kTilesPerSlab = BK / 16;
   constexpr int kSlabsPerWave = kWaveM / BK;
   constexpr int kDSlabs = BM / BK;
-  constexpr int kDPairs = kTilesPerSlab * TN, kDBatches = 3, kDBatch = (kDPairs + kDBatches - 1) / kDBatches;
-  static_assert(kWaveM % BK == 0 && TM == kSlabsPerWave * kTilesPerSlab && kSteps == 2, "D slabs must divide over the waves and the half steps");
+  constexpr int kDPairs = kTilesPerSlab * TN, kDBatch = kDPairs / 2;
+  static_assert(kWaveM % BK == 0 && TM == kSlabsPerWave * kTilesPerSlab && kSteps == 2 && TMH % (kTilesPerSlab / 2) == 0,
+                "D slabs must divide over the waves and the half steps");
   const int d_base = BM * BK + lcol * BK + 4 * ((lane >> 4) & 1);  // slab row lcol (+ 16 j), first or second half of a chunk
   const int d_swizzle = (lcol / kRowsPerSweep) % kChunks;          // the same for lcol + 16 j
   u32x2 d_vals[kDBatch];
@@ -364,7 +412,6 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
 #pragma unroll
     for (int n = 0; n < kDBatch; ++n) {
       const int pair = batch * kDBatch + n, ii = pair / TN, j = pair % TN;
-      if (pair >= kDPairs) break;
       const int chunk = (2 * ii + (lane >> 5)) ^ d_swizzle;
       d_vals[n] = *reinterpret_cast<const u32x2*>(smem + stage * kStageElems + d_base + j * 16 * BK + (chunk << 3));
     }
@@ -374,7 +421,6 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
 #pragma unroll
     for (int n = 0; n < kDBatch; ++n) {
       const int pair = batch * kDBatch + n, i = kFirstTile + pair / TN, j = pair % TN;
-      if (pair >= kDPairs) break;
       acc[i][j][0] += scale * __uint_as_float(d_vals[n].x << 16);
       acc[i][j][1] += scale * __uint_as_float(d_vals[n].x & 0xffff0000u);
       acc[i][j][2] += scale * __uint_as_float(d_vals[n].y << 16);
@@ -387,57 +433,54 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
     constexpr int kD = decltype(d_tag)::value;
     constexpr int kOwner = kD < 0 ? 0 : kD / kSlabsPerWave;
     using Part = std::integral_constant<int, kD < 0 ? 0 : kD % kSlabsPerWave>;
+    // the half step the first D batch rides on: the slab's tile rows (its first two, in a tile whose slab rows span both
+    // halves) meet their first MFMA there
+    constexpr int kDHalf = kD < 0 ? -4 : (Part::value * kTilesPerSlab >= TMH ? 1 : 0);
     const float scale = (kD >= 0 && wave_m == kOwner) ? d_scale : 0.0f;  // the other waves add zero times a finite value
+    auto d_before = [&](auto half_tag) {
+      constexpr int kBatch = decltype(half_tag)::value - kDHalf;
+      if constexpr (kBatch == 0 || kBatch == 1) {
+        d_read(stage, kBatch);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    auto d_after = [&](auto half_tag) {
+      constexpr int kBatch = decltype(half_tag)::value - kDHalf;
+      if constexpr (kBatch == 0 || kBatch == 1) d_add(Part{}, kBatch, scale);
+    };
     const int next_stage = stage + 1 == STAGES ? 0 : stage + 1;
     const int prev_stage = stage == 0 ? STAGES - 1 : stage - 1;
-#pragma unroll
-    for (int kk = 0; kk < kSteps; kk += 2) {
-      __builtin_amdgcn_s_waitcnt(kWaitLds);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (kD >= 0) {
-        d_read(stage, 0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (kk == 0) {
-        // second half of the refill of the stage the previous slab's barrier released (its P rows went out there)
-        const int k0 = k0_clamped(it - 1 + STAGES);
-        first_half(fb0, stage, kk, std::integral_constant<int, kLoadsQ>{}, [&](int l) { load_q(k0, prev_stage, l); });
-      } else {
-        first_half(fb0, stage, kk, Zero{}, [](int) {});
-      }
-      __builtin_amdgcn_s_waitcnt(kWaitLds);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (kD >= 0) {
-        d_add(Part{}, 0, scale);
-        d_read(stage, 1);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      second_half(fb0, fb1, stage, kk + 1, Zero{}, [](int) {});
-      __builtin_amdgcn_s_waitcnt(kWaitLds);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (kD >= 0) {
-        d_add(Part{}, 1, scale);
-        d_read(stage, 2);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      first_half(fb1, stage, kk + 1, Zero{}, [](int) {});
-      if (kk + 2 < kSteps) {
-        __builtin_amdgcn_s_waitcnt(kWaitLds);
-        __builtin_amdgcn_sched_barrier(0);
-        second_half(fb1, fb0, stage, kk + 2, Zero{}, [](int) {});
-      } else {
-        // last half step of the slab: the slab after it must have landed (the STAGES - 2 younger ones may be in
-        // flight); behind the barrier this slab's stage is free and its refill starts with the P rows
-        __builtin_amdgcn_s_waitcnt(kWaitNextSlab);
-        __syncthreads();
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (kD >= 0) {
-          d_add(Part{}, 2, scale);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        const int k0 = k0_clamped(it + STAGES);
-        second_half(fb1, fb0, next_stage, 0, std::integral_constant<int, kLoadsP>{}, [&](int l) { load_p(k0, stage, l); });
-      }
+    using H0 = std::integral_constant<int, 0>;
+    using H1 = std::integral_constant<int, 1>;
+    using H2 = std::integral_constant<int, 2>;
+    __builtin_amdgcn_s_waitcnt(kWaitLds);
+    __builtin_amdgcn_sched_barrier(0);
+    d_before(H0{});
+    {
+      // second half of the refill of the stage the previous slab's barrier released (its P rows went out there)
+      const int k0 = k0_clamped(it - 1 + STAGES);
+      first_half(fb0, stage, 0, std::integral_constant<int, kLoadsQ>{}, [&](int l) { load_q(k0, prev_stage, l); });
+    }
+    __builtin_amdgcn_s_waitcnt(kWaitLds);
+    __builtin_amdgcn_sched_barrier(0);
+    d_after(H0{});
+    d_before(H1{});
+    second_half(fb0, fb1, stage, 1, Zero{}, [](int) {});
+    __builtin_amdgcn_s_waitcnt(kWaitLds);
+    __builtin_amdgcn_sched_barrier(0);
+    d_after(H1{});
+    d_before(H2{});
+    first_half(fb1, stage, 1, Zero{}, [](int) {});
+    // last half step of the slab: the slab after it must have landed (the STAGES - 2 younger ones may be in
+    // flight); behind the barrier this slab's stage is free and its refill starts with the P rows
+    __builtin_amdgcn_s_waitcnt(kWaitNextSlab);
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    d_after(H2{});
+    if constexpr (kD >= 0) __builtin_amdgcn_sched_barrier(0);
+    {
+      const int k0 = k0_clamped(it + STAGES);
+      second_half(fb1, fb0, next_stage, 0, std::integral_constant<int, kLoadsP>{}, [&](int l) { load_p(k0, stage, l); });
     }
     stage = next_stage;
   };
@@ -448,7 +491,7 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
     for (int it = 0; it < first_d; ++it) slab(it, NoD{});
     auto d_slabs = [&](auto&& self, auto q_tag) -> void {
       constexpr int kQ = decltype(q_tag)::value;
-      slab(first_d + kQ, q_tag);
+      if (first_d + kQ < n_slabs) slab(first_d + kQ, q_tag);  // tile rows at or beyond K have no D (and no result)
       if constexpr (kQ + 1 < kDSlabs) self(self, std::integral_constant<int, kQ + 1>{});
     };
     d_slabs(d_slabs, Zero{});
@@ -461,7 +504,7 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
   // ---- K pieces: park the fp32 partial tile (row-major BM x BN); the fix-up kernel sums the pieces and
   // runs the epilogue.
   if (!whole) {
-    float* mine = sched.partials + (static_cast<int64_t>(piece_tile) * sched.splits + split) * (BM * BN);
+    float* mine = args.partials + (static_cast<int64_t>(a.partial_base) + piece_tile * a.splits + split) * (BM * BN);
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -480,7 +523,7 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
   uint16_t* __restrict__ C = static_cast<uint16_t*>(a.C);
   uint16_t* __restrict__ CT = static_cast<uint16_t*>(a.CT);
   int ldct = a.ldct;
-  if (a.symmetric) {  // mirror the off-diagonal tile
+  if (args.symmetric) {  // mirror the off-diagonal tile
     CT = tm != tn ? C : nullptr;
     ldct = a.ldc;
   }
@@ -494,10 +537,10 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[i][j][r] = a.alpha * acc[i][j][r];
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = args.alpha * acc[i][j][r];
   if (a.update_param != nullptr) {
     // the last product of a Muon step: the tile goes into the parameter (in the parameter's orientation) and nowhere else
-    if (!a.update_transposed) {
+    if (!(a.flags & kGemmUpdateTransposed)) {
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -508,7 +551,7 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
       __syncthreads();
       for (int c = tid; c < BM * kRowChunks; c += kThreads) {
         const int r = c / kRowChunks, cc = c - r * kRowChunks;
-        update_param8(a, row0 + r, col0 + cc * 8, *reinterpret_cast<const u32x4*>(stage_c + r * kLdS + cc * 8));
+        update_param8(a, args.update_dtype, row0 + r, col0 + cc * 8, *reinterpret_cast<const u32x4*>(stage_c + r * kLdS + cc * 8));
       }
     } else {
 #pragma unroll
@@ -521,12 +564,12 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
       __syncthreads();
       for (int c = tid; c < BN * kColChunks; c += kThreads) {
         const int r = c / kColChunks, cc = c - r * kColChunks;
-        update_param8(a, col0 + r, row0 + cc * 8, *reinterpret_cast<const u32x4*>(stage_c + r * kLdT + cc * 8));
+        update_param8(a, args.update_dtype, col0 + r, row0 + cc * 8, *reinterpret_cast<const u32x4*>(stage_c + r * kLdT + cc * 8));
       }
     }
     return;
   }
-  if (!a.skip_c) {
+  if (!(a.flags & kGemmSkipC)) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -567,53 +610,57 @@ gemm_nt_kernel(GemmNtArgs a, Schedule sched) {
 constexpr int kFixupThreads = 1024;
 template <int BM, int BN>
 __global__ void __launch_bounds__(kFixupThreads)
-splitk_fixup_kernel(GemmNtArgs a, Schedule sched) {
+splitk_fixup_kernel(LaunchArgs args) {
   constexpr int kSub = 64;
   constexpr int kSubsPerTile = (BM / kSub) * (BN / kSub);
   __shared__ __attribute__((aligned(16))) uint16_t transposed[kSub][kSub + 8];
-  const int tile = blockIdx.x / kSubsPerTile;
+  const int split_tile = blockIdx.x / kSubsPerTile;
   const int sub = blockIdx.x % kSubsPerTile;
+  const int problem = problem_of(args.split_begin, args.n, split_tile);
+  const GemmProblem& a = args.problem[problem];
+  const int tile = split_tile - args.split_begin[problem];
+  const int full_tiles = args.tile_begin[problem + 1] - args.tile_begin[problem];
   const int sub_row0 = (sub / (BN / kSub)) * kSub, sub_col0 = (sub % (BN / kSub)) * kSub;
   int tm, tn;
-  tile_coords(sched.group_m, sched.full_tiles + tile, sched.tiles_m, sched.tiles_n, a.symmetric != 0, &tm, &tn);
+  tile_coords(args.group_m, full_tiles + tile, (a.M + BM - 1) / BM, (a.N + BN - 1) / BN, args.symmetric != 0, &tm, &tn);
   const uint16_t* __restrict__ D = static_cast<const uint16_t*>(a.D);
   uint16_t* __restrict__ C = static_cast<uint16_t*>(a.C);
   uint16_t* __restrict__ CT = static_cast<uint16_t*>(a.CT);
   int ldct = a.ldct;
-  if (a.symmetric) {  // mirror the off-diagonal tile
+  if (args.symmetric) {  // mirror the off-diagonal tile
     CT = tm != tn ? C : nullptr;
     ldct = a.ldc;
   }
   const int t = threadIdx.x;
   const int r = t / 16, c = (t % 16) * 4;  // position inside the 64 x 64 block
   const int lrow = sub_row0 + r, lcol = sub_col0 + c;
-  const float* base = sched.partials + static_cast<int64_t>(tile) * sched.splits * (BM * BN) + lrow * BN + lcol;
+  const float* base = args.partials + (static_cast<int64_t>(a.partial_base) + static_cast<int64_t>(tile) * a.splits) * (BM * BN) + lrow * BN + lcol;
   // four loads in flight at a time; the sum itself stays in split order
   f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
   int s = 0;
-  for (; s + 4 <= sched.splits; s += 4) {
+  for (; s + 4 <= a.splits; s += 4) {
     f32x4 piece[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) piece[u] = *reinterpret_cast<const f32x4*>(base + static_cast<int64_t>(s + u) * (BM * BN));
 #pragma unroll
     for (int u = 0; u < 4; ++u) sum += piece[u];
   }
-  for (; s < sched.splits; ++s) sum += *reinterpret_cast<const f32x4*>(base + static_cast<int64_t>(s) * (BM * BN));
+  for (; s < a.splits; ++s) sum += *reinterpret_cast<const f32x4*>(base + static_cast<int64_t>(s) * (BM * BN));
   const int row = tm * BM + lrow, col = tn * BN + lcol;
-  float v[4] = {a.alpha * sum.x, a.alpha * sum.y, a.alpha * sum.z, a.alpha * sum.w};
+  float v[4] = {args.alpha * sum.x, args.alpha * sum.y, args.alpha * sum.z, args.alpha * sum.w};
   if (D != nullptr) {
     const u32x2 d = *reinterpret_cast<const u32x2*>(D + static_cast<int64_t>(row) * a.ldd + col);
-    v[0] += a.beta * bf16_bits_to_float(static_cast<uint16_t>(d.x));
-    v[1] += a.beta * bf16_bits_to_float(static_cast<uint16_t>(d.x >> 16));
-    v[2] += a.beta * bf16_bits_to_float(static_cast<uint16_t>(d.y));
-    v[3] += a.beta * bf16_bits_to_float(static_cast<uint16_t>(d.y >> 16));
+    v[0] += args.beta * bf16_bits_to_float(static_cast<uint16_t>(d.x));
+    v[1] += args.beta * bf16_bits_to_float(static_cast<uint16_t>(d.x >> 16));
+    v[2] += args.beta * bf16_bits_to_float(static_cast<uint16_t>(d.y));
+    v[3] += args.beta * bf16_bits_to_float(static_cast<uint16_t>(d.y >> 16));
   }
   const uint32_t lo = pack_bf16x2(v[0], v[1]);
   const uint32_t hi = pack_bf16x2(v[2], v[3]);
   if (a.update_param != nullptr) {  // uniform over the grid: the parameter update in place of the stores (see gemm_nt_kernel)
-    if (!a.update_transposed) {
+    if (!(a.flags & kGemmUpdateTransposed)) {
       const u32x4 packed = {lo, hi, 0u, 0u};  // this thread's four columns
-      update_param8(a, row, col, packed, 4);
+      update_param8(a, args.update_dtype, row, col, packed, 4);
       return;
     }
     transposed[c][r] = static_cast<uint16_t>(lo);
@@ -623,11 +670,11 @@ splitk_fixup_kernel(GemmNtArgs a, Schedule sched) {
     __syncthreads();
     if (t < kSub * 8) {
       const int tr = t / 8, chunk = t % 8;
-      update_param8(a, tn * BN + sub_col0 + tr, tm * BM + sub_row0 + chunk * 8, *reinterpret_cast<const u32x4*>(&transposed[tr][chunk * 8]));
+      update_param8(a, args.update_dtype, tn * BN + sub_col0 + tr, tm * BM + sub_row0 + chunk * 8, *reinterpret_cast<const u32x4*>(&transposed[tr][chunk * 8]));
     }
     return;
   }
-  if (!a.skip_c) {
+  if (!(a.flags & kGemmSkipC)) {
     const u32x2 packed = {lo, hi};
     *reinterpret_cast<u32x2*>(C + static_cast<int64_t>(row) * a.ldc + col) = packed;
   }
@@ -653,36 +700,142 @@ GemmTuning tuning_snapshot() {
 }
 
 // Tiles a product computes: every tile of a general product, the tiles on or below the diagonal of a symmetric one.
-int tile_count(const GemmNtArgs& a, int bm, int bn) {
-  const int tm = a.M / bm, tn = a.N / bn;
-  return a.symmetric ? tm * (tm + 1) / 2 : tm * tn;
+int tile_count(const GemmGroup& g, const GemmProblem& p, int tile) {
+  const int tm = (p.M + tile - 1) / tile, tn = (p.N + tile - 1) / tile;
+  return g.symmetric ? tm * (tm + 1) / 2 : tm * tn;
+}
+
+// Below this many slabs a tile is never cut: the pieces would be gone before the fix-up launch (4-5 us) has paid off, and
+// matrices this small keep the bits of their update whatever else the launch holds.
+constexpr int kMinSplitSlabs = 17;
+
+// What a tile variant costs, in microseconds: one slab of a tile when every CU holds as many workgroups as it can
+// (slab_us) and when it holds one (lone_slab_us), prologue and epilogue of a tile (tile_us).  From kernel traces: 256 x 256
+// tiles with K = 4096 take 102 us a round, two 128 x 128 tiles per CU 0.95 us a slab.  The choice they make is the faster
+// one on every group measured (whole Muon step, symmetric / general products forced to 256 or 128): hidden4096 7.28 ms
+// against 7.85 / 8.09 with small tiles, two hidden5120 matrices 11.0 against 12.1 / 12.8, five small ragged ones 0.344
+// against 0.427 / 0.406 with big ones, 24 of 1536 x 1024 1.23 against 1.27 / 1.29 with small ones.
+struct Variant {
+  int tile, per_cu;
+  double slab_us, lone_slab_us, tile_us;
+};
+constexpr Variant kVariants[3] = {{}, {256, 1, 1.45, 1.45, 9.0}, {128, 2, 0.95, 0.60, 5.0}};
+
+// When the workgroups of a launch end, if each starts on the slot that is free first (as they do, in block order).
+// Slots are kept as groups that are free at the same time; a launch of equal tiles costs a few steps per round.
+class SlotTimes {
+ public:
+  explicit SlotTimes(int slots) : groups_{{0.0, slots}} {}
+  void add(int workgroups, double us) {
+    while (workgroups > 0) {
+      Slots& first = groups_.front();
+      const int n = std::min(workgroups, first.count);
+      const Slots busy{first.time + us, n};
+      first.count -= n;
+      if (first.count == 0) groups_.erase(groups_.begin());
+      auto at = std::lower_bound(groups_.begin(), groups_.end(), busy, [](const Slots& x, const Slots& y) { return x.time < y.time; });
+      if (at != groups_.end() && at->time == busy.time) at->count += n;
+      else groups_.insert(at, busy);
+      workgroups -= n;
+    }
+  }
+  double end() const { return groups_.back().time; }
+
+ private:
+  struct Slots { double time; int count; };
+  std::vector<Slots> groups_;
+};
+
+GemmPlan make_plan(const GemmGroup& g, int variant, const GemmScratch& scratch, const GemmTuning& tuning) {
+  const Variant& v = kVariants[variant];
+  const int cus = device_cu_count(), slots = cus * v.per_cu;
+  GemmPlan plan;
+  plan.variant = variant;
+  for (int i = 0; i < g.n; ++i) plan.order[i] = i;
+  std::stable_sort(plan.order, plan.order + g.n, [&](int a, int b) { return g.problem[a].K > g.problem[b].K; });
+  int tiles[kMaxGemmGroup], slabs[kMaxGemmGroup], total = 0;
+  for (int i = 0; i < g.n; ++i) {
+    tiles[i] = tile_count(g, g.problem[plan.order[i]], v.tile);
+    slabs[i] = g.problem[plan.order[i]].K / kSlabK;
+    total += tiles[i];
+    plan.split_tiles[i] = 0;
+    plan.splits[i] = 1;
+  }
+  // The last total % slots tiles (those with the shortest K) are the ones that may be cut: the others fill whole rounds.
+  int rest[kMaxGemmGroup];
+  for (int i = g.n - 1, left = total % slots; i >= 0; --i) {
+    rest[i] = std::min(left, tiles[i]);
+    left -= rest[i];
+  }
+  const double tile_bytes = static_cast<double>(v.tile) * v.tile * 4;
+  // tries pieces of about `piece` slabs (0: nothing is cut) and keeps the plan if it is the fastest so far
+  auto consider = [&](int piece) {
+    int splits[kMaxGemmGroup], blocks = 0;
+    int64_t partial = 0;
+    for (int i = 0; i < g.n; ++i) {
+      splits[i] = 1;
+      if (piece > 0 && rest[i] > 0 && slabs[i] >= kMinSplitSlabs && 4 * slabs[i] > 5 * piece) splits[i] = std::min((slabs[i] + piece - 1) / piece, tuning.max_splits);
+      if (splits[i] > 1) partial += static_cast<int64_t>(rest[i]) * splits[i];
+      blocks += tiles[i] + rest[i] * (splits[i] - 1);
+    }
+    if (piece > 0 && (partial == 0 || partial > 0x7fffffff || partial * tile_bytes > static_cast<double>(scratch.partials_bytes))) return;
+    const double slab_us = blocks <= cus ? v.lone_slab_us : v.slab_us;
+    SlotTimes times(slots);
+    for (int i = 0; i < g.n; ++i) times.add(tiles[i] - (splits[i] > 1 ? rest[i] : 0), slabs[i] * slab_us + v.tile_us);
+    for (int i = 0; i < g.n; ++i)
+      if (splits[i] > 1) times.add(rest[i] * splits[i], (slabs[i] + splits[i] - 1) / splits[i] * slab_us + v.tile_us);
+    // the fix-up launch: 4 us, and the partial tiles written and read again at about 5 TB/s
+    const double us = times.end() + (partial > 0 ? 4.0 + partial * tile_bytes * 2.0 / 5.0e6 : 0.0);
+    if (piece > 0 && us >= plan.us) return;
+    plan.us = us;
+    for (int i = 0; i < g.n; ++i) {
+      plan.splits[i] = splits[i];
+      plan.split_tiles[i] = splits[i] > 1 ? rest[i] : 0;
+    }
+  };
+  consider(0);
+  if (!tuning.split_remainder || scratch.partials == nullptr) return plan;
+  // piece lengths worth a look: every fraction of the longest K that may be cut, and the other K themselves
+  int longest = 0, tried = 0;
+  for (int i = 0; i < g.n; ++i)
+    if (rest[i] > 0 && slabs[i] >= kMinSplitSlabs) longest = std::max(longest, slabs[i]);
+  for (int c = 2; longest > 0 && c <= tuning.max_splits; ++c) consider((longest + c - 1) / c);
+  for (int i = 1; i < g.n && tried < 4; ++i)
+    if (rest[i] > 0 && slabs[i] != slabs[i - 1] && slabs[i] < longest) {
+      consider(slabs[i]);
+      ++tried;
+    }
+  return plan;
 }
 
 template <int BM, int BN, int WM, int WN, int BK, int STAGES, int OCC>
-int launch(const GemmNtArgs& a, const GemmScratch& scratch, const GemmTuning& tuning, hipStream_t stream) {
-  constexpr int blocks_per_cu = OCC;
-  Schedule s{};
-  s.tiles_m = a.M / BM;
-  s.tiles_n = a.N / BN;
-  const int tiles = tile_count(a, BM, BN);
-  const int slots = device_cu_count() * blocks_per_cu;
-  const int k_slabs = a.K / BK;
-  s.full_tiles = tiles;
-  s.splits = 1;
-  s.partials = static_cast<float*>(scratch.partials);
-  s.group_m = std::max(1, tuning.group_m);
-  const int rem = tiles % slots;
-  if (tuning.split_remainder && rem != 0 && scratch.partials != nullptr) {
-    // fill the machine once more with pieces of the leftover tiles; cap the pieces per tile so that the summing stays short
-    int splits = std::min({slots / rem, k_slabs, tuning.max_splits});
-    const int64_t tile_bytes = static_cast<int64_t>(BM) * BN * 4;
-    while (splits > 1 && static_cast<int64_t>(rem) * splits * tile_bytes > scratch.partials_bytes) --splits;
-    if (splits > 1) {
-      s.full_tiles = tiles - rem;
-      s.splits = splits;
-    }
+int launch(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& scratch, const GemmTuning& tuning, hipStream_t stream) {
+  LaunchArgs args;
+  args.n = g.n;
+  args.symmetric = g.symmetric;
+  args.group_m = std::max(1, tuning.group_m);
+  args.round_tiles = std::max(kXcds, device_cu_count() * OCC / kXcds * kXcds);
+  args.update_dtype = g.update_dtype;
+  args.alpha = g.alpha;
+  args.beta = g.beta;
+  args.partials = static_cast<float*>(scratch.partials);
+  int tile = 0, piece = 0, split = 0, partial = 0, classes = 0;
+  for (int i = 0; i <= kMaxGemmGroup; ++i) {
+    args.tile_begin[i] = tile;
+    args.split_begin[i] = split;
+    args.piece_begin[i] = piece;
+    if (i >= g.n) continue;
+    GemmProblem& p = args.problem[i] = g.problem[plan.order[i]];
+    if (i == 0 || p.K != args.problem[i - 1].K) args.class_begin[classes++] = tile;
+    p.splits = plan.splits[i];
+    p.partial_base = partial;
+    tile += tile_count(g, p, BM) - plan.split_tiles[i];
+    split += plan.split_tiles[i];
+    piece += plan.split_tiles[i] * plan.splits[i];
+    partial += plan.split_tiles[i] * plan.splits[i];
   }
-  const int blocks = s.full_tiles + (tiles - s.full_tiles) * s.splits;
+  for (int i = 0; i <= kMaxGemmGroup; ++i) args.piece_begin[i] += tile;  // block ids: behind the whole tiles
+  for (int i = classes; i <= kMaxGemmGroup; ++i) args.class_begin[i] = tile;
   constexpr size_t smem_loop = static_cast<size_t>(STAGES) * (BM + BN) * BK * sizeof(uint16_t);
   constexpr size_t smem_c = static_cast<size_t>(BM) * (BN + 8) * sizeof(uint16_t), smem_ct = static_cast<size_t>(BN) * (BM + 8) * sizeof(uint16_t);
   constexpr size_t smem_epilogue = smem_c > smem_ct ? smem_c : smem_ct;
@@ -701,46 +854,13 @@ int launch(const GemmNtArgs& a, const GemmScratch& scratch, const GemmTuning& tu
       if (dev >= 0 && dev < 64) configured[dev] = true;
     }
   }
-  hipLaunchKernelGGL(kernel, dim3(blocks), dim3(WM * WN * 64), smem, stream, a, s);
+  hipLaunchKernelGGL(kernel, dim3(tile + piece), dim3(WM * WN * 64), smem, stream, args);
   MFSDP_CHECK_LAUNCH("gemm_nt_kernel");
-  if (s.splits > 1) {
-    const int fix_blocks = (tiles - s.full_tiles) * (BM / 64) * (BN / 64);
-    hipLaunchKernelGGL((splitk_fixup_kernel<BM, BN>), dim3(fix_blocks), dim3(kFixupThreads), 0, stream, a, s);
+  if (split > 0) {
+    hipLaunchKernelGGL((splitk_fixup_kernel<BM, BN>), dim3(split * (BM / 64) * (BN / 64)), dim3(kFixupThreads), 0, stream, args);
     MFSDP_CHECK_LAUNCH("splitk_fixup_kernel");
   }
   return MFSDP_OK;
-}
-
-// Which tiling a product runs with: 1 = 256 x 256, 2 = 128 x 128.
-int choose_variant(const GemmNtArgs& a, const GemmTuning& tuning) {
-  int variant = a.symmetric ? tuning.symmetric_variant : tuning.general_variant;
-  if (a.symmetric && variant == 3) {
-    // The triangle of a symmetric product rarely tiles the machine evenly.  Compare the two tilings in rounds of
-    // resident workgroups, the last partial round counting 1/splits (plus the partial-tile traffic, which grows with
-    // the splits) when its tiles are split along K: a round of 128x128 tiles (two per CU) takes about 0.6 of a round
-    // of 256x256 tiles.  m = 4096 on 256 CUs: 136 big tiles are one half-empty round (1.0) against 528 small ones in
-    // 1 + 1/16 rounds (0.83); m = 5120: 210 big tiles in one round (1.0) against 820 small ones in two (1.2) --
-    // measured 15 % faster with the big tiles.  Below three quarters of a round of big tiles (m <= 4096 on 256 CUs)
-    // only K-splitting would fill the machine and the small tiles win (m = 3072: 0.89 ms against 1.15 ms for the five
-    // iterations; m = 2048, k = 8192: 0.88 against 0.99).
-    auto rounds = [&](int tile, int per_cu) {
-      const int t = a.M / tile, tiles = t * (t + 1) / 2, slots = device_cu_count() * per_cu;
-      const int rem = tiles % slots;
-      double r = tiles / slots;
-      if (rem != 0) {
-        const int splits = tuning.split_remainder ? std::min({slots / rem, a.K / kSlabK, tuning.max_splits}) : 1;
-        r += splits > 1 ? 1.0 / splits + 0.02 * splits : 1.0;
-      }
-      return r;
-    };
-    const int big = a.M / 256, big_tiles = big * (big + 1) / 2;
-    variant = (4 * big_tiles >= 3 * device_cu_count() && rounds(256, 1) <= 0.6 * rounds(128, 2)) ? 1 : 2;
-    // On a machine shared with other matrices' kernels the CUs a part-filling triangle of big tiles leaves idle are
-    // not lost, and a big tile moves fewer LDS bytes per flop: three hidden4096 matrices on three streams take 7.97 ms
-    // with big tiles against 8.73 ms with small ones (8.47 ms one after the other).
-    if (a.shared && 4 * big_tiles >= device_cu_count()) variant = 1;
-  }
-  return variant;
 }
 
 }  // namespace
@@ -751,44 +871,58 @@ void set_gemm_tuning(const GemmTuning& t) {
 }
 GemmTuning get_gemm_tuning() { return tuning_snapshot(); }
 
-int64_t gemm_nt_executed_flops(const GemmNtArgs& a) {
+GemmPlan gemm_plan(const GemmGroup& g, const GemmScratch& scratch) {
   const GemmTuning tuning = tuning_snapshot();
-  const int tile = choose_variant(a, tuning) == 2 ? 128 : 256;
-  return 2 * static_cast<int64_t>(tile) * tile * a.K * tile_count(a, tile, tile);
+  const int variant = g.symmetric ? tuning.symmetric_variant : tuning.general_variant;
+  if (variant == 1 || variant == 2) return make_plan(g, variant, scratch, tuning);
+  const GemmPlan big = make_plan(g, 1, scratch, tuning);
+  // On a machine shared with other matrices' kernels the CUs a part-filling triangle of big tiles leaves idle are
+  // not lost, and a big tile moves fewer LDS bytes per flop.
+  if (g.symmetric && g.shared && 4 * tile_count(g, g.problem[0], 256) >= device_cu_count()) return big;
+  const GemmPlan small = make_plan(g, 2, scratch, tuning);
+  return big.us <= small.us ? big : small;
 }
 
-int gemm_nt_bf16(const GemmNtArgs& a, const GemmScratch& scratch, hipStream_t stream) {
-  if (a.M <= 0 || a.N <= 0 || a.K <= 0 || a.M % 256 || a.N % 256 || a.K % kSlabK)
-    return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: M=%d N=%d must be multiples of 256 and K=%d of %d", a.M, a.N, a.K, kSlabK);
-  if (a.symmetric && a.M != a.N) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: symmetric product needs M == N");
-  if (a.skip_c && (a.symmetric || !a.CT)) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: skip_c needs a transposed output and a general product");
-  if (!a.P || !a.Q || !a.C) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: null operand");
-  if (a.ldp < a.K || a.ldq < a.K || a.ldc < a.N || (a.D && a.ldd < a.N) || (a.CT && a.ldct < a.M))
-    return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: leading dimension smaller than the row length");
-  if ((a.ldp | a.ldq) % 8 || (reinterpret_cast<uintptr_t>(a.P) | reinterpret_cast<uintptr_t>(a.Q)) % 16)
-    return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: operands must be 16-byte aligned with leading dimensions multiple of 8");
-  if ((a.ldc % 8) || reinterpret_cast<uintptr_t>(a.C) % 16 || (a.D && ((a.ldd % 8) || reinterpret_cast<uintptr_t>(a.D) % 16)) ||
-      (a.CT && ((a.ldct % 8) || reinterpret_cast<uintptr_t>(a.CT) % 16)))
-    return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: C, D and the transposed output must be 16-byte aligned with leading dimensions multiple of 8");
-  if (a.D && (!a.d_transposed_is_q || a.K < a.M || a.alpha == 0.0f))
-    return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: a D operand needs D^T == Q (K >= M) and alpha != 0");
-  if (a.ldp > (1 << 22) || a.ldq > (1 << 22)) return fail(MFSDP_ERR_UNSUPPORTED, "gemm_nt_bf16: leading dimensions beyond 2^22 elements");
-  GemmNtArgs b = a;
-  if (a.update_param != nullptr) {
-    const int elem = a.update_dtype == MFSDP_F32 ? 4 : 2;
-    if (a.symmetric || (a.update_dtype != MFSDP_F32 && a.update_dtype != MFSDP_BF16) || a.update_rows <= 0 || a.update_cols <= 0 ||
-        a.update_rows > (a.update_transposed ? a.N : a.M) || a.update_cols > (a.update_transposed ? a.M : a.N) ||
-        reinterpret_cast<uintptr_t>(a.update_param) % elem)
-      return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: parameter update needs a general product, an f32 / bf16 parameter inside the result and an aligned pointer");
-    // groups of eight elements start at multiples of eight columns: whole 16-byte accesses when the rows keep that alignment
-    b.update_vectors = a.update_cols % 8 == 0 && reinterpret_cast<uintptr_t>(a.update_param) % 16 == 0;
+int64_t gemm_nt_executed_flops(const GemmGroup& g) {
+  GemmScratch scratch;
+  scratch.partials_bytes = kGemmPartialsBytes;
+  scratch.partials = &scratch;  // only its presence counts
+  const int tile = kVariants[gemm_plan(g, scratch).variant].tile;
+  int64_t flops = 0;
+  for (int i = 0; i < g.n; ++i) flops += 2 * static_cast<int64_t>(tile) * tile * g.problem[i].K * tile_count(g, g.problem[i], tile);
+  return flops;
+}
+
+int gemm_nt_bf16(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& scratch, hipStream_t stream) {
+  if (g.n < 1 || g.n > kMaxGemmGroup) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: %d problems in one launch", g.n);
+  for (int i = 0; i < g.n; ++i) {
+    const GemmProblem& a = g.problem[i];
+    if (a.M <= 0 || a.N <= 0 || a.K <= 0 || a.K % kSlabK)
+      return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: M=%d, N=%d must be positive and K=%d a multiple of %d", a.M, a.N, a.K, kSlabK);
+    if (g.symmetric && a.M != a.N) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: symmetric product needs M == N");
+    if ((a.flags & kGemmSkipC) && (g.symmetric || !a.CT)) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: skipping C needs a transposed output and a general product");
+    if (!a.P || !a.Q || !a.C) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: null operand");
+    // tiles reach beyond M and N: rows up to the next multiple of 256 must exist (the caller's word), columns are checked
+    const int mp = (a.M + 255) / 256 * 256, np = (a.N + 255) / 256 * 256;
+    if (a.ldp < a.K || a.ldq < a.K || a.ldc < np || (a.D && a.ldd < np) || (a.CT && a.ldct < mp))
+      return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: leading dimension smaller than the padded row length");
+    if ((a.ldp | a.ldq) % 8 || (reinterpret_cast<uintptr_t>(a.P) | reinterpret_cast<uintptr_t>(a.Q)) % 16)
+      return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: operands must be 16-byte aligned with leading dimensions multiple of 8");
+    if ((a.ldc % 8) || reinterpret_cast<uintptr_t>(a.C) % 16 || (a.D && ((a.ldd % 8) || reinterpret_cast<uintptr_t>(a.D) % 16)) ||
+        (a.CT && ((a.ldct % 8) || reinterpret_cast<uintptr_t>(a.CT) % 16)))
+      return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: C, D and the transposed output must be 16-byte aligned with leading dimensions multiple of 8");
+    if (a.D && (a.K < a.M || g.alpha == 0.0f)) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: a D operand needs K >= M and alpha != 0");
+    if (a.ldp > (1 << 22) || a.ldq > (1 << 22)) return fail(MFSDP_ERR_UNSUPPORTED, "gemm_nt_bf16: leading dimensions beyond 2^22 elements");
+    if (a.update_param != nullptr && (g.symmetric || (g.update_dtype != MFSDP_F32 && g.update_dtype != MFSDP_BF16) ||
+                                      reinterpret_cast<uintptr_t>(a.update_param) % (g.update_dtype == MFSDP_F32 ? 4 : 2)))
+      return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: parameter update needs a general product and an aligned f32 / bf16 parameter");
   }
   const GemmTuning tuning = tuning_snapshot();
   // Slabs of 32 (three to five deep) were measured too: each slab row is then half a 128-byte line, the vector
   // cache looks every line up twice, and the products run 15-25 % slower than with slabs of 64 two deep.
-  if (choose_variant(b, tuning) == 2)  // 128x128 tile, 4 waves of 64x64, two workgroups per CU
-    return launch<128, 128, 2, 2, 64, 2, 2>(b, scratch, tuning, stream);
-  return launch<256, 256, 2, 4, 64, 2, 1>(b, scratch, tuning, stream);  // 256x256 tile, 8 waves of 128x64, one workgroup per CU
+  if (plan.variant == 2)  // 128x128 tile, 4 waves of 64x64, two workgroups per CU
+    return launch<128, 128, 2, 2, 64, 2, 2>(g, plan, scratch, tuning, stream);
+  return launch<256, 256, 2, 4, 64, 2, 1>(g, plan, scratch, tuning, stream);  // 256x256 tile, 8 waves of 128x64, one workgroup per CU
 }
 
 }  // namespace mfsdp

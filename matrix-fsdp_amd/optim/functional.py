@@ -1,6 +1,7 @@
 """Tensor-level entry points of the HIP optimizer kernels (current stream, no synchronisation)."""
 from __future__ import annotations
 
+import ctypes
 import math
 import os
 
@@ -43,7 +44,9 @@ class MuonWorkspace:
         self.buffer: torch.Tensor | None = None
 
     def get(self, rows: int, cols: int) -> torch.Tensor:
-        need = muon_workspace_bytes(rows, cols)
+        return self.get_bytes(muon_workspace_bytes(rows, cols))
+
+    def get_bytes(self, need: int) -> torch.Tensor:
         if self.buffer is None or self.buffer.numel() < need:
             self.buffer = None  # release before growing
             self.buffer = torch.empty(need, dtype=torch.uint8, device=self.device)
@@ -57,6 +60,20 @@ def _check_matrix(t: torch.Tensor, what: str) -> None:
         raise RuntimeError(f"{what} must be a contiguous CUDA tensor")
     if t.dtype not in _DTYPE_CODES:
         raise RuntimeError(f"{what} must be float32 or bfloat16, got {t.dtype}")
+
+
+def _check_step(param: torch.Tensor, grad: torch.Tensor, momentum_buf: torch.Tensor, ns_steps: int) -> None:
+    if grad.ndim != 2:
+        raise ValueError("Param gradient must be a 2D matrix")
+    for t, what in ((param, "param"), (grad, "grad"), (momentum_buf, "momentum buffer")):
+        _check_matrix(t, what)
+    if not (param.dtype == grad.dtype == momentum_buf.dtype):
+        # Tensor.lerp_ rejects mixed dtypes; the reference's local shard, grad shard and state share one dtype
+        raise RuntimeError(f"param, grad and momentum buffer must share a dtype, got {param.dtype}, {grad.dtype}, {momentum_buf.dtype}")
+    if not (param.shape == grad.shape == momentum_buf.shape):
+        raise RuntimeError("param, grad and momentum buffer must share a shape")
+    if ns_steps >= 100:
+        raise ValueError("Number of steps must be less than 100 for computational efficiency")
 
 
 def newton_schulz(
@@ -111,19 +128,9 @@ def muon_step(
 ) -> None:
     """One matrix of ``_single_tensor_muon`` (torch/optim/_muon.py:285-318), in
     place on ``param`` and ``momentum_buf``.  ``shared_machine`` tells the
-    kernels that other matrices are updated on other streams at the same time
-    (``muon_step_many`` sets it)."""
-    if grad.ndim != 2:
-        raise ValueError("Param gradient must be a 2D matrix")
-    for t, what in ((param, "param"), (grad, "grad"), (momentum_buf, "momentum buffer")):
-        _check_matrix(t, what)
-    if not (param.dtype == grad.dtype == momentum_buf.dtype):
-        # Tensor.lerp_ rejects mixed dtypes; the reference's local shard, grad shard and state share one dtype
-        raise RuntimeError(f"param, grad and momentum buffer must share a dtype, got {param.dtype}, {grad.dtype}, {momentum_buf.dtype}")
-    if not (param.shape == grad.shape == momentum_buf.shape):
-        raise RuntimeError("param, grad and momentum buffer must share a shape")
-    if ns_steps >= 100:
-        raise ValueError("Number of steps must be less than 100 for computational efficiency")
+    kernels that the caller updates other matrices on other streams at the same
+    time."""
+    _check_step(param, grad, momentum_buf, ns_steps)
     rows, cols = param.shape
     workspace = workspace or MuonWorkspace(param.device)
     ws = workspace.get(rows, cols)
@@ -140,30 +147,9 @@ def muon_step(
         )
 
 
-class MuonStreamPool:
-    """Side streams (default priority) with one Newton-Schulz workspace each, for updating independent matrices at
-    the same time."""
-
-    def __init__(self, device, n_streams: int = 3) -> None:
-        self.device = torch.device(device)
-        self.streams = [torch.cuda.Stream(device=self.device) for _ in range(n_streams)]
-        self.workspaces = [MuonWorkspace(self.device) for _ in range(n_streams)]
-
-
-_STREAM_POOLS: dict[torch.device, MuonStreamPool] = {}
-
-
-def _underfills_the_machine(shape, compute_units: int) -> bool:
-    """Would the 256 x 256 tiles of this matrix's symmetric products (the lower triangle of an m x m result, m the
-    short side) occupy less than three quarters of the CUs?"""
-    t = -(-min(shape) // 256)
-    return 4 * (t * (t + 1) // 2) < 3 * compute_units
-
-
 def side_by_side_default() -> bool | None:
-    """``MATRIX_FSDP_MUON_SIDE_BY_SIDE``: ``0`` keeps every matrix on the calling stream (result bits that do not
-    depend on which other parameters the optimizer holds), ``1`` forces the side streams, unset / ``auto`` decides
-    per call."""
+    """``MATRIX_FSDP_MUON_SIDE_BY_SIDE``: ``0`` updates one matrix after the other (result bits that do not depend on
+    which other parameters the optimizer holds), anything else lets them share launches."""
     value = os.environ.get("MATRIX_FSDP_MUON_SIDE_BY_SIDE", "auto").strip().lower()
     if value in ("0", "false", "off", "no"):
         return False
@@ -172,23 +158,26 @@ def side_by_side_default() -> bool | None:
     return None
 
 
-def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, pool: MuonStreamPool | None = None,
-                   side_by_side: bool | None = None) -> None:
+def _job(param, grad, momentum_buf, *, lr, weight_decay, momentum, nesterov, ns_coefficients=NS_COEFFICIENTS, ns_steps=NS_STEPS, eps=NS_EPS, adjust_lr_fn=None):
+    """``(what the jobs of one library call share, fields of mfsdp_muon_job)``."""
+    _check_step(param, grad, momentum_buf, ns_steps)
+    rows, cols = param.shape
+    key = (_DTYPE_CODES[param.dtype], momentum, int(bool(nesterov)), *ns_coefficients, ns_steps, eps)
+    return key, (param.data_ptr(), grad.data_ptr(), momentum_buf.data_ptr(), rows, cols, lr, weight_decay, adjust_lr(lr, adjust_lr_fn, (rows, cols)))
+
+
+def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, side_by_side: bool | None = None) -> None:
     """Updates several matrices; ``jobs`` is a sequence of ``(param, grad, momentum_buf, keywords of muon_step)``.
 
-    The matrices of a rank are independent of each other.  When at least two of them are so small that the triangle
-    of their symmetric products leaves CUs idle (a hidden4096 layer on 256 CUs: 136 tiles), those are spread over up
-    to three side streams, longest first, so that the idle CUs work for another matrix (three hidden4096 matrices:
-    7.3 against 7.5 ms); the calling stream waits for the side streams before anything enqueued later runs.  Matrices
-    that keep the machine busy on their own run first, one after the other on the calling stream, as every matrix does
-    when fewer than two are small.
+    The matrices of a rank are independent of each other, so those that share their hyper-parameters (the learning
+    rate and weight decay may differ) go through every stage of the update as one launch, up to 32 at a time and as many
+    as 2.3 GiB of workspace hold (``mfsdp_muon_step_many``): small matrices fill the machine together and the number of
+    launches does not grow with theirs.
 
-    Reproducibility: a matrix updated on a side stream takes 256 x 256 tiles in its symmetric products where it would
-    take 128 x 128 tiles alone, so the order of its fp32 sums, and with it the last bits of the update, depends on
-    whether other small matrices are updated in the same call.  Both forms meet the same parity bar; a caller that
-    needs bits independent of the optimizer's other parameters passes ``side_by_side=False`` (or sets
-    ``MATRIX_FSDP_MUON_SIDE_BY_SIDE=0``), which keeps everything on the calling stream; ``True`` sends every 2-D
-    matrix to the side streams whatever its size."""
+    Reproducibility: how the K walk of a product is cut into pieces, and with it the order of its fp32 sums and the last
+    bits of an update, may depend on the other matrices of the call where a side is longer than 1024.  Both forms meet
+    the same parity bar; a caller that needs bits independent of the optimizer's other parameters passes
+    ``side_by_side=False`` (or sets ``MATRIX_FSDP_MUON_SIDE_BY_SIDE=0``), which updates one matrix after the other."""
     jobs = list(jobs)
     if not jobs:
         return
@@ -198,53 +187,26 @@ def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, pool: MuonSt
             raise RuntimeError("muon_step_many updates the matrices of one device")
     if side_by_side is None:
         side_by_side = side_by_side_default()
-    compute_units = torch.cuda.get_device_properties(device).multi_processor_count
+    workspace = workspace or MuonWorkspace(device)
     if side_by_side is False:
-        small = []
-    elif side_by_side:
-        small = [job for job in jobs if job[0].ndim == 2]
-    else:
-        small = [job for job in jobs if job[0].ndim == 2 and _underfills_the_machine(job[0].shape, compute_units)]
-        if len(small) < 2:
-            small = []
-    small_ids = {id(job) for job in small}
-    alone = [job for job in jobs if id(job) not in small_ids]
-    if alone:
-        workspace = workspace or MuonWorkspace(device)
-        for param, grad, buf, kw in alone:
+        for param, grad, buf, kw in jobs:
             muon_step(param, grad, buf, workspace=workspace, **kw)
-    jobs = small
-    if not jobs:
         return
-    if pool is None:
-        pool = _STREAM_POOLS.get(device)
-        if pool is None:
-            pool = _STREAM_POOLS[device] = MuonStreamPool(device)
-    n = min(len(pool.streams), len(jobs))
-    # longest first onto the least loaded stream (flops of the products: 4 m^2 n + 2 m^3 per step)
-    def cost(job):
-        m, k = min(job[0].shape), max(job[0].shape)
-        return 4 * m * m * k + 2 * m**3
-
-    loads, assigned = [0] * n, [[] for _ in range(n)]
-    for job in sorted(jobs, key=cost, reverse=True):
-        s = loads.index(min(loads))
-        assigned[s].append(job)
-        loads[s] += cost(job)
-    current = torch.cuda.current_stream(device)
-    fork = torch.cuda.Event()
-    fork.record(current)
-    for s in range(n):
-        side = pool.streams[s]
-        side.wait_event(fork)
-        with torch.cuda.stream(side):
-            for param, grad, buf, kw in assigned[s]:
-                for t in (param, grad, buf):
-                    t.record_stream(side)
-                muon_step(param, grad, buf, workspace=pool.workspaces[s], shared_machine=True, **kw)
-        join = torch.cuda.Event()
-        join.record(side)
-        current.wait_event(join)
+    alike: dict[tuple, list[tuple]] = {}
+    for param, grad, buf, kw in jobs:
+        key, fields = _job(param, grad, buf, **kw)
+        alike.setdefault(key, []).append(fields)
+    lib = _lib.lib()
+    stream = torch.cuda.current_stream(device).cuda_stream
+    with torch.cuda.device(device):
+        for (dtype, momentum, nesterov, a, b, c, ns_steps, eps), fields in alike.items():
+            n = len(fields)
+            rows, cols = (ctypes.c_int64 * n)(*(f[3] for f in fields)), (ctypes.c_int64 * n)(*(f[4] for f in fields))
+            need = lib.mfsdp_muon_many_workspace_bytes(n, rows, cols)
+            if need <= 0:
+                raise ValueError("Param gradient must be a 2D matrix")
+            ws = workspace.get_bytes(need)
+            _lib.check(lib.mfsdp_muon_step_many(n, (_lib.MuonJob * n)(*fields), dtype, momentum, nesterov, a, b, c, ns_steps, eps, ws.data_ptr(), ws.numel(), stream))
 
 
 def adamw_step(

@@ -310,3 +310,75 @@ def test_adamw_unaligned_views_and_errors():
         F.adamw_step(p, g, m, v, 0, lr=1e-3)
     with pytest.raises(RuntimeError, match="float32"):
         F.adamw_step(p.bfloat16(), g, m, v, 1, lr=1e-3)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("short", [1, 63, 64, 65, 127, 129, 255, 257])
+def test_muon_group_at_tile_edges(short, dtype):
+    """Matrices around the edges of 64, 128 and 256 tiles, wide and tall, in one launch per stage: the momentum and the
+    bits of a call of their own (every side is at most 1024, so no K walk is cut), and the oracle's update."""
+    shapes = [(short, short), (short, 200), (200, short), (short, 700), (700, short), (320, 256)]
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
+    params = [make(sh, 800 + i, 0.02).to(dtype) for i, sh in enumerate(shapes)]
+    grads = [make(sh, 820 + i).to(dtype) for i, sh in enumerate(shapes)]
+    bufs = [make(sh, 840 + i).to(dtype) for i, sh in enumerate(shapes)]
+    many_p, many_b = [p.to(DEV) for p in params], [b.to(DEV) for b in bufs]
+    F.muon_step_many([(p, g.to(DEV), b, kw) for p, g, b in zip(many_p, grads, many_b)])
+    for i in range(len(shapes)):
+        p, b = params[i].to(DEV), bufs[i].to(DEV)
+        F.muon_step(p, grads[i].to(DEV), b, **kw)
+        assert torch.equal(many_p[i], p) and torch.equal(many_b[i], b), shapes[i]
+        p_ref, b_ref = params[i].clone(), bufs[i].clone()
+        O.muon_step(p_ref, grads[i], b_ref, **kw)
+        # a bf16 parameter moves in steps of its own last bit (see test_muon_step_matches_oracle)
+        assert rel_fro((many_p[i].cpu() - params[i]).float(), (p_ref - params[i]).float()) < (MUON_TOL if dtype == torch.float32 else 5e-2), shapes[i]
+
+
+def test_muon_group_larger_than_a_launch_and_than_the_workspace():
+    """More matrices than one launch carries, a workspace that holds only the largest of them (so that every launch has
+    one or two) and parameters at odd offsets of a flat shard: bits of the one-by-one calls."""
+    import ctypes
+
+    from matrix_fsdp_amd import _lib
+
+    shapes = [(96, 160), (33, 70), (160, 96)] * 13
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.9, nesterov=False)
+    flats = [[torch.randn(r * c + 3, generator=torch.Generator().manual_seed(900 + 3 * i + k)) for k in range(3)] for i, (r, c) in enumerate(shapes)]
+
+    def views():
+        return [[f.to(DEV)[1 : 1 + r * c].view(r, c) for f in three] for three, (r, c) in zip(flats, shapes)]
+
+    one = views()
+    for p, g, b in one:
+        F.muon_step(p, g, b, **kw)
+    many = views()
+    F.muon_step_many([(p, g, b, kw) for p, g, b in many])
+    tight = views()
+    ws = torch.empty(F.muon_workspace_bytes(96, 160), dtype=torch.uint8, device=DEV)
+    jobs = (_lib.MuonJob * len(tight))(*((p.data_ptr(), g.data_ptr(), b.data_ptr(), *p.shape, 0.02, 0.1, F.adjust_lr(0.02, None, p.shape)) for p, g, b in tight))
+    args = (_lib.DT_F32, 0.9, 0, *F.NS_COEFFICIENTS, 5, F.NS_EPS)
+    _lib.check(_lib.lib().mfsdp_muon_step_many(len(tight), jobs, *args, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream))
+    for a, b, c in zip(one, many, tight):
+        assert torch.equal(a[0], b[0]) and torch.equal(a[2], b[2]) and torch.equal(a[0], c[0])
+    before = tight[0][0].clone()
+    jobs[5].rows = 0  # one bad job: nothing is enqueued
+    assert _lib.lib().mfsdp_muon_step_many(len(tight), jobs, *args, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream) == 1
+    jobs[5].rows = shapes[5][0]
+    assert _lib.lib().mfsdp_muon_step_many(len(tight), jobs, *args, ws.data_ptr(), ws.numel() - 256, torch.cuda.current_stream().cuda_stream) == 1
+    torch.cuda.synchronize()
+    assert torch.equal(tight[0][0], before)
+    assert _lib.lib().mfsdp_muon_many_workspace_bytes(1, (ctypes.c_int64 * 1)(96), (ctypes.c_int64 * 1)(160)) == ws.numel()
+
+
+def test_muon_group_with_cut_k_walks():
+    """Sides beyond 1024, where the tiles of the last round are cut along K: several K in one launch, against the oracle."""
+    shapes = [(192, 1088), (130, 2100), (4160, 200), (70, 8200)]
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
+    params = [make(sh, 860 + i, 0.02) for i, sh in enumerate(shapes)]
+    grads = [make(sh, 870 + i) for i, sh in enumerate(shapes)]
+    dev_p, dev_b = [p.to(DEV) for p in params], [torch.zeros(sh, device=DEV) for sh in shapes]
+    F.muon_step_many([(p, g.to(DEV), b, kw) for p, g, b in zip(dev_p, grads, dev_b)])
+    for i, sh in enumerate(shapes):
+        p_ref, b_ref = params[i].clone(), torch.zeros(sh)
+        O.muon_step(p_ref, grads[i], b_ref, **kw)
+        assert rel_fro(dev_p[i].cpu() - params[i], p_ref - params[i]) < MUON_TOL, sh
