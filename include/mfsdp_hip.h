@@ -178,10 +178,8 @@ int64_t mfsdp_segment_program_num_runs(const mfsdp_segment_program* program);
 /*
  * Replays the program: srcs[i] is the device base of source i and must hold
  * at least the src_numels[i] elements given at create time, dst at least
- * dst_numel.  One kernel launch per vector width in use (one for a layout whose
- * offsets are all 16-byte multiples); never allocates, never synchronises.  Base
- * pointers less aligned than the layout run the same tables at a narrower
- * vector width.
+ * dst_numel.  One kernel launch (one per block of 128 sources), whatever the alignment of
+ * offsets and base pointers; never allocates, never synchronises.
  */
 int mfsdp_segment_program_run(mfsdp_segment_program* program, const void* const* srcs, int32_t n_srcs,
                               void* dst, void* stream);

@@ -6,6 +6,13 @@
 // / store touches one contiguous 1 KiB span whenever the tile lies inside a row.  Strided 2-D runs (block shards)
 // find their row with a multiply-high by a host-computed reciprocal instead of a division.  By default there is one
 // workgroup per tile and no grid-stride loop; a persistent grid is a tuning option.
+//
+// Alignment.  A group is 16 bytes of the wider side wherever a segment starts: global memory takes vector accesses at any
+// element address, and the last group of a row is moved back so that it ends with the row (it overlaps its neighbour and
+// writes the same bytes again).  Only rows shorter than a group go element by element.  Tiles of long rows begin at
+// multiples of 128 bytes of the destination, so that stores stay whole lines and only the loads straddle.  (Groups as wide
+// as the common alignment of a run's ends took 42 us for the 23 MB of an odd-sized unit cut for three ranks: 2 bytes per
+// lane.)
 #include "mfsdp_common.h"
 
 #include <algorithm>
@@ -26,9 +33,9 @@ constexpr int kMaxBatch = 64;     // destination pointers (buffers) one launch c
 constexpr int kDefaultBlocksPerCu = 0;  // one workgroup per tile
 constexpr int kDefaultBlockThreads = 64;
 constexpr int kBlockThreads = 256;
-constexpr int kFillTileSpans = 8;  // spans of 256 * U groups a zero-fill tile covers (its group count must stay below 2^16)
+constexpr int kFillTileSpans = 8;  // spans of 256 * U groups a zero-fill tile covers (its units must stay below 2^16)
 constexpr int64_t kMaxGrid = (int64_t{1} << 31) - 1;  // grid-stride loops keep a capped grid correct
-constexpr int64_t kMaxUnitsPerRun = 0x7fffffff;  // a device run holds fewer than 2^31 units: the reciprocal division is exact below 2^31 groups, at any group width
+constexpr int64_t kMaxGroupsPerRun = 0x7fffffff;  // the reciprocal division is exact below 2^31 groups
 
 struct SourceTable {
   const char* p[kMaxSources];  // buffer b's source i at p[b * sources_per_buffer + i]
@@ -37,26 +44,28 @@ struct DestTable {
   char* p[kMaxBatch];
 };
 
-// One run in units of vector groups (device copy).
+// One run (device copy).  Offsets, pitches and row length in units (bytes; elements where the program converts).
 struct DevRun {
   int64_t src_off;
   int64_t dst_off;
   int64_t src_stride;
   int64_t dst_stride;
-  uint32_t row_groups;
+  uint32_t row_units;
+  uint32_t row_groups;  // vector groups per row, the last one moved back to end with the row
   uint32_t n_groups;
   uint32_t magic;  // row = umulhi(magic, g) >> shift   (unused when rows == 1 or row_groups == 1)
   uint32_t shift;
   int32_t src_id;
   uint32_t multi_row;
+  uint32_t reserved;
 };
 
 // One tile = the work of one workgroup, 16 bytes.  A tile that lies inside one row of its run is DIRECT: it carries
 // its own offsets, so the workgroup needs no run descriptor (one dependent scalar load before its data loads instead
 // of two, and no row arithmetic).  Runs whose rows are short get GENERIC tiles of 256 * U consecutive groups of the
 // run, which may span rows and go through the run descriptor.
-//   direct : a = source group offset | (source id + 1) << 48  (0: zero fill),  b = destination group offset | groups << 48
-//   generic: a = 1 << 63 | run index,                                           b = tile index within the run
+//   direct : a = source offset | (source id + 1) << 48  (0: zero fill),  b = destination offset | units << 48
+//   generic: a = 1 << 63 | run index,                                    b = tile index within the run
 struct DevTile {
   uint64_t a;
   uint64_t b;
@@ -67,6 +76,12 @@ constexpr uint64_t kTileOffsetMask = (uint64_t{1} << 48) - 1;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
+// 16 and 8 bytes at any address
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+typedef u32x2 u32x2_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef uint16_t u16_any __attribute__((aligned(1)));
+
 template <int NB>
 struct Words {
   uint32_t w[(NB + 3) / 4];
@@ -75,32 +90,20 @@ struct Words {
 template <int NB, bool NT>
 __device__ __forceinline__ Words<NB> load_bytes(const char* p) {
   Words<NB> r;
-  if constexpr (NB == 32) {
-    u32x4 a, b;
-    if constexpr (NT) {
-      a = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-      b = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p) + 1);
-    } else {
-      a = *reinterpret_cast<const u32x4*>(p);
-      b = *(reinterpret_cast<const u32x4*>(p) + 1);
-    }
-    r.w[0] = a.x; r.w[1] = a.y; r.w[2] = a.z; r.w[3] = a.w;
-    r.w[4] = b.x; r.w[5] = b.y; r.w[6] = b.z; r.w[7] = b.w;
-  } else if constexpr (NB == 16) {
+  if constexpr (NB == 16) {
     u32x4 a;
-    if constexpr (NT) a = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-    else a = *reinterpret_cast<const u32x4*>(p);
+    if constexpr (NT) a = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
+    else a = *reinterpret_cast<const u32x4_any*>(p);
     r.w[0] = a.x; r.w[1] = a.y; r.w[2] = a.z; r.w[3] = a.w;
   } else if constexpr (NB == 8) {
     u32x2 a;
-    if constexpr (NT) a = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p));
-    else a = *reinterpret_cast<const u32x2*>(p);
+    if constexpr (NT) a = __builtin_nontemporal_load(reinterpret_cast<const u32x2_any*>(p));
+    else a = *reinterpret_cast<const u32x2_any*>(p);
     r.w[0] = a.x; r.w[1] = a.y;
   } else if constexpr (NB == 4) {
-    if constexpr (NT) r.w[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p));
-    else r.w[0] = *reinterpret_cast<const uint32_t*>(p);
+    r.w[0] = *reinterpret_cast<const u32_any*>(p);
   } else if constexpr (NB == 2) {
-    r.w[0] = *reinterpret_cast<const uint16_t*>(p);
+    r.w[0] = *reinterpret_cast<const u16_any*>(p);
   } else {
     r.w[0] = *reinterpret_cast<const uint8_t*>(p);
   }
@@ -109,29 +112,18 @@ __device__ __forceinline__ Words<NB> load_bytes(const char* p) {
 
 template <int NB, bool NT>
 __device__ __forceinline__ void store_bytes(char* p, const Words<NB>& v) {
-  if constexpr (NB == 32) {
-    u32x4 a = {v.w[0], v.w[1], v.w[2], v.w[3]};
-    u32x4 b = {v.w[4], v.w[5], v.w[6], v.w[7]};
-    if constexpr (NT) {
-      __builtin_nontemporal_store(a, reinterpret_cast<u32x4*>(p));
-      __builtin_nontemporal_store(b, reinterpret_cast<u32x4*>(p) + 1);
-    } else {
-      *reinterpret_cast<u32x4*>(p) = a;
-      *(reinterpret_cast<u32x4*>(p) + 1) = b;
-    }
-  } else if constexpr (NB == 16) {
-    u32x4 a = {v.w[0], v.w[1], v.w[2], v.w[3]};
-    if constexpr (NT) __builtin_nontemporal_store(a, reinterpret_cast<u32x4*>(p));
-    else *reinterpret_cast<u32x4*>(p) = a;
+  if constexpr (NB == 16) {
+    const u32x4 a = {v.w[0], v.w[1], v.w[2], v.w[3]};
+    if constexpr (NT) __builtin_nontemporal_store(a, reinterpret_cast<u32x4_any*>(p));
+    else *reinterpret_cast<u32x4_any*>(p) = a;
   } else if constexpr (NB == 8) {
-    u32x2 a = {v.w[0], v.w[1]};
-    if constexpr (NT) __builtin_nontemporal_store(a, reinterpret_cast<u32x2*>(p));
-    else *reinterpret_cast<u32x2*>(p) = a;
+    const u32x2 a = {v.w[0], v.w[1]};
+    if constexpr (NT) __builtin_nontemporal_store(a, reinterpret_cast<u32x2_any*>(p));
+    else *reinterpret_cast<u32x2_any*>(p) = a;
   } else if constexpr (NB == 4) {
-    if constexpr (NT) __builtin_nontemporal_store(v.w[0], reinterpret_cast<uint32_t*>(p));
-    else *reinterpret_cast<uint32_t*>(p) = v.w[0];
+    *reinterpret_cast<u32_any*>(p) = v.w[0];
   } else if constexpr (NB == 2) {
-    *reinterpret_cast<uint16_t*>(p) = static_cast<uint16_t>(v.w[0]);
+    *reinterpret_cast<u16_any*>(p) = static_cast<uint16_t>(v.w[0]);
   } else {
     *reinterpret_cast<uint8_t*>(p) = static_cast<uint8_t>(v.w[0]);
   }
@@ -188,14 +180,47 @@ __device__ __forceinline__ Words<DST_B> convert_group(const Words<SRC_B>& in) {
 // stores finely interleaved -- what HBM serves best (a plain copy: 6.5 TB/s against 5.9 for a persistent grid); and the
 // finer the better: by default the 256 lanes of a tile are four workgroups of one wavefront each (THREADS = 64), which
 // all read the same 16-byte tile entry.
-// narrow_shift s > 0 runs the tables at a vector group 2^s times narrower than the one they were compiled for (base
-// pointers less aligned than the layout): a tile is then 2^s sub-tiles, and group g of the narrow grid lies in natural
-// group g >> s.
-template <int SRC_B, int DST_B, int U, bool NT, bool NTS = NT, bool HALF = false, int THREADS = kBlockThreads>
+template <int SRC_U, int DST_U>
+constexpr int group_units() {
+  // the wider side is one 16-byte access per lane, so that every wave-level access is one contiguous span (converting
+  // eight elements would make the 32-byte side two half-dense accesses: 51 % vs 67 % of HBM peak)
+  return SRC_U == DST_U ? 16 : 4;
+}
+
+// `n` units (fewer than a group), by one lane.
+template <int SRC_U, int DST_U, bool HALF>
+__device__ __forceinline__ void move_few(const char* src, char* dst, uint32_t n) {
+  if constexpr (SRC_U == DST_U) {
+    const bool fill = src == nullptr;
+    uint32_t at = 0;
+    auto part = [&](auto bytes) {
+      constexpr int B = decltype(bytes)::value;
+      if (n & B) {
+        Words<B> v = {};
+        if (!fill) v = load_bytes<B, false>(src + at);
+        store_bytes<B, false>(dst + at, v);
+        at += B;
+      }
+    };
+    part(std::integral_constant<int, 8>{});
+    part(std::integral_constant<int, 4>{});
+    part(std::integral_constant<int, 2>{});
+    part(std::integral_constant<int, 1>{});
+  } else {
+    for (uint32_t i = 0; i < n; ++i) {
+      Words<SRC_U> v = {};
+      if (src != nullptr) v = load_bytes<SRC_U, false>(src + i * SRC_U);
+      store_bytes<DST_U, false>(dst + i * DST_U, convert_group<SRC_U, DST_U, HALF>(v));
+    }
+  }
+}
+
+template <int SRC_U, int DST_U, int U, bool NT, bool NTS = NT, bool HALF = false, int THREADS = kBlockThreads>
 __global__ void __launch_bounds__(THREADS)
 segment_program_kernel(SourceTable srcs, DestTable dsts, const DevRun* __restrict__ runs, const DevTile* __restrict__ tiles,
-                       uint32_t n_tiles, uint32_t total_tiles, uint32_t srcs_per_buffer, uint32_t narrow_shift, uint32_t tiles_per_xcd_turn) {
-  const uint32_t s = narrow_shift;
+                       uint32_t n_tiles, uint32_t total_tiles, uint32_t srcs_per_buffer, uint32_t tiles_per_xcd_turn) {
+  constexpr uint32_t G = group_units<SRC_U, DST_U>();
+  constexpr int SRC_B = G * SRC_U, DST_B = G * DST_U;
   constexpr uint32_t kTileGroups = kBlockThreads * U;
   // a tile's 256 lanes may be spread over several smaller workgroups: lane = part * THREADS + threadIdx.x
   constexpr uint32_t kParts = kBlockThreads / THREADS;
@@ -227,17 +252,21 @@ segment_program_kernel(SourceTable srcs, DestTable dsts, const DevRun* __restric
     const DevTile tile = tiles[t];
     if (!(tile.a & kTileGeneric)) {
       const uint32_t id1 = static_cast<uint32_t>(tile.a >> 48);
-      const char* sbase = id1 == 0 ? nullptr : (srcs_per_buffer == 1 ? only_source : srcs.p[b * srcs_per_buffer + id1 - 1]);
-      const int64_t soff = static_cast<int64_t>(tile.a & kTileOffsetMask) << s;
-      const int64_t doff = static_cast<int64_t>(tile.b & kTileOffsetMask) << s;
-      const uint32_t n_groups = static_cast<uint32_t>(tile.b >> 48) << s;
-      for (uint32_t first = 0; first < n_groups; first += kTileGroups) {
+      const char* src = id1 == 0 ? nullptr : (srcs_per_buffer == 1 ? only_source : srcs.p[b * srcs_per_buffer + id1 - 1]);
+      if (src != nullptr) src += static_cast<int64_t>(tile.a & kTileOffsetMask) * SRC_U;
+      dst += static_cast<int64_t>(tile.b & kTileOffsetMask) * DST_U;
+      const uint32_t units = static_cast<uint32_t>(tile.b >> 48);
+      if (units < G) {
+        if (tile_lane == 0) move_few<SRC_U, DST_U, HALF>(src, dst, units);
+        continue;
+      }
+      for (uint32_t first = 0; first < units; first += kTileGroups * G) {
         Words<SRC_B> data[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const uint32_t g = first + u * kBlockThreads + tile_lane;
-          if (g < n_groups && sbase != nullptr) {
-            data[u] = load_bytes<SRC_B, NT>(sbase + (soff + g) * SRC_B);
+          const uint32_t at = first + (u * kBlockThreads + tile_lane) * G;
+          if (at < units && src != nullptr) {
+            data[u] = load_bytes<SRC_B, NT>(src + static_cast<uint64_t>(min(at, units - G)) * SRC_U);
           } else {
 #pragma unroll
             for (int i = 0; i < (SRC_B + 3) / 4; ++i) data[u].w[i] = 0;
@@ -245,45 +274,44 @@ segment_program_kernel(SourceTable srcs, DestTable dsts, const DevRun* __restric
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const uint32_t g = first + u * kBlockThreads + tile_lane;
-          if (g < n_groups) store_bytes<DST_B, NTS>(dst + (doff + g) * DST_B, convert_group<SRC_B, DST_B, HALF>(data[u]));
+          const uint32_t at = first + (u * kBlockThreads + tile_lane) * G;
+          if (at < units) store_bytes<DST_B, NTS>(dst + static_cast<uint64_t>(min(at, units - G)) * DST_U, convert_group<SRC_B, DST_B, HALF>(data[u]));
         }
       }
       continue;
     }
     const DevRun run = runs[static_cast<uint32_t>(tile.a)];
-    const uint32_t tile_index = static_cast<uint32_t>(tile.b);
-    const char* sbase = run.src_id >= 0 ? srcs.p[b * srcs_per_buffer + run.src_id] : nullptr;
-    const uint32_t n_groups = run.n_groups << s;
-    for (uint32_t sub = 0; sub < (1u << s); ++sub) {
-      const uint32_t first = ((tile_index << s) + sub) * kTileGroups;
-      if (first >= n_groups) break;
-      Words<SRC_B> data[U];
-      int64_t doff[U];
-      bool live[U];
+    const char* src = run.src_id >= 0 ? srcs.p[b * srcs_per_buffer + run.src_id] : nullptr;
+    const uint32_t first = static_cast<uint32_t>(tile.b) * kTileGroups;
+    Words<SRC_B> data[U];
+    int64_t doff[U];
+    bool live[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint32_t g = first + u * kBlockThreads + tile_lane;
-        live[u] = g < n_groups;
-        uint32_t row = 0, col = g;
-        if (run.multi_row) {
-          const uint32_t natural = g >> s;
-          row = run.row_groups == 1 ? natural : (__umulhi(run.magic, natural) >> run.shift);
-          col = g - ((row * run.row_groups) << s);
-        }
-        doff[u] = (run.dst_off << s) + static_cast<int64_t>(row) * (run.dst_stride << s) + col;
-        if (live[u] && sbase != nullptr) {
-          const int64_t soff = (run.src_off << s) + static_cast<int64_t>(row) * (run.src_stride << s) + col;
-          data[u] = load_bytes<SRC_B, NT>(sbase + soff * SRC_B);
-        } else {
-#pragma unroll
-          for (int i = 0; i < (SRC_B + 3) / 4; ++i) data[u].w[i] = 0;
-        }
+    for (int u = 0; u < U; ++u) {
+      const uint32_t g = first + u * kBlockThreads + tile_lane;
+      live[u] = g < run.n_groups;
+      uint32_t row = 0, col = g;
+      if (run.multi_row) {
+        row = run.row_groups == 1 ? g : (__umulhi(run.magic, g) >> run.shift);
+        col = g - row * run.row_groups;
       }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (live[u]) store_bytes<DST_B, NTS>(dst + doff[u] * DST_B, convert_group<SRC_B, DST_B, HALF>(data[u]));
+      const int64_t col_unit = run.row_units < G ? 0 : min(col * G, run.row_units - G);
+      doff[u] = run.dst_off + static_cast<int64_t>(row) * run.dst_stride + col_unit;
+      const int64_t soff = run.src_off + static_cast<int64_t>(row) * run.src_stride + col_unit;
+      if (run.row_units < G) {
+        if (live[u]) move_few<SRC_U, DST_U, HALF>(src == nullptr ? nullptr : src + soff * SRC_U, dst + doff[u] * DST_U, run.row_units);
+        live[u] = false;
       }
+      if (live[u] && src != nullptr) {
+        data[u] = load_bytes<SRC_B, NT>(src + soff * SRC_U);
+      } else {
+#pragma unroll
+        for (int i = 0; i < (SRC_B + 3) / 4; ++i) data[u].w[i] = 0;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (live[u]) store_bytes<DST_B, NTS>(dst + doff[u] * DST_U, convert_group<SRC_B, DST_B, HALF>(data[u]));
     }
   }
 }
@@ -295,9 +323,6 @@ struct Tuning {
   std::atomic<int> nontemporal{1};
   std::atomic<int> block_threads{0};  // threads per workgroup: 64, 128 or 256 (a tile's 256 lanes over 4, 2 or 1 workgroups); 0: default
   std::atomic<int> unroll{0};  // loads in flight per lane: 1, 2 or 4; 0: library default per kernel
-  // elements per lane when converting: 4 keeps the wider side at one 16-byte access per lane, so that every wave-level
-  // access is one contiguous span (8 elements would make the 32-byte side two half-dense accesses: 51 % vs 67 % of HBM peak)
-  static constexpr int convert_group = 4;
 };
 Tuning g_tuning;
 
@@ -305,9 +330,8 @@ bool is_half_conversion(int convert) { return convert == MFSDP_CONVERT_F16_TO_F3
 
 // ---- host side -------------------------------------------------------------------------------
 
-// Tables of one launch: the runs of one natural vector width whose sources fall into one block of kMaxSources.
+// Tables of one launch: the runs whose sources fall into one block of kMaxSources.
 struct Compiled {
-  int group_units = 0;   // natural group width G, in units
   int source_base = 0;   // first source id the launch's pointer table holds (a multiple of kMaxSources)
   int n_sources = 0;     // pointers per buffer in that table
   DevRun* runs = nullptr;
@@ -325,12 +349,6 @@ void reciprocal(uint32_t d, uint32_t* magic, uint32_t* shift) {
   *shift = l - 1;
 }
 
-int64_t gcd_pow2(int64_t v, int64_t cap) {  // largest power of two <= cap dividing v (v == 0 -> cap)
-  int64_t g = cap;
-  while (g > 1 && (v % g) != 0) g >>= 1;
-  return g;
-}
-
 }  // namespace
 }  // namespace mfsdp
 
@@ -343,7 +361,6 @@ struct mfsdp_segment_program {
   int convert = 0;
   int src_unit = 1;  // bytes per unit on the source side
   int dst_unit = 1;
-  int max_group = 16;  // widest vector group in units
   int64_t bytes_moved = 0;
   int device = 0;
   std::vector<Compiled> compiled;  // built once at create time; run() only reads it
@@ -359,60 +376,56 @@ void free_compiled(std::vector<Compiled>& v) {
   v.clear();
 }
 
-// Builds the device tables: runs bucketed by (natural vector width, block of kMaxSources sources), one tile per workgroup.
+// Builds the device tables: runs bucketed by blocks of kMaxSources sources, one tile per workgroup.
 int compile_tables(mfsdp_segment_program* prog, std::vector<Compiled>* out) {
   int unroll = g_tuning.unroll.load(std::memory_order_relaxed);
   // plain copies: one 16-byte load per lane (pack / unpack of the hidden4096 block layout with workgroups of one
   // wavefront: 6.56 / 6.39 TB/s against 6.22 / 6.14 with two loads; with 256 threads 6.06 / 6.20); converting programs move
   // half as much on their narrow side and like two (bf16 -> fp32 gradient fill of the hidden2048 layer 6.09 against 6.00)
-  if (unroll != 1 && unroll != 2 && unroll != 4) unroll = prog->src_unit != prog->dst_unit ? 2 : 1;
-  const uint32_t tile_groups = kBlockThreads * unroll;
-  std::map<std::pair<int, int>, std::pair<std::vector<DevRun>, std::vector<DevTile>>> buckets;
+  const bool converts = prog->src_unit != prog->dst_unit;
+  if (unroll != 1 && unroll != 2 && unroll != 4) unroll = converts ? 2 : 1;
+  const int64_t group = converts ? 4 : 16;
+  const int64_t tile_groups = kBlockThreads * unroll, tile_units = tile_groups * group;
+  const int64_t line = 128 / prog->dst_unit;  // destination units per 128 bytes
+  std::map<int, std::pair<std::vector<DevRun>, std::vector<DevTile>>> buckets;
   for (const auto& r : prog->runs) {
-    int64_t g = prog->max_group;
-    g = gcd_pow2(r.row_len, g);
-    g = gcd_pow2(r.dst_off, g);
-    if (r.src_id >= 0) g = gcd_pow2(r.src_off, g);
-    if (r.rows > 1) {
-      g = gcd_pow2(r.dst_stride, g);
-      if (r.src_id >= 0) g = gcd_pow2(r.src_stride, g);
-    }
     const int block = r.src_id >= 0 ? r.src_id / kMaxSources : 0;
-    auto& bucket = buckets[{static_cast<int>(g), block}];
-    const int64_t row_groups = r.row_len / g;
+    auto& bucket = buckets[block];
     const int32_t local_id = r.src_id >= 0 ? r.src_id - block * kMaxSources : -1;
-    const int64_t src_off = r.src_id >= 0 ? r.src_off / g : 0, dst_off = r.dst_off / g;
-    const int64_t src_stride = r.rows > 1 && r.src_id >= 0 ? r.src_stride / g : 0, dst_stride = r.rows > 1 ? r.dst_stride / g : 0;
+    const int64_t src_off = r.src_id >= 0 ? r.src_off : 0, src_stride = r.rows > 1 && r.src_id >= 0 ? r.src_stride : 0, dst_stride = r.rows > 1 ? r.dst_stride : 0;
+    const int64_t row_groups = (r.row_len + group - 1) / group;
     if (r.rows == 1 || row_groups >= tile_groups / 2) {
-      // direct tiles: every row is cut into equal pieces of at most one tile, a multiple of 128 bytes long where
-      // the row allows it, so that no workgroup is left with a sliver
+      // direct tiles: every row is cut into equal pieces of at most one tile, so that no workgroup is left with a sliver,
+      // at multiples of 128 bytes of the destination (of its offset: base pointers are at least that aligned as a rule)
       // Zero fill only stores: a wavefront that writes 1 KiB is gone before the next can be dispatched and the launch
       // runs at the dispatch rate (pad tails of the hidden5120 owner layouts: 4.2-4.6 TB/s); eight times the span per
       // workgroup, walked in the kernel's loop over a direct tile, lifts the fill to 5.3 TB/s (pack of such a layer
       // buffer 6.09 TB/s against 5.55-5.78; 32 spans no better; fill tiles spread evenly among the copying tiles
       // instead of behind each rank's segments: slower, 5.85-5.95).
-      const int64_t tile_cap = r.src_id < 0 ? kFillTileSpans * tile_groups : tile_groups;
-      const int64_t per_row = (row_groups + tile_cap - 1) / tile_cap;
-      const int64_t piece = std::min<int64_t>(tile_cap, ((row_groups + per_row - 1) / per_row + 7) / 8 * 8);
+      const int64_t tile_cap = r.src_id < 0 ? kFillTileSpans * tile_units : tile_units;
+      const int64_t per_row = (r.row_len + tile_cap - 1) / tile_cap;
+      const int64_t piece = std::min(tile_cap, ((r.row_len + per_row - 1) / per_row + line - 1) / line * line);
       for (int64_t row = 0; row < r.rows; ++row) {
-        for (int64_t col = 0; col < row_groups; col += piece) {
-          const uint64_t n = static_cast<uint64_t>(std::min(piece, row_groups - col));
-          bucket.second.push_back(DevTile{static_cast<uint64_t>(src_off + row * src_stride + col) | (static_cast<uint64_t>(local_id + 1) << 48),
-                                          static_cast<uint64_t>(dst_off + row * dst_stride + col) | (n << 48)});
+        const int64_t src = src_off + row * src_stride, dst = r.dst_off + row * dst_stride;
+        for (int64_t col = 0, n; col < r.row_len; col += n) {
+          n = std::min(piece - (dst + col) % line, r.row_len - col);
+          bucket.second.push_back(DevTile{static_cast<uint64_t>(src + col) | (static_cast<uint64_t>(local_id + 1) << 48),
+                                          static_cast<uint64_t>(dst + col) | (static_cast<uint64_t>(n) << 48)});
         }
       }
       continue;
     }
-    // generic tiles: short rows, several per tile; a device run holds fewer than 2^31 units so that the reciprocal
-    // division stays exact at any vector width (row_groups < tile_groups here, so only the row count is ever cut)
-    const int64_t rows_per_part = std::max<int64_t>(1, kMaxUnitsPerRun / g / row_groups);
+    // generic tiles: short rows, several per tile; a device run holds fewer than 2^31 groups so that the reciprocal
+    // division stays exact (row_groups < tile_groups here, so only the row count is ever cut)
+    const int64_t rows_per_part = std::max<int64_t>(1, kMaxGroupsPerRun / row_groups);
     for (int64_t row0 = 0; row0 < r.rows; row0 += rows_per_part) {
       const int64_t nrows = std::min(rows_per_part, r.rows - row0);
       DevRun d{};
       d.src_off = src_off + row0 * src_stride;
-      d.dst_off = dst_off + row0 * dst_stride;
+      d.dst_off = r.dst_off + row0 * dst_stride;
       d.src_stride = nrows > 1 ? src_stride : 0;
       d.dst_stride = nrows > 1 ? dst_stride : 0;
+      d.row_units = static_cast<uint32_t>(r.row_len);
       d.row_groups = static_cast<uint32_t>(row_groups);
       d.n_groups = static_cast<uint32_t>(row_groups * nrows);
       d.multi_row = nrows > 1 ? 1u : 0u;
@@ -422,15 +435,14 @@ int compile_tables(mfsdp_segment_program* prog, std::vector<Compiled>* out) {
       if (d.multi_row && d.row_groups > 1) reciprocal(d.row_groups, &d.magic, &d.shift);
       const uint64_t run_index = bucket.first.size();
       bucket.first.push_back(d);
-      const uint32_t ntiles = (d.n_groups + tile_groups - 1) / tile_groups;
+      const uint32_t ntiles = static_cast<uint32_t>((d.n_groups + tile_groups - 1) / tile_groups);
       for (uint32_t t = 0; t < ntiles; ++t) bucket.second.push_back(DevTile{kTileGeneric | run_index, t});
     }
   }
   const int n_srcs = static_cast<int>(prog->src_numels.size());
   for (auto& kv : buckets) {
     Compiled c;
-    c.group_units = kv.first.first;
-    c.source_base = kv.first.second * kMaxSources;
+    c.source_base = kv.first * kMaxSources;
     c.n_sources = std::max(0, std::min(kMaxSources, n_srcs - c.source_base));
     c.unroll = unroll;
     auto& runs = kv.second.first;
@@ -454,9 +466,8 @@ int compile_tables(mfsdp_segment_program* prog, std::vector<Compiled>* out) {
   return MFSDP_OK;
 }
 
-template <int SRC_B, int DST_B, bool HALF = false>
-int launch_one(const Compiled& c, const SourceTable& srcs, const DestTable& dsts, uint32_t batch, uint32_t narrow_shift,
-               hipStream_t stream) {
+template <int SRC_U, int DST_U, bool HALF = false>
+int launch_one(const Compiled& c, const SourceTable& srcs, const DestTable& dsts, uint32_t batch, hipStream_t stream) {
   const int cus = device_cu_count();
   const uint64_t total64 = static_cast<uint64_t>(c.n_tiles) * batch;
   if (total64 > 0xffffffffull) return fail(MFSDP_ERR_UNSUPPORTED, "a batch of %u buffers needs %llu tiles, more than one launch can address", batch, static_cast<unsigned long long>(total64));
@@ -475,8 +486,8 @@ int launch_one(const Compiled& c, const SourceTable& srcs, const DestTable& dsts
   const uint32_t tpl = batch == 1 ? 4u : 0u;
   const int nt = g_tuning.nontemporal.load(std::memory_order_relaxed);  // 0 none, 1 loads and stores, 2 loads only, 3 stores only
 #define MFSDP_LAUNCH(U_, NTL_, NTS_, T_)                                                                                  \
-  hipLaunchKernelGGL((segment_program_kernel<SRC_B, DST_B, U_, NTL_, NTS_, HALF, T_>), grid, dim3(T_), 0, stream, srcs, dsts, \
-                     c.runs, c.tiles, c.n_tiles, total, static_cast<uint32_t>(c.n_sources), narrow_shift, tpl)
+  hipLaunchKernelGGL((segment_program_kernel<SRC_U, DST_U, U_, NTL_, NTS_, HALF, T_>), grid, dim3(T_), 0, stream, srcs, dsts, \
+                     c.runs, c.tiles, c.n_tiles, total, static_cast<uint32_t>(c.n_sources), tpl)
 #define MFSDP_LAUNCH_T(U_, NTL_, NTS_)                                        \
   if (threads == 64) MFSDP_LAUNCH(U_, NTL_, NTS_, 64);                        \
   else if (threads == 128) MFSDP_LAUNCH(U_, NTL_, NTS_, 128);                 \
@@ -500,50 +511,29 @@ int launch_one(const Compiled& c, const SourceTable& srcs, const DestTable& dsts
   return MFSDP_OK;
 }
 
-// `cap` is the widest group (in units) the base pointers of this launch allow.
 int launch_compiled(const mfsdp_segment_program* prog, const Compiled& c, const SourceTable& srcs, const DestTable& dsts,
-                    uint32_t batch, int cap, hipStream_t stream) {
+                    uint32_t batch, hipStream_t stream) {
   if (c.n_tiles == 0) return MFSDP_OK;
-  const int group = std::min(c.group_units, cap);
-  uint32_t narrow_shift = 0;
-  while ((group << narrow_shift) < c.group_units) ++narrow_shift;
-  const int sb = group * prog->src_unit;
-  const int db = group * prog->dst_unit;
-#define MFSDP_CASE(S_, D_) \
-  if (sb == S_ && db == D_) return launch_one<S_, D_>(c, srcs, dsts, batch, narrow_shift, stream)
-#define MFSDP_CONVERTING(S_, D_) \
-  if (sb == S_ && db == D_) return half ? launch_one<S_, D_, true>(c, srcs, dsts, batch, narrow_shift, stream) : launch_one<S_, D_, false>(c, srcs, dsts, batch, narrow_shift, stream)
   const bool half = is_half_conversion(prog->convert);
-  MFSDP_CASE(16, 16); MFSDP_CASE(8, 8); MFSDP_CASE(4, 4); MFSDP_CASE(2, 2); MFSDP_CASE(1, 1);
-  MFSDP_CONVERTING(16, 32); MFSDP_CONVERTING(8, 16); MFSDP_CONVERTING(4, 8); MFSDP_CONVERTING(2, 4);
-  MFSDP_CONVERTING(32, 16); MFSDP_CONVERTING(16, 8); MFSDP_CONVERTING(8, 4); MFSDP_CONVERTING(4, 2);
-#undef MFSDP_CONVERTING
-#undef MFSDP_CASE
-  return fail(MFSDP_ERR_UNSUPPORTED, "no kernel for %d -> %d byte groups", sb, db);
+  if (prog->src_unit == prog->dst_unit) return launch_one<1, 1>(c, srcs, dsts, batch, stream);
+  if (prog->src_unit == 2) return half ? launch_one<2, 4, true>(c, srcs, dsts, batch, stream) : launch_one<2, 4, false>(c, srcs, dsts, batch, stream);
+  return half ? launch_one<4, 2, true>(c, srcs, dsts, batch, stream) : launch_one<4, 2, false>(c, srcs, dsts, batch, stream);
 }
 
-int pointer_alignment_units(const void* p, int unit_bytes, int max_group) {
-  // largest power-of-two group (in units) whose byte size (capped at 16) divides the address
-  int g = max_group;
-  const uintptr_t a = reinterpret_cast<uintptr_t>(p);
-  while (g > 1 && (a % static_cast<uintptr_t>(std::min(g * unit_bytes, 16))) != 0) g >>= 1;
-  return g;
-}
-
-int setup_units(int convert, int elem_bytes, int* src_unit, int* dst_unit, int* max_group, int* scale) {
+int setup_units(int convert, int elem_bytes, int* src_unit, int* dst_unit, int* scale) {
   switch (convert) {
     case MFSDP_CONVERT_NONE:
       if (elem_bytes != 1 && elem_bytes != 2 && elem_bytes != 4 && elem_bytes != 8)
         return fail(MFSDP_ERR_INVALID, "elem_bytes must be 1, 2, 4 or 8, got %d", elem_bytes);
-      *src_unit = 1; *dst_unit = 1; *max_group = 16; *scale = elem_bytes;  // units are bytes
+      *src_unit = 1; *dst_unit = 1; *scale = elem_bytes;  // units are bytes
       return MFSDP_OK;
     case MFSDP_CONVERT_BF16_TO_F32:
     case MFSDP_CONVERT_F16_TO_F32:
-      *src_unit = 2; *dst_unit = 4; *max_group = Tuning::convert_group; *scale = 1;
+      *src_unit = 2; *dst_unit = 4; *scale = 1;
       return MFSDP_OK;
     case MFSDP_CONVERT_F32_TO_BF16:
     case MFSDP_CONVERT_F32_TO_F16:
-      *src_unit = 4; *dst_unit = 2; *max_group = Tuning::convert_group; *scale = 1;
+      *src_unit = 4; *dst_unit = 2; *scale = 1;
       return MFSDP_OK;
     default:
       return fail(MFSDP_ERR_INVALID, "unknown conversion code %d", convert);
@@ -639,8 +629,8 @@ extern "C" int mfsdp_segment_program_create(const mfsdp_copy_run* runs, int64_t 
   if (n_srcs < 0) return fail(MFSDP_ERR_INVALID, "n_srcs must be non-negative, got %d", n_srcs);
   if (n_srcs > 0 && src_numels == nullptr) return fail(MFSDP_ERR_INVALID, "src_numels is null");
   if (dst_numel < 0) return fail(MFSDP_ERR_INVALID, "dst_numel must be non-negative");
-  int src_unit, dst_unit, max_group, scale;
-  if (int rc = setup_units(convert, elem_bytes, &src_unit, &dst_unit, &max_group, &scale)) return rc;
+  int src_unit, dst_unit, scale;
+  if (int rc = setup_units(convert, elem_bytes, &src_unit, &dst_unit, &scale)) return rc;
   for (int32_t i = 0; i < n_srcs; ++i)
     if (src_numels[i] < 0) return fail(MFSDP_ERR_INVALID, "src_numels[%d] is negative", i);
 
@@ -648,7 +638,6 @@ extern "C" int mfsdp_segment_program_create(const mfsdp_copy_run* runs, int64_t 
   prog->convert = convert;
   prog->src_unit = src_unit;
   prog->dst_unit = dst_unit;
-  prog->max_group = max_group;
   prog->dst_numel = dst_numel * scale;
   for (int32_t i = 0; i < n_srcs; ++i) prog->src_numels.push_back(src_numels[i] * scale);
   (void)hipGetDevice(&prog->device);
@@ -711,16 +700,12 @@ extern "C" int mfsdp_segment_program_run_many(mfsdp_segment_program* program, in
     return fail(MFSDP_ERR_INVALID, "program was created for %zu sources, got %d", program->src_numels.size(), n_srcs);
   if (program->runs.empty() || n_buffers == 0) return MFSDP_OK;
   if (dsts == nullptr || (n_srcs > 0 && srcs == nullptr)) return fail(MFSDP_ERR_INVALID, "pointer array is null");
-  // the narrowest alignment among all base pointers decides the vector width of every launch
-  int cap = program->max_group;
   for (int32_t b = 0; b < n_buffers; ++b) {
     if (dsts[b] == nullptr) return fail(MFSDP_ERR_INVALID, "dst is null (buffer %d)", b);
-    cap = std::min(cap, pointer_alignment_units(dsts[b], program->dst_unit, program->max_group));
     for (int32_t i = 0; i < n_srcs; ++i) {
       const void* p = srcs[static_cast<int64_t>(b) * n_srcs + i];
       if (program->src_numels[i] == 0) continue;
       if (p == nullptr) return fail(MFSDP_ERR_INVALID, "source %d is null (buffer %d)", i, b);
-      cap = std::min(cap, pointer_alignment_units(p, program->src_unit, program->max_group));
     }
   }
   hipStream_t s = as_stream(stream);
@@ -738,7 +723,7 @@ extern "C" int mfsdp_segment_program_run_many(mfsdp_segment_program* program, in
         for (int i = 0; i < c.n_sources; ++i)
           st.p[b * c.n_sources + i] = static_cast<const char*>(srcs[static_cast<int64_t>(b0 + b) * n_srcs + c.source_base + i]);
       }
-      if (int rc = launch_compiled(program, c, st, dt, static_cast<uint32_t>(batch), cap, s)) return rc;
+      if (int rc = launch_compiled(program, c, st, dt, static_cast<uint32_t>(batch), s)) return rc;
     }
   }
   return MFSDP_OK;
@@ -793,10 +778,18 @@ int stream_threads() {
   return (threads == 64 || threads == 128 || threads == 256) ? threads : kDefaultBlockThreads;
 }
 
-// dst[g] = convert(src[g]) over n_groups contiguous vector groups.
-template <int SRC_B, int DST_B, int U, bool NT, bool HALF = false>
+// dst = convert(src) over `units` contiguous units, in vector groups; the last one is moved back so that it ends with the
+// span (a span shorter than a group goes unit by unit).  Neither pointer needs more than its elements' alignment.
+template <int SRC_U, int DST_U, int U, bool NT, bool HALF = false>
 __global__ void __launch_bounds__(kBlockThreads)
-linear_kernel(const char* __restrict__ src, char* __restrict__ dst, int64_t n_groups) {
+linear_kernel(const char* __restrict__ src, char* __restrict__ dst, int64_t units) {
+  constexpr int G = group_units<SRC_U, DST_U>();
+  constexpr int SRC_B = G * SRC_U, DST_B = G * DST_U;
+  if (units < G) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) move_few<SRC_U, DST_U, HALF>(src, dst, static_cast<uint32_t>(units));
+    return;
+  }
+  const int64_t n_groups = (units + G - 1) / G;
   const int64_t span = static_cast<int64_t>(blockDim.x) * U;
   for (int64_t base = static_cast<int64_t>(blockIdx.x) * span; base < n_groups;
        base += static_cast<int64_t>(gridDim.x) * span) {
@@ -804,68 +797,40 @@ linear_kernel(const char* __restrict__ src, char* __restrict__ dst, int64_t n_gr
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t g = base + u * blockDim.x + threadIdx.x;
-      if (g < n_groups) data[u] = load_bytes<SRC_B, NT>(src + g * SRC_B);
+      if (g < n_groups) data[u] = load_bytes<SRC_B, NT>(src + (g + 1 < n_groups ? g * G : units - G) * SRC_U);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int64_t g = base + u * blockDim.x + threadIdx.x;
-      if (g < n_groups) store_bytes<DST_B, NT>(dst + g * DST_B, convert_group<SRC_B, DST_B, HALF>(data[u]));
+      if (g < n_groups) store_bytes<DST_B, NT>(dst + (g + 1 < n_groups ? g * G : units - G) * DST_U, convert_group<SRC_B, DST_B, HALF>(data[u]));
     }
   }
 }
 
-template <int SRC_B, int DST_B, bool HALF = false>
-int launch_linear(const char* src, char* dst, int64_t n_groups, hipStream_t stream) {
-  if (n_groups <= 0) return MFSDP_OK;
+template <int SRC_U, int DST_U, bool HALF = false>
+int launch_linear(const char* src, char* dst, int64_t units, hipStream_t stream) {
   // one workgroup per block of the tensor, not a persistent grid: workgroups are dispatched in order, so those in
   // flight sweep neighbouring addresses (bf16 -> fp32 of 202 M elements 5.83 against 5.65 TB/s with 16 per CU)
   // workgroups of one wavefront, one 16-byte load per lane for a plain copy (202 M bf16 elements: 6.55 TB/s; two loads 6.39,
   // four 6.21; 256 threads: 6.42 / 6.13 / 5.91), two for the conversions (bf16 -> fp32 6.44 against 6.23, fp32 -> bf16
   // 6.60 against 6.08)
   int unroll = g_tuning.unroll.load(std::memory_order_relaxed);
-  if (unroll != 1 && unroll != 2 && unroll != 4) unroll = SRC_B != DST_B ? 2 : 1;
+  if (unroll != 1 && unroll != 2 && unroll != 4) unroll = SRC_U != DST_U ? 2 : 1;
   const bool nt = g_tuning.nontemporal.load(std::memory_order_relaxed) != 0;
   auto go = [&](auto u_tag) {
     constexpr int U = decltype(u_tag)::value;
     const int threads = stream_threads();
-    const int64_t span = static_cast<int64_t>(threads) * U;
-    const int64_t want = (n_groups + span - 1) / span;
+    const int64_t span = static_cast<int64_t>(threads) * U * group_units<SRC_U, DST_U>();
+    const int64_t want = (units + span - 1) / span;
     const dim3 grid(static_cast<uint32_t>(std::max<int64_t>(1, std::min(want, kMaxGrid))));
-    if (nt) hipLaunchKernelGGL((linear_kernel<SRC_B, DST_B, U, true, HALF>), grid, dim3(threads), 0, stream, src, dst, n_groups);
-    else hipLaunchKernelGGL((linear_kernel<SRC_B, DST_B, U, false, HALF>), grid, dim3(threads), 0, stream, src, dst, n_groups);
+    if (nt) hipLaunchKernelGGL((linear_kernel<SRC_U, DST_U, U, true, HALF>), grid, dim3(threads), 0, stream, src, dst, units);
+    else hipLaunchKernelGGL((linear_kernel<SRC_U, DST_U, U, false, HALF>), grid, dim3(threads), 0, stream, src, dst, units);
   };
   if (unroll == 1) go(std::integral_constant<int, 1>{});
   else if (unroll == 2) go(std::integral_constant<int, 2>{});
   else go(std::integral_constant<int, 4>{});
   MFSDP_CHECK_LAUNCH("linear_kernel");
   return MFSDP_OK;
-}
-
-// Moves `units` contiguous units: a wide body sized by the pointers' common alignment, then a
-// unit-wide tail for the remainder.
-int linear_dispatch(const char* src, char* dst, int64_t units, int src_unit, int dst_unit, int max_group,
-                    hipStream_t stream, bool half = false) {
-  int g = std::min(pointer_alignment_units(src, src_unit, max_group), pointer_alignment_units(dst, dst_unit, max_group));
-  const int64_t body = units / g;
-  const int64_t tail = units - body * g;
-  const int sb = g * src_unit, db = g * dst_unit;
-  int rc = MFSDP_ERR_UNSUPPORTED;
-#define MFSDP_CASE(S_, D_) \
-  if (sb == S_ && db == D_) rc = launch_linear<S_, D_>(src, dst, body, stream)
-#define MFSDP_CONVERTING(S_, D_) \
-  if (sb == S_ && db == D_) rc = half ? launch_linear<S_, D_, true>(src, dst, body, stream) : launch_linear<S_, D_, false>(src, dst, body, stream)
-  MFSDP_CASE(16, 16); MFSDP_CASE(8, 8); MFSDP_CASE(4, 4); MFSDP_CASE(2, 2); MFSDP_CASE(1, 1);
-  MFSDP_CONVERTING(16, 32); MFSDP_CONVERTING(8, 16); MFSDP_CONVERTING(4, 8); MFSDP_CONVERTING(2, 4);
-  MFSDP_CONVERTING(32, 16); MFSDP_CONVERTING(16, 8); MFSDP_CONVERTING(8, 4); MFSDP_CONVERTING(4, 2);
-#undef MFSDP_CONVERTING
-#undef MFSDP_CASE
-  if (rc == MFSDP_ERR_UNSUPPORTED) return fail(rc, "no kernel for %d -> %d byte groups", sb, db);
-  if (rc != MFSDP_OK || tail == 0) return rc;
-  const char* ts = src + body * sb;
-  char* td = dst + body * db;
-  if (src_unit == 1) return launch_linear<1, 1>(ts, td, tail, stream);
-  if (src_unit == 2) return half ? launch_linear<2, 4, true>(ts, td, tail, stream) : launch_linear<2, 4, false>(ts, td, tail, stream);
-  return half ? launch_linear<4, 2, true>(ts, td, tail, stream) : launch_linear<4, 2, false>(ts, td, tail, stream);
 }
 
 }  // namespace
@@ -880,7 +845,7 @@ extern "C" int mfsdp_copy_range(const void* in, int64_t in_numel, void* out, int
   if (out_numel == 0) return MFSDP_OK;
   if (in == nullptr || out == nullptr) return fail(MFSDP_ERR_INVALID, "in or out is null");
   const char* src = static_cast<const char*>(in) + input_offset * elem_bytes;
-  return linear_dispatch(src, static_cast<char*>(out), out_numel * elem_bytes, 1, 1, 16, as_stream(stream));
+  return launch_linear<1, 1>(src, static_cast<char*>(out), out_numel * elem_bytes, as_stream(stream));
 }
 
 extern "C" int mfsdp_cast(const void* src, void* dst, int64_t numel, int convert, void* stream) {
@@ -890,8 +855,11 @@ extern "C" int mfsdp_cast(const void* src, void* dst, int64_t numel, int convert
   if (numel == 0) return MFSDP_OK;
   if (src == nullptr || dst == nullptr) return fail(MFSDP_ERR_INVALID, "src or dst is null");
   const bool widen = convert == MFSDP_CONVERT_BF16_TO_F32 || convert == MFSDP_CONVERT_F16_TO_F32;
-  return linear_dispatch(static_cast<const char*>(src), static_cast<char*>(dst), numel, widen ? 2 : 4, widen ? 4 : 2,
-                         Tuning::convert_group, as_stream(stream), is_half_conversion(convert));
+  const char* in = static_cast<const char*>(src);
+  char* out = static_cast<char*>(dst);
+  hipStream_t s = as_stream(stream);
+  if (widen) return is_half_conversion(convert) ? launch_linear<2, 4, true>(in, out, numel, s) : launch_linear<2, 4, false>(in, out, numel, s);
+  return is_half_conversion(convert) ? launch_linear<4, 2, true>(in, out, numel, s) : launch_linear<4, 2, false>(in, out, numel, s);
 }
 
 // ---- HBM probes: what the part sustains for pure reads and pure writes, measured with this library's own launch shape
@@ -958,7 +926,7 @@ __device__ __forceinline__ uint32_t add_word(uint32_t a, uint32_t b) {
   }
 }
 
-// n_vec 16-byte groups, then `tail` single elements starting at element `tail_first`
+// n_vec 16-byte groups (aligned to elements only), then `tail` single elements starting at element `tail_first`
 template <int FMT>
 __global__ void __launch_bounds__(kBlockThreads)
 accumulate_kernel(char* __restrict__ dst, const char* __restrict__ src, int64_t n_vec, int64_t tail_first, int64_t tail) {
@@ -989,9 +957,8 @@ extern "C" int mfsdp_accumulate(void* dst, const void* src, int64_t numel, int d
   if (numel == 0) return MFSDP_OK;
   if (dst == nullptr || src == nullptr) return fail(MFSDP_ERR_INVALID, "dst or src is null");
   const int elem = dtype == MFSDP_F32 ? 4 : 2;
-  const bool aligned = (reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) % 16 == 0;
   const int64_t per_vec = 16 / elem;
-  const int64_t n_vec = aligned ? numel / per_vec : 0;
+  const int64_t n_vec = numel / per_vec;
   const int64_t tail_first = n_vec * per_vec, tail = numel - tail_first;
   const int64_t work = std::max(n_vec, tail);
   const int threads = stream_threads();

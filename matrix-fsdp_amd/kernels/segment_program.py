@@ -96,8 +96,8 @@ def merge_runs(runs: np.ndarray) -> np.ndarray:
 
 class SegmentProgram:
     """Owns one ``mfsdp_segment_program``.  ``run`` is one kernel launch on
-    the current HIP stream (one per block of 128 sources and per vector width
-    in use); it neither allocates nor synchronises."""
+    the current HIP stream (one per block of 128 sources); it neither allocates
+    nor synchronises."""
 
     def __init__(
         self,

@@ -9,6 +9,7 @@ from matrix_fsdp_amd import LayoutSegment, ShardPlan
 from matrix_fsdp_amd.core.plans import block_grid_plan, contiguous_even_plan, fsdp2_chunk_plan
 from matrix_fsdp_amd.kernels import native
 from matrix_fsdp_amd.kernels.segment_program import (
+    RUN_DTYPE,
     SegmentProgram,
     compact_owner_program,
     grad_fill_program,
@@ -485,3 +486,38 @@ def test_uncached_segment_copy_entry_point():
     torch.cuda.synchronize()
     assert out.cpu().tolist() == [4, 5, 6, 7, 8, 9, 0, 0, 0, 1, 2, 3]
     assert _lib.lib().mfsdp_copy_rank_segments_to_full(local.data_ptr(), 10, out.data_ptr(), 12, arr([9]), arr([0]), arr([4]), 1, 4, None) != 0
+
+
+@pytest.mark.parametrize("src_dtype, dst_dtype", [(torch.uint8, torch.uint8), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)], ids=str)
+@pytest.mark.parametrize("row_len", [1, 2, 3, 4, 5, 7, 15, 16, 17, 31, 33, 63, 127, 129, 1023, 1025, 2047, 2049, 4095, 4097, 8205])
+def test_rows_of_any_length_at_any_offset(row_len, src_dtype, dst_dtype):
+    """Rows shorter than a vector group, with and without a remainder, one to several tiles long, at odd offsets and odd
+    pitches on both sides (many short rows of a run, single rows, and zero fill): every element exactly once, nothing
+    beside the rows."""
+    rows, pitch_s, pitch_d, first_s, first_d = 37, row_len + 3, row_len + 5, 3, 7
+    n_src, n_dst = first_s + rows * pitch_s + 11, first_d + (rows + 2) * pitch_d + 13
+    gen = torch.Generator().manual_seed(row_len)
+    src = torch.randint(0, 255, (n_src,), generator=gen).to(src_dtype)
+    runs = np.zeros(3, dtype=RUN_DTYPE)
+    runs[0] = (first_s, first_d, row_len, rows, pitch_s, pitch_d, 0, 0)
+    runs[1] = (first_s + 1, first_d + rows * pitch_d, row_len, 1, 0, 0, 0, 0)
+    runs[2] = (0, first_d + (rows + 1) * pitch_d, row_len, 1, 0, 0, -1, 0)
+    program = SegmentProgram(runs, (n_src,), n_dst, src_dtype=src_dtype, dst_dtype=dst_dtype, device=DEV, merge=False)
+    want = torch.full((n_dst,), 77, dtype=dst_dtype)
+    for r in range(rows):
+        want[first_d + r * pitch_d : first_d + r * pitch_d + row_len] = src[first_s + r * pitch_s : first_s + r * pitch_s + row_len].to(dst_dtype)
+    want[first_d + rows * pitch_d : first_d + rows * pitch_d + row_len] = src[first_s + 1 : first_s + 1 + row_len].to(dst_dtype)
+    want[first_d + (rows + 1) * pitch_d : first_d + (rows + 1) * pitch_d + row_len] = 0
+    for shift in (0, 1):
+        dst = torch.full((n_dst + shift,), 77, dtype=dst_dtype, device=DEV)[shift:]
+        held = torch.zeros(n_src + shift, dtype=src_dtype, device=DEV)[shift:]
+        held.copy_(src)
+        program.run((held,), dst)
+        assert torch.equal(dst.cpu(), want)
+        # one contiguous span through the range copy and the cast
+        span = torch.full((row_len + 2 + shift,), 77, dtype=dst_dtype, device=DEV)[shift:]
+        if src_dtype == dst_dtype:
+            native.copy_range(held, span[1 : 1 + row_len], 5)
+        else:
+            native.cast(held[5 : 5 + row_len], dst_dtype, out=span[1 : 1 + row_len])
+        assert torch.equal(span[1 : 1 + row_len].cpu(), src[5 : 5 + row_len].to(dst_dtype)) and float(span[0]) == 77 and float(span[-1]) == 77
