@@ -307,6 +307,24 @@ int mfsdp_adamw_step_ex(float* param, const void* grad, int grad_dtype, float* e
                         float* max_exp_avg_sq, int64_t numel, int64_t step, double lr, double beta1, double beta2,
                         double eps, double weight_decay, int maximize, void* stream);
 
+/*
+ * The same update of n spans that lie anywhere in memory, up to 56 of them per launch (spans that follow each other with
+ * different gradient types, with and without amsgrad, or with overlapping parameters take launches of their own, in the
+ * order given).  A null max_exp_avg_sq means no amsgrad.  Nothing is enqueued if any span is refused.
+ */
+typedef struct {
+  float* param;
+  const void* grad;
+  float* exp_avg;
+  float* exp_avg_sq;
+  float* max_exp_avg_sq;
+  int64_t numel;
+  int64_t step;
+  int32_t grad_dtype;
+} mfsdp_adamw_span;
+int mfsdp_adamw_step_many(int64_t n, const mfsdp_adamw_span* spans, double lr, double beta1, double beta2, double eps,
+                          double weight_decay, int maximize, void* stream);
+
 /* ------------------------------------------------------------------ measurement and experiments
  *
  * Nothing below is part of the drop-in surface: the reference has no counterpart for any of it and a binding of the

@@ -56,6 +56,21 @@ class MuonJob(Structure):
     ]
 
 
+class AdamWSpan(Structure):
+    """``mfsdp_adamw_span``."""
+
+    _fields_ = [
+        ("param", c_void_p),
+        ("grad", c_void_p),
+        ("exp_avg", c_void_p),
+        ("exp_avg_sq", c_void_p),
+        ("max_exp_avg_sq", c_void_p),
+        ("numel", c_int64),
+        ("step", c_int64),
+        ("grad_dtype", c_int32),
+    ]
+
+
 # name -> (restype, argtypes); every symbol include/mfsdp_hip.h declares
 SIGNATURES = {
     "mfsdp_last_error": (c_char_p, []),
@@ -115,6 +130,7 @@ SIGNATURES = {
         c_int,
         [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int64, c_int64, c_double, c_double, c_double, c_double, c_double, c_void_p],
     ),
+    "mfsdp_adamw_step_many": (c_int, [c_int64, POINTER(AdamWSpan), c_double, c_double, c_double, c_double, c_double, c_int, c_void_p]),
     "mfsdp_adamw_step_ex": (
         c_int,
         [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_double, c_double, c_double, c_double, c_double, c_int, c_void_p],

@@ -1,12 +1,12 @@
-"""``FusedAdamW``: AdamW on the HIP kernel, one launch per contiguous run of parameters.
+"""``FusedAdamW``: AdamW on the HIP kernel, one launch for the parameters of a group.
 
 Hyper-parameters, parameter-group keys and state keys (``step``, ``exp_avg``,
 ``exp_avg_sq``) are those of ``torch.optim.AdamW`` (``amsgrad`` and ``maximize`` included), the optimizer the reference
 builds for everything Muon does not take (matrix_fsdp/optim/wrapper.py:431-439);
 the arithmetic is the single-tensor path of torch/optim/adam.py:347-547.  When
 the parameters are views of one flat shard and their grads views of one local
-grad shard, neighbouring parameters are merged and the run is updated by a
-single launch: the moments this optimizer creates for such a run are laid out
+grad shard, neighbouring parameters are merged and the run is updated as one
+span: the moments this optimizer creates for such a run are laid out
 back to back as well (``initialize_flat_adamw_state`` does the same for a whole
 flat buffer up front and keeps the buffers addressable).
 """
@@ -39,7 +39,7 @@ class FusedAdamW(torch.optim.AdamW):
 
     def _init_states(self, params: list[Tensor], amsgrad: bool) -> None:
         """First step: parameters that follow each other in memory (views of one local shard) get moments that
-        follow each other too, so that the run can be updated by one launch.  Every parameter still has its own
+        follow each other too, so that the run can be updated as one span.  Every parameter still has its own
         ``exp_avg`` / ``exp_avg_sq`` tensors of its own shape."""
         fresh = sorted((p for p in params if len(self.state[p]) == 0), key=lambda p: p.data_ptr())
         names = ("exp_avg", "exp_avg_sq") + (("max_exp_avg_sq",) if amsgrad else ())
@@ -75,32 +75,37 @@ class FusedAdamW(torch.optim.AdamW):
                 if p.dtype != torch.float32:
                     raise RuntimeError(f"FusedAdamW updates float32 parameters, got {p.dtype}")
             self._init_states(active, amsgrad)
-            for p in active:
-                state = self.state[p]
+            states = [self.state[p] for p in active]
+            if states:
+                torch._foreach_add_([state["step"] for state in states], 1)
+            for p, state in zip(active, states):
                 if amsgrad and "max_exp_avg_sq" not in state:  # amsgrad switched on after the first step
                     state["max_exp_avg_sq"] = torch.zeros_like(p, memory_format=torch.preserve_format)
-                state["step"] += 1
                 tensors = [p.data, p.grad.contiguous(), state["exp_avg"], state["exp_avg_sq"]]
                 if amsgrad:
                     tensors.append(state["max_exp_avg_sq"])
                 entries.append((*tensors, int(state["step"].item())))
+            # the runs lie apart in memory and share one launch: for 15 parameters from 2048 to 3 M elements a launch each
+            # was 278 us of host work around 30 us of memory traffic
+            batch = F.AdamWBatch()
             for *tensors, step in _merge_contiguous(entries):
                 F.adamw_step(
                     *tensors[:4], step,
                     lr=group["lr"], betas=group["betas"], eps=group["eps"], weight_decay=group["weight_decay"],
-                    max_exp_avg_sq=tensors[4] if amsgrad else None, maximize=bool(group.get("maximize", False)),
+                    max_exp_avg_sq=tensors[4] if amsgrad else None, maximize=bool(group.get("maximize", False)), batch=batch,
                 )
+            batch.launch()
         return loss
 
 
 def _follows(prev: Tensor, nxt: Tensor) -> bool:
     return (
-        prev.dtype == nxt.dtype
+        prev.data_ptr() + prev.numel() * prev.element_size() == nxt.data_ptr()  # first: it settles most pairs
+        and prev.dtype == nxt.dtype
         and prev.device == nxt.device
         and prev.is_contiguous()
         and nxt.is_contiguous()
         and prev.untyped_storage().data_ptr() == nxt.untyped_storage().data_ptr()
-        and prev.data_ptr() + prev.numel() * prev.element_size() == nxt.data_ptr()
     )
 
 
@@ -126,5 +131,5 @@ def _merge_contiguous(entries):
 def _flat_span(first: Tensor, numel: int) -> Tensor:
     """1-D view of ``numel`` elements starting at ``first``'s first element."""
     if first.numel() == numel:
-        return first.reshape(-1)
+        return first if first.is_contiguous() else first.reshape(-1)
     return torch.as_strided(first, (numel,), (1,), first.storage_offset())

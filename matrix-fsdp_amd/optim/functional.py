@@ -209,6 +209,29 @@ def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, side_by_side
             _lib.check(lib.mfsdp_muon_step_many(n, (_lib.MuonJob * n)(*fields), dtype, momentum, nesterov, a, b, c, ns_steps, eps, ws.data_ptr(), ws.numel(), stream))
 
 
+class AdamWBatch:
+    """Spans that ``adamw_step(..., batch=...)`` has checked, updated by one launch per device (``mfsdp_adamw_step_many``)
+    when ``launch`` is called.  The tensors are held until then."""
+
+    def __init__(self) -> None:
+        self._spans: dict[tuple, list[tuple]] = {}
+        self._tensors: list[tuple] = []
+
+    def add(self, device: torch.device, hyper: tuple, span: tuple, tensors: tuple) -> None:
+        self._spans.setdefault((device, *hyper), []).append(span)
+        self._tensors.append(tensors)
+
+    def launch(self) -> None:
+        spans_by_key, self._spans = self._spans, {}
+        try:
+            for (device, *hyper), spans in spans_by_key.items():
+                with torch.cuda.device(device):
+                    stream = torch.cuda.current_stream(device).cuda_stream
+                    _lib.check(_lib.lib().mfsdp_adamw_step_many(len(spans), (_lib.AdamWSpan * len(spans))(*spans), *hyper, stream))
+        finally:
+            self._tensors.clear()
+
+
 def adamw_step(
     param: torch.Tensor,
     grad: torch.Tensor,
@@ -222,26 +245,32 @@ def adamw_step(
     weight_decay: float = 1e-2,
     max_exp_avg_sq: torch.Tensor | None = None,
     maximize: bool = False,
+    batch: AdamWBatch | None = None,
 ) -> None:
     """Fused AdamW over flat fp32 tensors; ``step`` is the 1-based count after
     this update (torch/optim/adam.py:347-547).  ``max_exp_avg_sq`` turns on
-    amsgrad, ``maximize`` negates the gradient."""
-    state = [(param, "param"), (exp_avg, "exp_avg"), (exp_avg_sq, "exp_avg_sq")]
+    amsgrad, ``maximize`` negates the gradient.  With ``batch`` the checked span
+    is left to ``batch.launch()``."""
+    numel = param.numel()
+    state = ((param, "param"), (exp_avg, "exp_avg"), (exp_avg_sq, "exp_avg_sq"))
     if max_exp_avg_sq is not None:
-        state.append((max_exp_avg_sq, "max_exp_avg_sq"))
+        state += ((max_exp_avg_sq, "max_exp_avg_sq"),)
     for t, what in state:
         if not t.is_cuda or not t.is_contiguous() or t.dtype != torch.float32:
             raise RuntimeError(f"{what} must be a contiguous float32 CUDA tensor")
-        if t.numel() != param.numel():
-            raise RuntimeError(f"{what} has {t.numel()} elements, param has {param.numel()}")
-    if not grad.is_cuda or not grad.is_contiguous() or grad.dtype not in _DTYPE_CODES or grad.numel() != param.numel():
+        if t.numel() != numel:
+            raise RuntimeError(f"{what} has {t.numel()} elements, param has {numel}")
+    if not grad.is_cuda or not grad.is_contiguous() or grad.dtype not in _DTYPE_CODES or grad.numel() != numel:
         raise RuntimeError("grad must be a contiguous float32 or bfloat16 CUDA tensor of the param's size")
-    stream = torch.cuda.current_stream(param.device).cuda_stream
-    with torch.cuda.device(param.device):
-        _lib.check(
-            _lib.lib().mfsdp_adamw_step_ex(
-                param.data_ptr(), grad.data_ptr(), _DTYPE_CODES[grad.dtype], exp_avg.data_ptr(), exp_avg_sq.data_ptr(),
-                None if max_exp_avg_sq is None else max_exp_avg_sq.data_ptr(),
-                param.numel(), int(step), lr, betas[0], betas[1], eps, weight_decay, int(bool(maximize)), stream,
-            )
-        )
+    span = (
+        param.data_ptr(), grad.data_ptr(), exp_avg.data_ptr(), exp_avg_sq.data_ptr(), None if max_exp_avg_sq is None else max_exp_avg_sq.data_ptr(),
+        numel, int(step), _DTYPE_CODES[grad.dtype],
+    )
+    hyper = (lr, betas[0], betas[1], eps, weight_decay, int(bool(maximize)))
+    tensors = (param, grad, exp_avg, exp_avg_sq, max_exp_avg_sq)
+    if batch is not None:
+        batch.add(param.device, hyper, span, tensors)
+        return
+    batch = AdamWBatch()
+    batch.add(param.device, hyper, span, tensors)
+    batch.launch()

@@ -382,3 +382,45 @@ def test_muon_group_with_cut_k_walks():
         p_ref, b_ref = params[i].clone(), torch.zeros(sh)
         O.muon_step(p_ref, grads[i], b_ref, **kw)
         assert rel_fro(dev_p[i].cpu() - params[i], p_ref - params[i]) < MUON_TOL, sh
+
+
+@pytest.mark.parametrize("amsgrad", [False, True])
+@pytest.mark.parametrize("count", [1, 4, 5, 56, 57, 130])
+def test_adamw_batch_has_the_bits_of_single_spans(count, amsgrad):
+    """Spans of 0 to a few thousand elements at any element offset, with step counts and gradient types of their own, in
+    launches of up to 56: the bits of one call per span, and nothing outside the spans is touched."""
+    edges = [0, 1, 3, 4, 5, 255, 256, 257, 511, 512, 513, 1023, 1025, 4099]
+    sizes = [edges[(7 * i + count) % len(edges)] for i in range(count)]
+    starts = [sum(sizes[:i]) + i + 1 for i in range(count)]  # a gap of one element before every span
+    total = sum(sizes) + count + 8
+    flats = [make((total,), 70 + k, 0.02).to(DEV) for k in range(5)]
+    flats[3].abs_()
+    flats[4].abs_()
+    expect = [f.clone() for f in flats]
+
+    def run(tensors, batch):
+        p, g, m, v, x = tensors
+        for i, (a, n) in enumerate(zip(starts, sizes)):
+            cut = slice(a, a + n)
+            grad = g[cut].bfloat16() if i % 5 == 3 else g[cut]
+            F.adamw_step(p[cut], grad, m[cut], v[cut], 1 + i % 3, lr=1e-3, betas=(0.9, 0.95), eps=1e-8, weight_decay=0.1,
+                         max_exp_avg_sq=x[cut] if amsgrad else None, batch=batch)
+
+    run(expect, None)
+    batch = F.AdamWBatch()
+    run(flats, batch)
+    batch.launch()
+    for have, want in zip(flats, expect):
+        assert torch.equal(have, want)
+    batch.launch()  # nothing is left in it
+    assert torch.equal(flats[0], expect[0])
+    # overlapping parameters keep their order
+    p, q = flats[0].clone(), flats[0].clone()
+    g, m, v = flats[1], torch.zeros(total, device=DEV), torch.zeros(total, device=DEV)
+    for target, b in ((p, None), (q, F.AdamWBatch())):
+        first, second = (torch.zeros(4, device=DEV) for _ in range(2))
+        F.adamw_step(target[0:4], g[0:4], first, second, 1, lr=0.1, batch=b)
+        F.adamw_step(target[2:6], g[2:6], m[2:6].clone(), v[2:6].clone(), 1, lr=0.1, batch=b)
+        if b is not None:
+            b.launch()
+    assert torch.equal(p, q)
