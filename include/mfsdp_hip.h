@@ -364,8 +364,8 @@ void mfsdp_set_copy_tuning(int blocks_per_cu, int nontemporal, int unroll, int b
 
 /* Kernel selection for experiments (values <= 0 keep the current setting):
  * tile variant of the general and of the symmetric Newton-Schulz products (1: 256x256 tile / 8 waves / one
- * workgroup per CU, 2: 128x128 tile / 4 waves / two per CU; for the symmetric products also 3, the default:
- * whichever of the two fills the CUs better for the size at hand), the tile rows the general products walk together
+ * workgroup per CU, 2: 128x128 tile / 4 waves / two per CU, 4: 64x64 tile / K cut among 8 waves; 3, the default:
+ * whichever is expected to be fastest for the launch at hand), the tile rows the general products walk together
  * (default 4), K-splitting of the last partial round of tiles on (1) / off (2), and its cap. */
 void mfsdp_set_muon_tuning(int general_variant, int symmetric_variant, int group_m, int split_remainder, int max_splits);
 

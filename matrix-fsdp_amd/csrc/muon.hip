@@ -10,7 +10,7 @@
 //
 // A step's matrices do not depend on each other: up to 32 of them go through every stage as ONE launch (momentum, norm,
 // scale + transpose, three products per iteration), so that small matrices fill the machine together and a step costs
-// 3 + 3 x steps launches instead of that many per matrix.
+// 2 or 3 + 3 x steps launches instead of that many per matrix.
 #include "mfsdp_common.h"
 #include "muon_elementwise.h"
 #include "muon_gemm.h"
@@ -113,8 +113,7 @@ void finish_group(Group* g, char* shared) {
 // at least one step the last product writes the parameters themselves; otherwise O is left in X[steps & 1] (wide) or
 // XT[steps & 1] (tall).
 int run_newton_schulz(const Group& group, float a, float b, float c, int steps, float eps, bool shared, int update_dtype, hipStream_t stream) {
-  if (int rc = muon_norm(group.elementwise, eps, stream)) return rc;
-  if (int rc = muon_scale_transpose(group.elementwise, stream)) return rc;
+  if (int rc = muon_scale_transpose(group.elementwise, eps, stream)) return rc;
   GemmGroup g;
   g.n = group.n;
   GemmPlan gram, poly, update;  // made in the first iteration

@@ -37,11 +37,8 @@ int muon_momentum_partials(int64_t numel);
 // (without momentum: xraw <- bf16(g)).
 int muon_momentum(const MuonMatrices& g, int dtype, double momentum, int nesterov, bool with_momentum, hipStream_t stream);
 
-// norms[i] = max(bf16(sqrt(sum of matrix i's partials)), bf16(eps)).
-int muon_norm(const MuonMatrices& g, float eps, hipStream_t stream);
-
-// same[r][c] = bf16(x[r][c] / norm), trans[c][r] = same[r][c].
-int muon_scale_transpose(const MuonMatrices& g, hipStream_t stream);
+// same[r][c] = bf16(x[r][c] / norm), trans[c][r] = same[r][c], with norm = max(bf16(sqrt(sum of the partials)), bf16(eps)).
+int muon_scale_transpose(const MuonMatrices& g, float eps, hipStream_t stream);
 
 // p <- p*decay - adj_lr * O (torch/optim/_muon.py:313-315).
 int muon_apply(void* param, int dtype, const void* ortho, int rows, int cols, int ldo, float decay, float neg_lr,

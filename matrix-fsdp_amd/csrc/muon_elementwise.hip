@@ -211,6 +211,13 @@ momentum_kernel(GroupArgs args, float momentum, float one_minus_momentum, int ne
 }
 
 constexpr int kNormThreads = 1024;
+constexpr int kFoldPartials = 1024;
+
+__device__ __forceinline__ float norm_of(double sum, float eps) {
+  const float norm = bf16_to_f32(f32_to_bf16(sqrtf(static_cast<float>(sum))));
+  const float floor_ = bf16_to_f32(f32_to_bf16(eps));
+  return norm > floor_ ? norm : floor_;
+}
 
 // norms[i] = max(bf16(sqrt(sum partials)), bf16(eps)); one workgroup per matrix, the sum in double and in a fixed order
 __global__ void __launch_bounds__(kNormThreads)
@@ -241,11 +248,7 @@ norm_kernel(MuonMatrices args, float eps) {
     if (static_cast<int>(threadIdx.x) < off) lds[threadIdx.x] += lds[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    const float norm = bf16_to_f32(f32_to_bf16(sqrtf(static_cast<float>(lds[0]))));
-    const float floor_ = bf16_to_f32(f32_to_bf16(eps));
-    args.norms[blockIdx.x] = norm > floor_ ? norm : floor_;
-  }
+  if (threadIdx.x == 0) args.norms[blockIdx.x] = norm_of(lds[0], eps);
 }
 
 // 64 x 64 tile of the outputs per block:
@@ -253,14 +256,38 @@ norm_kernel(MuonMatrices args, float eps) {
 //   trans[c][r]  = same[r][c]             (ld_trans)
 // with x = 0 outside rows x cols.  Every thread handles groups of four consecutive elements: 64-bit stores on
 // both outputs (their rows are 256-element aligned), 64-bit loads that need element alignment only.
+// FOLD_NORM: every workgroup sums its matrix's partials itself (all of them in the same order) instead of reading the norm
+// that a launch of its own has left: for matrices of up to kFoldPartials partials, 4 KiB that stay in L2, the launch saved
+// is worth more (a launch in this chain takes 5-7 us whatever it does; the sum adds 1-2 us to this one).
+template <bool FOLD_NORM>
 __global__ void __launch_bounds__(kThreads)
-scale_transpose_kernel(GroupArgs args) {
+scale_transpose_kernel(GroupArgs args, float eps) {
   __shared__ uint16_t tile[64][68];
   const int index = matrix_of(args, blockIdx.x);
   const MuonMatrix& m = args.g.m[index];
   const int block = blockIdx.x - args.begin[index];
   const int rows = m.rows, cols = m.cols, tile_cols = (cols + 63) / 64;
-  const float norm = args.g.norms[index];
+  float norm;
+  if constexpr (FOLD_NORM) {
+    static_assert(kFoldPartials % kThreads == 0);
+    __shared__ double wave_sums[kThreads / 64];
+    float part[kFoldPartials / kThreads];
+#pragma unroll
+    for (int u = 0; u < kFoldPartials / kThreads; ++u) {
+      const int i = u * kThreads + static_cast<int>(threadIdx.x);
+      part[u] = i < m.n_partials ? m.partials[i] : 0.0f;
+    }
+    double s = 0.0;
+#pragma unroll
+    for (int u = 0; u < kFoldPartials / kThreads; ++u) s += static_cast<double>(part[u]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (threadIdx.x % 64 == 0) wave_sums[threadIdx.x / 64] = s;
+    __syncthreads();
+    norm = norm_of((wave_sums[0] + wave_sums[1]) + (wave_sums[2] + wave_sums[3]), eps);
+  } else {
+    norm = args.g.norms[index];
+  }
   const uint16_t* __restrict__ xraw = m.xraw;
   uint16_t* __restrict__ same = m.same;
   uint16_t* __restrict__ trans = m.trans;
@@ -383,16 +410,18 @@ int muon_momentum(const MuonMatrices& g, int dtype, double momentum, int nestero
   return MFSDP_OK;
 }
 
-int muon_norm(const MuonMatrices& g, float eps, hipStream_t stream) {
-  hipLaunchKernelGGL(norm_kernel, dim3(g.n), dim3(kNormThreads), 0, stream, g, eps);
-  MFSDP_CHECK_LAUNCH("norm_kernel");
-  return MFSDP_OK;
-}
-
-int muon_scale_transpose(const MuonMatrices& g, hipStream_t stream) {
+int muon_scale_transpose(const MuonMatrices& g, float eps, hipStream_t stream) {
   GroupArgs args;
   const dim3 grid(fill_group(&args, g, [](const MuonMatrix& m) { return ((m.rows + 63) / 64) * ((m.cols + 63) / 64); }));
-  hipLaunchKernelGGL(scale_transpose_kernel, grid, dim3(kThreads), 0, stream, args);
+  int most = 0;
+  for (int i = 0; i < g.n; ++i) most = std::max(most, g.m[i].n_partials);
+  if (most <= kFoldPartials) {
+    hipLaunchKernelGGL(scale_transpose_kernel<true>, grid, dim3(kThreads), 0, stream, args, eps);
+  } else {
+    hipLaunchKernelGGL(norm_kernel, dim3(g.n), dim3(kNormThreads), 0, stream, g, eps);
+    MFSDP_CHECK_LAUNCH("norm_kernel");
+    hipLaunchKernelGGL(scale_transpose_kernel<false>, grid, dim3(kThreads), 0, stream, args, eps);
+  }
   MFSDP_CHECK_LAUNCH("scale_transpose_kernel");
   return MFSDP_OK;
 }

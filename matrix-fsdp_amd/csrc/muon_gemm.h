@@ -60,7 +60,7 @@ struct GemmScratch {
 constexpr int64_t kGemmPartialsBytes = 64ll << 20;
 
 // Tile variants: 1 = 256 x 256 tile / 8 waves / one workgroup per CU, 2 = 128 x 128 tile / 4 waves / two per CU,
-// 3 = whichever is expected to be faster for the launch at hand.
+// 4 = 64 x 64 tile / K cut among 8 waves, 3 = whichever is expected to be faster for the launch at hand.
 struct GemmTuning {
   int general_variant = 3;
   int symmetric_variant = 3;

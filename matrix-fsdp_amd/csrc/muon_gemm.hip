@@ -691,6 +691,168 @@ splitk_fixup_kernel(LaunchArgs args) {
   }
 }
 
+// ---- 64 x 64 tiles for launches that leave most CUs idle otherwise.
+// A chain of products of matrices of a few hundred rows is bound by the latency of each launch: with 128 x 128 tiles a
+// handful of CUs walk all of K slab by slab, a load latency and a barrier per slab.  Here the eight waves of a workgroup
+// cut K among themselves: each computes the whole 64 x 64 tile over its share, straight from global memory to registers
+// (the loads of four k32 steps are in flight, no barrier in the walk), and the partial tiles are summed through LDS in a
+// fixed order.  A tile moves four times the operand bytes of a 256 x 256 one per flop, so this pays only while the launch
+// is latency bound.  Whole Muon step, 128 x 128 tiles -> these, us: 512x256 with 256x512 162 -> 124, 512x512 171 -> 142,
+// two of 512x1536 220 -> 201, 1024x1024 251 -> 204, four of 64x256 117 -> 91.
+template <int N>
+struct SmallArgs {
+  int begin[N];  // first workgroup of a problem; entries past n are the end
+  int n;
+  int symmetric;
+  int group_m;
+  int update_dtype;
+  float alpha, beta;
+  GemmProblem problem[N];
+};
+static_assert(sizeof(SmallArgs<kMaxGemmGroup>) <= 4096, "kernel arguments are limited to 4 KiB");
+
+constexpr int kSmallTile = 64;
+constexpr int kSmallWaves = 8;
+constexpr int kSmallThreads = kSmallWaves * 64;
+constexpr int kSmallPitch = kSmallTile + 4;  // floats per row of a partial tile in LDS: skews the banks of a lane's four rows
+
+template <int N>
+__global__ void __launch_bounds__(kSmallThreads, 2)
+gemm_small_kernel(SmallArgs<N> args) {
+  constexpr int kTiles = kSmallTile / 16;
+  __shared__ __attribute__((aligned(16))) float sums[4 * kSmallTile * kSmallPitch];
+  int problem = 0;
+#pragma unroll
+  for (int i = 1; i < N; ++i) problem += static_cast<int>(blockIdx.x) >= args.begin[i] ? 1 : 0;
+  const GemmProblem a = args.problem[problem];  // a copy: all of its fields in one go instead of a scalar load at each use
+  int tm, tn;
+  tile_coords(args.group_m, blockIdx.x - args.begin[problem], (a.M + kSmallTile - 1) / kSmallTile, (a.N + kSmallTile - 1) / kSmallTile,
+              args.symmetric != 0, &tm, &tn);
+  const int row0 = tm * kSmallTile, col0 = tn * kSmallTile;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+
+  // D values of the epilogue (thread t: eight columns of row t / 8), fetched under the products
+  const int orow = tid / 8, ocol = (tid % 8) * 8;
+  u32x4 d = {0u, 0u, 0u, 0u};
+  if (a.D != nullptr) d = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.D) + static_cast<int64_t>(row0 + orow) * a.ldd + col0 + ocol);
+
+  // 16x16x32 MFMA operands: lane l supplies row l % 16 of a 16-row block and the 8 k values of chunk l / 16
+  const int steps = a.K / 32;
+  const int first = steps * wave / kSmallWaves, last = steps * (wave + 1) / kSmallWaves;
+  const __bf16* __restrict__ P = static_cast<const __bf16*>(a.P) + static_cast<int64_t>(row0 + (lane & 15)) * a.ldp + (lane >> 4) * 8;
+  const __bf16* __restrict__ Q = static_cast<const __bf16*>(a.Q) + static_cast<int64_t>(col0 + (lane & 15)) * a.ldq + (lane >> 4) * 8;
+  const int64_t p_block = static_cast<int64_t>(16) * a.ldp, q_block = static_cast<int64_t>(16) * a.ldq;
+  f32x4 acc[kTiles][kTiles];
+#pragma unroll
+  for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+    for (int j = 0; j < kTiles; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // kSteps k32 steps: every load is issued before the first product (left to itself the compiler sinks them to their uses
+  // and waits out a memory latency for each)
+  auto batch = [&](int step, auto steps_tag) {
+    constexpr int kSteps = decltype(steps_tag)::value;
+    bf16x8 fp[kSteps][kTiles], fq[kSteps][kTiles];
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) {
+#pragma unroll
+      for (int i = 0; i < kTiles; ++i) fp[s][i] = *reinterpret_cast<const bf16x8*>(P + i * p_block + (step + s) * 32);
+#pragma unroll
+      for (int j = 0; j < kTiles; ++j) fq[s][j] = *reinterpret_cast<const bf16x8*>(Q + j * q_block + (step + s) * 32);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+      for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+        for (int j = 0; j < kTiles; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp[s][i], fq[s][j], acc[i][j], 0, 0, 0);
+  };
+  int step = first;
+  for (; step + 4 <= last; step += 4) batch(step, std::integral_constant<int, 4>{});
+  switch (last - step) {
+    case 3: batch(step, std::integral_constant<int, 3>{}); break;
+    case 2: batch(step, std::integral_constant<int, 2>{}); break;
+    case 1: batch(step, std::integral_constant<int, 1>{}); break;
+    default: break;
+  }
+
+  // ---- partial tiles: waves 4 .. 7 hand theirs to waves 0 .. 3 lane by lane, then every thread sums four
+  f32x4* raw = reinterpret_cast<f32x4*>(sums);
+  if (wave >= 4) {
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+      for (int j = 0; j < kTiles; ++j) raw[((wave - 4) * kTiles * kTiles + i * kTiles + j) * 64 + lane] = acc[i][j];
+  }
+  __syncthreads();
+  if (wave < 4) {
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+      for (int j = 0; j < kTiles; ++j) acc[i][j] += raw[(wave * kTiles * kTiles + i * kTiles + j) * 64 + lane];
+  }
+  __syncthreads();
+  if (wave < 4) {
+    // accumulator register r of lane l holds C[4*(l/16) + r][l%16] of its 16x16 tile
+    float* mine = sums + (wave * kSmallTile + (lane >> 4) * 4) * kSmallPitch + (lane & 15);
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i)
+#pragma unroll
+      for (int j = 0; j < kTiles; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) mine[(i * 16 + r) * kSmallPitch + j * 16] = acc[i][j][r];
+  }
+  __syncthreads();
+  f32x4 lo = {0.0f, 0.0f, 0.0f, 0.0f}, hi = lo;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const f32x4* from = reinterpret_cast<const f32x4*>(sums + (w * kSmallTile + orow) * kSmallPitch + ocol);
+    lo += from[0];
+    hi += from[1];
+  }
+  u32x4 packed;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float v0 = args.alpha * (e < 2 ? lo[2 * e] : hi[2 * e - 4]), v1 = args.alpha * (e < 2 ? lo[2 * e + 1] : hi[2 * e - 3]);
+    if (a.D != nullptr) {
+      v0 += args.beta * __uint_as_float(d[e] << 16);
+      v1 += args.beta * __uint_as_float(d[e] & 0xffff0000u);
+    }
+    packed[e] = pack_bf16x2(v0, v1);
+  }
+
+  // ---- epilogue, as in gemm_nt_kernel: C, the transposed / mirrored tile, or the parameter
+  uint16_t* __restrict__ C = static_cast<uint16_t*>(a.C);
+  uint16_t* __restrict__ CT = static_cast<uint16_t*>(a.CT);
+  int ldct = a.ldct;
+  if (args.symmetric) {
+    CT = tm != tn ? C : nullptr;
+    ldct = a.ldc;
+  }
+  const bool update = a.update_param != nullptr, update_transposed = update && (a.flags & kGemmUpdateTransposed) != 0;
+  if (update && !update_transposed) {
+    update_param8(a, args.update_dtype, row0 + orow, col0 + ocol, packed);
+    return;
+  }
+  if (!update) {
+    if (!(a.flags & kGemmSkipC)) *reinterpret_cast<u32x4*>(C + static_cast<int64_t>(row0 + orow) * a.ldc + col0 + ocol) = packed;
+    if (CT == nullptr) return;  // uniform over the workgroup
+  }
+  __syncthreads();  // every thread has read its sums
+  constexpr int kLdT = kSmallTile + 8;
+  uint16_t* transposed = reinterpret_cast<uint16_t*>(sums);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    transposed[(ocol + 2 * e) * kLdT + orow] = static_cast<uint16_t>(packed[e]);
+    transposed[(ocol + 2 * e + 1) * kLdT + orow] = static_cast<uint16_t>(packed[e] >> 16);
+  }
+  __syncthreads();
+  const u32x4 eight = *reinterpret_cast<const u32x4*>(transposed + orow * kLdT + ocol);  // column orow of the tile
+  if (update_transposed) update_param8(a, args.update_dtype, col0 + orow, row0 + ocol, eight);
+  else *reinterpret_cast<u32x4*>(CT + static_cast<int64_t>(col0 + orow) * ldct + row0 + ocol) = eight;
+}
+
 GemmTuning g_tuning;
 std::mutex g_tuning_mutex;  // the setter may be called while other threads launch: every launch works on one snapshot
 
@@ -705,8 +867,7 @@ int tile_count(const GemmGroup& g, const GemmProblem& p, int tile) {
   return g.symmetric ? tm * (tm + 1) / 2 : tm * tn;
 }
 
-// Below this many slabs a tile is never cut: the pieces would be gone before the fix-up launch (4-5 us) has paid off, and
-// matrices this small keep the bits of their update whatever else the launch holds.
+// Below this many slabs a tile is never cut: the pieces would be gone before the fix-up launch (4-5 us) has paid off.
 constexpr int kMinSplitSlabs = 17;
 
 // What a tile variant costs, in microseconds: one slab of a tile when every CU holds as many workgroups as it can
@@ -715,11 +876,12 @@ constexpr int kMinSplitSlabs = 17;
 // one on every group measured (whole Muon step, symmetric / general products forced to 256 or 128): hidden4096 7.28 ms
 // against 7.85 / 8.09 with small tiles, two hidden5120 matrices 11.0 against 12.1 / 12.8, five small ragged ones 0.344
 // against 0.427 / 0.406 with big ones, 24 of 1536 x 1024 1.23 against 1.27 / 1.29 with small ones.
+constexpr int kSmallVariant = 4;
 struct Variant {
   int tile, per_cu;
   double slab_us, lone_slab_us, tile_us;
 };
-constexpr Variant kVariants[3] = {{}, {256, 1, 1.45, 1.45, 9.0}, {128, 2, 0.95, 0.60, 5.0}};
+constexpr Variant kVariants[5] = {{}, {256, 1, 1.45, 1.45, 9.0}, {128, 2, 0.95, 0.60, 5.0}, {}, {kSmallTile, 1, 0.43, 0.43, 5.0}};
 
 // When the workgroups of a launch end, if each starts on the slot that is free first (as they do, in block order).
 // Slots are kept as groups that are free at the same time; a launch of equal tiles costs a few steps per round.
@@ -794,7 +956,7 @@ GemmPlan make_plan(const GemmGroup& g, int variant, const GemmScratch& scratch, 
     }
   };
   consider(0);
-  if (!tuning.split_remainder || scratch.partials == nullptr) return plan;
+  if (variant == kSmallVariant || !tuning.split_remainder || scratch.partials == nullptr) return plan;
   // piece lengths worth a look: every fraction of the longest K that may be cut, and the other K themselves
   int longest = 0, tried = 0;
   for (int i = 0; i < g.n; ++i)
@@ -863,6 +1025,27 @@ int launch(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& scratch,
   return MFSDP_OK;
 }
 
+template <int N>
+int launch_small(const GemmGroup& g, const GemmPlan& plan, const GemmTuning& tuning, hipStream_t stream) {
+  SmallArgs<N> args;
+  args.n = g.n;
+  args.symmetric = g.symmetric;
+  args.group_m = std::max(1, tuning.group_m);
+  args.update_dtype = g.update_dtype;
+  args.alpha = g.alpha;
+  args.beta = g.beta;
+  int tile = 0;
+  for (int i = 0; i < g.n; ++i) {
+    args.problem[i] = g.problem[plan.order[i]];
+    args.begin[i] = tile;
+    tile += tile_count(g, args.problem[i], kSmallTile);
+  }
+  for (int i = g.n; i < N; ++i) args.begin[i] = tile;
+  hipLaunchKernelGGL(gemm_small_kernel<N>, dim3(tile), dim3(kSmallThreads), 0, stream, args);
+  MFSDP_CHECK_LAUNCH("gemm_small_kernel");
+  return MFSDP_OK;
+}
+
 }  // namespace
 
 void set_gemm_tuning(const GemmTuning& t) {
@@ -874,13 +1057,21 @@ GemmTuning get_gemm_tuning() { return tuning_snapshot(); }
 GemmPlan gemm_plan(const GemmGroup& g, const GemmScratch& scratch) {
   const GemmTuning tuning = tuning_snapshot();
   const int variant = g.symmetric ? tuning.symmetric_variant : tuning.general_variant;
-  if (variant == 1 || variant == 2) return make_plan(g, variant, scratch, tuning);
+  if (variant == 1 || variant == 2 || variant == kSmallVariant) return make_plan(g, variant, scratch, tuning);
   const GemmPlan big = make_plan(g, 1, scratch, tuning);
   // On a machine shared with other matrices' kernels the CUs a part-filling triangle of big tiles leaves idle are
   // not lost, and a big tile moves fewer LDS bytes per flop.
   if (g.symmetric && g.shared && 4 * tile_count(g, g.problem[0], 256) >= device_cu_count()) return big;
   const GemmPlan small = make_plan(g, 2, scratch, tuning);
-  return big.us <= small.us ? big : small;
+  const GemmPlan& better = big.us <= small.us ? big : small;
+  // 64 x 64 tiles for one round at most: a second round costs as much as the first (1024 x 1536 update: 384 of them 279 us a
+  // step against 241 with 128 x 128 tiles; eight matrices of 512 x 1536: 495 against 281).  Within a round the model decides;
+  // K beyond about 2000 goes to 128 x 128 tiles cut along K (gram of 768 x 2304).
+  int tiles = 0;
+  for (int i = 0; i < g.n; ++i) tiles += tile_count(g, g.problem[i], kSmallTile);
+  if (tiles > device_cu_count()) return better;
+  const GemmPlan smallest = make_plan(g, kSmallVariant, scratch, tuning);
+  return smallest.us < better.us ? smallest : better;
 }
 
 int64_t gemm_nt_executed_flops(const GemmGroup& g) {
@@ -920,6 +1111,7 @@ int gemm_nt_bf16(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& sc
   const GemmTuning tuning = tuning_snapshot();
   // Slabs of 32 (three to five deep) were measured too: each slab row is then half a 128-byte line, the vector
   // cache looks every line up twice, and the products run 15-25 % slower than with slabs of 64 two deep.
+  if (plan.variant == kSmallVariant) return g.n <= 8 ? launch_small<8>(g, plan, tuning, stream) : launch_small<kMaxGemmGroup>(g, plan, tuning, stream);
   if (plan.variant == 2)  // 128x128 tile, 4 waves of 64x64, two workgroups per CU
     return launch<128, 128, 2, 2, 64, 2, 2>(g, plan, scratch, tuning, stream);
   return launch<256, 256, 2, 4, 64, 2, 1>(g, plan, scratch, tuning, stream);  // 256x256 tile, 8 waves of 128x64, one workgroup per CU

@@ -175,7 +175,7 @@ def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, side_by_side
     launches does not grow with theirs.
 
     Reproducibility: how the K walk of a product is cut into pieces, and with it the order of its fp32 sums and the last
-    bits of an update, may depend on the other matrices of the call where a side is longer than 1024.  Both forms meet
+    bits of an update, may depend on the other matrices of the call.  Both forms meet
     the same parity bar; a caller that needs bits independent of the optimizer's other parameters passes
     ``side_by_side=False`` (or sets ``MATRIX_FSDP_MUON_SIDE_BY_SIDE=0``), which updates one matrix after the other."""
     jobs = list(jobs)

@@ -424,3 +424,36 @@ def test_adamw_batch_has_the_bits_of_single_spans(count, amsgrad):
         if b is not None:
             b.launch()
     assert torch.equal(p, q)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shapes", [[(1, 1)], [(64, 64), (65, 63)], [(1024, 1024)], [(960, 1100)], [(1000, 40), (40, 1000), (33, 2047)], [(512, 1536)] * 2,
+                                    [(200, 3000)], [(128, 130)] * 9, [(100, 300)] * 33])
+def test_muon_small_tiles_against_the_oracle(shapes, dtype):
+    """Launches of at most one round of 64 x 64 tiles: every K length of a wave's share (no step, one to four, several
+    batches), up to 8 and more problems per launch, matrices whose norm is summed on the way and larger ones, wide and
+    tall.  The same launches forced to 128 x 128 tiles give the same update to bf16 rounding."""
+    from matrix_fsdp_amd import _lib
+
+    params = [make(s, 300 + i, 0.02).to(dtype) for i, s in enumerate(shapes)]
+    grads = [make(s, 400 + i).to(dtype) for i, s in enumerate(shapes)]
+    bufs = [make(s, 500 + i).to(dtype) for i, s in enumerate(shapes)]
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
+    results = []
+    try:
+        for variant in (4, 2, 3):
+            _lib.lib().mfsdp_set_muon_tuning(variant, variant, 0, 0, 0)
+            p, b = [t.to(DEV) for t in params], [t.to(DEV) for t in bufs]
+            F.muon_step_many([(pi, g.to(DEV), bi, kw) for pi, g, bi in zip(p, grads, b)])
+            results.append(p)
+    finally:
+        _lib.lib().mfsdp_set_muon_tuning(3, 3, 0, 0, 0)
+    for i in range(0, len(shapes), 8):
+        want_p, want_b = params[i].clone(), bufs[i].clone()
+        O.muon_step(want_p, grads[i], want_b, **kw)
+        step = (want_p.double() - params[i].double()).norm()
+        # bf16 rounding of the five iterations' products in another order: the bar the other variants are held to; a bf16
+        # parameter adds its own rounding, 2^-9 of its value on either side
+        bar = 1e-2 * step + (0.0 if dtype == torch.float32 else 2.0**-8 * params[i].double().norm())
+        for have in results:
+            assert (have[i].double().cpu() - want_p.double()).norm() <= bar, shapes[i]
