@@ -19,6 +19,7 @@ from functools import lru_cache
 import torch
 
 from .. import _lib
+from .launch import device_guard, stream_handle
 from ..core.layout import LayoutSegment
 from .segment_program import SegmentProgram, local_segments_program
 
@@ -157,8 +158,8 @@ def copy_rank_segments_to_full(
         if not workspace.is_cuda or not workspace.is_contiguous() or workspace.device != output_tensor.device:
             raise RuntimeError("workspace must be a contiguous CUDA tensor on the output's device")
         ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-    stream = torch.cuda.current_stream(output_tensor.device).cuda_stream
-    with torch.cuda.device(output_tensor.device):
+    stream = stream_handle(output_tensor.device)
+    with device_guard(output_tensor.device):
         _lib.check(
             _lib.lib().mfsdp_copy_rank_segments_to_full_device(
                 local_tensor.data_ptr(), local_tensor.numel(), output_tensor.data_ptr(), output_tensor.numel(),
@@ -203,8 +204,8 @@ def copy_range(input_tensor: torch.Tensor, output_tensor: torch.Tensor, input_of
         raise RuntimeError("input_tensor and output_tensor must be contiguous")
     if input_tensor.dtype != output_tensor.dtype:
         raise RuntimeError("source and destination dtype mismatch")
-    stream = torch.cuda.current_stream(output_tensor.device).cuda_stream
-    with torch.cuda.device(output_tensor.device):
+    stream = stream_handle(output_tensor.device)
+    with device_guard(output_tensor.device):
         _lib.check(
             _lib.lib().mfsdp_copy_range(
                 input_tensor.data_ptr(),
@@ -232,8 +233,8 @@ def accumulate(destination: torch.Tensor, source: torch.Tensor) -> torch.Tensor:
         raise RuntimeError(f"accumulate adds float32, bfloat16 or float16 tensors of one dtype, got {destination.dtype} += {source.dtype}")
     if destination.numel() != source.numel():
         raise RuntimeError(f"destination has {destination.numel()} elements, source has {source.numel()}")
-    stream = torch.cuda.current_stream(destination.device).cuda_stream
-    with torch.cuda.device(destination.device):
+    stream = stream_handle(destination.device)
+    with device_guard(destination.device):
         _lib.check(
             _lib.lib().mfsdp_accumulate(destination.data_ptr(), source.data_ptr(), destination.numel(), _ACCUMULATE_DTYPES[destination.dtype], stream)
         )
@@ -263,7 +264,7 @@ def cast(source: torch.Tensor, dtype: torch.dtype, out: torch.Tensor | None = No
         out = torch.empty(source.shape, dtype=dtype, device=source.device)
     elif out.dtype != dtype or out.numel() != source.numel() or not out.is_contiguous() or out.device != source.device:
         raise RuntimeError("cast output must be contiguous, on the source's device, of the target dtype and size")
-    stream = torch.cuda.current_stream(source.device).cuda_stream
-    with torch.cuda.device(source.device):
+    stream = stream_handle(source.device)
+    with device_guard(source.device):
         _lib.check(_lib.lib().mfsdp_cast(source.data_ptr(), out.data_ptr(), source.numel(), code, stream))
     return out

@@ -27,6 +27,7 @@ import numpy as np
 import torch
 
 from .. import _lib
+from .launch import device_guard, stream_handle
 
 RUN_DTYPE = np.dtype(
     [
@@ -142,7 +143,7 @@ class SegmentProgram:
             )
         self._handle = handle
         self.bytes_moved = int(_lib.lib().mfsdp_segment_program_bytes(handle))
-        self._src_array = (ctypes.c_void_p * max(1, len(self.src_numels)))()
+        self._src_array_type = ctypes.c_void_p * max(1, len(self.src_numels))
 
     def run(self, srcs: Sequence[torch.Tensor], dst: torch.Tensor) -> torch.Tensor:
         if self._handle is None:
@@ -150,15 +151,16 @@ class SegmentProgram:
         if len(srcs) != len(self.src_numels):
             raise RuntimeError(f"segment program expects {len(self.src_numels)} sources, got {len(srcs)}.")
         _check_tensor(dst, self.dst_dtype, self.dst_numel, "destination")
-        for i, (t, n) in enumerate(zip(srcs, self.src_numels)):
-            _check_tensor(t, self.src_dtype, n, f"source {i}")
-            if t.device != dst.device:
+        device, pointers = dst.device, []
+        for t, n in zip(srcs, self.src_numels):
+            if not _fits(t, self.src_dtype, n):
+                _check_tensor(t, self.src_dtype, n, f"source {len(pointers)}")
+            if t.device != device:
                 raise RuntimeError("sources and destination must be on one device.")
-            self._src_array[i] = t.data_ptr()
-        stream = torch.cuda.current_stream(dst.device).cuda_stream
-        with torch.cuda.device(dst.device):
+            pointers.append(t.data_ptr())
+        with device_guard(device):
             _lib.check(
-                _lib.lib().mfsdp_segment_program_run(self._handle, self._src_array, len(self.src_numels), dst.data_ptr(), stream)
+                _lib.lib().mfsdp_segment_program_run(self._handle, self._src_array_type(*pointers), len(pointers), dst.data_ptr(), stream_handle(device))
             )
         return dst
 
@@ -188,8 +190,8 @@ class SegmentProgram:
                 if t.device != device:
                     raise RuntimeError("sources and destination must be on one device.")
                 src_array[b * n_srcs + i] = t.data_ptr()
-        stream = torch.cuda.current_stream(device).cuda_stream
-        with torch.cuda.device(device):
+        stream = stream_handle(device)
+        with device_guard(device):
             _lib.check(_lib.lib().mfsdp_segment_program_run_many(self._handle, len(dsts), src_array, n_srcs, dst_array, stream))
 
     def destroy(self) -> None:
@@ -204,9 +206,15 @@ class SegmentProgram:
             pass
 
 
+def _fits(t: torch.Tensor, dtype: torch.dtype, min_numel: int) -> bool:
+    return t.is_cuda and t.is_contiguous() and t.dtype == dtype and t.numel() >= min_numel
+
+
 def _check_tensor(t: torch.Tensor, dtype: torch.dtype, min_numel: int, what: str) -> None:
     """The preconditions the reference checks before its copy kernels
     (matrix_fsdp/kernels/native.py:353-360, kernels/native/matrix_copy.cpp:60-78)."""
+    if _fits(t, dtype, min_numel):
+        return
     if not t.is_cuda:
         raise RuntimeError(f"{what} must be a CUDA tensor")
     if not t.is_contiguous():

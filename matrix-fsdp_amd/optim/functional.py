@@ -8,6 +8,7 @@ import os
 import torch
 
 from .. import _lib
+from ..kernels.launch import device_guard, stream_handle
 
 NS_COEFFICIENTS = (3.4445, -4.7750, 2.0315)
 NS_EPS = 1e-7
@@ -99,8 +100,8 @@ def newton_schulz(
     if out is None:
         out = torch.empty((rows, cols), dtype=torch.bfloat16, device=update.device)
     a, b, c = ns_coefficients
-    stream = torch.cuda.current_stream(update.device).cuda_stream
-    with torch.cuda.device(update.device):
+    stream = stream_handle(update.device)
+    with device_guard(update.device):
         _lib.check(
             _lib.lib().mfsdp_newton_schulz(
                 update.data_ptr(), _DTYPE_CODES[update.dtype], rows, cols, a, b, c, ns_steps, eps,
@@ -135,8 +136,8 @@ def muon_step(
     workspace = workspace or MuonWorkspace(param.device)
     ws = workspace.get(rows, cols)
     a, b, c = ns_coefficients
-    stream = torch.cuda.current_stream(param.device).cuda_stream
-    with torch.cuda.device(param.device):
+    stream = stream_handle(param.device)
+    with device_guard(param.device):
         _lib.check(
             _lib.lib().mfsdp_muon_step_ex(
                 param.data_ptr(), grad.data_ptr(), momentum_buf.data_ptr(), _DTYPE_CODES[param.dtype], rows, cols,
@@ -197,8 +198,8 @@ def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, side_by_side
         key, fields = _job(param, grad, buf, **kw)
         alike.setdefault(key, []).append(fields)
     lib = _lib.lib()
-    stream = torch.cuda.current_stream(device).cuda_stream
-    with torch.cuda.device(device):
+    stream = stream_handle(device)
+    with device_guard(device):
         for (dtype, momentum, nesterov, a, b, c, ns_steps, eps), fields in alike.items():
             n = len(fields)
             rows, cols = (ctypes.c_int64 * n)(*(f[3] for f in fields)), (ctypes.c_int64 * n)(*(f[4] for f in fields))
@@ -225,8 +226,8 @@ class AdamWBatch:
         spans_by_key, self._spans = self._spans, {}
         try:
             for (device, *hyper), spans in spans_by_key.items():
-                with torch.cuda.device(device):
-                    stream = torch.cuda.current_stream(device).cuda_stream
+                with device_guard(device):
+                    stream = stream_handle(device)
                     _lib.check(_lib.lib().mfsdp_adamw_step_many(len(spans), (_lib.AdamWSpan * len(spans))(*spans), *hyper, stream))
         finally:
             self._tensors.clear()

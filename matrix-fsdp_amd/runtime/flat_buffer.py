@@ -240,7 +240,7 @@ class MatrixFlatBuffer:
                 raise NotImplementedError("MatrixFSDP V0 cannot expose multi-segment parameters yet.")
             else:
                 view = views[0]
-                data = self.local_shard[view.shard_start : view.shard_end]
+                data = self.local_shard.narrow(0, view.shard_start, view.shard_end - view.shard_start)
                 mp.param.data = data.view(mp.shape) if view.numel == mp.numel else data
         self.clear_full_params()
 
@@ -249,7 +249,7 @@ class MatrixFlatBuffer:
         if self.full_buffer is None:
             raise RuntimeError("Full parameter buffer is not materialized.")
         for mp in self.managed_params:
-            mp.param.data = self.full_buffer[mp.offset : mp.end].view(mp.shape)
+            mp.param.data = self.full_buffer.narrow(0, mp.offset, mp.end - mp.offset).view(mp.shape)
 
     def param_data_alias_full_buffer(self) -> bool:
         if self.full_buffer is None:
@@ -554,7 +554,7 @@ class MatrixFlatBuffer:
                 mp.param.grad = None
                 continue
             view = views[0]
-            grad = self.local_grad_shard[view.shard_start : view.shard_end]
+            grad = self.local_grad_shard.narrow(0, view.shard_start, view.shard_end - view.shard_start)
             mp.param.grad = grad.view(mp.shape) if view.numel == mp.numel else grad
 
     def prepare_grad_bucket(self) -> bool:

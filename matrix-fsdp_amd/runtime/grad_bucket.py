@@ -182,10 +182,10 @@ def fill_reduce_scatter_input(
         raise ValueError(f"packed has {packed.numel()} elements, expected {expected}.")
     if backend not in _BACKENDS:
         raise ValueError("backend must be 'auto', 'flat_cat', 'foreach_copy', 'chunk_cat', or 'segment_copy'.")
-    kind = classify_copy_in_layout(bucket)
-    if backend in ("flat_cat", "foreach_copy") and kind != "flat_contiguous":
+    # only the backends that need a layout look at it: the classification walks every parameter of every rank
+    if backend in ("flat_cat", "foreach_copy") and classify_copy_in_layout(bucket) != "flat_contiguous":
         raise ValueError(f"{backend} backend requires an equal, rank-contiguous flat bucket layout.")
-    if backend == "chunk_cat" and kind != "fsdp2_chunk":
+    if backend == "chunk_cat" and classify_copy_in_layout(bucket) != "fsdp2_chunk":
         raise ValueError("chunk_cat backend requires an FSDP2-style per-parameter chunk bucket layout.")
     grads = []
     for pg in bucket.param_grads:
