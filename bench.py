@@ -64,7 +64,7 @@ def parse_args():
                     "devcopy (the device-metadata rank-segment copy, the reference extension's own entry point), gemm (one plain 8192^3 product beside "
                     "the library's), muon, adamw, mixed")
     ap.add_argument("--muon-form", default="both", choices=("both", "serial", "side-by-side"),
-                    help="which form of the Muon leg to run: one matrix at a time on the calling stream, the three side by side on side streams, "
+                    help="which form of the Muon leg to run: one matrix at a time, the three sharing every launch, "
                     "or both (serial alone makes every kernel of a rocprofv3 trace run by itself)")
     ap.add_argument("--skip-cpu", action="store_true", help="do not time the CPU baselines")
     ap.add_argument("--hold-muon-seconds", type=float, default=0.0,
@@ -432,7 +432,7 @@ def main() -> int:
                 F.muon_step(p, g, buf, workspace=ws, **kw)
 
         def muon_all():
-            # the step of the optimizer: independent matrices side by side on the library's side streams, joined on this stream
+            # the step of the optimizer: independent matrices share every launch
             F.muon_step_many([(p, g, buf, kw) for p, g, buf in mats])
 
         med_one_stream = med = None
@@ -473,8 +473,8 @@ def main() -> int:
             "ns_TFLOPs_reference_flop_count": round(tflops, 1),
             "pct_bf16_mfma_peak": round(100 * tflops / BF16_MFMA_PEAK_TFLOPS, 2),
             "flop_count": "5 * (4 m^2 n + 2 m^3) per matrix, full GEMMs as the reference executes them; the time is the whole "
-            "update (momentum, norm, Newton-Schulz, parameter update) of the three matrices, which muon_step_many runs side by side on "
-            "three streams; per_matrix times are each matrix alone",
+            "update (momentum, norm, Newton-Schulz, parameter update) of the three matrices, which muon_step_many takes through "
+            "every stage as one launch; per_matrix times are each matrix alone",
             "dtype_variant": "fp32 params / momentum, bf16-valued fp32 grads",
             "per_matrix": per_matrix,
         }

@@ -95,8 +95,8 @@ __device__ __forceinline__ void store_once(P* p, V v) { __builtin_nontemporal_st
 // stores mix.  One span of 41 M elements: one wavefront per workgroup with two vectors per thread 6.22 TB/s (one vector
 // 5.55, four 6.01; 256 threads with four vectors 5.93, with two 5.94; 16 persistent workgroups per CU 5.71); 5.1-5.5 TB/s
 // with cached loads or stores.  One launch
-// for all spans of a step: 15 parameters of 1000 to 3 M elements (5.1 M in all) take 132 us of host and device time a step
-// against 294 us with a launch each.
+// for all spans of a step: 15 parameters of 1000 to 6.1 M elements (8.2 M in all) take 127 us of host and device time a
+// step against 293 us with a launch each.
 template <bool GRAD_BF16, bool AMSGRAD, int N>
 __global__ void __launch_bounds__(kThreads)
 adamw_kernel(SpanTable<N> table) {

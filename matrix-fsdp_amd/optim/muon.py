@@ -5,8 +5,8 @@ per-parameter state (``momentum_buffer = zeros_like(grad)``) follow
 torch/optim/_muon.py:87-202, which is the optimizer the reference
 instantiates for owner-rank matrices (matrix_fsdp/optim/wrapper.py:416-429).
 ``step()`` runs momentum, Newton-Schulz and the parameter update of every
-matrix through ``mfsdp_muon_step_ex`` (independent matrices side by side where
-that pays); nothing falls back to torch arithmetic.
+matrix through ``mfsdp_muon_step_many`` (the matrices share every launch);
+nothing falls back to torch arithmetic.
 """
 from __future__ import annotations
 
@@ -72,7 +72,7 @@ class Muon(torch.optim.Muon):
                     adjust_lr_fn=group["adjust_lr_fn"],
                 )
                 jobs.append((p.data, grad.contiguous(), state["momentum_buffer"], keywords))
-        # the matrices are independent: one device's share goes to muon_step_many, which runs small ones side by side
+        # the matrices are independent: one device's share goes to muon_step_many, where they share every launch
         by_device: dict[torch.device, list] = {}
         for job in jobs:
             by_device.setdefault(job[0].device, []).append(job)
