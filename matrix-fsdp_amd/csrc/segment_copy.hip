@@ -33,7 +33,7 @@ constexpr int kMaxBatch = 64;     // destination pointers (buffers) one launch c
 constexpr int kDefaultBlocksPerCu = 0;  // one workgroup per tile
 constexpr int kDefaultBlockThreads = 64;
 constexpr int kBlockThreads = 256;
-constexpr int kFillTileSpans = 8;  // spans of 256 * U groups a zero-fill tile covers (its units must stay below 2^16)
+constexpr int kFillTileSpans = 8;  // spans of 256 * U groups a zero-fill tile covers, as far as its length can be held
 constexpr int64_t kMaxGrid = (int64_t{1} << 31) - 1;  // grid-stride loops keep a capped grid correct
 constexpr int64_t kMaxGroupsPerRun = 0x7fffffff;  // the reciprocal division is exact below 2^31 groups
 
@@ -80,6 +80,8 @@ struct DevTile {
 };
 constexpr uint64_t kTileGeneric = uint64_t{1} << 63;
 constexpr uint64_t kTileOffsetMask = (uint64_t{1} << 48) - 1;
+constexpr int64_t kMaxTileUnits = 65408;  // longest direct tile: 16 bits of length, whole 128-byte lines of the destination
+static_assert(kMaxTileUnits < (1 << 16) && kMaxTileUnits % 128 == 0 && 4 * kBlockThreads * 16 <= kMaxTileUnits, "a copying tile is never shortened by it");
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -410,7 +412,7 @@ int compile_tables(mfsdp_segment_program* prog, std::vector<Compiled>* out) {
       // workgroup, walked in the kernel's loop over a direct tile, lifts the fill to 5.3 TB/s (pack of such a layer
       // buffer 6.09 TB/s against 5.55-5.78; 32 spans no better; fill tiles spread evenly among the copying tiles
       // instead of behind each rank's segments: slower, 5.85-5.95).
-      const int64_t tile_cap = r.src_id < 0 ? kFillTileSpans * tile_units : tile_units;
+      const int64_t tile_cap = r.src_id < 0 ? std::min(kFillTileSpans * tile_units, kMaxTileUnits) : tile_units;
       const int64_t per_row = (r.row_len + tile_cap - 1) / tile_cap;
       const int64_t piece = std::min(tile_cap, ((r.row_len + per_row - 1) / per_row + line - 1) / line * line);
       for (int64_t row = 0; row < r.rows; ++row) {

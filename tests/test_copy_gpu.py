@@ -521,3 +521,29 @@ def test_rows_of_any_length_at_any_offset(row_len, src_dtype, dst_dtype):
         else:
             native.cast(held[5 : 5 + row_len], dst_dtype, out=span[1 : 1 + row_len])
         assert torch.equal(span[1 : 1 + row_len].cpu(), src[5 : 5 + row_len].to(dst_dtype)) and float(span[0]) == 77 and float(span[-1]) == 77
+
+
+@pytest.mark.parametrize("unroll", [0, 1, 2, 4])
+def test_long_zero_fills_at_every_unroll(unroll):
+    """Zero-fill runs around what the 16-bit length of one tile holds, for programs created at every unroll of the tuning
+    call, plain (a unit is a byte) and converting: every element of the runs cleared, nothing beside them."""
+    from matrix_fsdp_amd import _lib
+
+    lengths = (1, 32768, 65408, 65535, 65536, 65537, 100000, 131072, 1 << 20)
+    starts = [sum(lengths[:i]) + 9 * (i + 1) for i in range(len(lengths))]
+    runs = np.zeros(len(lengths), dtype=RUN_DTYPE)
+    for run, at, n in zip(runs, starts, lengths):
+        run["dst_off"], run["row_len"], run["rows"], run["src_id"] = at, n, 1, -1
+    total = starts[-1] + lengths[-1] + 5
+    for src_dtype, dst_dtype in ((torch.uint8, torch.uint8), (torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)):
+        _lib.lib().mfsdp_set_copy_tuning(-1, 1, unroll, 0)
+        try:
+            program = SegmentProgram(runs, (), total, src_dtype=src_dtype, dst_dtype=dst_dtype, device=DEV, merge=False)
+        finally:
+            _lib.lib().mfsdp_set_copy_tuning(-1, 1, 0, 0)
+        dst = torch.full((total,), 77, dtype=dst_dtype, device=DEV)
+        program.run((), dst)
+        want = torch.full((total,), 77, dtype=dst_dtype)
+        for at, n in zip(starts, lengths):
+            want[at : at + n] = 0
+        assert torch.equal(dst.cpu(), want), (src_dtype, dst_dtype)
