@@ -181,10 +181,12 @@ int check_iteration(float a, float b, float c, int steps) {
   return MFSDP_OK;
 }
 
-int check_matrix(int64_t rows, int64_t cols, Matrix* w) {
+int check_matrix(int64_t rows, int64_t cols, int steps, Matrix* w) {
   if (!plan_matrix(rows, cols, nullptr, w))
     return fail(MFSDP_ERR_INVALID, "Input tensor gradient must be a 2D matrix with positive sizes, got %lld x %lld",
                 static_cast<long long>(rows), static_cast<long long>(cols));
+  if (steps > 0 && w->np > kMaxGemmLeading)  // of the products' operands; without a product there is no limit
+    return fail(MFSDP_ERR_UNSUPPORTED, "leading dimensions beyond 2^22 elements, got %lld x %lld", static_cast<long long>(rows), static_cast<long long>(cols));
   return MFSDP_OK;
 }
 
@@ -288,7 +290,7 @@ extern "C" int mfsdp_newton_schulz(const void* update, int update_dtype, int64_t
                                    int steps, float eps, void* out_bf16, void* workspace, int64_t workspace_bytes, void* stream) {
   Group g;
   if (int rc = check_iteration(a, b, c, steps)) return rc;
-  if (int rc = check_matrix(rows, cols, &g.w[0])) return rc;
+  if (int rc = check_matrix(rows, cols, steps, &g.w[0])) return rc;
   if (int rc = check_workspace(workspace, workspace_bytes, g.w[0].bytes + kSharedBytes)) return rc;
   if (update_dtype != MFSDP_F32 && update_dtype != MFSDP_BF16) return fail(MFSDP_ERR_INVALID, "update dtype must be f32 or bf16");
   if (!update || !out_bf16) return fail(MFSDP_ERR_INVALID, "null tensor pointer");
@@ -310,7 +312,7 @@ extern "C" int mfsdp_muon_step_ex(void* param, const void* grad, void* momentum_
   const StepArgs s{dtype, momentum, nesterov, a, b, c, steps, eps, (flags & MFSDP_MUON_SHARED_MACHINE) != 0};
   Matrix w;
   if (int rc = check_step(s)) return rc;
-  if (int rc = check_matrix(rows, cols, &w)) return rc;
+  if (int rc = check_matrix(rows, cols, steps, &w)) return rc;
   if (int rc = check_workspace(workspace, workspace_bytes, w.bytes + kSharedBytes)) return rc;
   if (int rc = check_tensors(param, grad, momentum_buf, dtype, lr, weight_decay)) return rc;
   if (flags & ~MFSDP_MUON_SHARED_MACHINE) return fail(MFSDP_ERR_INVALID, "unknown flags 0x%x", flags);
@@ -338,7 +340,7 @@ extern "C" int mfsdp_muon_step_many(int64_t n, const mfsdp_muon_job* jobs, int d
   int64_t largest = 0;
   for (int64_t i = 0; i < n; ++i) {
     Matrix w;
-    if (int rc = check_matrix(jobs[i].rows, jobs[i].cols, &w)) return rc;
+    if (int rc = check_matrix(jobs[i].rows, jobs[i].cols, steps, &w)) return rc;
     if (int rc = check_tensors(jobs[i].param, jobs[i].grad, jobs[i].momentum_buf, dtype, jobs[i].lr, jobs[i].weight_decay)) return rc;
     order.emplace_back(w.bytes, i);
     largest = std::max(largest, w.bytes);

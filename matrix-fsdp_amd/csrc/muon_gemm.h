@@ -38,6 +38,7 @@ struct GemmProblem {
   int splits, partial_base;
 };
 
+constexpr int kMaxGemmLeading = 1 << 22;  // largest leading dimension of P and Q: a tile's rows are reached by 31-bit byte offsets
 constexpr int kMaxGemmGroup = 32;  // problems one launch carries by value in its kernel arguments
 
 // Products of one launch.  symmetric: every P*Q^T is known to be symmetric (M == N); only tiles on or below the diagonal

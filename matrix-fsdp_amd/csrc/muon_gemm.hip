@@ -1108,7 +1108,7 @@ int gemm_nt_bf16(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& sc
         (a.CT && ((a.ldct % 8) || reinterpret_cast<uintptr_t>(a.CT) % 16)))
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: C, D and the transposed output must be 16-byte aligned with leading dimensions multiple of 8");
     if (a.D && (a.K < a.M || g.alpha == 0.0f)) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: a D operand needs K >= M and alpha != 0");
-    if (a.ldp > (1 << 22) || a.ldq > (1 << 22)) return fail(MFSDP_ERR_UNSUPPORTED, "gemm_nt_bf16: leading dimensions beyond 2^22 elements");
+    if (a.ldp > kMaxGemmLeading || a.ldq > kMaxGemmLeading) return fail(MFSDP_ERR_UNSUPPORTED, "gemm_nt_bf16: leading dimensions beyond 2^22 elements");
     if (a.update_param != nullptr && (g.symmetric || (g.update_dtype != MFSDP_F32 && g.update_dtype != MFSDP_BF16) ||
                                       reinterpret_cast<uintptr_t>(a.update_param) % (g.update_dtype == MFSDP_F32 ? 4 : 2)))
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: parameter update needs a general product and an aligned f32 / bf16 parameter");

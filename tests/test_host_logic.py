@@ -532,3 +532,30 @@ def test_mixed_optimizer_constructor_surface_of_the_reference():
         MixedMuonAdamWOptimizer([matrix], [], momentum=0.9)
     with pytest.raises(RuntimeError, match="at least one non-empty parameter"):
         MixedMuonAdamWOptimizer([], [])
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the pointers are made up: only without a device is a call that passes the checks harmless")
+def test_muon_refuses_long_sides_before_anything_is_enqueued():
+    """A product's leading dimension is limited to 2^22 elements: a matrix with a longer side is refused with
+    MFSDP_ERR_UNSUPPORTED by the checks, wherever it stands in a list.  Without a device a call that passes the checks
+    fails at its first launch (MFSDP_ERR_HIP), which is what a side of exactly 2^22 and a step without products do."""
+    lib = _lib.lib()
+    fake, room = 1 << 40, 1 << 50
+    ns = (3.4445, -4.7750, 2.0315)
+
+    def many(shapes, steps=5):
+        jobs = (_lib.MuonJob * len(shapes))(*((fake, fake, fake, r, c, 0.1, 0.0, 0.1) for r, c in shapes))
+        return lib.mfsdp_muon_step_many(len(shapes), jobs, _lib.DT_F32, 0.9, 1, *ns, steps, 1e-7, fake, room, None)
+
+    def single(rows, cols, steps=5):
+        return lib.mfsdp_muon_step(fake, fake, fake, _lib.DT_F32, rows, cols, 0.1, 0.0, 0.9, 1, *ns, steps, 1e-7, 0.1, fake, room, None)
+
+    def orthogonalise(rows, cols, steps=5):
+        return lib.mfsdp_newton_schulz(fake, _lib.DT_F32, rows, cols, *ns, steps, 1e-7, fake, fake, room, None)
+
+    limit = 1 << 22
+    for rows, cols in ((8, limit + 1), (limit + 1, 8), (8, 5_000_000)):
+        for rc in (single(rows, cols), orthogonalise(rows, cols), many([(rows, cols)]), many([(64, 64), (rows, cols)]), many([(rows, cols), (64, 64), (32, 8)])):
+            assert rc == 3 and b"2^22" in lib.mfsdp_last_error(), (rows, cols, rc)
+        assert single(rows, cols, steps=0) == orthogonalise(rows, cols, steps=0) == many([(64, 64), (rows, cols)], steps=0) == 2
+    assert single(8, limit) == orthogonalise(limit, 8) == many([(64, 64), (8, limit)]) == 2

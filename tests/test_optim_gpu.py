@@ -370,6 +370,19 @@ def test_muon_group_larger_than_a_launch_and_than_the_workspace():
     assert _lib.lib().mfsdp_muon_many_workspace_bytes(1, (ctypes.c_int64 * 1)(96), (ctypes.c_int64 * 1)(160)) == ws.numel()
 
 
+def test_muon_group_with_a_side_too_long_is_refused_whole():
+    """A matrix whose long side no product takes, behind an ordinary one: the call raises and neither has changed."""
+    shapes = [(64, 96), (1, (1 << 22) + 1)]
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.9, nesterov=True)
+    mats = [[make(sh, 950 + 3 * i + k).to(DEV) for k in range(3)] for i, sh in enumerate(shapes)]
+    before = [[t.clone() for t in three] for three in mats]
+    with pytest.raises(RuntimeError, match="2\\^22"):
+        F.muon_step_many([(p, g, b, kw) for p, g, b in mats])
+    torch.cuda.synchronize()
+    assert all(torch.equal(t, u) for three, old in zip(mats, before) for t, u in zip(three, old))
+    torch.cuda.empty_cache()  # the workspace of the long matrix
+
+
 def test_muon_group_with_cut_k_walks():
     """Sides beyond 1024, where the tiles of the last round are cut along K: several K in one launch, against the oracle."""
     shapes = [(192, 1088), (130, 2100), (4160, 200), (70, 8200)]
