@@ -148,6 +148,52 @@ def muon_step(
         )
 
 
+class MuonStreamPool:
+    """Side streams (default priority) with one Newton-Schulz workspace each, for a caller that wants independent matrices
+    updated on streams of its own (``muon_step_many(..., pool=...)``)."""
+
+    def __init__(self, device, n_streams: int = 3) -> None:
+        self.device = torch.device(device)
+        self.streams = [torch.cuda.Stream(device=self.device) for _ in range(n_streams)]
+        self.workspaces = [MuonWorkspace(self.device) for _ in range(n_streams)]
+
+
+def _underfills_the_machine(shape, compute_units: int) -> bool:
+    """Would the 256 x 256 tiles of this matrix's symmetric products (the lower triangle of an m x m result, m the
+    short side) occupy less than three quarters of the CUs?"""
+    t = -(-min(shape) // 256)
+    return 4 * (t * (t + 1) // 2) < 3 * compute_units
+
+
+def _step_on_streams(jobs, pool: MuonStreamPool) -> None:
+    """Every matrix on one of the pool's streams, longest first onto the least loaded one; the calling stream waits for
+    them before anything enqueued later runs."""
+    n = min(len(pool.streams), len(jobs))
+
+    def cost(job):  # flops of the products: 4 m^2 n + 2 m^3 per step
+        m, k = min(job[0].shape), max(job[0].shape)
+        return 4 * m * m * k + 2 * m**3
+
+    loads, assigned = [0] * n, [[] for _ in range(n)]
+    for job in sorted(jobs, key=cost, reverse=True):
+        s = loads.index(min(loads))
+        assigned[s].append(job)
+        loads[s] += cost(job)
+    current = torch.cuda.current_stream(jobs[0][0].device)
+    fork = torch.cuda.Event()
+    fork.record(current)
+    for side, workspace, share in zip(pool.streams, pool.workspaces, assigned):
+        side.wait_event(fork)
+        with torch.cuda.stream(side):
+            for param, grad, buf, kw in share:
+                for t in (param, grad, buf):
+                    t.record_stream(side)
+                muon_step(param, grad, buf, workspace=workspace, **{**kw, "shared_machine": True})
+        join = torch.cuda.Event()
+        join.record(side)
+        current.wait_event(join)
+
+
 def side_by_side_default() -> bool | None:
     """``MATRIX_FSDP_MUON_SIDE_BY_SIDE``: ``0`` updates one matrix after the other (result bits that do not depend on
     which other parameters the optimizer holds), anything else lets them share launches."""
@@ -167,7 +213,8 @@ def _job(param, grad, momentum_buf, *, lr, weight_decay, momentum, nesterov, ns_
     return key, (param.data_ptr(), grad.data_ptr(), momentum_buf.data_ptr(), rows, cols, lr, weight_decay, adjust_lr(lr, adjust_lr_fn, (rows, cols)))
 
 
-def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, side_by_side: bool | None = None) -> None:
+def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, pool: MuonStreamPool | None = None,
+                   side_by_side: bool | None = None) -> None:
     """Updates several matrices; ``jobs`` is a sequence of ``(param, grad, momentum_buf, keywords of muon_step)``.
 
     The matrices of a rank are independent of each other, so those that share their hyper-parameters (the learning
@@ -178,7 +225,11 @@ def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, side_by_side
     Reproducibility: how the K walk of a product is cut into pieces, and with it the order of its fp32 sums and the last
     bits of an update, may depend on the other matrices of the call.  Both forms meet
     the same parity bar; a caller that needs bits independent of the optimizer's other parameters passes
-    ``side_by_side=False`` (or sets ``MATRIX_FSDP_MUON_SIDE_BY_SIDE=0``), which updates one matrix after the other."""
+    ``side_by_side=False`` (or sets ``MATRIX_FSDP_MUON_SIDE_BY_SIDE=0``), which updates one matrix after the other.
+
+    With a ``pool`` the matrices take launches of their own on the pool's streams instead: those that leave CUs idle, when
+    there are at least two of them (all of them with ``side_by_side=True``), the others one after the other on the calling
+    stream.  A job whose keywords hold ``shared_machine`` is updated by ``muon_step``."""
     jobs = list(jobs)
     if not jobs:
         return
@@ -189,9 +240,22 @@ def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, side_by_side
     if side_by_side is None:
         side_by_side = side_by_side_default()
     workspace = workspace or MuonWorkspace(device)
+    spread = []
     if side_by_side is False:
-        for param, grad, buf, kw in jobs:
-            muon_step(param, grad, buf, workspace=workspace, **kw)
+        alone, jobs = jobs, []
+    elif pool is not None:
+        compute_units = torch.cuda.get_device_properties(device).multi_processor_count
+        small = [job[0].ndim == 2 and (bool(side_by_side) or _underfills_the_machine(job[0].shape, compute_units)) for job in jobs]
+        if sum(small) < 2 and not side_by_side:
+            small = [False] * len(jobs)
+        alone, spread, jobs = [j for j, s in zip(jobs, small) if not s], [j for j, s in zip(jobs, small) if s], []
+    else:
+        alone, jobs = [j for j in jobs if "shared_machine" in j[3]], [j for j in jobs if "shared_machine" not in j[3]]
+    for param, grad, buf, kw in alone:
+        muon_step(param, grad, buf, workspace=workspace, **kw)
+    if spread:
+        _step_on_streams(spread, pool)
+    if not jobs:
         return
     alike: dict[tuple, list[tuple]] = {}
     for param, grad, buf, kw in jobs:

@@ -217,6 +217,43 @@ def test_muon_step_many_side_by_side_switch(monkeypatch):
             assert torch.equal(bs[i], alone_b[i])  # the momentum does not depend on the tiling
 
 
+@pytest.mark.parametrize("side_by_side", [None, True, False])
+def test_muon_step_many_on_the_streams_of_a_pool(side_by_side):
+    """A caller's own side streams, used twice with new gradients: the update of one call per matrix within the parity bar,
+    the momentum exactly, and work enqueued afterwards on the calling stream sees them.  A machine-filling matrix rides
+    along; its launches stay on the calling stream unless every matrix is sent to the streams."""
+    shapes = [(512, 768), (768, 512), (100, 36), (5120, 5120), (1024, 512)]
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
+    params = [make(sh, 960 + i, 0.02).to(DEV) for i, sh in enumerate(shapes)]
+    bufs = [make(sh, 970 + i).to(DEV) for i, sh in enumerate(shapes)]
+    one_p, one_b = [p.clone() for p in params], [b.clone() for b in bufs]
+    many_p, many_b = [p.clone() for p in params], [b.clone() for b in bufs]
+    pool, ws = F.MuonStreamPool(DEV), F.MuonWorkspace(DEV)
+    for step in range(2):
+        grads = [make(sh, 980 + 10 * step + i).to(DEV) for i, sh in enumerate(shapes)]
+        for p, g, b in zip(one_p, grads, one_b):
+            F.muon_step(p, g, b, workspace=ws, **kw)
+        F.muon_step_many([(p, g, b, kw) for p, g, b in zip(many_p, grads, many_b)], workspace=ws, pool=pool, side_by_side=side_by_side)
+        seen = [p.clone() for p in many_p]  # enqueued right behind the call
+        torch.cuda.synchronize()
+        for i in range(len(shapes)):
+            assert torch.equal(many_b[i], one_b[i]) and torch.equal(many_p[i], seen[i])
+            assert rel_fro(many_p[i] - params[i], one_p[i] - params[i]) < MUON_TOL, shapes[i]
+
+
+def test_muon_step_many_takes_the_keywords_of_muon_step():
+    """``shared_machine`` among a job's keywords: that matrix gets the bits of ``muon_step`` with the flag."""
+    shapes = [(3072, 3072), (200, 100)]
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
+    params, grads = [make(sh, 990 + i, 0.02).to(DEV) for i, sh in enumerate(shapes)], [make(sh, 995 + i).to(DEV) for i, sh in enumerate(shapes)]
+    many_p, one_p = [p.clone() for p in params], [p.clone() for p in params]
+    keywords = [dict(kw, shared_machine=True), kw]
+    F.muon_step_many([(p, g, torch.zeros_like(p), k) for p, g, k in zip(many_p, grads, keywords)])
+    for p, g, k, have in zip(one_p, grads, keywords, many_p):
+        F.muon_step(p, g, torch.zeros_like(p), **k)
+        assert torch.equal(p, have)
+
+
 def test_muon_argument_errors():
     p = torch.zeros(8, 8, device=DEV)
     with pytest.raises(ValueError, match="2D"):
