@@ -261,9 +261,10 @@ int mfsdp_muon_step_ex(void* param, const void* grad, void* momentum_buf, int dt
 /*
  * The whole matrices of a rank in one call (the loop of torch/optim/_muon.py:285-318): mfsdp_muon_step of every job, all
  * with the same dtype, momentum, coefficients and number of steps.  The matrices are independent; up to 32 at a time go
- * through each stage of the update as one launch, so that small ones fill the machine together.  How many do is a matter
- * of the workspace: mfsdp_muon_many_workspace_bytes is what the library makes best use of (bounded: 2.3 GiB, or what the
- * largest matrix needs), mfsdp_muon_workspace_bytes of the largest job is the least it takes.  Every job is checked before
+ * through each stage of the update as one launch, so that small ones fill the machine together; one that fills it by itself
+ * (a short side beyond 4864 on 256 CUs) has launches of its own.  How many go together is a matter of the workspace:
+ * mfsdp_muon_many_workspace_bytes is what the library makes best use of (bounded: 1.4 GiB, or what the largest matrix
+ * needs), mfsdp_muon_workspace_bytes of the largest job is the least it takes.  Every job is checked before
  * anything is enqueued.  Results do not depend on the other jobs beyond the summation order inside a product (how its
  * K is cut), and not at all where every side is at most 1024.
  */

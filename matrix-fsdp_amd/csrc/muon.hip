@@ -17,7 +17,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <utility>
 #include <vector>
 
 namespace mfsdp {
@@ -72,9 +71,16 @@ static_assert(kMaxMuonGroup <= kMaxGemmGroup && kMaxMuonGroup * sizeof(float) <=
 // the sums of squares of the momentum kernel are consumed by the norm before the first product runs
 static_assert(static_cast<int64_t>(kMaxMuonGroup) * kMuonMaxPartials * 4 <= kGemmPartialsBytes, "the partial sums borrow the products' scratch");
 
-// Most workspace a group is given beyond what its largest matrix needs anyway: three 15360 x 5120 matrices.  Matrices
-// that large fill the machine on their own, more of them side by side only cost memory.
-constexpr int64_t kGroupBytes = 2304ll << 20;
+// Most workspace a group is given beyond what its largest matrix needs anyway: three 12288 x 4096 matrices.
+constexpr int64_t kGroupBytes = 1344ll << 20;
+
+// Does the triangle of 256 x 256 tiles of the matrix's symmetric products occupy three quarters of the CUs?  Such a matrix
+// goes through the stages on its own: others beside it would cost their workspace and gain next to nothing (15360 x 5120
+// and 5120 x 13824 in bf16 together 11.01 ms with 1.4 GiB, one after the other 11.33 ms with 0.75 GiB).
+bool fills_machine(const Matrix& w) {
+  const int t = w.mp / 256;
+  return 4 * (t * (t + 1) / 2) >= 3 * device_cu_count();
+}
 
 // A group of matrices that go through every stage of the update together, one launch per stage.
 struct Group {
@@ -249,6 +255,27 @@ int run_step(Group* g, char* shared, const StepArgs& s, hipStream_t stream) {
   return MFSDP_OK;
 }
 
+// A matrix of a call that waits for its group.
+struct Pending {
+  bool alone;  // see fills_machine
+  int64_t bytes;
+  int64_t job;
+};
+
+// Those that go alone first, then the largest first, so that a group holds matrices of like size; equals in the order given.
+void sort_pending(std::vector<Pending>* order) {
+  std::stable_sort(order->begin(), order->end(), [](const Pending& x, const Pending& y) { return x.alone != y.alone ? x.alone : x.bytes > y.bytes; });
+}
+
+// The group that starts at `first` ends before the returned position: as many as one launch carries and `room` holds, at
+// least one.
+size_t group_end(const std::vector<Pending>& order, size_t first, int64_t room, int64_t* bytes) {
+  size_t end = first + 1;
+  *bytes = order[first].bytes;
+  while (!order[first].alone && end < order.size() && end - first < kMaxMuonGroup && *bytes + order[end].bytes <= room) *bytes += order[end++].bytes;
+  return end;
+}
+
 }  // namespace
 }  // namespace mfsdp
 
@@ -261,14 +288,20 @@ extern "C" int64_t mfsdp_muon_workspace_bytes(int64_t rows, int64_t cols) {
 
 extern "C" int64_t mfsdp_muon_many_workspace_bytes(int64_t n, const int64_t* rows, const int64_t* cols) {
   if (n <= 0 || rows == nullptr || cols == nullptr) return 0;
-  int64_t sum = 0, largest = 0;
+  std::vector<Pending> order;
   for (int64_t i = 0; i < n; ++i) {
     Matrix w;
     if (!plan_matrix(rows[i], cols[i], nullptr, &w)) return 0;
-    sum += w.bytes;
-    largest = std::max(largest, w.bytes);
+    order.push_back(Pending{fills_machine(w), w.bytes, i});
   }
-  return std::max(largest, std::min(sum, kGroupBytes)) + kSharedBytes;
+  sort_pending(&order);
+  int64_t largest = 0;
+  for (size_t next = 0; next < order.size();) {
+    int64_t bytes = 0;
+    next = group_end(order, next, kGroupBytes, &bytes);
+    largest = std::max(largest, bytes);
+  }
+  return largest + kSharedBytes;
 }
 
 extern "C" int64_t mfsdp_muon_executed_flops(int64_t rows, int64_t cols, int steps, int flags) {
@@ -336,29 +369,27 @@ extern "C" int mfsdp_muon_step_many(int64_t n, const mfsdp_muon_job* jobs, int d
   if (n == 0) return MFSDP_OK;
   const StepArgs s{dtype, momentum, nesterov, a, b, c, steps, eps, false};
   if (int rc = check_step(s)) return rc;
-  std::vector<std::pair<int64_t, int64_t>> order;  // (bytes, job): the largest first, so that a group holds matrices of like size
+  std::vector<Pending> order;
   int64_t largest = 0;
   for (int64_t i = 0; i < n; ++i) {
     Matrix w;
     if (int rc = check_matrix(jobs[i].rows, jobs[i].cols, steps, &w)) return rc;
     if (int rc = check_tensors(jobs[i].param, jobs[i].grad, jobs[i].momentum_buf, dtype, jobs[i].lr, jobs[i].weight_decay)) return rc;
-    order.emplace_back(w.bytes, i);
+    order.push_back(Pending{fills_machine(w), w.bytes, i});
     largest = std::max(largest, w.bytes);
   }
   if (int rc = check_workspace(workspace, workspace_bytes, largest + kSharedBytes)) return rc;
-  std::stable_sort(order.begin(), order.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+  sort_pending(&order);
   char* base = static_cast<char*>(workspace);
-  const int64_t room = workspace_bytes - kSharedBytes;
   for (size_t next = 0; next < order.size();) {
     Group g;
-    int64_t used = 0;
-    while (next < order.size() && g.n < kMaxMuonGroup && used + order[next].first <= room) {
-      const mfsdp_muon_job& job = jobs[order[next].second];
+    int64_t bytes = 0, used = 0;
+    for (const size_t end = group_end(order, next, workspace_bytes - kSharedBytes, &bytes); next < end; ++next) {
+      const mfsdp_muon_job& job = jobs[order[next].job];
       Matrix w;
       plan_matrix(job.rows, job.cols, base + used, &w);
       add_to_group(&g, w, job.param, job.grad, job.momentum_buf, job.lr, job.weight_decay, job.adjusted_lr);
       used += w.bytes;
-      ++next;
     }
     if (int rc = run_step(&g, base + used, s, as_stream(stream))) return rc;
   }

@@ -219,7 +219,7 @@ def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, pool: MuonSt
 
     The matrices of a rank are independent of each other, so those that share their hyper-parameters (the learning
     rate and weight decay may differ) go through every stage of the update as one launch, up to 32 at a time and as many
-    as 2.3 GiB of workspace hold (``mfsdp_muon_step_many``): small matrices fill the machine together and the number of
+    as 1.4 GiB of workspace hold (``mfsdp_muon_step_many``; one that fills the machine goes alone): small matrices fill the machine together and the number of
     launches does not grow with theirs.
 
     Reproducibility: how the K walk of a product is cut into pieces, and with it the order of its fp32 sums and the last

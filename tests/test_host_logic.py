@@ -559,3 +559,26 @@ def test_muon_refuses_long_sides_before_anything_is_enqueued():
             assert rc == 3 and b"2^22" in lib.mfsdp_last_error(), (rows, cols, rc)
         assert single(rows, cols, steps=0) == orthogonalise(rows, cols, steps=0) == many([(64, 64), (rows, cols)], steps=0) == 2
     assert single(8, limit) == orthogonalise(limit, 8) == many([(64, 64), (8, limit)]) == 2
+
+
+@pytest.mark.parametrize(
+    "shapes, like",
+    [
+        ([(15360, 5120), (5120, 13824)] * 3, 1),          # each fills the machine: the scratch of the largest alone
+        ([(5120, 5120), (12288, 4096), (64, 64)] * 4, 3),
+        ([(12288, 4096), (11008, 4096), (4096, 4096)] * 8, 3),
+        ([(4096, 11008)], 1),
+        ([(8, 8)] * 100, 32),
+    ],
+)
+def test_muon_scratch_of_many_matrices_is_bounded(shapes, like):
+    """The workspace ``muon_step_many`` allocates: no more than ``like`` workspaces of the largest matrix, and never more
+    than three of a 12288 x 4096 one unless a single matrix needs it."""
+    lib = _lib.lib()
+    column = lambda k: (ctypes.c_int64 * len(shapes))(*(s[k] for s in shapes))
+    need = lib.mfsdp_muon_many_workspace_bytes(len(shapes), column(0), column(1))
+    largest = max(lib.mfsdp_muon_workspace_bytes(*s) for s in shapes)
+    assert largest <= need <= like * largest
+    assert need <= max(largest, 3 * lib.mfsdp_muon_workspace_bytes(12288, 4096))
+    if like == 1:
+        assert need == largest

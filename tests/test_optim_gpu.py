@@ -420,6 +420,27 @@ def test_muon_group_with_a_side_too_long_is_refused_whole():
     torch.cuda.empty_cache()  # the workspace of the long matrix
 
 
+def test_muon_step_many_machine_filling_matrices_go_alone():
+    """Two matrices that fill the machine between small ones: they get the bits of a call of their own and the small ones
+    those of a call without them, whether or not the workspace has room for more."""
+    shapes = [(64, 96), (4865, 5120), (300, 520), (5120, 4900), (96, 64)]
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
+    params = [make(sh, 940 + i, 0.02).to(DEV) for i, sh in enumerate(shapes)]
+    grads = [make(sh, 945 + i).to(DEV) for i, sh in enumerate(shapes)]
+
+    def update(which, workspace=None):
+        ps, bs = [params[i].clone() for i in which], [torch.zeros_like(params[i]) for i in which]
+        F.muon_step_many([(p, grads[i], b, kw) for i, p, b in zip(which, ps, bs)], workspace=workspace)
+        return dict(zip(which, ps))
+
+    want = {**update([0, 2, 4]), **update([1]), **update([3])}
+    roomy = F.MuonWorkspace(DEV)
+    roomy.get_bytes(3 * F.muon_workspace_bytes(5120, 5120))
+    for workspace in (None, roomy):
+        have = update(list(range(5)), workspace)
+        assert all(torch.equal(have[i], want[i]) for i in range(5))
+
+
 def test_muon_group_with_cut_k_walks():
     """Sides beyond 1024, where the tiles of the last round are cut along K: several K in one launch, against the oracle."""
     shapes = [(192, 1088), (130, 2100), (4160, 200), (70, 8200)]
