@@ -105,9 +105,12 @@ __device__ __forceinline__ void update_param8(const GemmProblem& a, int dtype, i
 
 // Kernel argument: the problems of a launch and which workgroup does what.  Block ids [0, tile_begin[n]) compute one
 // whole tile each, problem after problem (longest K first); behind them come the K pieces of the split tiles.
-// Two sizes: a launch of up to N = 8 problems, the usual number, is 0.8 us shorter with 1 KiB of arguments than with the
-// 4 KiB that 32 problems take (empty kernels: 2.9 against 3.7 us), and has fewer entries to search (whole Muon
-// step: five ragged matrices 342 -> 330 us, two of 2048x5000 1101 -> 1077, a hidden2048 layer 2092 -> 2067).
+// Three sizes.  One problem: nothing is searched and every field sits at a fixed place, so that a workgroup's first loads need
+// no address from an earlier one (a product is 0.8 to 1.0 us shorter than with the table of eight; whole Muon step of one
+// matrix: 2048x2048 413 -> 402 us, 4096x4096 1300 -> 1285, 1024x4096 256 -> 246).  Up to 8, the usual number of several: 0.8 us
+// shorter with 1 KiB of arguments than with the 4 KiB that 32 problems take (empty kernels: 2.9 against 3.7 us), and fewer
+// entries to search (whole Muon step: five ragged matrices 342 -> 330 us, two of 2048x5000 1101 -> 1077, a hidden2048 layer
+// 2092 -> 2067).
 template <int N>
 struct LaunchArgs {
   int tile_begin[N + 1];   // first whole-tile block of a problem; entries past n repeat the end
@@ -129,6 +132,7 @@ static_assert(sizeof(LaunchArgs<kMaxGemmGroup>) <= 4096, "kernel arguments are l
 // dependent loads would wait out the memory latency at every step).
 template <int N>
 __device__ __forceinline__ int problem_of(const int (&begin)[N], int n, int block) {
+  if constexpr (N == 2) return 0;  // a launch for one problem
   if (n == 1) return 0;  // fewer classes than problems: their entries past the last repeat the end, too
   int p = 0;
 #pragma unroll
@@ -1120,13 +1124,14 @@ int gemm_nt_bf16(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& sc
     return g.n <= 2   ? launch_small<2>(g, plan, tuning, stream)
            : g.n <= 8 ? launch_small<8>(g, plan, tuning, stream)
                       : launch_small<kMaxGemmGroup>(g, plan, tuning, stream);
-  const bool few = g.n <= 8;
   if (plan.variant == 2)  // 128x128 tile, 4 waves of 64x64, two workgroups per CU
-    return few ? launch<128, 128, 2, 2, 64, 2, 2, 8>(g, plan, scratch, tuning, stream)
-               : launch<128, 128, 2, 2, 64, 2, 2, kMaxGemmGroup>(g, plan, scratch, tuning, stream);
+    return g.n == 1  ? launch<128, 128, 2, 2, 64, 2, 2, 1>(g, plan, scratch, tuning, stream)
+           : g.n <= 8 ? launch<128, 128, 2, 2, 64, 2, 2, 8>(g, plan, scratch, tuning, stream)
+                      : launch<128, 128, 2, 2, 64, 2, 2, kMaxGemmGroup>(g, plan, scratch, tuning, stream);
   // 256x256 tile, 8 waves of 128x64, one workgroup per CU
-  return few ? launch<256, 256, 2, 4, 64, 2, 1, 8>(g, plan, scratch, tuning, stream)
-             : launch<256, 256, 2, 4, 64, 2, 1, kMaxGemmGroup>(g, plan, scratch, tuning, stream);
+  return g.n == 1  ? launch<256, 256, 2, 4, 64, 2, 1, 1>(g, plan, scratch, tuning, stream)
+         : g.n <= 8 ? launch<256, 256, 2, 4, 64, 2, 1, 8>(g, plan, scratch, tuning, stream)
+                    : launch<256, 256, 2, 4, 64, 2, 1, kMaxGemmGroup>(g, plan, scratch, tuning, stream);
 }
 
 }  // namespace mfsdp
