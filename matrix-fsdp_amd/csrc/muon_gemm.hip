@@ -151,12 +151,16 @@ __device__ __forceinline__ void tile_coords(int group_m, int logical, int tiles_
     *tn = logical - i * (i + 1) / 2;
     return;
   }
-  // Columns of kSuper tiles, walked down all rows in blocks of group_m x kSuper / 2 tiles: what the whole machine works on
-  // at a time is then nearly square (16 x 16 tiles where a round has 256), and so is what one XCD works on.
+  // Super columns of up to kSuper tiles, all of nearly one width, walked down all rows in blocks of group_m x half a width:
+  // what the whole machine works on at a time is then nearly square (16 x 16 tiles where a round has 256), and so is what
+  // one XCD works on.  Widths as even as they come: a last super column of 4 of 20 tiles makes an XCD's share of it tall and
+  // narrow, which reads more panels (256-tiles of 5120 x 5120 253 -> 241 us, of 5120 x 13824 603 -> 594 with 14, 14, 14, 12
+  // instead of 16, 16, 16, 6).
   constexpr int kSuper = 16;
-  const int per_super = kSuper * tiles_m;
+  const int supers = (tiles_n + kSuper - 1) / kSuper, width = (tiles_n + supers - 1) / supers;
+  const int per_super = width * tiles_m;
   const int super = logical / per_super;
-  const int first_n = super * kSuper, cols = min(kSuper, tiles_n - first_n);
+  const int first_n = super * width, cols = min(width, tiles_n - first_n);
   int in = logical - super * per_super;
   const int band = in / (group_m * cols);  // group_m rows of this super column
   const int first_m = band * group_m, rows = min(group_m, tiles_m - first_m);
