@@ -76,7 +76,7 @@ constexpr int64_t kGroupBytes = 1344ll << 20;
 
 // Does the triangle of 256 x 256 tiles of the matrix's symmetric products occupy three quarters of the CUs?  Such a matrix
 // goes through the stages on its own: others beside it would cost their workspace and gain next to nothing (15360 x 5120
-// and 5120 x 13824 in bf16 together 11.01 ms with 1.4 GiB, one after the other 11.33 ms with 0.75 GiB).
+// and 5120 x 13824 in bf16 together 11.14 ms with 1.4 GiB, one after the other 11.27 ms with 0.75 GiB).
 bool fills_machine(const Matrix& w) {
   const int t = w.mp / 256;
   return 4 * (t * (t + 1) / 2) >= 3 * device_cu_count();

@@ -880,21 +880,26 @@ int tile_count(const GemmGroup& g, const GemmProblem& p, int tile) {
   return g.symmetric ? tm * (tm + 1) / 2 : tm * tn;
 }
 
-// Below this many slabs a tile is never cut: the pieces would be gone before the fix-up launch (4-5 us) has paid off.
+// Below this many slabs a tile is never cut: the pieces would be gone before the fix-up launch (4 us and more) has paid off.
 constexpr int kMinSplitSlabs = 17;
 
-// What a tile variant costs, in microseconds: one slab of a tile when every CU holds as many workgroups as it can
-// (slab_us) and when it holds one (lone_slab_us), prologue and epilogue of a tile (tile_us).  From kernel traces: 256 x 256
-// tiles with K = 4096 take 102 us a round, two 128 x 128 tiles per CU 0.95 us a slab.  The choice they make is the faster
-// one on every group measured (whole Muon step, symmetric / general products forced to 256 or 128): hidden4096 7.28 ms
-// against 7.85 / 8.09 with small tiles, two hidden5120 matrices 11.0 against 12.1 / 12.8, five small ragged ones 0.344
-// against 0.427 / 0.406 with big ones, 24 of 1536 x 1024 1.23 against 1.27 / 1.29 with small ones.
+// What a tile variant costs, in microseconds: one slab of a tile when few CUs are busy (lone_slab_us: for the variant with two
+// workgroups per CU, while each has one of its own) and when the machine is full (slab_us: power and LDS shared by all; in
+// between it grows with the workgroups of the launch), prologue and epilogue of a tile (tile_us).  The constants, and those of
+// the fix-up launch below, follow 682 traced products: 25 matrices of 512 to 13824, both tiles, whole and cut into 2 to 16
+// pieces (11 % rms; the plans they choose are 1.7 % slower than the best measured one in the mean.  With one rate for every
+// launch beyond a workgroup per CU it was 23 % and 3.3 %, and the gram product of 2560 x 6912 was not cut: 69 us where two
+// pieces take 55).  The tile they choose
+// is the faster one on the groups measured (whole Muon step, symmetric / general products forced to 256 or 128):
+// hidden4096 7.28 ms against 7.85 / 8.09 with small tiles, two hidden5120 matrices 11.0 against 12.1 / 12.8, five small ragged
+// ones 0.344 against 0.427 / 0.406 with big ones, 24 of 1536 x 1024 1.23 against 1.27 / 1.29 with small ones.
 constexpr int kSmallVariant = 4;
 struct Variant {
   int tile, per_cu;
   double slab_us, lone_slab_us, tile_us;
 };
-constexpr Variant kVariants[5] = {{}, {256, 1, 1.45, 1.45, 9.0}, {128, 2, 0.95, 0.60, 5.0}, {}, {kSmallTile, 1, 0.43, 0.43, 5.0}};
+constexpr Variant kVariants[5] = {{}, {256, 1, 1.35, 1.00, 8.6}, {128, 2, 0.86, 0.65, 4.7}, {}, {kSmallTile, 1, 0.45, 0.45, 4.6}};
+constexpr double kFixupUs = 3.2, kFixupBytesPerUs = 3.0e6;  // of the fix-up launch: its partial tiles written and read again
 
 // When the workgroups of a launch end, if each starts on the slot that is free first (as they do, in block order).
 // Slots are kept as groups that are free at the same time; a launch of equal tiles costs a few steps per round.
@@ -954,13 +959,13 @@ GemmPlan make_plan(const GemmGroup& g, int variant, const GemmScratch& scratch, 
       blocks += tiles[i] + rest[i] * (splits[i] - 1);
     }
     if (piece > 0 && (partial == 0 || partial > 0x7fffffff || partial * tile_bytes > static_cast<double>(scratch.partials_bytes))) return;
-    const double slab_us = blocks <= cus ? v.lone_slab_us : v.slab_us;
+    const double full = std::min(1.0, std::max(0.0, static_cast<double>(blocks) / cus - (v.per_cu - 1)));
+    const double slab_us = v.lone_slab_us + (v.slab_us - v.lone_slab_us) * full;
     SlotTimes times(slots);
     for (int i = 0; i < g.n; ++i) times.add(tiles[i] - (splits[i] > 1 ? rest[i] : 0), slabs[i] * slab_us + v.tile_us);
     for (int i = 0; i < g.n; ++i)
       if (splits[i] > 1) times.add(rest[i] * splits[i], (slabs[i] + splits[i] - 1) / splits[i] * slab_us + v.tile_us);
-    // the fix-up launch: 4 us, and the partial tiles written and read again at about 5 TB/s
-    const double us = times.end() + (partial > 0 ? 4.0 + partial * tile_bytes * 2.0 / 5.0e6 : 0.0);
+    const double us = times.end() + (partial > 0 ? kFixupUs + partial * tile_bytes / kFixupBytesPerUs : 0.0);
     if (piece > 0 && us >= plan.us) return;
     plan.us = us;
     for (int i = 0; i < g.n; ++i) {
