@@ -69,7 +69,8 @@ bool plan_matrix(int64_t rows, int64_t cols, char* base, Matrix* w) {
 constexpr int64_t kSharedBytes = kAlign + kGemmPartialsBytes;
 static_assert(kMaxMuonGroup <= kMaxGemmGroup && kMaxMuonGroup * sizeof(float) <= kAlign, "a group travels through both kinds of launch");
 // the sums of squares of the momentum kernel are consumed by the norm before the first product runs
-static_assert(static_cast<int64_t>(kMaxMuonGroup) * kMuonMaxPartials * 4 <= kGemmPartialsBytes, "the partial sums borrow the products' scratch");
+static_assert(kMuonMaxPartials % 4 == 0 && static_cast<int64_t>(kMaxMuonGroup) * kMuonMaxPartials * 4 <= kGemmPartialsBytes,
+              "the partial sums borrow the products' scratch");
 
 // Most workspace a group is given beyond what its largest matrix needs anyway: three 12288 x 4096 matrices.
 constexpr int64_t kGroupBytes = 1344ll << 20;
@@ -111,7 +112,7 @@ void finish_group(Group* g, char* shared) {
     m.cols = w.cols;
     m.n_partials = muon_momentum_partials(static_cast<int64_t>(w.rows) * w.cols);
     m.partials = partials;
-    partials += m.n_partials;
+    partials += round_up(m.n_partials, 4);  // the norm reads groups of four
   }
 }
 

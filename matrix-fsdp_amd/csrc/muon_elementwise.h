@@ -18,7 +18,7 @@ struct MuonMatrix {
   uint16_t* xraw;    // rows x cols unscaled bf16 update
   uint16_t* same;
   uint16_t* trans;
-  float* partials;   // sums of squares, one per workgroup of the momentum kernel
+  float* partials;   // sums of squares, one per workgroup of the momentum kernel; 16-byte aligned
   int n_partials;
   int rows, cols;
   int ld_same, ld_trans;

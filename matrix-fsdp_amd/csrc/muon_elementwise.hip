@@ -396,6 +396,8 @@ int muon_momentum(const MuonMatrices& g, int dtype, double momentum, int nestero
   // the scalars torch hands to lerp_ are the Python doubles 1 - momentum and momentum, rounded to fp32 by the kernel
   const float one_minus = static_cast<float>(1.0 - momentum);
   const float weight = static_cast<float>(momentum);
+  for (int i = 0; i < g.n; ++i)  // the norm kernel reads them four at a time
+    if (reinterpret_cast<uintptr_t>(g.m[i].partials) % 16) return fail(MFSDP_ERR_INVALID, "muon_momentum: partial sums must be 16-byte aligned");
   GroupArgs args;
   const dim3 grid(fill_group(&args, g, [](const MuonMatrix& m) { return m.n_partials; }));
 #define MFSDP_MOMENTUM(T_, MOM_) \

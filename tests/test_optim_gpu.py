@@ -441,6 +441,27 @@ def test_muon_step_many_machine_filling_matrices_go_alone():
         assert all(torch.equal(have[i], want[i]) for i in range(5))
 
 
+def test_muon_group_with_ragged_partial_sums():
+    """Matrices whose numbers of partial sums leave every remainder by four, beside ones so large that the norms are summed
+    by a launch of their own: the oracle's update and momentum."""
+    shapes = [(1, 7), (33, 70), (40, 60), (20, 200), (777, 1411), (600, 900), (1, 700)]
+    partials = [max(1, -(-(r * c // 4) // 128)) for r, c in shapes]
+    assert {n % 4 for n in partials} == {0, 1, 2, 3} and max(partials) > 1024
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
+    params = [make(sh, 600 + i, 0.02) for i, sh in enumerate(shapes)]
+    grads = [make(sh, 610 + i, 1e-3 * 4.0**i) for i, sh in enumerate(shapes)]  # norms far apart
+    bufs = [make(sh, 620 + i, 1e-3 * 4.0**i) for i, sh in enumerate(shapes)]
+    for order in (range(len(shapes)), reversed(range(len(shapes)))):
+        order = list(order)
+        dev_p, dev_b = [params[i].to(DEV) for i in order], [bufs[i].to(DEV) for i in order]
+        F.muon_step_many([(p, grads[i].to(DEV), b, kw) for i, p, b in zip(order, dev_p, dev_b)])
+        for i, p, b in zip(order, dev_p, dev_b):
+            p_ref, b_ref = params[i].clone(), bufs[i].clone()
+            O.muon_step(p_ref, grads[i], b_ref, **kw)
+            assert rel_fro(p.cpu() - params[i], p_ref - params[i]) < MUON_TOL, shapes[i]
+            assert torch.allclose(b.cpu(), b_ref, rtol=1e-6, atol=1e-6 * float(b_ref.abs().max()))
+
+
 def test_muon_group_with_cut_k_walks():
     """Sides beyond 1024, where the tiles of the last round are cut along K: several K in one launch, against the oracle."""
     shapes = [(192, 1088), (130, 2100), (4160, 200), (70, 8200)]
