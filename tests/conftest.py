@@ -25,6 +25,28 @@ def pytest_collection_modifyitems(config, items):
             item.add_marker(skip)
 
 
+def _muon_tiles():
+    """What the tile choice shows: the flops a step of some sizes executes (the flops of a product depend on its tile)."""
+    from matrix_fsdp_amd import _lib
+
+    return [_lib.lib().mfsdp_muon_executed_flops(*shape, 1, 0) for shape in ((300, 520), (1000, 3000), (2050, 2050), (5120, 5120))]
+
+
+_DEFAULT_MUON_TILES = []
+
+
+@pytest.fixture(autouse=True)
+def default_muon_tuning(request):
+    """A GPU test that selects kernels leaves the library's own choice behind for the tests after it."""
+    if "gpu" not in request.keywords:
+        yield
+        return
+    if not _DEFAULT_MUON_TILES:
+        _DEFAULT_MUON_TILES.extend(_muon_tiles())
+    yield
+    assert _muon_tiles() == _DEFAULT_MUON_TILES, "the test left mfsdp_set_muon_tuning changed"
+
+
 @pytest.fixture(scope="session")
 def golden():
     with open(os.path.join(ROOT, "tests", "golden", "reference_vectors.json")) as f:

@@ -306,7 +306,7 @@ def test_tile_variants_forced(shape, variant, general):
     try:
         have = F.newton_schulz(u.to(DEV)).float().cpu()
     finally:
-        _lib.lib().mfsdp_set_muon_tuning(1, 3, 0, 0, 0)
+        _lib.lib().mfsdp_set_muon_tuning(3, 3, 0, 0, 0)
     assert rel_fro(have, want) < MUON_TOL
 
 
