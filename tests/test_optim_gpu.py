@@ -537,15 +537,44 @@ def test_muon_small_tiles_against_the_oracle(shapes, dtype):
             _lib.lib().mfsdp_set_muon_tuning(variant, variant, 0, 0, 0)
             p, b = [t.to(DEV) for t in params], [t.to(DEV) for t in bufs]
             F.muon_step_many([(pi, g.to(DEV), bi, kw) for pi, g, bi in zip(p, grads, b)])
-            results.append(p)
+            results.append((p, b))
     finally:
         _lib.lib().mfsdp_set_muon_tuning(3, 3, 0, 0, 0)
-    for i in range(0, len(shapes), 8):
+    for i in range(len(shapes)):
         want_p, want_b = params[i].clone(), bufs[i].clone()
         O.muon_step(want_p, grads[i], want_b, **kw)
         step = (want_p.double() - params[i].double()).norm()
         # bf16 rounding of the five iterations' products in another order: the bar the other variants are held to; a bf16
         # parameter adds its own rounding, 2^-9 of its value on either side
         bar = 1e-2 * step + (0.0 if dtype == torch.float32 else 2.0**-8 * params[i].double().norm())
-        for have in results:
-            assert (have[i].double().cpu() - want_p.double()).norm() <= bar, shapes[i]
+        for have_p, have_b in results:
+            assert (have_p[i].double().cpu() - want_p.double()).norm() <= bar, shapes[i]
+            # one lerp in fp32, in bf16 rounded once: a last bit where the host fuses a multiply-add
+            assert rel_fro(have_b[i], want_b) < (1e-6 if dtype == torch.float32 else 4e-3), shapes[i]
+
+
+@pytest.mark.parametrize("variant", [1, 2, 3])
+def test_muon_many_matrices_of_several_k_over_several_rounds(variant):
+    """Thirteen matrices in one launch per stage (the argument table of 32), of three K lengths in every product, with more
+    tiles than the machine holds at a time (update product: 423 of 256 x 256, 1479 of 128 x 128), wide and tall, by 256 and
+    128 tiles and as the library chooses: ``torch.optim.Muon`` on this GPU, every matrix and its momentum."""
+    from matrix_fsdp_amd import _lib
+
+    shapes = [(1024, 1024), (1100, 2100), (4100, 640)] * 2 + [(1024, 1024), (2100, 1100)] * 2 + [(1024, 1024), (2100, 1100), (1024, 1024)]
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
+    params, grads, bufs = ([make(sh, base + i, std).to(DEV) for i, sh in enumerate(shapes)] for base, std in ((1000, 0.02), (1020, 1e-3), (1040, 1e-3)))
+    have_p, have_b = [p.clone() for p in params], [b.clone() for b in bufs]
+    _lib.lib().mfsdp_set_muon_tuning(variant, variant, 0, 0, 0)
+    try:
+        F.muon_step_many([(p, g, b, kw) for p, g, b in zip(have_p, grads, have_b)])
+    finally:
+        _lib.lib().mfsdp_set_muon_tuning(3, 3, 0, 0, 0)
+    torch_params = [torch.nn.Parameter(p.clone()) for p in params]
+    optimizer = torch.optim.Muon(torch_params, **kw)
+    for p, g, b in zip(torch_params, grads, bufs):
+        optimizer.state[p]["momentum_buffer"] = b.clone()
+        p.grad = g
+    optimizer.step()
+    for i, p in enumerate(torch_params):
+        assert rel_fro(have_p[i] - params[i], p.detach() - params[i]) < MUON_TOL, (i, shapes[i])
+        assert torch.allclose(have_b[i], optimizer.state[p]["momentum_buffer"], rtol=1e-6, atol=1e-9)
