@@ -265,8 +265,9 @@ int mfsdp_muon_step_ex(void* param, const void* grad, void* momentum_buf, int dt
  * (a short side beyond 4864 on 256 CUs) has launches of its own.  How many go together is a matter of the workspace:
  * mfsdp_muon_many_workspace_bytes is what the library makes best use of (bounded: 1.4 GiB, or what the largest matrix
  * needs), mfsdp_muon_workspace_bytes of the largest job is the least it takes.  Every job is checked before
- * anything is enqueued.  Results do not depend on the other jobs beyond the summation order inside a product (how its
- * K is cut), and not at all where every side is at most 1024.
+ * anything is enqueued.  Results depend on the other jobs, and on the workspace, only through the order in which a product
+ * sums: which tile a launch takes and how its K walk is cut follow from all matrices of the launch, at any size.  The
+ * momentum does not depend on them.  A caller that needs bits independent of the other matrices makes one call per matrix.
  */
 typedef struct mfsdp_muon_job {
   void* param;

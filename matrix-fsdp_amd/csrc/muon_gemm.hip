@@ -410,8 +410,8 @@ gemm_nt_kernel(LaunchArgs<N> args) {
   // the rows of kTilesPerSlab MFMA tile rows of the waves with wave_m == q / kSlabsPerWave; a lane's four rows of one
   // column are four consecutive k of one slab row: one 64-bit LDS read per MFMA tile, in two batches that are read at the
   // start of a half step and added at its end, so that every tile row gets its D between its two MFMAs of the slab.
-  // Every tile variant therefore adds in the same order: the bits of a result do not depend on the tile it was computed
-  // in (only on whether its K walk was cut into pieces).
+  // The 256 and the 128 tiles therefore add in the same order: a result has the same bits in either (unless its K walk was
+  // cut into pieces; the 64 tiles, whose waves share K and add D at the end, sum in an order of their own).
   constexpr int kTilesPerSlab = BK / 16;
   constexpr int kSlabsPerWave = kWaveM / BK;
   constexpr int kDSlabs = BM / BK;

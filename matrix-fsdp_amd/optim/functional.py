@@ -219,13 +219,13 @@ def muon_step_many(jobs, *, workspace: MuonWorkspace | None = None, pool: MuonSt
 
     The matrices of a rank are independent of each other, so those that share their hyper-parameters (the learning
     rate and weight decay may differ) go through every stage of the update as one launch, up to 32 at a time and as many
-    as 1.4 GiB of workspace hold (``mfsdp_muon_step_many``; one that fills the machine goes alone): small matrices fill the machine together and the number of
-    launches does not grow with theirs.
+    as 1.4 GiB of workspace hold (``mfsdp_muon_step_many``; one that fills the machine goes alone): small matrices fill
+    the machine together and the number of launches does not grow with theirs.
 
-    Reproducibility: how the K walk of a product is cut into pieces, and with it the order of its fp32 sums and the last
-    bits of an update, may depend on the other matrices of the call.  Both forms meet
-    the same parity bar; a caller that needs bits independent of the optimizer's other parameters passes
-    ``side_by_side=False`` (or sets ``MATRIX_FSDP_MUON_SIDE_BY_SIDE=0``), which updates one matrix after the other.
+    Reproducibility: which tiles a product takes and how its K walk is cut into pieces, and with them the order of its
+    fp32 sums and the last bits of an update, depend on the other matrices of the call.  Both forms meet the same parity
+    bar; a caller that needs bits independent of the optimizer's other parameters passes ``side_by_side=False`` (or sets
+    ``MATRIX_FSDP_MUON_SIDE_BY_SIDE=0``), which updates one matrix after the other.
 
     With a ``pool`` the matrices take launches of their own on the pool's streams instead: those that leave CUs idle, when
     there are at least two of them (all of them with ``side_by_side=True``), the others one after the other on the calling

@@ -156,9 +156,9 @@ def test_muon_step_matches_torch_optim_muon_on_device_inputs():
 
 
 def test_muon_step_many_matches_one_matrix_at_a_time():
-    """Independent matrices spread over side streams: the same bits as one call per matrix on the calling stream (for
-    matrices this small the flag does not change the tiling), work enqueued afterwards sees the updates, and an
-    optimizer over several parameter groups goes the same way."""
+    """Independent matrices of two sets of hyper-parameters, which share launches with their like: the same bits as one
+    call per matrix (together they are few enough for the 64 x 64 tiles that each takes alone), work enqueued afterwards
+    sees the updates, and an optimizer over several parameter groups goes the same way."""
     shapes = [(512, 768), (768, 512), (256, 256), (320, 200), (1024, 512)]
     hypers = [dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True), dict(lr=0.01, weight_decay=0.0, momentum=0.9, nesterov=False, adjust_lr_fn="match_rms_adamw")]
     params = [make(sh, 100 + i, 0.02) for i, sh in enumerate(shapes)]
@@ -179,17 +179,17 @@ def test_muon_step_many_matches_one_matrix_at_a_time():
         assert rel_fro(many_p[i].cpu() - params[i], p_ref - params[i]) < MUON_TOL
     assert float(total) == float(sum(p.sum() for p in one_p))
     F.muon_step_many([])
-    F.muon_step_many([(many_p[0], dev_grads[0], many_b[0], hypers[0])])  # a single matrix stays on the calling stream
+    F.muon_step_many([(many_p[0], dev_grads[0], many_b[0], hypers[0])])
     F.muon_step(one_p[0], dev_grads[0], one_b[0], workspace=ws, **hypers[0])
     assert torch.equal(many_p[0], one_p[0])
 
 
-def test_muon_step_many_side_by_side_switch(monkeypatch):
-    """Matrices large enough that the side-by-side form changes the tiling of their symmetric products (m = 3072: the
-    triangle of 256 x 256 tiles occupies 78 of the CUs): with ``side_by_side=False`` (argument or environment) every
-    matrix gets the bits of a call of its own, whatever else the batch holds; the side-by-side form stays within the
-    parity bar of the same result."""
-    shapes = [(3072, 3072), (3072, 3328), (3072, 3072)]
+@pytest.mark.parametrize("shapes", [[(3072, 3072), (3072, 3328), (3072, 3072)], [(512, 512), (512, 300)] * 8])
+def test_muon_step_many_side_by_side_switch(monkeypatch, shapes):
+    """With ``side_by_side=False`` (argument or environment) every matrix gets the bits of a call of its own, whatever else
+    the call holds; sharing launches stays within the parity bar of the same result.  Matrices that change tiles and K
+    cuts together (m = 3072: the triangle of 256 x 256 tiles occupies 78 of the CUs), and sixteen small ones that are more
+    than one round of the 64 x 64 tiles each takes alone."""
     kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
     params = [make(sh, 400 + i, 0.02).to(DEV) for i, sh in enumerate(shapes)]
     grads = [make(sh, 500 + i).bfloat16().float().to(DEV) for i, sh in enumerate(shapes)]
@@ -214,7 +214,7 @@ def test_muon_step_many_side_by_side_switch(monkeypatch):
         ps, bs = batch(**how)
         for i in range(len(shapes)):
             assert rel_fro((ps[i] - params[i]).cpu(), (alone_p[i] - params[i]).cpu()) < MUON_TOL
-            assert torch.equal(bs[i], alone_b[i])  # the momentum does not depend on the tiling
+            assert torch.equal(bs[i], alone_b[i])  # the momentum depends on no product
 
 
 @pytest.mark.parametrize("side_by_side", [None, True, False])
@@ -353,7 +353,8 @@ def test_adamw_unaligned_views_and_errors():
 @pytest.mark.parametrize("short", [1, 63, 64, 65, 127, 129, 255, 257])
 def test_muon_group_at_tile_edges(short, dtype):
     """Matrices around the edges of 64, 128 and 256 tiles, wide and tall, in one launch per stage: the momentum and the
-    bits of a call of their own (every side is at most 1024, so no K walk is cut), and the oracle's update."""
+    bits of a call of their own (all of them together are within one round of 64 x 64 tiles, which each takes alone too,
+    and no K walk is cut), and the oracle's update."""
     shapes = [(short, short), (short, 200), (200, short), (short, 700), (700, short), (320, 256)]
     kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
     params = [make(sh, 800 + i, 0.02).to(dtype) for i, sh in enumerate(shapes)]
