@@ -23,6 +23,7 @@ CPU oracle (a port of the reference's per-segment slice-copy loops and of
 from __future__ import annotations
 
 import argparse
+import ctypes
 import json
 import os
 import sys
@@ -491,7 +492,11 @@ def main() -> int:
                 n_hold += 20
             held = (time.perf_counter() - t_hold) / n_hold * 1e3
             legs["muon_hidden4096"]["held"] = {"seconds": args.hold_muon_seconds, "ms_per_step": round(held, 4), "ns_TFLOPs_reference_flop_count": round(flops / (held * 1e-3) / 1e12, 1)}
-        executed = sum(int(_lib.lib().mfsdp_muon_executed_flops(sh[0], sh[1], 5, 0 if args.muon_form == "serial" else _lib.MUON_SHARED_MACHINE)) for sh in MUON_HIDDEN4096_SHAPES)
+        if args.muon_form == "serial":
+            executed = sum(int(_lib.lib().mfsdp_muon_executed_flops(sh[0], sh[1], 5, 0)) for sh in MUON_HIDDEN4096_SHAPES)
+        else:
+            sides = [(ctypes.c_int64 * len(mats))(*(sh[k] for sh in MUON_HIDDEN4096_SHAPES)) for k in (0, 1)]
+            executed = int(_lib.lib().mfsdp_muon_many_executed_flops(len(mats), *sides, 5, _lib.lib().mfsdp_muon_many_workspace_bytes(len(mats), *sides)))
         tflops_executed = executed / (med * 1e-3) / 1e12
         legs["muon_hidden4096"]["ns_TFLOPs_executed"] = round(tflops_executed, 1)
         result["roofline_muon"] = {

@@ -336,10 +336,13 @@ int mfsdp_adamw_step_many(int64_t n, const mfsdp_adamw_span* spans, double lr, d
 
 /*
  * Flops the Newton-Schulz kernels execute for `steps` iterations on a rows x cols matrix with the current tuning
- * and the flags of mfsdp_muon_step_ex (operands zero-padded to multiples of 256; the two symmetric products of a step compute only the tiles on or below
- * the diagonal).  The reference executes full products: steps * (4 m^2 n + 2 m^3) with m the short side.
+ * and the flags of mfsdp_muon_step_ex (sides rounded up to whole tiles, K to 64; the two symmetric products of a step
+ * compute only the tiles on or below the diagonal).  The reference executes full products: steps * (4 m^2 n + 2 m^3) with
+ * m the short side.  mfsdp_muon_many_executed_flops counts for mfsdp_muon_step_many with a workspace of that size, where
+ * the tile of a launch follows from all of its matrices; 0 where that call would refuse the sizes or the workspace.
  */
 int64_t mfsdp_muon_executed_flops(int64_t rows, int64_t cols, int steps, int flags);
+int64_t mfsdp_muon_many_executed_flops(int64_t n, const int64_t* rows, const int64_t* cols, int steps, int64_t workspace_bytes);
 
 /*
  * Measurement aid (no counterpart in the reference): one pass of pure reads (kind 0: `bytes` of src are loaded

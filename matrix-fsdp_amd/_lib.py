@@ -104,6 +104,7 @@ SIGNATURES = {
     "mfsdp_cast": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_void_p]),
     "mfsdp_muon_workspace_bytes": (c_int64, [c_int64, c_int64]),
     "mfsdp_muon_executed_flops": (c_int64, [c_int64, c_int64, c_int, c_int]),
+    "mfsdp_muon_many_executed_flops": (c_int64, [c_int64, POINTER(c_int64), POINTER(c_int64), c_int, c_int64]),
     "mfsdp_newton_schulz": (
         c_int,
         [c_void_p, c_int, c_int64, c_int64, c_float, c_float, c_float, c_int, c_float, c_void_p, c_void_p, c_int64, c_void_p],

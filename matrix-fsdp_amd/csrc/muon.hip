@@ -277,6 +277,26 @@ size_t group_end(const std::vector<Pending>& order, size_t first, int64_t room, 
   return end;
 }
 
+// Flops the products of one Newton-Schulz step of `n` matrices that share their launches execute.
+int64_t executed_flops(const Matrix* w, int n, bool shared) {
+  GemmGroup gram, poly, update;
+  gram.n = poly.n = update.n = n;
+  gram.symmetric = poly.symmetric = 1;
+  gram.shared = poly.shared = shared;
+  auto size = [](GemmProblem* p, int rows, int cols, int k) {
+    *p = GemmProblem{};
+    p->M = rows;
+    p->N = cols;
+    p->K = static_cast<int>(round_up(k, kTileK));
+  };
+  for (int i = 0; i < n; ++i) {
+    size(&gram.problem[i], w[i].m, w[i].m, w[i].n);
+    size(&poly.problem[i], w[i].m, w[i].m, w[i].m);
+    size(&update.problem[i], w[i].m, w[i].n, w[i].m);
+  }
+  return gemm_nt_executed_flops(gram) + gemm_nt_executed_flops(poly) + gemm_nt_executed_flops(update);
+}
+
 }  // namespace
 }  // namespace mfsdp
 
@@ -308,16 +328,28 @@ extern "C" int64_t mfsdp_muon_many_workspace_bytes(int64_t n, const int64_t* row
 extern "C" int64_t mfsdp_muon_executed_flops(int64_t rows, int64_t cols, int steps, int flags) {
   Matrix w;
   if (steps < 0 || !plan_matrix(rows, cols, nullptr, &w)) return 0;
-  GemmGroup gram, poly, update;
-  gram.n = poly.n = update.n = 1;
-  gram.symmetric = poly.symmetric = 1;
-  gram.shared = poly.shared = (flags & MFSDP_MUON_SHARED_MACHINE) != 0;
-  gram.problem[0] = poly.problem[0] = update.problem[0] = GemmProblem{};
-  auto size = [](GemmProblem& p, int64_t m, int64_t n, int64_t k) { p.M = static_cast<int>(m); p.N = static_cast<int>(n); p.K = static_cast<int>(round_up(k, kTileK)); };
-  size(gram.problem[0], w.m, w.m, w.n);
-  size(poly.problem[0], w.m, w.m, w.m);
-  size(update.problem[0], w.m, w.n, w.m);
-  return steps * (gemm_nt_executed_flops(gram) + gemm_nt_executed_flops(poly) + gemm_nt_executed_flops(update));
+  return steps * executed_flops(&w, 1, (flags & MFSDP_MUON_SHARED_MACHINE) != 0);
+}
+
+extern "C" int64_t mfsdp_muon_many_executed_flops(int64_t n, const int64_t* rows, const int64_t* cols, int steps, int64_t workspace_bytes) {
+  if (n <= 0 || rows == nullptr || cols == nullptr || steps < 0) return 0;
+  std::vector<Pending> order;
+  for (int64_t i = 0; i < n; ++i) {
+    Matrix w;
+    if (!plan_matrix(rows[i], cols[i], nullptr, &w) || w.bytes + kSharedBytes > workspace_bytes) return 0;
+    order.push_back(Pending{fills_machine(w), w.bytes, i});
+  }
+  sort_pending(&order);
+  int64_t flops = 0;
+  for (size_t next = 0; next < order.size();) {
+    Matrix w[kMaxMuonGroup];
+    int64_t bytes = 0;
+    int count = 0;
+    for (const size_t end = group_end(order, next, workspace_bytes - kSharedBytes, &bytes); next < end; ++next)
+      plan_matrix(rows[order[next].job], cols[order[next].job], nullptr, &w[count++]);
+    flops += executed_flops(w, count, false);
+  }
+  return steps * flops;
 }
 
 extern "C" int mfsdp_newton_schulz(const void* update, int update_dtype, int64_t rows, int64_t cols, float a, float b, float c,

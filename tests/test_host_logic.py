@@ -582,3 +582,26 @@ def test_muon_scratch_of_many_matrices_is_bounded(shapes, like):
     assert need <= max(largest, 3 * lib.mfsdp_muon_workspace_bytes(12288, 4096))
     if like == 1:
         assert need == largest
+
+
+def test_muon_executed_flops_of_many_matrices():
+    """The count for a list follows the launches of ``mfsdp_muon_step_many``: one matrix, matrices that go alone and a
+    workspace for one at a time count as single calls; sixteen small matrices share launches of larger tiles than each
+    takes alone; the three hidden4096 matrices too, still less than full products."""
+    lib = _lib.lib()
+
+    def many(shapes, workspace=None, steps=5):
+        sides = [(ctypes.c_int64 * len(shapes))(*(s[k] for s in shapes)) for k in (0, 1)]
+        return lib.mfsdp_muon_many_executed_flops(len(shapes), *sides, steps, lib.mfsdp_muon_many_workspace_bytes(len(shapes), *sides) if workspace is None else workspace)
+
+    def single(shapes, steps=5):
+        return sum(lib.mfsdp_muon_executed_flops(*s, steps, 0) for s in shapes)
+
+    small, large = [(500, 600)] * 16, [(15360, 5120), (5120, 13824)]
+    assert many([(300, 520)]) == single([(300, 520)]) > 0
+    assert many(large) == single(large)
+    assert many(small, lib.mfsdp_muon_workspace_bytes(500, 600)) == single(small) < many(small)
+    layer = [(4096, 4096), (12288, 4096), (11008, 4096)]
+    full = sum(5 * (4 * min(s) ** 2 * max(s) + 2 * min(s) ** 3) for s in layer)
+    assert 0.5 * full < single(layer) <= many(layer) < full
+    assert many(layer, steps=0) == many([(0, 5)], 1 << 40) == many(small, lib.mfsdp_muon_workspace_bytes(500, 600) - 1) == 0
