@@ -49,7 +49,7 @@ extern "C" {
 #define MFSDP_CONVERT_F32_TO_F16 4   /* round-to-nearest-even, NaN -> sign | 0x7E00 (Tensor.to(float16)) */
 
 const char* mfsdp_last_error(void);
-/* ABI version of the library; bumped on any signature change. */
+/* ABI version of the library; bumped when an entry point or a structure is added, changed or removed. */
 int mfsdp_abi_version(void);
 
 /* ------------------------------------------------------------------ copy */

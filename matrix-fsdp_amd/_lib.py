@@ -21,7 +21,7 @@ CONVERT_F32_TO_F16 = 4
 DT_F32 = 0
 DT_BF16 = 1
 DT_F16 = 2  # mfsdp_accumulate only
-ABI_VERSION = 6
+ABI_VERSION = 7
 MUON_SHARED_MACHINE = 1
 NOALLOC_MAX_SEGMENTS = 131071  # MFSDP_NOALLOC_MAX_SEGMENTS
 
@@ -157,14 +157,14 @@ def lib() -> ctypes.CDLL:
             "(there is no CPU fallback for the HIP path)."
         )
     handle = ctypes.CDLL(LIB_PATH)
-    for name, (restype, argtypes) in SIGNATURES.items():
-        fn = getattr(handle, name)  # AttributeError here means the library is stale
-        fn.restype = restype
-        fn.argtypes = argtypes
-    if handle.mfsdp_abi_version() != ABI_VERSION:
+    if handle.mfsdp_abi_version() != ABI_VERSION:  # before the symbols: another version may not have them all
         raise NativeLibraryError(
             f"{LIB_PATH} has ABI version {handle.mfsdp_abi_version()}, this binding expects {ABI_VERSION}: rebuild it."
         )
+    for name, (restype, argtypes) in SIGNATURES.items():
+        fn = getattr(handle, name)
+        fn.restype = restype
+        fn.argtypes = argtypes
     _LIB = handle
     return handle
 

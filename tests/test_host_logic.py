@@ -1,6 +1,7 @@
 """CPU tests of the host-side mirror: shard metadata, layout classification, closed-form plans, the
 C-ABI library's symbols, and the run compiler (host part of the library)."""
 import ctypes
+import hashlib
 import os
 import re
 
@@ -605,3 +606,28 @@ def test_muon_executed_flops_of_many_matrices():
     full = sum(5 * (4 * min(s) ** 2 * max(s) + 2 * min(s) ** 3) for s in layer)
     assert 0.5 * full < single(layer) <= many(layer) < full
     assert many(layer, steps=0) == many([(0, 5)], 1 << 40) == many(small, lib.mfsdp_muon_workspace_bytes(500, 600) - 1) == 0
+
+
+def test_stale_library_is_refused_by_its_version(monkeypatch):
+    """A library of another version is named as such, whatever symbols it lacks."""
+
+    class Stale:
+        @staticmethod
+        def mfsdp_abi_version():
+            return _lib.ABI_VERSION - 1
+
+    monkeypatch.setattr(_lib, "_LIB", None)
+    monkeypatch.setattr(_lib.ctypes, "CDLL", lambda path: Stale())
+    with pytest.raises(_lib.NativeLibraryError, match=f"ABI version {_lib.ABI_VERSION - 1}"):
+        _lib.lib()
+    assert _lib._LIB is None
+
+
+def test_abi_version_belongs_to_the_interface():
+    """The version a set of entry points and structures has: who changes one gives the other a new number, here and in the
+    library, and writes the new pair down."""
+    name = lambda t: t.__name__ if t is not None else "void"
+    interface = sorted((symbol, name(restype), [name(t) for t in args]) for symbol, (restype, args) in _lib.SIGNATURES.items())
+    interface += [(s.__name__, [(f, name(t)) for f, t in s._fields_]) for s in (_lib.CopyRun, _lib.MuonJob, _lib.AdamWSpan)]
+    digest = hashlib.sha256(repr(interface).encode()).hexdigest()[:16]
+    assert (_lib.ABI_VERSION, digest) == (7, "215ac545616d72c8")
