@@ -17,7 +17,8 @@
 
 #include <algorithm>
 #include <cmath>
-#include <vector>
+#include <memory>
+#include <new>
 
 namespace mfsdp {
 namespace {
@@ -78,9 +79,9 @@ constexpr int64_t kGroupBytes = 1344ll << 20;
 // Does the triangle of 256 x 256 tiles of the matrix's symmetric products occupy three quarters of the CUs?  Such a matrix
 // goes through the stages on its own: others beside it would cost their workspace and gain next to nothing (15360 x 5120
 // and 5120 x 13824 in bf16 together 11.14 ms with 1.4 GiB, one after the other 11.27 ms with 0.75 GiB).
-bool fills_machine(const Matrix& w) {
+bool fills_machine(const Matrix& w, int cus) {
   const int t = w.mp / 256;
-  return 4 * (t * (t + 1) / 2) >= 3 * device_cu_count();
+  return 4 * (t * (t + 1) / 2) >= 3 * cus;
 }
 
 // A group of matrices that go through every stage of the update together, one launch per stage.
@@ -263,19 +264,33 @@ struct Pending {
   int64_t job;
 };
 
-// Those that go alone first, then the largest first, so that a group holds matrices of like size; equals in the order given.
-void sort_pending(std::vector<Pending>* order) {
-  std::stable_sort(order->begin(), order->end(), [](const Pending& x, const Pending& y) { return x.alone != y.alone ? x.alone : x.bytes > y.bytes; });
-}
+// The matrices of a call.  Without host memory for them `data` is null: nothing of this may throw out of an extern "C" function.
+struct PendingList {
+  explicit PendingList(int64_t n) : data(new (std::nothrow) Pending[n]), cus(device_cu_count()) {}
+  void add(const Matrix& w) {
+    data[size] = Pending{fills_machine(w, cus), w.bytes, size};
+    ++size;
+  }
+  // Those that go alone first, then the largest first, so that a group holds matrices of like size; equals in the order given.
+  void sort() {
+    std::sort(data.get(), data.get() + size, [](const Pending& x, const Pending& y) {
+      return x.alone != y.alone ? x.alone : x.bytes != y.bytes ? x.bytes > y.bytes : x.job < y.job;
+    });
+  }
+  // The group that starts at `first` ends before the returned position: as many as one launch carries and `room` holds, at
+  // least one.
+  int64_t group_end(int64_t first, int64_t room, int64_t* bytes) const {
+    int64_t end = first + 1;
+    *bytes = data[first].bytes;
+    while (!data[first].alone && end < size && end - first < kMaxMuonGroup && *bytes + data[end].bytes <= room) *bytes += data[end++].bytes;
+    return end;
+  }
+  std::unique_ptr<Pending[]> data;
+  int64_t size = 0;
+  int cus;
+};
 
-// The group that starts at `first` ends before the returned position: as many as one launch carries and `room` holds, at
-// least one.
-size_t group_end(const std::vector<Pending>& order, size_t first, int64_t room, int64_t* bytes) {
-  size_t end = first + 1;
-  *bytes = order[first].bytes;
-  while (!order[first].alone && end < order.size() && end - first < kMaxMuonGroup && *bytes + order[end].bytes <= room) *bytes += order[end++].bytes;
-  return end;
-}
+int out_of_host_memory(int64_t n) { return fail(MFSDP_ERR_UNSUPPORTED, "out of host memory for %lld matrices", static_cast<long long>(n)); }
 
 // Flops the products of one Newton-Schulz step of `n` matrices that share their launches execute.
 int64_t executed_flops(const Matrix* w, int n, bool shared) {
@@ -309,17 +324,18 @@ extern "C" int64_t mfsdp_muon_workspace_bytes(int64_t rows, int64_t cols) {
 
 extern "C" int64_t mfsdp_muon_many_workspace_bytes(int64_t n, const int64_t* rows, const int64_t* cols) {
   if (n <= 0 || rows == nullptr || cols == nullptr) return 0;
-  std::vector<Pending> order;
+  PendingList order(n);
+  if (!order.data) return out_of_host_memory(n), 0;
   for (int64_t i = 0; i < n; ++i) {
     Matrix w;
     if (!plan_matrix(rows[i], cols[i], nullptr, &w)) return 0;
-    order.push_back(Pending{fills_machine(w), w.bytes, i});
+    order.add(w);
   }
-  sort_pending(&order);
+  order.sort();
   int64_t largest = 0;
-  for (size_t next = 0; next < order.size();) {
+  for (int64_t next = 0; next < n;) {
     int64_t bytes = 0;
-    next = group_end(order, next, kGroupBytes, &bytes);
+    next = order.group_end(next, kGroupBytes, &bytes);
     largest = std::max(largest, bytes);
   }
   return largest + kSharedBytes;
@@ -333,20 +349,21 @@ extern "C" int64_t mfsdp_muon_executed_flops(int64_t rows, int64_t cols, int ste
 
 extern "C" int64_t mfsdp_muon_many_executed_flops(int64_t n, const int64_t* rows, const int64_t* cols, int steps, int64_t workspace_bytes) {
   if (n <= 0 || rows == nullptr || cols == nullptr || steps < 0) return 0;
-  std::vector<Pending> order;
+  PendingList order(n);
+  if (!order.data) return out_of_host_memory(n), 0;
   for (int64_t i = 0; i < n; ++i) {
     Matrix w;
     if (!plan_matrix(rows[i], cols[i], nullptr, &w) || w.bytes + kSharedBytes > workspace_bytes) return 0;
-    order.push_back(Pending{fills_machine(w), w.bytes, i});
+    order.add(w);
   }
-  sort_pending(&order);
+  order.sort();
   int64_t flops = 0;
-  for (size_t next = 0; next < order.size();) {
+  for (int64_t next = 0; next < n;) {
     Matrix w[kMaxMuonGroup];
     int64_t bytes = 0;
     int count = 0;
-    for (const size_t end = group_end(order, next, workspace_bytes - kSharedBytes, &bytes); next < end; ++next)
-      plan_matrix(rows[order[next].job], cols[order[next].job], nullptr, &w[count++]);
+    for (const int64_t end = order.group_end(next, workspace_bytes - kSharedBytes, &bytes); next < end; ++next)
+      plan_matrix(rows[order.data[next].job], cols[order.data[next].job], nullptr, &w[count++]);
     flops += executed_flops(w, count, false);
   }
   return steps * flops;
@@ -402,23 +419,24 @@ extern "C" int mfsdp_muon_step_many(int64_t n, const mfsdp_muon_job* jobs, int d
   if (n == 0) return MFSDP_OK;
   const StepArgs s{dtype, momentum, nesterov, a, b, c, steps, eps, false};
   if (int rc = check_step(s)) return rc;
-  std::vector<Pending> order;
+  PendingList order(n);
+  if (!order.data) return out_of_host_memory(n);
   int64_t largest = 0;
   for (int64_t i = 0; i < n; ++i) {
     Matrix w;
     if (int rc = check_matrix(jobs[i].rows, jobs[i].cols, steps, &w)) return rc;
     if (int rc = check_tensors(jobs[i].param, jobs[i].grad, jobs[i].momentum_buf, dtype, jobs[i].lr, jobs[i].weight_decay)) return rc;
-    order.push_back(Pending{fills_machine(w), w.bytes, i});
+    order.add(w);
     largest = std::max(largest, w.bytes);
   }
   if (int rc = check_workspace(workspace, workspace_bytes, largest + kSharedBytes)) return rc;
-  sort_pending(&order);
+  order.sort();
   char* base = static_cast<char*>(workspace);
-  for (size_t next = 0; next < order.size();) {
+  for (int64_t next = 0; next < n;) {
     Group g;
     int64_t bytes = 0, used = 0;
-    for (const size_t end = group_end(order, next, workspace_bytes - kSharedBytes, &bytes); next < end; ++next) {
-      const mfsdp_muon_job& job = jobs[order[next].job];
+    for (const int64_t end = order.group_end(next, workspace_bytes - kSharedBytes, &bytes); next < end; ++next) {
+      const mfsdp_muon_job& job = jobs[order.data[next].job];
       Matrix w;
       plan_matrix(job.rows, job.cols, base + used, &w);
       add_to_group(&g, w, job.param, job.grad, job.momentum_buf, job.lr, job.weight_decay, job.adjusted_lr);

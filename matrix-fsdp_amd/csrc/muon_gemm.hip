@@ -31,7 +31,6 @@
 #include <mutex>
 #include <type_traits>
 #include <utility>
-#include <vector>
 
 namespace mfsdp {
 namespace {
@@ -902,28 +901,34 @@ constexpr Variant kVariants[5] = {{}, {256, 1, 1.35, 1.00, 8.6}, {128, 2, 0.86, 
 constexpr double kFixupUs = 3.2, kFixupBytesPerUs = 3.0e6;  // of the fix-up launch: its partial tiles written and read again
 
 // When the workgroups of a launch end, if each starts on the slot that is free first (as they do, in block order).
-// Slots are kept as groups that are free at the same time; a launch of equal tiles costs a few steps per round.
+// Slots are kept as groups that are free at the same time; a launch of equal tiles costs a few steps per round.  Every call
+// of add leaves at most one group more (a group is taken whole for each one that comes in, but for the last), so the groups
+// of a launch's whole tiles and pieces fit an array.
 class SlotTimes {
  public:
-  explicit SlotTimes(int slots) : groups_{{0.0, slots}} {}
+  explicit SlotTimes(int slots) : groups_{{0.0, slots}}, n_(1) {}
   void add(int workgroups, double us) {
     while (workgroups > 0) {
-      Slots& first = groups_.front();
-      const int n = std::min(workgroups, first.count);
-      const Slots busy{first.time + us, n};
-      first.count -= n;
-      if (first.count == 0) groups_.erase(groups_.begin());
-      auto at = std::lower_bound(groups_.begin(), groups_.end(), busy, [](const Slots& x, const Slots& y) { return x.time < y.time; });
-      if (at != groups_.end() && at->time == busy.time) at->count += n;
-      else groups_.insert(at, busy);
-      workgroups -= n;
+      const Slots busy{groups_[0].time + us, std::min(workgroups, groups_[0].count)};
+      groups_[0].count -= busy.count;
+      workgroups -= busy.count;
+      if (groups_[0].count == 0) std::copy(groups_ + 1, groups_ + n_--, groups_);
+      Slots* at = std::lower_bound(groups_, groups_ + n_, busy, [](const Slots& x, const Slots& y) { return x.time < y.time; });
+      if (at != groups_ + n_ && at->time == busy.time) {
+        at->count += busy.count;
+      } else {
+        std::copy_backward(at, groups_ + n_, groups_ + n_ + 1);
+        *at = busy;
+        ++n_;
+      }
     }
   }
-  double end() const { return groups_.back().time; }
+  double end() const { return groups_[n_ - 1].time; }
 
  private:
   struct Slots { double time; int count; };
-  std::vector<Slots> groups_;
+  Slots groups_[2 * kMaxGemmGroup + 2];
+  int n_;
 };
 
 GemmPlan make_plan(const GemmGroup& g, int variant, const GemmScratch& scratch, const GemmTuning& tuning) {

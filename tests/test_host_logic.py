@@ -4,6 +4,8 @@ import ctypes
 import hashlib
 import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -631,3 +633,34 @@ def test_abi_version_belongs_to_the_interface():
     interface += [(s.__name__, [(f, name(t)) for f, t in s._fields_]) for s in (_lib.CopyRun, _lib.MuonJob, _lib.AdamWSpan)]
     digest = hashlib.sha256(repr(interface).encode()).hexdigest()[:16]
     assert (_lib.ABI_VERSION, digest) == (7, "215ac545616d72c8")
+
+
+def test_out_of_host_memory_is_an_error_code():
+    """The entry points that take lists of any length need host memory in proportion to it: without it they return an error,
+    and no C++ exception leaves the library (that would end the process).  In a child whose address space is limited once
+    the list is made."""
+    child = """
+import ctypes, resource
+import numpy as np
+from matrix_fsdp_amd import _lib
+
+lib, n = _lib.lib(), 4_000_000
+jobs = np.zeros(n, dtype=np.dtype([("param", "u8"), ("grad", "u8"), ("buf", "u8"), ("rows", "i8"), ("cols", "i8"), ("lr", "f8"), ("wd", "f8"), ("alr", "f8")]))
+assert jobs.itemsize == ctypes.sizeof(_lib.MuonJob)
+for name in ("param", "grad", "buf"):
+    jobs[name] = 1 << 40
+jobs["rows"] = jobs["cols"] = 64
+sides = np.full(n, 64, dtype=np.int64)
+pointer = sides.ctypes.data_as(ctypes.POINTER(ctypes.c_int64))
+size = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (size + (24 << 20), resource.RLIM_INFINITY))
+flops = lib.mfsdp_muon_many_executed_flops(n, pointer, pointer, 5, 1 << 40)
+room = lib.mfsdp_muon_many_workspace_bytes(n, pointer, pointer)
+rc = lib.mfsdp_muon_step_many(n, jobs.ctypes.data_as(ctypes.POINTER(_lib.MuonJob)), _lib.DT_F32, 0.9, 1, 3.0, -4.0, 2.0, 5, 1e-7, 1 << 40, 0, None)
+message = lib.mfsdp_last_error()
+resource.setrlimit(resource.RLIMIT_AS, (resource.RLIM_INFINITY, resource.RLIM_INFINITY))
+print(flops, room, rc, message.decode())
+"""
+    done = subprocess.run([sys.executable, "-c", child], cwd=ROOT, capture_output=True, text=True, timeout=120)
+    assert done.returncode == 0, (done.returncode, done.stderr[-500:])
+    assert done.stdout.strip() == "0 0 3 out of host memory for 4000000 matrices"
