@@ -39,12 +39,11 @@ struct Span {
 
 constexpr int kMaxSpans = 56;  // of one launch: its kernel arguments carry the table
 
-// Kernel arguments of up to N spans: one, whose fields then need no lookup, a few or many, because 4 KiB of arguments make a launch 1.2 us longer than a few hundred bytes
-// (3.7 against 2.5 us for an empty kernel), which is most of a small update.
+// Kernel arguments of up to N spans: one, whose fields then need no lookup, a few or many, because 4 KiB of arguments make a
+// launch 1.2 us longer than a few hundred bytes (3.7 against 2.5 us for an empty kernel), which is most of a small update.
 template <int N>
 struct SpanTable {
-  uint32_t begin[N];  // first workgroup of a span; entries past n are the end
-  int n;
+  uint32_t begin[N];  // first workgroup of a span; entries past the last span are beyond every workgroup
   AdamWArgs a;
   Span span[N];
 };
@@ -184,7 +183,6 @@ int check_span(const mfsdp_adamw_span& s) {
 template <int N>
 int launch(const mfsdp_adamw_span* const* spans, int n, const AdamWArgs& a, double lr, double beta1, double beta2, hipStream_t stream) {
   SpanTable<N> table;
-  table.n = n;
   table.a = a;
   uint32_t blocks = 0;
   int64_t step = 0;

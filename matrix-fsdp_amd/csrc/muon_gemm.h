@@ -48,8 +48,8 @@ struct GemmGroup {
   float alpha = 1.0f, beta = 0.0f;
   int symmetric = 0;
   int update_dtype = 0;  // of the parameters (MFSDP_F32 / MFSDP_BF16)
-  int shared = 0;        // other matrices' products run beside this launch on other streams: a symmetric product then takes
-                         // the 256 x 256 tiles even where their triangle fills only part of the CUs
+  int shared = 0;        // other matrices' products run beside this launch of one problem on other streams: a symmetric product
+                         // then takes the 256 x 256 tiles even where their triangle fills only part of the CUs
   GemmProblem problem[kMaxGemmGroup];
 };
 

@@ -713,8 +713,7 @@ splitk_fixup_kernel(LaunchArgs<N> args) {
 // two of 512x1536 220 -> 201, 1024x1024 251 -> 204, four of 64x256 117 -> 91.
 template <int N>
 struct SmallArgs {
-  int begin[N];  // first workgroup of a problem; entries past n are the end
-  int n;
+  int begin[N];  // first workgroup of a problem; entries past the last problem are the end
   int symmetric;
   int group_m;
   int update_dtype;
@@ -1051,7 +1050,6 @@ int launch(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& scratch,
 template <int N>
 int launch_small(const GemmGroup& g, const GemmPlan& plan, const GemmTuning& tuning, hipStream_t stream) {
   SmallArgs<N> args;
-  args.n = g.n;
   args.symmetric = g.symmetric;
   args.group_m = std::max(1, tuning.group_m);
   args.update_dtype = g.update_dtype;

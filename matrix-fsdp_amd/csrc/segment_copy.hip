@@ -38,8 +38,8 @@ constexpr int64_t kMaxGrid = (int64_t{1} << 31) - 1;  // grid-stride loops keep 
 constexpr int64_t kMaxGroupsPerRun = 0x7fffffff;  // the reciprocal division is exact below 2^31 groups
 
 // Pointer tables of two sizes travel in the kernel arguments: most programs have one buffer of a few sources, and a launch
-// with 0.1 KiB of arguments is shorter than one with 1.6 KiB (pack + unpack +
-// gradient fill: two-layer MLP 19.5 -> 18.4 us, a hidden4096 layer in 2 x 2 blocks 462.5 -> 457.1).
+// with 0.1 KiB of arguments is shorter than one with 1.6 KiB (pack + unpack + gradient fill: two-layer MLP 19.6 -> 18.7 us, an
+// odd-sized unit for three ranks 33.7 -> 32.7; a large layer does not notice: 459 us for a hidden4096 one in 2 x 2 blocks).
 constexpr int kFewSources = 8;
 template <int N>
 struct SourcePointers {
@@ -509,7 +509,7 @@ int launch_one(const Compiled& c, const SourceTable& srcs, const DestTable& dsts
     case 3: MFSDP_LAUNCH_T(U_, false, true); break;  \
     default: MFSDP_LAUNCH_T(U_, true, true); break;  \
   }
-  if (batch == 1 && c.n_sources <= kFewSources && threads == kDefaultBlockThreads && (nt == 1 || nt < 0)) {
+  if (batch == 1 && c.n_sources <= kFewSources && threads == kDefaultBlockThreads && nt == 1) {
     SourcePointers<kFewSources> few;
     for (int i = 0; i < kFewSources; ++i) few.p[i] = i < c.n_sources ? srcs.p[i] : nullptr;
     const DestPointers<1> one{{dsts.p[0]}};
