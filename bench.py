@@ -233,7 +233,6 @@ def main() -> int:
     if "ceiling" in want:
         # -------------------------------------------------------------- what this part sustains: a plain contiguous copy of one
         # layer buffer's size through the library's range copy, pure reads and pure writes in the same launch shape
-        import ctypes
 
         n_el = w.total_numel
         a_buf = torch.empty(n_el, dtype=torch.bfloat16, device=dev).normal_(0.0, 0.02)
@@ -330,7 +329,6 @@ def main() -> int:
     if "devcopy" in want:
         # -------------------------------------------------------------- the boundary function itself: copy_rank_segments_to_full with
         # DEVICE metadata (kernels/native/matrix_copy.cpp:53-83), one rank's shard of one hidden4096 layer buffer into the full buffer
-        import ctypes
 
         from matrix_fsdp_amd.kernels import native as N
         from matrix_fsdp_amd.kernels.segment_program import local_segments_program
