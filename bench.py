@@ -37,17 +37,18 @@ BF16_MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense bf16, vendor figure
 NS_COEFFS = (3.4445, -4.7750, 2.0315)
 # Figures QUOTED from the committed rocprofv3 counter profiles (counters cannot be read from inside this process).  They
 # describe the library as it was when the profile was taken (its `head` line) and are reported under keys that say so.
-PROFILED_TRAFFIC = {"bytes_per_launch": 812_818_425, "source": "profiles/segment_program_hbm_traffic.md"}
+PROFILED_TRAFFIC = {"bytes_per_launch": 812_836_848, "source": "profiles/segment_program_hbm_traffic.md"}
 PROFILED_MUON = {
     # SQ_VALU_MFMA_BUSY_CYCLES over the SIMD cycles of the dispatch (all 256 CUs), per kernel and launch shape
     "mfma_busy": {
-        "gemm_nt_kernel<256,256> general product, 768 workgroups (12288x4096)": 0.565,
-        "gemm_nt_kernel<256,256> general product, 688 workgroups (11008x4096)": 0.508,
-        "gemm_nt_kernel<256,256> general product, 256 workgroups (4096x4096)": 0.597,
-        "gemm_nt_kernel<128,128> symmetric products, one matrix at a time, 768 workgroups": 0.470,
+        "gemm_nt_kernel<256,256> update products of the three matrices in one launch, 1712 workgroups": 0.546,
+        "gemm_nt_kernel<256,256> gram products of the three in one launch, 440 workgroups": 0.511,
+        "gemm_nt_kernel<256,256> poly products of the three in one launch, 408 workgroups": 0.508,
+        "gemm_nt_kernel<256,256> update product alone, 768 workgroups (12288x4096)": 0.562,
+        "gemm_nt_kernel<128,128> gram products alone, 768 workgroups (11008x4096, 12288x4096)": 0.492,
     },
-    # the dominant launch, B X on 12288 x 4096 (768 workgroups): FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000, in bytes
-    "traffic_bytes_per_launch": (2 * 295_250 + 176_947) * 1024,
+    # the dominant launch, the three update products together (1712 workgroups): FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000, in bytes
+    "traffic_bytes_per_launch": (2 * 788_322 + 438_631) * 1024,
     "source": "profiles/gemm_nt_kernel_muon_hidden4096_counters.md, profiles/gemm_nt_kernel_muon_hbm_traffic.md",
 }
 
