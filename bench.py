@@ -468,7 +468,7 @@ def main() -> int:
         tflops = flops / (med * 1e-3) / 1e12
         legs["muon_hidden4096"] = {
             "ms_per_step": round(med, 4),
-            "form_timed": {"both": "side by side (muon_step_many)", "serial": "one matrix at a time", "side-by-side": "side by side (muon_step_many)"}[args.muon_form],
+            "form_timed": {"both": "sharing launches (muon_step_many)", "serial": "one matrix at a time", "side-by-side": "sharing launches (muon_step_many)"}[args.muon_form],
             "ms_per_step_one_matrix_at_a_time": None if med_one_stream is None else round(med_one_stream, 4),
             "ns_TFLOPs_reference_flop_count": round(tflops, 1),
             "pct_bf16_mfma_peak": round(100 * tflops / BF16_MFMA_PEAK_TFLOPS, 2),

@@ -262,8 +262,8 @@ def test_muon_step_full_size_all_bf16(shape):
 
 
 def test_hidden4096_matrices_side_by_side_against_torch_muon():
-    """The three matrices of a hidden4096 layer updated at the same time on side streams (their symmetric products then
-    run on 256 x 256 tiles): every parameter delta against ``torch.optim.Muon.step`` on this GPU and, for the square
+    """The three matrices of a hidden4096 layer sharing every launch (their symmetric products run on 256 x 256 tiles, on
+    128 x 128 alone): every parameter delta against ``torch.optim.Muon.step`` on this GPU and, for the square
     one, against the CPU oracle."""
     torch.set_num_threads(16)
     shapes = [(4096, 4096), (12288, 4096), (11008, 4096)]
