@@ -652,6 +652,7 @@ for name in ("param", "grad", "buf"):
 jobs["rows"] = jobs["cols"] = 64
 sides = np.full(n, 64, dtype=np.int64)
 pointer = sides.ctypes.data_as(ctypes.POINTER(ctypes.c_int64))
+assert lib.mfsdp_muon_many_workspace_bytes(1, pointer, pointer) > 0  # the runtime is set up without the limit
 size = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
 resource.setrlimit(resource.RLIMIT_AS, (size + (24 << 20), resource.RLIM_INFINITY))
 flops = lib.mfsdp_muon_many_executed_flops(n, pointer, pointer, 5, 1 << 40)

@@ -463,6 +463,38 @@ def test_muon_group_with_ragged_partial_sums():
             assert torch.allclose(b.cpu(), b_ref, rtol=1e-6, atol=1e-6 * float(b_ref.abs().max()))
 
 
+@pytest.mark.parametrize("variant", [1, 2, 3, 4])
+def test_muon_group_reads_nothing_stale_and_nothing_of_its_neighbours(variant):
+    """Sides around the 64 that operands are zero-padded to, some K walks cut: a workspace full of NaN gives the bits of a
+    cleared one, and a matrix whose gradient is NaN or infinite leaves those of the others alone."""
+    from matrix_fsdp_amd import _lib
+
+    shapes = [(63, 65), (130, 2100), (64, 1153), (300, 257), (1, 7), (1200, 190)]
+    kw = dict(lr=0.02, weight_decay=0.1, momentum=0.95, nesterov=True)
+    params, grads = [make(sh, 700 + i, 0.02).to(DEV) for i, sh in enumerate(shapes)], [make(sh, 710 + i).to(DEV) for i, sh in enumerate(shapes)]
+
+    def update(fill, bad=None):
+        ps, bs, gs = [p.clone() for p in params], [torch.zeros_like(p) for p in params], [g.clone() for g in grads]
+        if bad is not None:
+            gs[1][5, 7] = bad
+            gs[3][0, 0] = bad
+        workspace = F.MuonWorkspace(DEV)
+        workspace.get_bytes(256 << 20).fill_(fill)
+        F.muon_step_many([(p, g, b, kw) for p, g, b in zip(ps, gs, bs)], workspace=workspace)
+        return ps
+
+    _lib.lib().mfsdp_set_muon_tuning(variant, variant, 0, 0, 0)
+    try:
+        want, stale = update(0), update(0xFF)
+        spoiled = [update(0, float("nan")), update(0xFF, float("inf"))]
+    finally:
+        _lib.lib().mfsdp_set_muon_tuning(3, 3, 0, 0, 0)
+    for i in range(len(shapes)):
+        assert torch.isfinite(want[i]).all() and torch.equal(stale[i], want[i]), shapes[i]
+        for ps in spoiled:
+            assert torch.isnan(ps[i]).all() if i in (1, 3) else torch.equal(ps[i], want[i]), shapes[i]
+
+
 def test_muon_group_with_cut_k_walks():
     """Sides beyond 1024, where the tiles of the last round are cut along K: several K in one launch, against the oracle."""
     shapes = [(192, 1088), (130, 2100), (4160, 200), (70, 8200)]
