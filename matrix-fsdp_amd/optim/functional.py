@@ -209,7 +209,8 @@ def _job(param, grad, momentum_buf, *, lr, weight_decay, momentum, nesterov, ns_
     """``(what the jobs of one library call share, fields of mfsdp_muon_job)``."""
     _check_step(param, grad, momentum_buf, ns_steps)
     rows, cols = param.shape
-    key = (_DTYPE_CODES[param.dtype], momentum, int(bool(nesterov)), *ns_coefficients, ns_steps, eps)
+    # plain floats: equal values share a launch whatever number type they come in
+    key = (_DTYPE_CODES[param.dtype], float(momentum), int(bool(nesterov)), *map(float, ns_coefficients), ns_steps, float(eps))
     return key, (param.data_ptr(), grad.data_ptr(), momentum_buf.data_ptr(), rows, cols, lr, weight_decay, adjust_lr(lr, adjust_lr_fn, (rows, cols)))
 
 
@@ -331,7 +332,7 @@ def adamw_step(
         param.data_ptr(), grad.data_ptr(), exp_avg.data_ptr(), exp_avg_sq.data_ptr(), None if max_exp_avg_sq is None else max_exp_avg_sq.data_ptr(),
         numel, int(step), _DTYPE_CODES[grad.dtype],
     )
-    hyper = (lr, betas[0], betas[1], eps, weight_decay, int(bool(maximize)))
+    hyper = (float(lr), float(betas[0]), float(betas[1]), float(eps), float(weight_decay), int(bool(maximize)))
     tensors = (param, grad, exp_avg, exp_avg_sq, max_exp_avg_sq)
     if batch is not None:
         batch.add(param.device, hyper, span, tensors)

@@ -3,6 +3,7 @@
 Tolerances: the Muon update must be within rel-Frobenius 1e-2 of the reference arithmetic on the
 same seeded inputs (bf16 products, fp32 accumulation; only the summation order differs); AdamW is
 fp32 element-wise and must agree to 1e-6 relative."""
+import numpy as np
 import pytest
 import torch
 
@@ -507,6 +508,25 @@ def test_muon_group_with_cut_k_walks():
         p_ref, b_ref = params[i].clone(), torch.zeros(sh)
         O.muon_step(p_ref, grads[i], b_ref, **kw)
         assert rel_fro(dev_p[i].cpu() - params[i], p_ref - params[i]) < MUON_TOL, sh
+
+
+@pytest.mark.parametrize("number", [np.array, np.float64, torch.tensor, lambda x: torch.tensor(x, device=DEV)], ids=["0-d array", "numpy scalar", "tensor", "device tensor"])
+def test_hyper_parameters_of_any_number_type(number):
+    """Learning rates and the like as numpy or torch numbers, which a scheduler may leave in a group: the bits of floats."""
+    p0, g0 = make((40, 60), 1, 0.02).to(DEV), make((40, 60), 2).to(DEV)
+    adam = dict(lr=1e-3, eps=1e-8, weight_decay=0.1)
+    muon = dict(lr=0.02, weight_decay=0.1, momentum=0.95, eps=1e-7)
+    results = []
+    for convert in (float, lambda x: number(float(x))):
+        p, q, r = p0.clone(), p0.clone(), p0.clone()
+        F.adamw_step(p, g0, torch.zeros_like(p), torch.zeros_like(p), 1, betas=(convert(0.5), convert(0.75)), **{k: convert(v) for k, v in adam.items()})
+        F.muon_step_many([(t, g0, torch.zeros_like(t), dict(nesterov=True, ns_coefficients=tuple(convert(c) for c in (3.0, -4.0, 2.0)), **{k: convert(v) for k, v in muon.items()}))
+                          for t in (q, r)])
+        results.append((p, q, r))
+    tight = number is np.array or number is np.float64
+    for have, want in zip(results[1], results[0]):
+        # a torch number is rounded to fp32 on its way
+        assert torch.equal(have, want) if tight else rel_fro(have - p0, want - p0) < 1e-4
 
 
 @pytest.mark.parametrize("amsgrad", [False, True])
