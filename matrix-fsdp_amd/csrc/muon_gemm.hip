@@ -157,11 +157,14 @@ __device__ __forceinline__ void tile_coords(int group_m, int logical, int tiles_
   // narrow, which reads more panels (256-tiles of 5120 x 5120 253 -> 241 us, of 5120 x 13824 603 -> 594 with 14, 14, 14, 12
   // instead of 16, 16, 16, 6).
   constexpr int kSuper = 16;
-  const int supers = (tiles_n + kSuper - 1) / kSuper, width = (tiles_n + supers - 1) / supers;
-  const int per_super = width * tiles_m;
-  const int super = logical / per_super;
-  const int first_n = super * width, cols = min(width, tiles_n - first_n);
-  int in = logical - super * per_super;
+  int first_n = 0, cols = tiles_n, in = logical;
+  if (tiles_n > kSuper) {
+    const int supers = (tiles_n + kSuper - 1) / kSuper, width = (tiles_n + supers - 1) / supers;
+    const int super = logical / (width * tiles_m);
+    first_n = super * width;
+    cols = min(width, tiles_n - first_n);
+    in -= super * width * tiles_m;
+  }
   const int band = in / (group_m * cols);  // group_m rows of this super column
   const int first_m = band * group_m, rows = min(group_m, tiles_m - first_m);
   in -= band * group_m * cols;
