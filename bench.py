@@ -186,7 +186,7 @@ def main() -> int:
         avg_launch_ms = ms_per_step / (2 * layers)
     achieved = bytes_per_launch / (avg_launch_ms * 1e-3) / 1e9
     roofline = {
-        "kernel": "segment_program_kernel<16,16> (pack / unpack of one hidden4096 layer buffer)",
+        "kernel": "segment_program_kernel (pack / unpack of one hidden4096 layer buffer)",
         "bound": "hbm",
         "achieved": round(achieved, 1),
         "peak": HBM_PEAK_GBPS,
