@@ -1,10 +1,10 @@
 // Owner-rank Muon update of one matrix: momentum -> Newton-Schulz (bf16 MFMA GEMMs) -> parameter update.
 //
-// The iteration keeps X (m x n, m <= n) AND X^T (n x m) so that all three products of a step are
-// K-contiguous "NT" GEMMs:
+// The iteration keeps X (m x n, m <= n) and, where that is faster (stores_transposes), X^T (n x m), so that all three
+// products of a step are K-contiguous "NT" GEMMs; elsewhere the update product reads X by columns:
 //     A  = X X^T                    P = Q = X          (symmetric: lower-triangle tiles, mirrored store)
 //     B  = b A + c A A = b A + c A A^T   P = Q = A     (symmetric)
-//     X' = a X + B X                P = B, Q = X^T     (writes X' and X'^T)
+//     X' = a X + B X                P = B, Q = X^T or X     (writes X' and, where kept, X'^T)
 // Every product is rounded to bf16, as the reference's bf16 addmm / mm do.  Buffers are padded to multiples of 256 so
 // the GEMM needs no edge handling; what a product reads beyond a matrix's sides along K is zero.
 //
@@ -63,6 +63,7 @@ struct Matrix {
   int rows, cols;          // of the parameter
   int m, n, mp, np;        // short / long side and their padded sizes
   bool tall;               // rows > cols: the iteration runs on the transpose
+  bool keeps_xt;           // X^T is stored beside X, see stores_transposes
   bool folded;             // of this group's iteration, see choose_folding
   uint16_t* X[2];          // mp x np
   uint16_t* XT[2];         // np x mp
@@ -79,6 +80,7 @@ bool plan_matrix(int64_t rows, int64_t cols, char* base, Matrix* w) {
   w->cols = static_cast<int>(cols);
   w->tall = rows > cols;
   w->folded = false;
+  w->keeps_xt = true;
   w->m = static_cast<int>(std::min(rows, cols));
   w->n = static_cast<int>(std::max(rows, cols));
   w->mp = static_cast<int>(round_up(w->m, kPad));
@@ -115,7 +117,7 @@ constexpr int64_t kGroupBytes = 1360ll << 20;
 // goes through the stages on its own: others beside it would cost their workspace and gain next to nothing (15360 x 5120
 // and 5120 x 13824 in bf16 together 11.14 ms with 1.4 GiB, one after the other 11.27 ms with 0.75 GiB).
 bool fills_machine(const Matrix& w, int cus) {
-  const int t = w.mp / 256;
+  const int t = (w.m + 255) / 256;
   return 4 * (t * (t + 1) / 2) >= 3 * cus;
 }
 
@@ -214,6 +216,12 @@ struct Products {
     p.ldp = w.mp; p.ldq = w.mp; p.ldd = w.np; p.ldc = w.np; p.ldct = w.mp;
     p.alpha = 1.0f; p.beta = diagonal ? 0.0f : it.a;
     p.flags = diagonal ? kGemmDiagP : 0;
+    if (!w.keeps_xt) {
+      p.Q = w.X[cur];
+      p.ldq = w.np;
+      p.flags |= kGemmQColumns;
+      if (!(last && w.tall)) p.CT = nullptr;
+    }
     if (last) {  // only has to leave O in the parameter's orientation
       if (w.tall) p.flags |= kGemmSkipC;
       else p.CT = nullptr;
@@ -287,6 +295,38 @@ int for_each_launch(const Matrix* w, int n, const Iteration& it, bool shared, La
   return MFSDP_OK;
 }
 
+// Does the group store X^T beside X?  The update product can take X itself (kGemmQColumns), and the epilogues of the update
+// products and the scale kernel then store one orientation of X instead of two; its walk over X is some percent slower.
+// Whole step with X^T -> without, us: 24 of 1536x1024 1241 -> 1090, a hidden2048 layer 1720 -> 1647, six of 1536x4096 in bf16 1365
+// -> 1227, 3072x9216 1561 -> 1478, 5120x15360 5842 -> 5717.  So:
+// * on 256 tiles (on 128 ones 1024x2048 226 -> 251, 1000x3000 with four smaller 316 -> 331; 64 tiles read their operands
+//   straight into registers, K-contiguous);
+// * where the tiles fill more than a round, so that their stores compete (200 tiles 745 -> 756, 288 1172 -> 1175, 324 1908 -> 1853);
+// * where X and X' are about what the memory-side cache of 256 MB holds (X of 157 MB: gains 2 %; the three matrices of a hidden4096
+//   step, 224 MB, lose 2 %).  This bounds X far below the 2 GiB that kGemmQColumns takes, too.
+constexpr int64_t kOneOrientationBytes = 192ll << 20;
+bool stores_transposes(const Group& group, const Iteration& it) {
+  GemmGroup g;
+  int64_t bytes = 0, tiles = 0;
+  g.n = group.n;
+  for (int i = 0; i < g.n; ++i) {
+    const Matrix& w = group.w[i];
+    g.problem[i] = Products{w, it}.update(0, false, false);
+    bytes += static_cast<int64_t>(w.m) * w.n * 2;
+    tiles += static_cast<int64_t>((w.m + 255) / 256) * ((w.n + 255) / 256);
+  }
+  return bytes > kOneOrientationBytes || 4 * tiles < 5 * device_cu_count() || !on_256_tiles(gemm_plan(g, group.scratch));
+}
+
+void choose_transposes(Group* group, const Iteration& it) {
+  if (it.steps == 0 || stores_transposes(*group, it)) return;  // without a product the result is taken from either
+  for (int i = 0; i < group->n; ++i) {
+    Matrix& w = group->w[i];
+    w.keeps_xt = false;
+    (w.tall ? group->elementwise.m[i].same : group->elementwise.m[i].trans) = nullptr;
+  }
+}
+
 // The plans of a step's launches so far, by the kinds of their products and the matrices they belong to.
 class Plans {
  public:
@@ -312,6 +352,7 @@ class Plans {
 // at least one step the last product writes the parameters themselves; otherwise O is left in X[steps & 1] (wide) or
 // XT[steps & 1] (tall).
 int run_newton_schulz(Group& group, const Iteration& it, float eps, bool shared, int update_dtype, hipStream_t stream) {
+  choose_transposes(&group, it);
   if (int rc = muon_scale_transpose(group.elementwise, eps, stream)) return rc;
   choose_folding(group.w, group.n, it, update_dtype == MFSDP_BF16);
   Plans plans;

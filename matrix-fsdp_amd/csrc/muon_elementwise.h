@@ -11,7 +11,7 @@ constexpr int kMuonMaxPartials = 1 << 18;  // upper bound on the workgroups of a
 constexpr int kMaxMuonGroup = 32;          // matrices one launch carries by value in its kernel arguments
 
 // One matrix of a launch.  `same` / `trans` receive the scaled update and its transpose: rows x cols with ld_same, cols x
-// rows with ld_trans, both zero up to the next multiples of 64.
+// rows with ld_trans, both zero up to the next multiples of 64; either may be null.
 struct MuonMatrix {
   const void* grad;
   void* buf;         // momentum buffer

@@ -315,8 +315,9 @@ scale_transpose_kernel(GroupArgs args, float eps) {
     }
     const u32x2 packed = {static_cast<uint32_t>(v[0]) | (static_cast<uint32_t>(v[1]) << 16),
                           static_cast<uint32_t>(v[2]) | (static_cast<uint32_t>(v[3]) << 16)};
-    *reinterpret_cast<u32x2*>(same + static_cast<int64_t>(r) * m.ld_same + c) = packed;
+    if (same != nullptr) *reinterpret_cast<u32x2*>(same + static_cast<int64_t>(r) * m.ld_same + c) = packed;
   }
+  if (trans == nullptr) return;
   __syncthreads();
   for (int e = threadIdx.x; e < 64 * 16; e += kThreads) {
     const int lc = e >> 4, lr = (e & 15) * 4;  // a row of trans = a column of the tile, four rows of the tile at a time

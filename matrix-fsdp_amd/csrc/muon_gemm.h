@@ -23,6 +23,9 @@ namespace mfsdp {
 // kGemmSymmetric: P Q^T is known to be symmetric (M == N); only tiles on or below the diagonal are computed and each
 // off-diagonal tile is also written mirrored into C.
 //
+// kGemmQColumns: Q is given as K x N row-major (ldq), rows beyond M taken as zero, K spanning M, less than 2 GiB of it; general
+// products on 256 tiles (gemm_plan takes no others for them).  D is then the same matrix.
+//
 // Diagonals to more than bf16.  A square operand S (leading dimension ld) may carry behind its last row, at S + ld * ld, ld
 // floats with what the rounding of each diagonal element left over (residual_of).  With kGemmDiagC a symmetric product adds
 // `shift` to its diagonal, takes the residuals of P and Q into it (kGemmDiagP / kGemmDiagQ: alpha (P_ii dq_i + dp_i Q_ii) +
@@ -36,6 +39,7 @@ enum GemmFlags {
   kGemmDiagP = 16,
   kGemmDiagQ = 32,
   kGemmDiagC = 64,
+  kGemmQColumns = 128,
 };
 struct GemmProblem {
   const void* P;
@@ -102,6 +106,7 @@ struct GemmPlan {
   int split_tiles[kMaxGemmGroup], splits[kMaxGemmGroup];  // by position in `order`
 };
 GemmPlan gemm_plan(const GemmGroup& group, const GemmScratch& scratch);
+bool on_256_tiles(const GemmPlan& plan);
 
 // Enqueues the products on `stream` as one launch (and a fix-up launch when tiles are split along K); returns an MFSDP_*
 // status.  `plan` is gemm_plan's for a group of these sizes.

@@ -1,6 +1,6 @@
 // bf16 MFMA GEMM for the Newton-Schulz iteration: C = bf16(alpha * P Q^T + beta * D) on gfx950.
 //
-// Both operands are K-contiguous (an "NT" product), which is what every Newton-Schulz product
+// Both operands are K-contiguous (an "NT" product; a Q of K rows has a walk of its own), which is what every Newton-Schulz product
 // reduces to once X and X^T are both kept: X X^T, A A^T (A symmetric) and B (X^T)^T.  A workgroup owns
 // a BM x BN tile of C; its waves each own a (BM/WM) x (BN/WN) sub-tile built from 16x16x32 bf16 MFMAs
 // with fp32 accumulators.  K is walked in slabs of BK = 64: the slab of P and Q is staged in LDS as
@@ -275,7 +275,8 @@ gemm_nt_kernel(LaunchArgs<N> args) {
   const int wave_n = wave % WN;
 
   const __bf16* __restrict__ P = static_cast<const __bf16*>(a.P) + static_cast<int64_t>(row0) * a.ldp;
-  const __bf16* __restrict__ Q = static_cast<const __bf16*>(a.Q) + static_cast<int64_t>(col0) * a.ldq;
+  const bool q_columns = BM == 256 && (a.flags & kGemmQColumns) != 0;
+  const __bf16* __restrict__ Q = static_cast<const __bf16*>(a.Q) + (q_columns ? col0 : static_cast<int64_t>(col0) * a.ldq);
 
   // ---- slab loader.  A slab row holds BK bf16 = kChunks 16-byte chunks; chunk c of row r is stored at chunk
   // position c ^ ((r / kRowsPerSweep) % kChunks).  One wave-level direct-to-LDS load fills 1 KiB = kRowsPerLoad
@@ -289,13 +290,15 @@ gemm_nt_kernel(LaunchArgs<N> args) {
   const int dl_row = wave * kRowsPerLoad + lane / kChunks;
   const int dl_chunk = (lane % kChunks) ^ ((dl_row / kRowsPerSweep) % kChunks);
   const uint32_t lane_offset_p = static_cast<uint32_t>(dl_row * a.ldp + dl_chunk * 8) * 2u;
-  const uint32_t lane_offset_q = static_cast<uint32_t>(dl_row * a.ldq + dl_chunk * 8) * 2u;
   auto operand_rsrc = [](const __bf16* base, int64_t rows, int ld) {
     const int64_t bytes = rows * ld * 2;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(base), 0, static_cast<int>(bytes < 0x7fffffff ? bytes : 0x7fffffff), 0x00020000);
   };
   const __amdgpu_buffer_rsrc_t rsrc_p = operand_rsrc(P, a.M - row0, a.ldp);
-  const __amdgpu_buffer_rsrc_t rsrc_q = operand_rsrc(Q, a.N - col0, a.ldq);
+  // a Q of K rows: its rows beyond M read as zero, as P's do (K runs over M)
+  const __amdgpu_buffer_rsrc_t rsrc_q =
+      q_columns ? __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(Q), 0, static_cast<int>((static_cast<int64_t>(a.M) * a.ldq - col0) * 2), 0x00020000)
+                : operand_rsrc(Q, a.N - col0, a.ldq);
   typedef __attribute__((address_space(3))) void* LdsPtr;
   // One load at a time: a wave that issues several of these back to back stalls on the address queue, and its
   // MFMAs wait with it, so the main loop slips them in between MFMAs.
@@ -304,20 +307,10 @@ gemm_nt_kernel(LaunchArgs<N> args) {
     const int scalar_offset = (i * kWaves * kRowsPerLoad * a.ldp + k0) * 2;
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_p, (LdsPtr)(smem + stage * kStageElems + r0 * BK), 16, lane_offset_p, scalar_offset, 0, 0);
   };
-  auto load_q = [&](int k0, int stage, int i) {
-    const int r0 = (i * kWaves + wave) * kRowsPerLoad;
-    const int scalar_offset = (i * kWaves * kRowsPerLoad * a.ldq + k0) * 2;
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_q, (LdsPtr)(smem + stage * kStageElems + BM * BK + r0 * BK), 16, lane_offset_q, scalar_offset, 0, 0);
-  };
   auto stream_p = [&](int k0, int stage) {
 #pragma unroll
     for (int i = 0; i < kLoadsP; ++i) load_p(k0, stage, i);
   };
-  auto stream_q = [&](int k0, int stage) {
-#pragma unroll
-    for (int i = 0; i < kLoadsQ; ++i) load_q(k0, stage, i);
-  };
-
   // Accumulator register r of lane l holds C[4*(l/16) + r][l%16] of its 16x16 tile.
   const int lcol = wave_n * kWaveN + (lane & 15);
   const int lrow = wave_m * kWaveM + (lane >> 4) * 4;
@@ -340,6 +333,42 @@ gemm_nt_kernel(LaunchArgs<N> args) {
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.0f;
+
+  // The K walk, for a Q of N rows (K-contiguous, as P) and for one of K rows (kGemmQColumns: X itself in the update product, so
+  // that no transpose of X is ever stored).  A slab of the latter is BK rows of BN bf16 in LDS, in chunks of 32 bytes: chunk c of
+  // row r sits at c ^ f(r), f(r) the row's bits 0, 1 and 3, so that the eight rows that half a wave reads at a time (four
+  // consecutive ones of two blocks of eight) cover all banks.  ds_read_b64_tr_b16 turns four rows by sixteen columns into four
+  // consecutive k of a lane's column: two of them are a fragment, one is a lane's D values.
+  auto walk = [&](auto q_columns_tag) __attribute__((always_inline)) {
+  constexpr bool kQColumns = decltype(q_columns_tag)::value;
+  constexpr int kQRowLanes = BN / 8, kQRowsPerLoad = 64 / kQRowLanes;
+  static_assert(kWaves * kQRowsPerLoad == 16 && BK / kQRowsPerLoad / kWaves == kLoadsQ, "the swizzle must repeat from one row group of a wave to the next");
+  const int q_row = wave * kQRowsPerLoad + lane / kQRowLanes;
+  const int q_chunk = ((lane % kQRowLanes) >> 1) ^ ((q_row & 3) | ((q_row >> 1) & 4));
+  const uint32_t lane_offset_q = kQColumns ? static_cast<uint32_t>(q_row * a.ldq + q_chunk * 16 + (lane & 1) * 8) * 2u
+                                           : static_cast<uint32_t>(dl_row * a.ldq + dl_chunk * 8) * 2u;
+  auto load_q = [&](int k0, int stage, int i) {
+    const int r0 = kQColumns ? (i * kWaves + wave) * 512 : (i * kWaves + wave) * kRowsPerLoad * BK;  // first element in LDS
+    const int scalar_offset = kQColumns ? (k0 + i * 16) * a.ldq * 2 : (i * kWaves * kRowsPerLoad * a.ldq + k0) * 2;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_q, (LdsPtr)(smem + stage * kStageElems + BM * BK + r0), 16, lane_offset_q, scalar_offset, 0, 0);
+  };
+  auto stream_q = [&](int k0, int stage) {
+#pragma unroll
+    for (int i = 0; i < kLoadsQ; ++i) load_q(k0, stage, i);
+  };
+  // lane 4 e + q of a group of sixteen reads four columns of row e
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) s16x4* TrPtr;
+  const int tr_e = (lane & 15) >> 2, tr_group = lane >> 4, tr_chunk0 = wave_n * kWaveN / 16;
+  auto read_tr = [&](int elements) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((TrPtr)(smem + elements)); };
+  const int tr_frag = BM * BK + (8 * tr_group + tr_e) * BN + (lane & 3) * 4 + (tr_chunk0 ^ ((tr_group & 1) * 4)) * 16;
+  const int tr_d = BM * BK + (4 * tr_group + tr_e) * BN + (lane & 3) * 4 + (tr_chunk0 ^ ((tr_group >> 1) * 4)) * 16;
+  static_assert(TN == 4, "a wave's column blocks are the low two bits of the chunk");
+  auto read_q = [&](int stage, int kk, int j) {
+    const int at = tr_frag + stage * kStageElems + kk * 32 * BN + ((j ^ tr_e) << 4);
+    const s16x4 lo = read_tr(at), hi = read_tr(at + 4 * BN);
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
 
   // 16x16x32 MFMA operands: lane l supplies row l % 16 of its 16-row block and the 8 k values of chunk l / 16 of
   // the 32 wide step.  (At equal peak rate this shape draws less power than 32x32x16 on operands with random
@@ -387,15 +416,20 @@ gemm_nt_kernel(LaunchArgs<N> args) {
 #pragma unroll
     for (int i = 0; i < TMH; ++i) fa_lo[i] = *reinterpret_cast<const bf16x8*>(frag_p + off + i * 16 * BK);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) fb0[j] = *reinterpret_cast<const bf16x8*>(frag_q + off + j * 16 * BK);
+    for (int j = 0; j < TN; ++j) {
+      if constexpr (kQColumns) fb0[j] = read_q(0, 0, j);
+      else fb0[j] = *reinterpret_cast<const bf16x8*>(frag_q + off + j * 16 * BK);
+    }
   }
   // One half step: the TMH x TN MFMAs on the fragments in hand (use_a for tile rows row0.., use_b), kReads LDS
   // reads (read(r), one behind each of the first MFMAs) and kLoads slab loads, interleaved instruction by
   // instruction: MFMA, LDS read, MFMA, LDS read, ..., slab load, ...  The matrix pipe is handed to the oldest wave
   // that has an MFMA ready, so whenever one of the two waves of a SIMD sits at the barrier the other runs alone,
   // and then every clump of other instructions between two MFMAs is a bubble in the pipe.
-  auto half_step = [&](auto row0_tag, const bf16x8 (&use_a)[TMH], const bf16x8 (&use_b)[TN], auto reads_tag, auto&& read,
+  // The first kPairs reads are two instructions each.
+  auto half_step = [&](auto row0_tag, const bf16x8 (&use_a)[TMH], const bf16x8 (&use_b)[TN], auto reads_tag, auto pairs_tag, auto&& read,
                        auto loads_tag, auto&& load) {
+    constexpr int kPairs = decltype(pairs_tag)::value;
     constexpr int kRow0 = decltype(row0_tag)::value;
     constexpr int kReads = decltype(reads_tag)::value;
     constexpr int kLoads = decltype(loads_tag)::value;
@@ -413,7 +447,8 @@ gemm_nt_kernel(LaunchArgs<N> args) {
 #pragma unroll
       for (int n = c * kPer; n < (c + 1) * kPer; ++n) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-        if (n < kReads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
+        if (n < kPairs) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        else if (n < kReads) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read
       }
       __builtin_amdgcn_sched_barrier(0);
       if constexpr (kLoads > 0) {
@@ -427,17 +462,19 @@ gemm_nt_kernel(LaunchArgs<N> args) {
   // first half of step kk (fragments in fa_lo / use_b): reads the second half's P fragments
   auto first_half = [&](const bf16x8 (&use_b)[TN], int read_stage, int kk, auto loads_tag, auto&& load) {
     const int off = frag_off(read_stage, kk);
-    half_step(Zero{}, fa_lo, use_b, std::integral_constant<int, TMH>{},
+    half_step(Zero{}, fa_lo, use_b, std::integral_constant<int, TMH>{}, Zero{},
               [&](int r) { fa_hi[r] = *reinterpret_cast<const bf16x8*>(frag_p + off + (TMH + r) * 16 * BK); }, loads_tag, load);
   };
   // second half (fa_hi / use_b): reads the Q fragments and the first-half P fragments of the step after it
   auto second_half = [&](const bf16x8 (&use_b)[TN], bf16x8 (&next_b)[TN], int read_stage, int read_kk, auto loads_tag, auto&& load) {
     const int off = frag_off(read_stage, read_kk);
-    half_step(Upper{}, fa_hi, use_b, std::integral_constant<int, TN + TMH>{},
+    half_step(Upper{}, fa_hi, use_b, std::integral_constant<int, TN + TMH>{}, std::integral_constant<int, kQColumns ? TN : 0>{},
               [&](int r) {
                 // Q fragments first: the next step's first MFMAs need every one of them but only the first P fragment
-                if (r < TN) next_b[r] = *reinterpret_cast<const bf16x8*>(frag_q + off + r * 16 * BK);
-                else fa_lo[r - TN] = *reinterpret_cast<const bf16x8*>(frag_p + off + (r - TN) * 16 * BK);
+                if (r < TN) {
+                  if constexpr (kQColumns) next_b[r] = read_q(read_stage, read_kk, r);
+                  else next_b[r] = *reinterpret_cast<const bf16x8*>(frag_q + off + r * 16 * BK);
+                } else fa_lo[r - TN] = *reinterpret_cast<const bf16x8*>(frag_p + off + (r - TN) * 16 * BK);
               },
               loads_tag, load);
   };
@@ -466,6 +503,10 @@ gemm_nt_kernel(LaunchArgs<N> args) {
 #pragma unroll
     for (int n = 0; n < kDBatch; ++n) {
       const int pair = batch * kDBatch + n, ii = pair / TN, j = pair % TN;
+      if constexpr (kQColumns) {
+        d_vals[n] = __builtin_bit_cast(u32x2, read_tr(tr_d + stage * kStageElems + ii * 16 * BN + ((j ^ tr_e) << 4)));
+        continue;
+      }
       const int chunk = (2 * ii + (lane >> 5)) ^ d_swizzle;
       d_vals[n] = *reinterpret_cast<const u32x2*>(smem + stage * kStageElems + d_base + j * 16 * BK + (chunk << 3));
     }
@@ -557,6 +598,13 @@ gemm_nt_kernel(LaunchArgs<N> args) {
     for (int it = first_d + kDSlabs; it < n_slabs; ++it) slab(it, NoD{});
   } else {
     for (int it = 0; it < n_slabs; ++it) slab(it, NoD{});
+  }
+  };  // walk
+  if constexpr (BM == 256) {
+    if (q_columns) walk(std::true_type{});
+    else walk(std::false_type{});
+  } else {  // without the code it never runs
+    walk(std::false_type{});
   }
   __builtin_amdgcn_s_waitcnt(0x0070);  // the loads past the end of the walk have landed too; LDS is free
 
@@ -1161,6 +1209,9 @@ GemmPlan gemm_plan(const GemmGroup& g, const GemmScratch& scratch) {
   bool symmetric = true;  // every problem of the launch
   for (int i = 0; i < g.n; ++i) symmetric = symmetric && (g.problem[i].flags & kGemmSymmetric) != 0;
   const int variant = symmetric ? tuning.symmetric_variant : tuning.general_variant;
+  bool q_columns = false;
+  for (int i = 0; i < g.n; ++i) q_columns = q_columns || (g.problem[i].flags & kGemmQColumns) != 0;
+  if (q_columns) return make_plan(g, 1, scratch, tuning);
   if (variant == 1 || variant == 2 || variant == kSmallVariant) return make_plan(g, variant, scratch, tuning);
   const GemmPlan big = make_plan(g, 1, scratch, tuning);
   // On a machine shared with other matrices' kernels the CUs a part-filling triangle of big tiles leaves idle are
@@ -1177,6 +1228,8 @@ GemmPlan gemm_plan(const GemmGroup& g, const GemmScratch& scratch) {
   const GemmPlan smallest = make_plan(g, kSmallVariant, scratch, tuning);
   return smallest.us < better.us ? smallest : better;
 }
+
+bool on_256_tiles(const GemmPlan& plan) { return kVariants[plan.variant].tile == 256; }
 
 int64_t gemm_nt_executed_flops(const GemmGroup& g) {
   GemmScratch scratch;
@@ -1200,7 +1253,10 @@ int gemm_nt_bf16(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& sc
     if (!a.P || !a.Q || !a.C) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: null operand");
     // tiles reach beyond M and N: rows up to the next multiple of 256 must exist (the caller's word), columns are checked
     const int mp = (a.M + 255) / 256 * 256, np = (a.N + 255) / 256 * 256;
-    if (a.ldp < a.K || a.ldq < a.K || (!update && a.ldc < np) || (a.D && a.ldd < np) || (a.CT && a.ldct < mp))
+    const bool q_columns = (a.flags & kGemmQColumns) != 0;
+    if (q_columns && (symmetric || plan.variant != 1 || a.K < a.M || static_cast<int64_t>(mp) * a.ldq >= 1 << 30))
+      return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: a Q of K rows needs a general product over M on 256 x 256 tiles and less than 2 GiB");
+    if (a.ldp < a.K || a.ldq < (q_columns ? np : a.K) || (!update && a.ldc < np) || (a.D && a.ldd < np) || (a.CT && a.ldct < mp))
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: leading dimension smaller than the padded row length");
     if ((a.ldp | a.ldq) % 8 || (reinterpret_cast<uintptr_t>(a.P) | reinterpret_cast<uintptr_t>(a.Q)) % 16)
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: operands must be 16-byte aligned with leading dimensions multiple of 8");
