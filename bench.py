@@ -499,7 +499,7 @@ def main() -> int:
         tflops_executed = executed / (med * 1e-3) / 1e12
         legs["muon_hidden4096"]["ns_TFLOPs_executed"] = round(tflops_executed, 1)
         result["roofline_muon"] = {
-            "kernel": "gemm_nt_kernel (Newton-Schulz products; the whole Muon step is timed: momentum, norm, 15 products of the square matrix and 17 of each of the others, whose first three iterations are folded, update)",
+            "kernel": "gemm_nt_kernel (Newton-Schulz products; the whole Muon step is timed: momentum, norm, 15 products per matrix, update)",
             "bound": "mfma",
             # the reference's count: full GEMMs, 5 * (4 m^2 n + 2 m^3) per matrix
             "achieved": round(tflops, 1),

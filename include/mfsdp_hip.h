@@ -266,9 +266,8 @@ int mfsdp_muon_step_ex(void* param, const void* grad, void* momentum_buf, int dt
  * mfsdp_muon_many_workspace_bytes is what the library makes best use of (bounded: 1.4 GiB, or what the largest matrix
  * needs), mfsdp_muon_workspace_bytes of the largest job is the least it takes.  Every job is checked before
  * anything is enqueued.  Results depend on the other jobs, and on the workspace, only through the order in which a product
- * sums and the order of the products: which tile a launch takes and how its K walk is cut follow from all matrices of the
- * launch, at any size, and so does whether the first three of five or more Newton-Schulz iterations of fp32 matrices with a
- * short side of 2048 or more are folded into one (no less precise, see csrc/muon.hip).  The momentum does not depend on them.  A caller that needs bits independent of the other matrices makes one call per matrix.
+ * sums: which tile a launch takes and how its K walk is cut follow from all matrices of the launch, at any size.  The
+ * momentum does not depend on them.  A caller that needs bits independent of the other matrices makes one call per matrix.
  */
 typedef struct mfsdp_muon_job {
   void* param;
@@ -336,9 +335,9 @@ int mfsdp_adamw_step_many(int64_t n, const mfsdp_adamw_span* spans, double lr, d
  */
 
 /*
- * Flops the Newton-Schulz kernels execute for `steps` iterations with the default coefficients on a rows x cols fp32 matrix
- * with the current tuning and the flags of mfsdp_muon_step_ex (sides rounded up to whole tiles, K to 64; symmetric products
- * compute only the tiles on or below the diagonal; folded iterations count as they run).  The reference executes full products: steps * (4 m^2 n + 2 m^3) with
+ * Flops the Newton-Schulz kernels execute for `steps` iterations on a rows x cols matrix with the current tuning
+ * and the flags of mfsdp_muon_step_ex (sides rounded up to whole tiles, K to 64; the two symmetric products of a step
+ * compute only the tiles on or below the diagonal).  The reference executes full products: steps * (4 m^2 n + 2 m^3) with
  * m the short side.  mfsdp_muon_many_executed_flops counts for mfsdp_muon_step_many with a workspace of that size, where
  * the tile of a launch follows from all of its matrices; 0 where that call would refuse the sizes or the workspace.
  */

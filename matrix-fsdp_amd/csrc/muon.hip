@@ -11,18 +11,6 @@
 // A step's matrices do not depend on each other: up to 32 of them go through every stage as ONE launch (momentum, norm,
 // scale + transpose, three products per iteration), so that small matrices fill the machine together and a step costs
 // 2 or 3 + 3 x steps launches instead of that many per matrix.
-//
-// Three iterations folded into one.  X' = (a + b A + c A A) X = P X with a symmetric P, so three iterations are
-//     X3 = P2 P1 P0 X,    A1 = P0 A0 P0,    A2 = P1 A1 P1
-// on m x m matrices, and X itself is multiplied once instead of three times and its Gram matrix formed once.  With a
-// symmetric product counted half, three iterations cost 3 (3 m^2 n + m^3) multiply-adds one by one and 3 m^2 n + 9 m^3 folded:
-// 18 against 30 m^3 at n = 3 m, the same at n = m.  See kFoldSide for where it is taken.
-// What would be lost is precision: A and the P have a dominant diagonal, whose rounding to bf16 no longer averages out over
-// the n elements of the rows of a rounded X.  Folded iterations therefore carry what the rounding of a diagonal leaves over in
-// fp32 (kGemmDiagC).  Error of five to eight iterations against 64-bit arithmetic, folded / one by one, of random, spiked,
-// low-rank, power-law and geometric spectra and of graded rows and columns: 0.2 to 0.99 at 2048x2048 and 2048x8192, 0.90 to 0.97
-// at 4096x11008 and 5120x13824; up to 1.02 at 1024x1536, 1.3 at 512 and 5.7 at 64.  Folding the last two as well: up to
-// 2 at 1024 (graded columns), so those stay.
 #include "mfsdp_common.h"
 #include "muon_elementwise.h"
 #include "muon_gemm.h"
@@ -39,22 +27,6 @@ constexpr int64_t kPad = 256;
 constexpr int64_t kAlign = 256;  // byte alignment of every workspace region
 constexpr int kTileK = 64;       // K of every product is rounded up to this: the operands are zero up to there
 
-// Where the first three iterations are folded (see above).
-// By precision: from short sides of 2048 on the error is no larger than that of the single iterations.  Fewer than five
-// iterations, or other coefficients than those the error was measured with (torch/optim/_muon.py:36-39), stay single.  So do
-// bf16 parameters.  Folded and torch's updates, each about 0.01 from 64-bit arithmetic, are 0.007 from each other where single
-// ones are 0.003, because the X between the folded iterations are not rounded; a bf16 parameter that moves by one or two of its
-// rounding steps shows that as 5 % of its move instead of 3 %.
-// By time: folding saves 6 (n - m) m^2 multiply-adds and costs a launch more and the lower rate of the symmetric products.  It
-// pays once the matrices of a group together save about 45e9 of them (whole step, single -> folded, us: 2048x4096 alone 511 ->
-// 510, 4096x5120 1716 -> 1657, 2048x3072 459 -> 474, four of them 1258 -> 1191, 4096x12288 3246 -> 2640, 5120x15360 5966 ->
-// 4652) and no square one is among those folded (4096x4096 1324 -> 1415, four of 2048x2048 880 -> 961; 5120x5120 2478 -> 2422
-// is let go).
-constexpr int kFoldSide = 2048;
-constexpr int kFolded = 3;
-constexpr double kFoldSaving = 45e9;
-bool may_fold(int m, int n) { return m >= kFoldSide && 5 * static_cast<int64_t>(n) >= 6 * static_cast<int64_t>(m); }
-
 int64_t round_up(int64_t v, int64_t to) { return (v + to - 1) / to * to; }
 
 // One matrix in the workspace.  Leading dimensions are padded to multiples of 256, so that tiles of every variant stay
@@ -64,12 +36,10 @@ struct Matrix {
   int m, n, mp, np;        // short / long side and their padded sizes
   bool tall;               // rows > cols: the iteration runs on the transpose
   bool keeps_xt;           // X^T is stored beside X, see stores_transposes
-  bool folded;             // of this group's iteration, see choose_folding
   uint16_t* X[2];          // mp x np
   uint16_t* XT[2];         // np x mp
-  uint16_t* A;             // mp x mp, of a matrix that may fold with room for the residuals of their diagonals behind them
-  uint16_t* B;
-  uint16_t* T[3];          // three more of them, in the place of X[1] and XT[1]: used up before those are written
+  uint16_t* A;             // mp x mp
+  uint16_t* B;             // mp x mp
   int64_t bytes;
   uint16_t* xraw() const { return X[1]; }  // rows x cols unscaled bf16 update
 };
@@ -79,7 +49,6 @@ bool plan_matrix(int64_t rows, int64_t cols, char* base, Matrix* w) {
   w->rows = static_cast<int>(rows);
   w->cols = static_cast<int>(cols);
   w->tall = rows > cols;
-  w->folded = false;
   w->keeps_xt = true;
   w->m = static_cast<int>(std::min(rows, cols));
   w->n = static_cast<int>(std::max(rows, cols));
@@ -89,17 +58,13 @@ bool plan_matrix(int64_t rows, int64_t cols, char* base, Matrix* w) {
   // (The square matrices, padded the same way, are no faster.)
   if (w->np % 2048 == 0 && w->mp >= 1024 && w->np < kMaxGemmLeading) w->np += kPad;
   const int64_t x_bytes = round_up(static_cast<int64_t>(w->mp) * w->np * 2, kAlign);
-  // 2 MiB-aligned as without the residuals: at odd multiples of 4 KiB the hidden4096 step takes 0.5 % longer
-  const int64_t a_bytes = may_fold(w->m, w->n) ? round_up(static_cast<int64_t>(w->mp) * (w->mp * 2 + 4), 1 << 21) : round_up(static_cast<int64_t>(w->mp) * w->mp * 2, kAlign);
+  const int64_t a_bytes = round_up(static_cast<int64_t>(w->mp) * w->mp * 2, kAlign);
   int64_t off = 0;
-  auto at = [&](int64_t offset) { return reinterpret_cast<uint16_t*>(base ? base + offset : nullptr); };
-  auto take = [&](int64_t bytes) { uint16_t* r = at(off); off += bytes; return r; };
+  auto take = [&](int64_t bytes) { char* r = base ? base + off : nullptr; off += bytes; return reinterpret_cast<uint16_t*>(r); };
   w->X[0] = take(x_bytes);
-  w->X[1] = at(off);
-  w->XT[1] = at(off + x_bytes);
-  for (int i = 0; i < 3; ++i) w->T[i] = at(off + i * a_bytes);
-  off += std::max(2 * x_bytes, may_fold(w->m, w->n) ? 3 * a_bytes : 0);
+  w->X[1] = take(x_bytes);
   w->XT[0] = take(x_bytes);
+  w->XT[1] = take(x_bytes);
   w->A = take(a_bytes);
   w->B = take(a_bytes);
   w->bytes = off;
@@ -157,145 +122,11 @@ void finish_group(Group* g, char* shared) {
   }
 }
 
-// Coefficients and number of the iterations.
-struct Iteration {
-  float a, b, c;
-  int steps;
-};
-
-// Which matrices of a group fold their first iterations; see may_fold.
-void choose_folding(Matrix* w, int n, const Iteration& it, bool bf16_parameters) {
-  double saved = 0.0;
-  if (!bf16_parameters && it.steps >= 5 && it.a == 3.4445f && it.b == -4.7750f && it.c == 2.0315f)
-    for (int i = 0; i < n; ++i)
-      if (may_fold(w[i].m, w[i].n)) saved += 6.0 * (w[i].n - w[i].m) * w[i].m * w[i].m;
-  for (int i = 0; i < n; ++i) w[i].folded = saved >= kFoldSaving && may_fold(w[i].m, w[i].n);
-}
-
-// What a product's size depends on: products of one kind of the same matrices run by the same plan.
-enum ProductKind : uint8_t { kGram, kSquare, kUpdate };
-
-// The products of one matrix, stage by stage: every stage needs the one before it.
-struct Products {
-  const Matrix& w;
-  const Iteration& it;
-
-  static constexpr int kFoldedStages = 10;  // in the place of 3 x kFolded
-  int stages() const { return 3 * it.steps + (w.folded ? kFoldedStages - 3 * kFolded : 0); }
-
-  // X X^T into A; `diagonal`: with the residuals of the diagonals, here and below
-  GemmProblem gram(int cur, bool diagonal) const {
-    GemmProblem p{};
-    p.P = w.X[cur]; p.Q = w.X[cur]; p.C = w.A;
-    p.M = w.m; p.N = w.m; p.K = static_cast<int>(round_up(w.n, kTileK));
-    p.ldp = w.np; p.ldq = w.np; p.ldc = w.mp;
-    p.alpha = 1.0f;
-    p.flags = kGemmSymmetric | (diagonal ? kGemmDiagC : 0);
-    return p;
-  }
-  GemmProblem square(const uint16_t* P, const uint16_t* Q, uint16_t* C, bool diagonal = true) const {
-    GemmProblem p{};
-    p.P = P; p.Q = Q; p.C = C;
-    p.M = w.m; p.N = w.m; p.K = static_cast<int>(round_up(w.m, kTileK));
-    p.ldp = w.mp; p.ldq = w.mp; p.ldc = w.mp;
-    p.alpha = 1.0f;
-    p.flags = kGemmSymmetric | (diagonal ? kGemmDiagP | kGemmDiagQ | kGemmDiagC : 0);
-    return p;
-  }
-  // c A A + b A into C; with residuals, + a on the diagonal
-  GemmProblem polynomial(uint16_t* C, bool diagonal) const {
-    GemmProblem p = square(w.A, w.A, C, diagonal);
-    p.D = w.A;  // A is symmetric: D^T is Q
-    p.ldd = w.mp;
-    p.alpha = it.c; p.beta = it.b;
-    p.shift = diagonal ? it.a : 0.0f;
-    return p;
-  }
-  // B X + a X from X[cur] into X[cur ^ 1]; with residuals, B has a on its diagonal and D brings them
-  GemmProblem update(int cur, bool last, bool diagonal) const {
-    GemmProblem p{};
-    p.P = w.B; p.Q = w.XT[cur]; p.D = w.X[cur]; p.C = w.X[cur ^ 1]; p.CT = w.XT[cur ^ 1];  // Q = X^T
-    p.M = w.m; p.N = w.n; p.K = static_cast<int>(round_up(w.m, kTileK));
-    p.ldp = w.mp; p.ldq = w.mp; p.ldd = w.np; p.ldc = w.np; p.ldct = w.mp;
-    p.alpha = 1.0f; p.beta = diagonal ? 0.0f : it.a;
-    p.flags = diagonal ? kGemmDiagP : 0;
-    if (!w.keeps_xt) {
-      p.Q = w.X[cur];
-      p.ldq = w.np;
-      p.flags |= kGemmQColumns;
-      if (!(last && w.tall)) p.CT = nullptr;
-    }
-    if (last) {  // only has to leave O in the parameter's orientation
-      if (w.tall) p.flags |= kGemmSkipC;
-      else p.CT = nullptr;
-    }
-    return p;
-  }
-
-  // The products of stage `s`: one, or two that do not depend on each other.
-  int stage(int s, GemmProblem* out, ProductKind* kind) const {
-    *kind = kSquare;
-    if (w.folded && s < kFoldedStages) {
-      uint16_t *A = w.A, *B = w.B, *const *T = w.T;
-      switch (s) {
-        case 0: *kind = kGram; *out = gram(0, true); return 1;
-        case 1: *out = polynomial(B, true); return 1;                                         // P0
-        case 2: *out = square(B, A, T[0]); return 1;                                    // P0 A0
-        case 3: *out = square(B, T[0], A); return 1;                                    // A1 = P0 A0 P0
-        case 4: *out = polynomial(T[1], true); return 1;                                      // P1
-        case 5: out[0] = square(T[1], A, T[0]); out[1] = square(T[1], B, T[2]); return 2;  // P1 A1, P1 P0
-        case 6: *out = square(T[1], T[0], A); return 1;                                 // A2 = P1 A1 P1
-        case 7: *out = polynomial(T[1], true); return 1;                                      // P2
-        case 8: *out = square(T[1], T[2], B); return 1;                                 // P2 P1 P0
-        default: *kind = kUpdate; *out = update(0, false, true); return 1;
-      }
-    }
-    if (w.folded) s += 3 * kFolded - kFoldedStages;
-    const int cur = w.folded ? (s / 3 - kFolded + 1) & 1 : (s / 3) & 1;
-    switch (s % 3) {
-      case 0: *kind = kGram; *out = gram(cur, false); return 1;
-      case 1: *out = polynomial(w.B, false); return 1;
-      default: *kind = kUpdate; *out = update(cur, s / 3 + 1 == it.steps, false); return 1;
-    }
-  }
-};
-
-// Calls launch(group, kinds, matrices) for every launch of the iterations of `n` matrices: stage s of each of them, with the
-// kind of every product and the matrix it belongs to.
-template <class Launch>
-int for_each_launch(const Matrix* w, int n, const Iteration& it, bool shared, Launch&& launch) {
-  int stages = 0;
-  for (int i = 0; i < n; ++i) stages = std::max(stages, Products{w[i], it}.stages());
-  for (int s = 0; s < stages; ++s) {
-    GemmGroup first, second;  // the second products of a stage go along where there is room
-    ProductKind kinds[2][kMaxGemmGroup];
-    int matrix[2][kMaxGemmGroup];
-    for (int i = 0; i < n; ++i) {
-      const Products products{w[i], it};
-      if (s >= products.stages()) continue;
-      GemmProblem p[2];
-      ProductKind kind;
-      const int count = products.stage(s, p, &kind);
-      matrix[0][first.n] = i;
-      kinds[0][first.n] = kind;
-      first.problem[first.n++] = p[0];
-      if (count == 1) continue;
-      matrix[1][second.n] = i;
-      kinds[1][second.n] = kind;
-      second.problem[second.n++] = p[1];
-    }
-    const bool together = first.n + second.n <= kMaxGemmGroup;
-    for (int i = 0; together && i < second.n; ++i) {
-      matrix[0][first.n] = matrix[1][i];
-      kinds[0][first.n] = kinds[1][i];
-      first.problem[first.n++] = second.problem[i];
-    }
-    first.shared = shared && first.n == 1;
-    if (int rc = launch(first, kinds[0], matrix[0])) return rc;
-    if (together || second.n == 0) continue;
-    if (int rc = launch(second, kinds[1], matrix[1])) return rc;
-  }
-  return MFSDP_OK;
+// The size of the update product.
+void update_size(const Matrix& w, GemmProblem* p) {
+  p->M = w.m;
+  p->N = w.n;
+  p->K = static_cast<int>(round_up(w.m, kTileK));
 }
 
 // Does the group store X^T beside X?  The update product can take X itself (kGemmQColumns), and the epilogues of the update
@@ -308,21 +139,22 @@ int for_each_launch(const Matrix* w, int n, const Iteration& it, bool shared, La
 // * where X and X' are about what the memory-side cache of 256 MB holds (X of 157 MB: gains 2 %; the three matrices of a hidden4096
 //   step, 224 MB, lose 2 %).  This bounds X far below the 2 GiB that kGemmQColumns takes, too.
 constexpr int64_t kOneOrientationBytes = 192ll << 20;
-bool stores_transposes(const Group& group, const Iteration& it) {
+bool stores_transposes(const Group& group) {
   GemmGroup g;
   int64_t bytes = 0, tiles = 0;
   g.n = group.n;
   for (int i = 0; i < g.n; ++i) {
     const Matrix& w = group.w[i];
-    g.problem[i] = Products{w, it}.update(0, false, false);
+    g.problem[i] = GemmProblem{};
+    update_size(w, &g.problem[i]);
     bytes += static_cast<int64_t>(w.m) * w.n * 2;
     tiles += static_cast<int64_t>((w.m + 255) / 256) * ((w.n + 255) / 256);
   }
   return bytes > kOneOrientationBytes || 4 * tiles < 5 * device_cu_count() || !on_256_tiles(gemm_plan(g, group.scratch));
 }
 
-void choose_transposes(Group* group, const Iteration& it) {
-  if (it.steps == 0 || stores_transposes(*group, it)) return;  // without a product the result is taken from either
+void choose_transposes(Group* group, int steps) {
+  if (steps == 0 || stores_transposes(*group)) return;  // without a product the result is taken from either
   for (int i = 0; i < group->n; ++i) {
     Matrix& w = group->w[i];
     w.keeps_xt = false;
@@ -330,70 +162,79 @@ void choose_transposes(Group* group, const Iteration& it) {
   }
 }
 
-// The plans of a step's launches so far, by the kinds of their products and the matrices they belong to.
-class Plans {
- public:
-  const GemmPlan& of(const GemmGroup& g, const ProductKind* kinds, const int* matrix, const GemmScratch& scratch) {
-    for (int i = 0; i < n_; ++i)
-      if (sizes_[i] == g.n && std::equal(kinds, kinds + g.n, kinds_[i]) && std::equal(matrix, matrix + g.n, matrix_[i])) return plans_[i];
-    const int at = n_ < kPlans ? n_++ : kPlans - 1;
-    sizes_[at] = g.n;
-    std::copy(kinds, kinds + g.n, kinds_[at]);
-    std::copy(matrix, matrix + g.n, matrix_[at]);
-    return plans_[at] = gemm_plan(g, scratch);
-  }
-
- private:
-  static constexpr int kPlans = 12;  // more than the launches of one kind that a group with folded and single matrices has
-  int n_ = 0;
-  int sizes_[kPlans], matrix_[kPlans][kMaxGemmGroup];
-  ProductKind kinds_[kPlans][kMaxGemmGroup];
-  GemmPlan plans_[kPlans];
-};
-
 // Newton-Schulz on the updates already sitting in xraw with their partial sums of squares.  With `update_dtype` >= 0 and
 // at least one step the last product writes the parameters themselves; otherwise O is left in X[steps & 1] (wide) or
 // XT[steps & 1] (tall).
-int run_newton_schulz(Group& group, const Iteration& it, float eps, bool shared, int update_dtype, hipStream_t stream) {
-  choose_transposes(&group, it);
+int run_newton_schulz(Group& group, float a, float b, float c, int steps, float eps, bool shared, int update_dtype, hipStream_t stream) {
+  choose_transposes(&group, steps);
   if (int rc = muon_scale_transpose(group.elementwise, eps, stream)) return rc;
-  choose_folding(group.w, group.n, it, update_dtype == MFSDP_BF16);
-  Plans plans;
-  int done[kMaxMuonGroup] = {};  // update products of a matrix so far
-  return for_each_launch(group.w, group.n, it, shared, [&](GemmGroup& g, const ProductKind* kinds, const int* matrix) -> int {
-    for (int i = 0; i < g.n; ++i) {
-      GemmProblem& p = g.problem[i];
-      const int m = matrix[i];
-      const Matrix& w = group.w[m];
-      if (kinds[i] != kUpdate) continue;
-      done[m] += w.folded && done[m] == 0 ? kFolded : 1;
-      if (update_dtype < 0 || done[m] < it.steps) continue;
-      // the last product goes straight into the parameter: O is never stored
-      g.update_dtype = update_dtype;
-      p.C = group.param[m];
-      p.CT = nullptr;
-      p.update_decay = group.decay[m];
-      p.update_neg_lr = group.neg_lr[m];
-      p.flags = (p.flags & ~kGemmSkipC) | kGemmUpdate | (w.tall ? kGemmUpdateTransposed : 0);
+  GemmGroup g;
+  g.n = group.n;
+  GemmPlan gram, poly, update;  // made in the first iteration
+  for (int s = 0; s < steps; ++s) {
+    const int cur = s & 1, nxt = cur ^ 1;
+    g.alpha = 1.0f; g.beta = 0.0f; g.symmetric = 1; g.shared = shared;
+    for (int i = 0; i < group.n; ++i) {
+      const Matrix& w = group.w[i];
+      GemmProblem& p = g.problem[i] = GemmProblem{};
+      p.P = w.X[cur]; p.Q = w.X[cur]; p.C = w.A;
+      p.M = w.m; p.N = w.m; p.K = static_cast<int>(round_up(w.n, kTileK));
+      p.ldp = w.np; p.ldq = w.np; p.ldc = w.mp;
     }
-    if (kinds[0] == kSquare && it.c == 0.0f) {
+    if (s == 0) gram = gemm_plan(g, group.scratch);
+    if (int rc = gemm_nt_bf16(g, gram, group.scratch, stream)) return rc;
+    if (c == 0.0f) {
       // addmm with alpha = 0 leaves beta * A (the product is not formed at all, torch/optim/_muon.py:61 with a
-      // quadratic polynomial); the GEMM's D path needs alpha != 0 (it adds (beta / alpha) D to the accumulators).  With such
-      // coefficients nothing is folded: every product of the launch is the polynomial.
+      // quadratic polynomial); the GEMM's D path needs alpha != 0 (it adds (beta / alpha) D to the accumulators)
       for (int i = 0; i < group.n; ++i)
-        if (int rc = muon_scale_bf16(group.w[i].B, group.w[i].A, static_cast<int64_t>(group.w[i].mp) * group.w[i].mp, it.b, stream)) return rc;
-      return MFSDP_OK;
+        if (int rc = muon_scale_bf16(group.w[i].B, group.w[i].A, static_cast<int64_t>(group.w[i].mp) * group.w[i].mp, b, stream)) return rc;
+    } else {
+      g.alpha = c; g.beta = b;
+      for (int i = 0; i < group.n; ++i) {
+        const Matrix& w = group.w[i];
+        GemmProblem& p = g.problem[i] = GemmProblem{};
+        p.P = w.A; p.Q = w.A; p.D = w.A; p.C = w.B;  // A is symmetric: D^T is Q
+        p.M = w.m; p.N = w.m; p.K = static_cast<int>(round_up(w.m, kTileK));
+        p.ldp = w.mp; p.ldq = w.mp; p.ldd = w.mp; p.ldc = w.mp;
+      }
+      if (s == 0) poly = gemm_plan(g, group.scratch);
+      if (int rc = gemm_nt_bf16(g, poly, group.scratch, stream)) return rc;
     }
-    return gemm_nt_bf16(g, plans.of(g, kinds, matrix, group.scratch), group.scratch, stream);
-  });
+    g.alpha = 1.0f; g.beta = a; g.symmetric = 0; g.shared = 0;
+    for (int i = 0; i < group.n; ++i) {
+      const Matrix& w = group.w[i];
+      GemmProblem& p = g.problem[i] = GemmProblem{};
+      p.P = w.B; p.Q = w.XT[cur]; p.D = w.X[cur]; p.C = w.X[nxt]; p.CT = w.XT[nxt];  // Q = X^T
+      update_size(w, &p);
+      p.ldp = w.mp; p.ldq = w.mp; p.ldd = w.np; p.ldc = w.np; p.ldct = w.mp;
+      if (!w.keeps_xt) {
+        p.Q = w.X[cur];
+        p.ldq = w.np;
+        p.flags |= kGemmQColumns;
+        if (s + 1 < steps) p.CT = nullptr;
+      }
+      if (s + 1 == steps) {  // the last step only has to leave O in the parameter's orientation
+        if (w.tall) p.flags |= kGemmSkipC;
+        else p.CT = nullptr;
+        if (update_dtype >= 0) {  // ... or take it straight into the parameter: O is never stored
+          g.update_dtype = update_dtype;
+          p.update_param = group.param[i];
+          p.update_decay = group.decay[i];
+          p.update_neg_lr = group.neg_lr[i];
+          if (w.tall) p.flags |= kGemmUpdateTransposed;
+        }
+      }
+    }
+    if (s == 0) update = gemm_plan(g, group.scratch);
+    if (int rc = gemm_nt_bf16(g, update, group.scratch, stream)) return rc;
+  }
+  return MFSDP_OK;
 }
 
 const uint16_t* result_of(const Matrix& w, int steps) { return w.tall ? w.XT[steps & 1] : w.X[steps & 1]; }
 
 // everything that can be refused is refused before the first kernel is enqueued (a step must not be left half applied)
-int check_iteration(const Iteration& it) {
-  const float a = it.a, b = it.b, c = it.c;
-  const int steps = it.steps;
+int check_iteration(float a, float b, float c, int steps) {
   if (!std::isfinite(a) || !std::isfinite(b) || !std::isfinite(c) || (c != 0.0f && !std::isfinite(b / c)))
     return fail(MFSDP_ERR_INVALID, "Newton-Schulz coefficients must be finite (and b / c representable), got (%g, %g, %g)", a, b, c);
   if (steps < 0 || steps >= 100) return fail(MFSDP_ERR_INVALID, "Number of steps must be less than 100 for computational efficiency");
@@ -421,13 +262,14 @@ struct StepArgs {
   int dtype;
   double momentum;
   int nesterov;
-  Iteration iteration;
+  float a, b, c;
+  int steps;
   float eps;
   bool shared;
 };
 
 int check_step(const StepArgs& s) {
-  if (int rc = check_iteration(s.iteration)) return rc;
+  if (int rc = check_iteration(s.a, s.b, s.c, s.steps)) return rc;
   if (s.dtype != MFSDP_F32 && s.dtype != MFSDP_BF16) return fail(MFSDP_ERR_INVALID, "dtype must be f32 or bf16");
   if (!(s.momentum >= 0.0)) return fail(MFSDP_ERR_INVALID, "momentum should be >= 0 but is: %g", s.momentum);
   return MFSDP_OK;
@@ -458,8 +300,8 @@ void add_to_group(Group* g, const Matrix& w, void* param, const void* grad, void
 int run_step(Group* g, char* shared, const StepArgs& s, hipStream_t stream) {
   finish_group(g, shared);
   if (int rc = muon_momentum(g->elementwise, s.dtype, s.momentum, s.nesterov, true, stream)) return rc;
-  if (int rc = run_newton_schulz(*g, s.iteration, s.eps, s.shared, s.dtype, stream)) return rc;
-  if (s.iteration.steps > 0) return MFSDP_OK;  // the last product has updated the parameters
+  if (int rc = run_newton_schulz(*g, s.a, s.b, s.c, s.steps, s.eps, s.shared, s.dtype, stream)) return rc;
+  if (s.steps > 0) return MFSDP_OK;  // the last product has updated the parameters
   for (int i = 0; i < g->n; ++i) {
     const Matrix& w = g->w[i];
     if (int rc = muon_apply(g->param[i], s.dtype, result_of(w, 0), w.rows, w.cols, w.tall ? w.mp : w.np, g->decay[i], g->neg_lr[i], stream)) return rc;
@@ -502,17 +344,24 @@ struct PendingList {
 
 int out_of_host_memory(int64_t n) { return fail(MFSDP_ERR_UNSUPPORTED, "out of host memory for %lld matrices", static_cast<long long>(n)); }
 
-// Flops the products of `steps` Newton-Schulz steps (default coefficients, fp32 parameters) of `n` matrices that share their
-// launches execute.
-int64_t executed_flops(Matrix* w, int n, int steps, bool shared) {
-  const Iteration it{3.4445f, -4.7750f, 2.0315f, steps};
-  choose_folding(w, n, it, false);
-  int64_t flops = 0;
-  for_each_launch(w, n, it, shared, [&](const GemmGroup& g, const ProductKind*, const int*) {
-    flops += gemm_nt_executed_flops(g);
-    return MFSDP_OK;
-  });
-  return flops;
+// Flops the products of one Newton-Schulz step of `n` matrices that share their launches execute.
+int64_t executed_flops(const Matrix* w, int n, bool shared) {
+  GemmGroup gram, poly, update;
+  gram.n = poly.n = update.n = n;
+  gram.symmetric = poly.symmetric = 1;
+  gram.shared = poly.shared = shared;
+  auto size = [](GemmProblem* p, int rows, int cols, int k) {
+    *p = GemmProblem{};
+    p->M = rows;
+    p->N = cols;
+    p->K = static_cast<int>(round_up(k, kTileK));
+  };
+  for (int i = 0; i < n; ++i) {
+    size(&gram.problem[i], w[i].m, w[i].m, w[i].n);
+    size(&poly.problem[i], w[i].m, w[i].m, w[i].m);
+    size(&update.problem[i], w[i].m, w[i].n, w[i].m);
+  }
+  return gemm_nt_executed_flops(gram) + gemm_nt_executed_flops(poly) + gemm_nt_executed_flops(update);
 }
 
 }  // namespace
@@ -547,7 +396,7 @@ extern "C" int64_t mfsdp_muon_many_workspace_bytes(int64_t n, const int64_t* row
 extern "C" int64_t mfsdp_muon_executed_flops(int64_t rows, int64_t cols, int steps, int flags) {
   Matrix w;
   if (steps < 0 || !plan_matrix(rows, cols, nullptr, &w)) return 0;
-  return executed_flops(&w, 1, steps, (flags & MFSDP_MUON_SHARED_MACHINE) != 0);
+  return steps * executed_flops(&w, 1, (flags & MFSDP_MUON_SHARED_MACHINE) != 0);
 }
 
 extern "C" int64_t mfsdp_muon_many_executed_flops(int64_t n, const int64_t* rows, const int64_t* cols, int steps, int64_t workspace_bytes) {
@@ -567,16 +416,15 @@ extern "C" int64_t mfsdp_muon_many_executed_flops(int64_t n, const int64_t* rows
     int count = 0;
     for (const int64_t end = order.group_end(next, workspace_bytes - kSharedBytes, &bytes); next < end; ++next)
       plan_matrix(rows[order.data[next].job], cols[order.data[next].job], nullptr, &w[count++]);
-    flops += executed_flops(w, count, steps, false);
+    flops += executed_flops(w, count, false);
   }
-  return flops;
+  return steps * flops;
 }
 
 extern "C" int mfsdp_newton_schulz(const void* update, int update_dtype, int64_t rows, int64_t cols, float a, float b, float c,
                                    int steps, float eps, void* out_bf16, void* workspace, int64_t workspace_bytes, void* stream) {
   Group g;
-  const Iteration it{a, b, c, steps};
-  if (int rc = check_iteration(it)) return rc;
+  if (int rc = check_iteration(a, b, c, steps)) return rc;
   if (int rc = check_matrix(rows, cols, steps, &g.w[0])) return rc;
   if (int rc = check_workspace(workspace, workspace_bytes, g.w[0].bytes + kSharedBytes)) return rc;
   if (update_dtype != MFSDP_F32 && update_dtype != MFSDP_BF16) return fail(MFSDP_ERR_INVALID, "update dtype must be f32 or bf16");
@@ -589,14 +437,14 @@ extern "C" int mfsdp_newton_schulz(const void* update, int update_dtype, int64_t
   add_to_group(&g, w, nullptr, update, nullptr, 0.0, 0.0, 0.0);
   finish_group(&g, base + w.bytes);
   if (int rc = muon_momentum(g.elementwise, update_dtype, 0.0, 0, false, s)) return rc;
-  if (int rc = run_newton_schulz(g, it, eps, false, -1, s)) return rc;
+  if (int rc = run_newton_schulz(g, a, b, c, steps, eps, false, -1, s)) return rc;
   return muon_extract(out_bf16, result_of(w, steps), w.rows, w.cols, w.tall ? w.mp : w.np, s);
 }
 
 extern "C" int mfsdp_muon_step_ex(void* param, const void* grad, void* momentum_buf, int dtype, int64_t rows, int64_t cols, double lr,
                                   double weight_decay, double momentum, int nesterov, float a, float b, float c, int steps, float eps,
                                   double adjusted_lr, int flags, void* workspace, int64_t workspace_bytes, void* stream) {
-  const StepArgs s{dtype, momentum, nesterov, {a, b, c, steps}, eps, (flags & MFSDP_MUON_SHARED_MACHINE) != 0};
+  const StepArgs s{dtype, momentum, nesterov, a, b, c, steps, eps, (flags & MFSDP_MUON_SHARED_MACHINE) != 0};
   Matrix w;
   if (int rc = check_step(s)) return rc;
   if (int rc = check_matrix(rows, cols, steps, &w)) return rc;
@@ -621,7 +469,7 @@ extern "C" int mfsdp_muon_step_many(int64_t n, const mfsdp_muon_job* jobs, int d
                                     float c, int steps, float eps, void* workspace, int64_t workspace_bytes, void* stream) {
   if (n < 0 || (n > 0 && jobs == nullptr)) return fail(MFSDP_ERR_INVALID, "jobs is null or n negative");
   if (n == 0) return MFSDP_OK;
-  const StepArgs s{dtype, momentum, nesterov, {a, b, c, steps}, eps, false};
+  const StepArgs s{dtype, momentum, nesterov, a, b, c, steps, eps, false};
   if (int rc = check_step(s)) return rc;
   PendingList order(n);
   if (!order.data) return out_of_host_memory(n);
@@ -659,7 +507,6 @@ extern "C" int mfsdp_gemm_nt_bf16(const void* p, const void* q, void* c, int m, 
   a.P = p; a.Q = q; a.C = c;
   a.M = m; a.N = n; a.K = k;
   a.ldp = k; a.ldq = k; a.ldc = n;
-  a.alpha = 1.0f;
   GemmScratch scratch;
   scratch.partials = partials;
   scratch.partials_bytes = partials ? partials_bytes : 0;

@@ -15,31 +15,17 @@ namespace mfsdp {
 //   D may be null (beta ignored); with D, Q must hold its transpose: Q[n][k] == D[k][n] for k < K, where K covers M
 //   (whole tiles pick their D values out of the Q slabs on their way through LDS; the fix-up of K-split pieces reads D
 //   itself).  CT, when non-null, also receives the transpose: CT[n][m] = C[m][n] (ldct); with kGemmSkipC only CT is written.
-// Parameter update in the epilogue (the last product of a Muon step): with kGemmUpdate, C is the parameter and every element
-// o = bf16(alpha P Q^T + beta D) of the M x N result goes into it,
+// Parameter update in the epilogue (the last product of a Muon step): when update_param is set, nothing is stored to
+// C / CT; every element o = bf16(alpha P Q^T + beta D) of the M x N result instead goes into
 //     param <- round(param * update_decay) + update_neg_lr * o        (torch/optim/_muon.py:313-315)
-// contiguous and row-major (M x N, or N x M with kGemmUpdateTransposed); nothing else is stored.  General products only.
-//
-// kGemmSymmetric: P Q^T is known to be symmetric (M == N); only tiles on or below the diagonal are computed and each
-// off-diagonal tile is also written mirrored into C.
+// on the contiguous row-major parameter (M x N, or N x M with kGemmUpdateTransposed).  General products only.
 //
 // kGemmQColumns: Q is given as K x N row-major (ldq), rows beyond M taken as zero, K spanning M, less than 2 GiB of it; general
 // products on 256 tiles (gemm_plan takes no others for them).  D is then the same matrix.
-//
-// Diagonals to more than bf16.  A square operand S (leading dimension ld) may carry behind its last row, at S + ld * ld, ld
-// floats with what the rounding of each diagonal element left over (residual_of).  With kGemmDiagC a symmetric product adds
-// `shift` to its diagonal, takes the residuals of P and Q into it (kGemmDiagP / kGemmDiagQ: alpha (P_ii dq_i + dp_i Q_ii) +
-// beta dq_i) and leaves C's own residuals behind C.  With kGemmDiagP a general product takes its D operand times
-// beta + alpha dp_i, row by row, so that diag(dp) Q^T is part of the result.
 enum GemmFlags {
   kGemmSkipC = 1,
   kGemmUpdateTransposed = 2,
-  kGemmUpdate = 4,
-  kGemmSymmetric = 8,
-  kGemmDiagP = 16,
-  kGemmDiagQ = 32,
-  kGemmDiagC = 64,
-  kGemmQColumns = 128,
+  kGemmQColumns = 4,
 };
 struct GemmProblem {
   const void* P;
@@ -47,27 +33,24 @@ struct GemmProblem {
   const void* D;
   void* C;
   void* CT;
+  void* update_param;
   int M, N, K;
   int ldp, ldq, ldd, ldc, ldct;
-  float alpha, beta, shift;
   float update_decay, update_neg_lr;
   int flags;
   // filled by the launch: K pieces per split tile, first partial tile of the problem in the scratch
   int splits, partial_base;
 };
 
-// The residuals behind a square matrix of leading dimension `ld` (see above).
-template <class T>
-__host__ __device__ inline float* residual_of(T* square, int ld) {
-  return reinterpret_cast<float*>(const_cast<uint16_t*>(static_cast<const uint16_t*>(square)) + static_cast<int64_t>(ld) * ld);
-}
-
 constexpr int kMaxGemmLeading = 1 << 22;  // largest leading dimension of P and Q: a tile's rows are reached by 31-bit byte offsets
 constexpr int kMaxGemmGroup = 32;  // problems one launch carries by value in its kernel arguments
 
-// Products of one launch.
+// Products of one launch.  symmetric: every P*Q^T is known to be symmetric (M == N); only tiles on or below the diagonal
+// are computed and each off-diagonal tile is also written mirrored into C.
 struct GemmGroup {
   int n = 0;
+  float alpha = 1.0f, beta = 0.0f;
+  int symmetric = 0;
   int update_dtype = 0;  // of the parameters (MFSDP_F32 / MFSDP_BF16)
   int shared = 0;        // other matrices' products run beside this launch of one problem on other streams: a symmetric product
                          // then takes the 256 x 256 tiles even where their triangle fills only part of the CUs

@@ -72,7 +72,7 @@ __device__ __forceinline__ void update_param8(const GemmProblem& a, int dtype, i
   }
   const float decay = a.update_decay, neg_lr = a.update_neg_lr;
   if (dtype == MFSDP_F32) {
-    float* p = static_cast<float*>(a.C) + at;
+    float* p = static_cast<float*>(a.update_param) + at;
     if (n == 8) {
       f32x4 lo = reinterpret_cast<const f32x4_a4*>(p)[0], hi = reinterpret_cast<const f32x4_a4*>(p)[1];
 #pragma unroll
@@ -86,7 +86,7 @@ __device__ __forceinline__ void update_param8(const GemmProblem& a, int dtype, i
       for (int e = 0; e < n; ++e) p[e] = p[e] * decay + neg_lr * o[e];
     }
   } else {
-    uint16_t* p = static_cast<uint16_t*>(a.C) + at;
+    uint16_t* p = static_cast<uint16_t*>(a.update_param) + at;
     auto one = [&](uint16_t old, float ov) {
       const float scaled = bf16_bits_to_float(__builtin_bit_cast(uint16_t, static_cast<__bf16>(bf16_bits_to_float(old) * decay)));
       return __builtin_bit_cast(uint16_t, static_cast<__bf16>(scaled + neg_lr * ov));
@@ -101,32 +101,6 @@ __device__ __forceinline__ void update_param8(const GemmProblem& a, int dtype, i
       for (int e = 0; e < n; ++e) p[e] = one(p[e], o[e]);
     }
   }
-}
-
-// What a general product multiplies row `row` of D with; a symmetric one takes the residuals into its diagonal only.
-__device__ __forceinline__ float row_beta(const GemmProblem& a, int row) {
-  const bool residuals = (a.flags & (kGemmDiagP | kGemmSymmetric)) == kGemmDiagP;
-  return a.beta + (residuals ? a.alpha * residual_of(a.P, a.ldp)[row] : 0.0f);
-}
-
-// Diagonal element `row` of a kGemmDiagC product: `v` is alpha P Q^T + beta D from the bf16 operands; returns it with the
-// residuals of the operands and the shift taken in, and stores what its rounding to bf16 leaves over.
-__device__ __forceinline__ float finish_diagonal(const GemmProblem& a, int row, float v) {
-  float rest = 0.0f;  // rows beyond the result stay zero: the next product's K runs over them
-  if (row < a.M) {
-    const float dp = a.flags & kGemmDiagP ? residual_of(a.P, a.ldp)[row] : 0.0f;
-    const float dq = a.flags & kGemmDiagQ ? residual_of(a.Q, a.ldq)[row] : 0.0f;
-    if (a.flags & (kGemmDiagP | kGemmDiagQ)) {
-      const float p = bf16_bits_to_float(static_cast<const uint16_t*>(a.P)[static_cast<int64_t>(row) * a.ldp + row]);
-      const float q = bf16_bits_to_float(static_cast<const uint16_t*>(a.Q)[static_cast<int64_t>(row) * a.ldq + row]);
-      v += a.alpha * (p * dq + dp * q);
-      if (a.D != nullptr) v += a.beta * dq;
-    }
-    v += a.shift;
-    rest = v - bf16_bits_to_float(__builtin_bit_cast(uint16_t, static_cast<__bf16>(v)));
-  }
-  residual_of(a.C, a.ldc)[row] = rest;
-  return v;
 }
 
 // Kernel argument: the problems of a launch and which workgroup does what.  Block ids [0, tile_begin[n]) compute one
@@ -144,9 +118,11 @@ struct LaunchArgs {
   int split_begin[N + 1];  // first split tile (the fix-up kernel's order)
   int class_begin[N + 1];  // first whole-tile block of a class: neighbouring problems with the same K
   int n;
+  int symmetric;
   int group_m;      // tile rows per block of the general products' tile order
   int round_tiles;  // resident workgroups, a multiple of 8
   int update_dtype;
+  float alpha, beta;
   float* partials;  // fp32 BM x BN tiles, problem p's from partial_base on: [its split tiles][splits]
   GemmProblem problem[N];
 };
@@ -200,9 +176,7 @@ __device__ __forceinline__ void tile_coords(int group_m, int logical, int tiles_
 }
 
 // OCC workgroups are meant to share a CU: the register budget per wave is set for OCC * WM * WN / 4 waves per SIMD.
-// DIAG: some problem of the launch has residuals of diagonals (kGemmDiagP and the like).  A kernel of its own, because the
-// factor per row in the D pick-up and the work on the diagonal cost the others 2 % (24 matrices of 1536x1024 1223 -> 1244 us).
-template <int BM, int BN, int WM, int WN, int BK, int STAGES, int OCC, int N, bool DIAG>
+template <int BM, int BN, int WM, int WN, int BK, int STAGES, int OCC, int N>
 __global__ void __launch_bounds__(WM * WN * 64, (OCC * WM * WN + 3) / 4)
 gemm_nt_kernel(LaunchArgs<N> args) {
   constexpr int kThreads = WM * WN * 64;
@@ -254,11 +228,9 @@ gemm_nt_kernel(LaunchArgs<N> args) {
     logical = args.tile_begin[problem + 1] - args.tile_begin[problem] + piece_tile;
   }
   int tm, tn;
-  tile_coords(args.group_m, logical, tiles_m, tiles_n, (a.flags & kGemmSymmetric) != 0, &tm, &tn);
+  tile_coords(args.group_m, logical, tiles_m, tiles_n, args.symmetric != 0, &tm, &tn);
   const int row0 = tm * BM;
   const int col0 = tn * BN;
-  // held in a register: loaded where it is used it would cost the epilogue a memory latency
-  const float alpha = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(a.alpha)));
   const int k_slabs_total = a.K / BK;
   const int ks_begin = whole ? 0 : static_cast<int>(static_cast<int64_t>(k_slabs_total) * split / a.splits);
   const int ks_end = whole ? k_slabs_total : static_cast<int>(static_cast<int64_t>(k_slabs_total) * (split + 1) / a.splits);
@@ -322,10 +294,7 @@ gemm_nt_kernel(LaunchArgs<N> args) {
   // cost a 256 x 256 tile with K = 4096 11 of its 121 microseconds: every CU wants its 128 KiB from HBM at the same
   // moment, and the tile has to be staged through LDS because its rows do not match the accumulator layout.)
   const bool d_in_slabs = whole && a.D != nullptr;
-  // With DIAG the factor is one per row, row_beta / alpha: BM floats in LDS behind the slab stages.
-  float* d_scales = reinterpret_cast<float*>(smem_raw + STAGES * kStageElems * sizeof(__bf16));
-  float d_scale = 0.0f;
-  if (d_in_slabs && (!DIAG || tid < BM)) d_scale = (DIAG ? row_beta(a, row0 + tid) : a.beta) / alpha;
+  const float d_scale = d_in_slabs ? args.beta / args.alpha : 0.0f;
   f32x4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
@@ -408,7 +377,6 @@ gemm_nt_kernel(LaunchArgs<N> args) {
       stream_p(k0_clamped(sidx), sidx);
       if (sidx + 1 < STAGES) stream_q(k0_clamped(sidx), sidx);  // the Q rows of the last one go out under the first MFMAs
     }
-    if (DIAG && d_in_slabs && tid < BM) d_scales[tid] = d_scale;
     constexpr int kAfterFirst = (STAGES - 2) * kLoadsPerSlab + kLoadsP;
     __builtin_amdgcn_s_waitcnt(0x0F70 | (kAfterFirst & 0xF) | ((kAfterFirst >> 4) << 14));
     __syncthreads();
@@ -492,14 +460,8 @@ gemm_nt_kernel(LaunchArgs<N> args) {
                 "D slabs must divide over the waves and the half steps");
   const int d_base = BM * BK + lcol * BK + 4 * ((lane >> 4) & 1);  // slab row lcol (+ 16 j), first or second half of a chunk
   const int d_swizzle = (lcol / kRowsPerSweep) % kChunks;          // the same for lcol + 16 j
-  constexpr int kDRows = kDBatch / TN;  // MFMA tile rows of a batch
-  static_assert(kDBatch % TN == 0, "a batch holds whole MFMA tile rows");
   u32x2 d_vals[kDBatch];
-  f32x4 d_row_scale[DIAG ? kDRows : 1];  // of the lane's four rows
-  auto d_read = [&](auto qq_tag, int stage, int batch) {
-    constexpr int kFirstTile = decltype(qq_tag)::value * kTilesPerSlab;
-#pragma unroll
-    for (int n = 0; n < (DIAG ? kDRows : 0); ++n) d_row_scale[n] = *reinterpret_cast<const f32x4*>(d_scales + lrow + (kFirstTile + batch * kDRows + n) * 16);
+  auto d_read = [&](int stage, int batch) {
 #pragma unroll
     for (int n = 0; n < kDBatch; ++n) {
       const int pair = batch * kDBatch + n, ii = pair / TN, j = pair % TN;
@@ -511,20 +473,15 @@ gemm_nt_kernel(LaunchArgs<N> args) {
       d_vals[n] = *reinterpret_cast<const u32x2*>(smem + stage * kStageElems + d_base + j * 16 * BK + (chunk << 3));
     }
   };
-  auto d_add = [&](auto qq_tag, int batch, bool owner) {
+  auto d_add = [&](auto qq_tag, int batch, float scale) {
     constexpr int kFirstTile = decltype(qq_tag)::value * kTilesPerSlab;
 #pragma unroll
-    for (int n = 0; n < (DIAG ? kDRows : 1); ++n)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) d_row_scale[n][r] = owner ? (DIAG ? d_row_scale[n][r] : d_scale) : 0.0f;  // the other waves add zero times a finite value
-#pragma unroll
     for (int n = 0; n < kDBatch; ++n) {
-      const f32x4 scale = d_row_scale[DIAG ? n / TN : 0];
       const int pair = batch * kDBatch + n, i = kFirstTile + pair / TN, j = pair % TN;
-      acc[i][j][0] += scale[0] * __uint_as_float(d_vals[n].x << 16);
-      acc[i][j][1] += scale[1] * __uint_as_float(d_vals[n].x & 0xffff0000u);
-      acc[i][j][2] += scale[2] * __uint_as_float(d_vals[n].y << 16);
-      acc[i][j][3] += scale[3] * __uint_as_float(d_vals[n].y & 0xffff0000u);
+      acc[i][j][0] += scale * __uint_as_float(d_vals[n].x << 16);
+      acc[i][j][1] += scale * __uint_as_float(d_vals[n].x & 0xffff0000u);
+      acc[i][j][2] += scale * __uint_as_float(d_vals[n].y << 16);
+      acc[i][j][3] += scale * __uint_as_float(d_vals[n].y & 0xffff0000u);
     }
   };
   int stage = 0;
@@ -536,17 +493,17 @@ gemm_nt_kernel(LaunchArgs<N> args) {
     // the half step the first D batch rides on: the slab's tile rows (its first two, in a tile whose slab rows span both
     // halves) meet their first MFMA there
     constexpr int kDHalf = kD < 0 ? -4 : (Part::value * kTilesPerSlab >= TMH ? 1 : 0);
-    const bool owner = wave_m == kOwner;
+    const float scale = (kD >= 0 && wave_m == kOwner) ? d_scale : 0.0f;  // the other waves add zero times a finite value
     auto d_before = [&](auto half_tag) {
       constexpr int kBatch = decltype(half_tag)::value - kDHalf;
       if constexpr (kBatch == 0 || kBatch == 1) {
-        d_read(Part{}, stage, kBatch);
+        d_read(stage, kBatch);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
     auto d_after = [&](auto half_tag) {
       constexpr int kBatch = decltype(half_tag)::value - kDHalf;
-      if constexpr (kBatch == 0 || kBatch == 1) d_add(Part{}, kBatch, owner);
+      if constexpr (kBatch == 0 || kBatch == 1) d_add(Part{}, kBatch, scale);
     };
     const int next_stage = stage + 1 == STAGES ? 0 : stage + 1;
     const int prev_stage = stage == 0 ? STAGES - 1 : stage - 1;
@@ -630,7 +587,7 @@ gemm_nt_kernel(LaunchArgs<N> args) {
   uint16_t* __restrict__ C = static_cast<uint16_t*>(a.C);
   uint16_t* __restrict__ CT = static_cast<uint16_t*>(a.CT);
   int ldct = a.ldct;
-  if (a.flags & kGemmSymmetric) {  // mirror the off-diagonal tile
+  if (args.symmetric) {  // mirror the off-diagonal tile
     CT = tm != tn ? C : nullptr;
     ldct = a.ldc;
   }
@@ -644,22 +601,8 @@ gemm_nt_kernel(LaunchArgs<N> args) {
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) acc[i][j][r] = alpha * acc[i][j][r];
-  if (DIAG && (a.flags & kGemmDiagC) && tm == tn) {
-    const int on = (lane & 15) - (lane >> 4) * 4;  // which of the lane's four rows meets its column
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        if (wave_m * kWaveM + i * 16 != wave_n * kWaveN + j * 16) continue;
-        if (on < 0 || on > 3) continue;
-        const float v = on == 0 ? acc[i][j][0] : on == 1 ? acc[i][j][1] : on == 2 ? acc[i][j][2] : acc[i][j][3];
-        const float fixed = finish_diagonal(a, row0 + wave_m * kWaveM + i * 16 + (lane & 15), v);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[i][j][r] = r == on ? fixed : acc[i][j][r];
-      }
-  }
-  if (a.flags & kGemmUpdate) {
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = args.alpha * acc[i][j][r];
+  if (a.update_param != nullptr) {
     // the last product of a Muon step: the tile goes into the parameter (in the parameter's orientation) and nowhere else
     if (!(a.flags & kGemmUpdateTransposed)) {
 #pragma unroll
@@ -729,7 +672,7 @@ gemm_nt_kernel(LaunchArgs<N> args) {
 // 1024 threads finishes a 64 x 64 block of a tile, thread t four consecutive columns of row t / 16; the transposed /
 // mirrored copy goes through LDS so that both orientations leave in whole 16-byte, row-contiguous stores.
 constexpr int kFixupThreads = 1024;
-template <int BM, int BN, int N, bool DIAG>
+template <int BM, int BN, int N>
 __global__ void __launch_bounds__(kFixupThreads)
 splitk_fixup_kernel(LaunchArgs<N> args) {
   constexpr int kSub = 64;
@@ -743,12 +686,12 @@ splitk_fixup_kernel(LaunchArgs<N> args) {
   const int full_tiles = args.tile_begin[problem + 1] - args.tile_begin[problem];
   const int sub_row0 = (sub / (BN / kSub)) * kSub, sub_col0 = (sub % (BN / kSub)) * kSub;
   int tm, tn;
-  tile_coords(args.group_m, full_tiles + tile, (a.M + BM - 1) / BM, (a.N + BN - 1) / BN, (a.flags & kGemmSymmetric) != 0, &tm, &tn);
+  tile_coords(args.group_m, full_tiles + tile, (a.M + BM - 1) / BM, (a.N + BN - 1) / BN, args.symmetric != 0, &tm, &tn);
   const uint16_t* __restrict__ D = static_cast<const uint16_t*>(a.D);
   uint16_t* __restrict__ C = static_cast<uint16_t*>(a.C);
   uint16_t* __restrict__ CT = static_cast<uint16_t*>(a.CT);
   int ldct = a.ldct;
-  if (a.flags & kGemmSymmetric) {  // mirror the off-diagonal tile
+  if (args.symmetric) {  // mirror the off-diagonal tile
     CT = tm != tn ? C : nullptr;
     ldct = a.ldc;
   }
@@ -768,23 +711,17 @@ splitk_fixup_kernel(LaunchArgs<N> args) {
   }
   for (; s < a.splits; ++s) sum += *reinterpret_cast<const f32x4*>(base + static_cast<int64_t>(s) * (BM * BN));
   const int row = tm * BM + lrow, col = tn * BN + lcol;
-  float v[4] = {a.alpha * sum.x, a.alpha * sum.y, a.alpha * sum.z, a.alpha * sum.w};
+  float v[4] = {args.alpha * sum.x, args.alpha * sum.y, args.alpha * sum.z, args.alpha * sum.w};
   if (D != nullptr) {
     const u32x2 d = *reinterpret_cast<const u32x2*>(D + static_cast<int64_t>(row) * a.ldd + col);
-    const float beta = DIAG ? row_beta(a, row) : a.beta;
-    v[0] += beta * bf16_bits_to_float(static_cast<uint16_t>(d.x));
-    v[1] += beta * bf16_bits_to_float(static_cast<uint16_t>(d.x >> 16));
-    v[2] += beta * bf16_bits_to_float(static_cast<uint16_t>(d.y));
-    v[3] += beta * bf16_bits_to_float(static_cast<uint16_t>(d.y >> 16));
-  }
-  if (DIAG && (a.flags & kGemmDiagC) && row >= col && row < col + 4) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (row == col + e) v[e] = finish_diagonal(a, row, v[e]);
+    v[0] += args.beta * bf16_bits_to_float(static_cast<uint16_t>(d.x));
+    v[1] += args.beta * bf16_bits_to_float(static_cast<uint16_t>(d.x >> 16));
+    v[2] += args.beta * bf16_bits_to_float(static_cast<uint16_t>(d.y));
+    v[3] += args.beta * bf16_bits_to_float(static_cast<uint16_t>(d.y >> 16));
   }
   const uint32_t lo = pack_bf16x2(v[0], v[1]);
   const uint32_t hi = pack_bf16x2(v[2], v[3]);
-  if (a.flags & kGemmUpdate) {  // uniform over the grid: the parameter update in place of the stores (see gemm_nt_kernel)
+  if (a.update_param != nullptr) {  // uniform over the grid: the parameter update in place of the stores (see gemm_nt_kernel)
     if (!(a.flags & kGemmUpdateTransposed)) {
       const u32x4 packed = {lo, hi, 0u, 0u};  // this thread's four columns
       update_param8(a, args.update_dtype, row, col, packed, 4);
@@ -829,8 +766,10 @@ splitk_fixup_kernel(LaunchArgs<N> args) {
 template <int N>
 struct SmallArgs {
   int begin[N];  // first workgroup of a problem; entries past the last problem are the end
+  int symmetric;
   int group_m;
   int update_dtype;
+  float alpha, beta;
   GemmProblem problem[N];
 };
 static_assert(sizeof(SmallArgs<kMaxGemmGroup>) <= 4096, "kernel arguments are limited to 4 KiB");
@@ -840,7 +779,7 @@ constexpr int kSmallWaves = 8;
 constexpr int kSmallThreads = kSmallWaves * 64;
 constexpr int kSmallPitch = kSmallTile + 4;  // floats per row of a partial tile in LDS: skews the banks of a lane's four rows
 
-template <int N, bool DIAG>
+template <int N>
 __global__ void __launch_bounds__(kSmallThreads, 2)
 gemm_small_kernel(SmallArgs<N> args) {
   constexpr int kTiles = kSmallTile / 16;
@@ -851,7 +790,7 @@ gemm_small_kernel(SmallArgs<N> args) {
   const GemmProblem a = args.problem[problem];  // a copy: all of its fields in one go instead of a scalar load at each use
   int tm, tn;
   tile_coords(args.group_m, blockIdx.x - args.begin[problem], (a.M + kSmallTile - 1) / kSmallTile, (a.N + kSmallTile - 1) / kSmallTile,
-              (a.flags & kGemmSymmetric) != 0, &tm, &tn);
+              args.symmetric != 0, &tm, &tn);
   const int row0 = tm * kSmallTile, col0 = tn * kSmallTile;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -935,19 +874,13 @@ gemm_small_kernel(SmallArgs<N> args) {
     lo += from[0];
     hi += from[1];
   }
-  const float beta = DIAG && a.D != nullptr ? row_beta(a, row0 + orow) : a.beta;
-  const bool diagonal = DIAG && (a.flags & kGemmDiagC) != 0 && tm == tn;
   u32x4 packed;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    float v0 = a.alpha * (e < 2 ? lo[2 * e] : hi[2 * e - 4]), v1 = a.alpha * (e < 2 ? lo[2 * e + 1] : hi[2 * e - 3]);
+    float v0 = args.alpha * (e < 2 ? lo[2 * e] : hi[2 * e - 4]), v1 = args.alpha * (e < 2 ? lo[2 * e + 1] : hi[2 * e - 3]);
     if (a.D != nullptr) {
-      v0 += beta * __uint_as_float(d[e] << 16);
-      v1 += beta * __uint_as_float(d[e] & 0xffff0000u);
-    }
-    if (diagonal) {
-      if (orow == ocol + 2 * e) v0 = finish_diagonal(a, row0 + orow, v0);
-      if (orow == ocol + 2 * e + 1) v1 = finish_diagonal(a, row0 + orow, v1);
+      v0 += args.beta * __uint_as_float(d[e] << 16);
+      v1 += args.beta * __uint_as_float(d[e] & 0xffff0000u);
     }
     packed[e] = pack_bf16x2(v0, v1);
   }
@@ -956,11 +889,11 @@ gemm_small_kernel(SmallArgs<N> args) {
   uint16_t* __restrict__ C = static_cast<uint16_t*>(a.C);
   uint16_t* __restrict__ CT = static_cast<uint16_t*>(a.CT);
   int ldct = a.ldct;
-  if (a.flags & kGemmSymmetric) {
+  if (args.symmetric) {
     CT = tm != tn ? C : nullptr;
     ldct = a.ldc;
   }
-  const bool update = (a.flags & kGemmUpdate) != 0, update_transposed = update && (a.flags & kGemmUpdateTransposed) != 0;
+  const bool update = a.update_param != nullptr, update_transposed = update && (a.flags & kGemmUpdateTransposed) != 0;
   if (update && !update_transposed) {
     update_param8(a, args.update_dtype, row0 + orow, col0 + ocol, packed);
     return;
@@ -992,9 +925,9 @@ GemmTuning tuning_snapshot() {
 }
 
 // Tiles a product computes: every tile of a general product, the tiles on or below the diagonal of a symmetric one.
-int tile_count(const GemmProblem& p, int tile) {
+int tile_count(const GemmGroup& g, const GemmProblem& p, int tile) {
   const int tm = (p.M + tile - 1) / tile, tn = (p.N + tile - 1) / tile;
-  return p.flags & kGemmSymmetric ? tm * (tm + 1) / 2 : tm * tn;
+  return g.symmetric ? tm * (tm + 1) / 2 : tm * tn;
 }
 
 // Below this many slabs a tile is never cut: the pieces would be gone before the fix-up launch (4 us and more) has paid off.
@@ -1058,7 +991,7 @@ GemmPlan make_plan(const GemmGroup& g, int variant, const GemmScratch& scratch, 
   std::stable_sort(plan.order, plan.order + g.n, [&](int a, int b) { return g.problem[a].K > g.problem[b].K; });
   int tiles[kMaxGemmGroup], slabs[kMaxGemmGroup], total = 0;
   for (int i = 0; i < g.n; ++i) {
-    tiles[i] = tile_count(g.problem[plan.order[i]], v.tile);
+    tiles[i] = tile_count(g, g.problem[plan.order[i]], v.tile);
     slabs[i] = g.problem[plan.order[i]].K / kSlabK;
     total += tiles[i];
     plan.split_tiles[i] = 0;
@@ -1111,13 +1044,16 @@ GemmPlan make_plan(const GemmGroup& g, int variant, const GemmScratch& scratch, 
   return plan;
 }
 
-template <int BM, int BN, int WM, int WN, int BK, int STAGES, int OCC, int N, bool DIAG>
+template <int BM, int BN, int WM, int WN, int BK, int STAGES, int OCC, int N>
 int launch(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& scratch, const GemmTuning& tuning, hipStream_t stream) {
   LaunchArgs<N> args;
   args.n = g.n;
+  args.symmetric = g.symmetric;
   args.group_m = std::max(1, tuning.group_m);
   args.round_tiles = std::max(kXcds, device_cu_count() * OCC / kXcds * kXcds);
   args.update_dtype = g.update_dtype;
+  args.alpha = g.alpha;
+  args.beta = g.beta;
   args.partials = static_cast<float*>(scratch.partials);
   int tile = 0, piece = 0, split = 0, partial = 0, classes = 0;
   for (int i = 0; i <= N; ++i) {
@@ -1129,18 +1065,18 @@ int launch(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& scratch,
     if (i == 0 || p.K != args.problem[i - 1].K) args.class_begin[classes++] = tile;
     p.splits = plan.splits[i];
     p.partial_base = partial;
-    tile += tile_count(p, BM) - plan.split_tiles[i];
+    tile += tile_count(g, p, BM) - plan.split_tiles[i];
     split += plan.split_tiles[i];
     piece += plan.split_tiles[i] * plan.splits[i];
     partial += plan.split_tiles[i] * plan.splits[i];
   }
   for (int i = 0; i <= N; ++i) args.piece_begin[i] += tile;  // block ids: behind the whole tiles
   for (int i = classes; i <= N; ++i) args.class_begin[i] = tile;
-  constexpr size_t smem_loop = static_cast<size_t>(STAGES) * (BM + BN) * BK * sizeof(uint16_t) + (DIAG ? BM * sizeof(float) : 0);
+  constexpr size_t smem_loop = static_cast<size_t>(STAGES) * (BM + BN) * BK * sizeof(uint16_t);
   constexpr size_t smem_c = static_cast<size_t>(BM) * (BN + 8) * sizeof(uint16_t), smem_ct = static_cast<size_t>(BN) * (BM + 8) * sizeof(uint16_t);
   constexpr size_t smem_epilogue = smem_c > smem_ct ? smem_c : smem_ct;
   constexpr size_t smem = smem_loop > smem_epilogue ? smem_loop : smem_epilogue;
-  auto kernel = gemm_nt_kernel<BM, BN, WM, WN, BK, STAGES, OCC, N, DIAG>;
+  auto kernel = gemm_nt_kernel<BM, BN, WM, WN, BK, STAGES, OCC, N>;
   {
     // raising the dynamic LDS limit is needed once per kernel and device
     static std::mutex mu;
@@ -1157,43 +1093,30 @@ int launch(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& scratch,
   hipLaunchKernelGGL(kernel, dim3(tile + piece), dim3(WM * WN * 64), smem, stream, args);
   MFSDP_CHECK_LAUNCH("gemm_nt_kernel");
   if (split > 0) {
-    hipLaunchKernelGGL((splitk_fixup_kernel<BM, BN, N, DIAG>), dim3(split * (BM / 64) * (BN / 64)), dim3(kFixupThreads), 0, stream, args);
+    hipLaunchKernelGGL((splitk_fixup_kernel<BM, BN, N>), dim3(split * (BM / 64) * (BN / 64)), dim3(kFixupThreads), 0, stream, args);
     MFSDP_CHECK_LAUNCH("splitk_fixup_kernel");
   }
   return MFSDP_OK;
 }
 
-template <int N, bool DIAG>
+template <int N>
 int launch_small(const GemmGroup& g, const GemmPlan& plan, const GemmTuning& tuning, hipStream_t stream) {
   SmallArgs<N> args;
+  args.symmetric = g.symmetric;
   args.group_m = std::max(1, tuning.group_m);
   args.update_dtype = g.update_dtype;
+  args.alpha = g.alpha;
+  args.beta = g.beta;
   int tile = 0;
   for (int i = 0; i < g.n; ++i) {
     args.problem[i] = g.problem[plan.order[i]];
     args.begin[i] = tile;
-    tile += tile_count(args.problem[i], kSmallTile);
+    tile += tile_count(g, args.problem[i], kSmallTile);
   }
   for (int i = g.n; i < N; ++i) args.begin[i] = tile;
-  hipLaunchKernelGGL((gemm_small_kernel<N, DIAG>), dim3(tile), dim3(kSmallThreads), 0, stream, args);
+  hipLaunchKernelGGL(gemm_small_kernel<N>, dim3(tile), dim3(kSmallThreads), 0, stream, args);
   MFSDP_CHECK_LAUNCH("gemm_small_kernel");
   return MFSDP_OK;
-}
-
-template <bool DIAG>
-int launch_plan(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& scratch, const GemmTuning& tuning, hipStream_t stream) {
-  if (plan.variant == kSmallVariant)
-    return g.n <= 2   ? launch_small<2, DIAG>(g, plan, tuning, stream)
-           : g.n <= 8 ? launch_small<8, DIAG>(g, plan, tuning, stream)
-                      : launch_small<kMaxGemmGroup, DIAG>(g, plan, tuning, stream);
-  if (plan.variant == 2)  // 128x128 tile, 4 waves of 64x64, two workgroups per CU
-    return g.n == 1  ? launch<128, 128, 2, 2, 64, 2, 2, 1, DIAG>(g, plan, scratch, tuning, stream)
-           : g.n <= 8 ? launch<128, 128, 2, 2, 64, 2, 2, 8, DIAG>(g, plan, scratch, tuning, stream)
-                      : launch<128, 128, 2, 2, 64, 2, 2, kMaxGemmGroup, DIAG>(g, plan, scratch, tuning, stream);
-  // 256x256 tile, 8 waves of 128x64, one workgroup per CU
-  return g.n == 1  ? launch<256, 256, 2, 4, 64, 2, 1, 1, DIAG>(g, plan, scratch, tuning, stream)
-         : g.n <= 8 ? launch<256, 256, 2, 4, 64, 2, 1, 8, DIAG>(g, plan, scratch, tuning, stream)
-                    : launch<256, 256, 2, 4, 64, 2, 1, kMaxGemmGroup, DIAG>(g, plan, scratch, tuning, stream);
 }
 
 }  // namespace
@@ -1206,9 +1129,7 @@ GemmTuning get_gemm_tuning() { return tuning_snapshot(); }
 
 GemmPlan gemm_plan(const GemmGroup& g, const GemmScratch& scratch) {
   const GemmTuning tuning = tuning_snapshot();
-  bool symmetric = true;  // every problem of the launch
-  for (int i = 0; i < g.n; ++i) symmetric = symmetric && (g.problem[i].flags & kGemmSymmetric) != 0;
-  const int variant = symmetric ? tuning.symmetric_variant : tuning.general_variant;
+  const int variant = g.symmetric ? tuning.symmetric_variant : tuning.general_variant;
   bool q_columns = false;
   for (int i = 0; i < g.n; ++i) q_columns = q_columns || (g.problem[i].flags & kGemmQColumns) != 0;
   if (q_columns) return make_plan(g, 1, scratch, tuning);
@@ -1216,14 +1137,14 @@ GemmPlan gemm_plan(const GemmGroup& g, const GemmScratch& scratch) {
   const GemmPlan big = make_plan(g, 1, scratch, tuning);
   // On a machine shared with other matrices' kernels the CUs a part-filling triangle of big tiles leaves idle are
   // not lost, and a big tile moves fewer LDS bytes per flop.
-  if (symmetric && g.shared && 4 * tile_count(g.problem[0], 256) >= device_cu_count()) return big;
+  if (g.symmetric && g.shared && 4 * tile_count(g, g.problem[0], 256) >= device_cu_count()) return big;
   const GemmPlan small = make_plan(g, 2, scratch, tuning);
   const GemmPlan& better = big.us <= small.us ? big : small;
   // 64 x 64 tiles for one round at most: a second round costs as much as the first (1024 x 1536 update: 384 of them 279 us a
   // step against 241 with 128 x 128 tiles; eight matrices of 512 x 1536: 495 against 281).  Within a round the model decides;
   // K beyond about 2000 goes to 128 x 128 tiles cut along K (gram of 768 x 2304).
   int tiles = 0;
-  for (int i = 0; i < g.n; ++i) tiles += tile_count(g.problem[i], kSmallTile);
+  for (int i = 0; i < g.n; ++i) tiles += tile_count(g, g.problem[i], kSmallTile);
   if (tiles > device_cu_count()) return better;
   const GemmPlan smallest = make_plan(g, kSmallVariant, scratch, tuning);
   return smallest.us < better.us ? smallest : better;
@@ -1237,7 +1158,7 @@ int64_t gemm_nt_executed_flops(const GemmGroup& g) {
   scratch.partials = &scratch;  // only its presence counts
   const int tile = kVariants[gemm_plan(g, scratch).variant].tile;
   int64_t flops = 0;
-  for (int i = 0; i < g.n; ++i) flops += 2 * static_cast<int64_t>(tile) * tile * g.problem[i].K * tile_count(g.problem[i], tile);
+  for (int i = 0; i < g.n; ++i) flops += 2 * static_cast<int64_t>(tile) * tile * g.problem[i].K * tile_count(g, g.problem[i], tile);
   return flops;
 }
 
@@ -1247,37 +1168,42 @@ int gemm_nt_bf16(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& sc
     const GemmProblem& a = g.problem[i];
     if (a.M <= 0 || a.N <= 0 || a.K <= 0 || a.K % kSlabK)
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: M=%d, N=%d must be positive and K=%d a multiple of %d", a.M, a.N, a.K, kSlabK);
-    const bool symmetric = (a.flags & kGemmSymmetric) != 0, update = (a.flags & kGemmUpdate) != 0;
-    if (symmetric && a.M != a.N) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: symmetric product needs M == N");
-    if ((a.flags & kGemmSkipC) && !update && (symmetric || !a.CT)) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: skipping C needs a transposed output and a general product");
+    if (g.symmetric && a.M != a.N) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: symmetric product needs M == N");
+    if ((a.flags & kGemmSkipC) && (g.symmetric || !a.CT)) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: skipping C needs a transposed output and a general product");
     if (!a.P || !a.Q || !a.C) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: null operand");
     // tiles reach beyond M and N: rows up to the next multiple of 256 must exist (the caller's word), columns are checked
     const int mp = (a.M + 255) / 256 * 256, np = (a.N + 255) / 256 * 256;
     const bool q_columns = (a.flags & kGemmQColumns) != 0;
-    if (q_columns && (symmetric || plan.variant != 1 || a.K < a.M || static_cast<int64_t>(mp) * a.ldq >= 1 << 30))
+    if (q_columns && (g.symmetric || plan.variant != 1 || a.K < a.M || static_cast<int64_t>(mp) * a.ldq >= 1 << 30))
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: a Q of K rows needs a general product over M on 256 x 256 tiles and less than 2 GiB");
-    if (a.ldp < a.K || a.ldq < (q_columns ? np : a.K) || (!update && a.ldc < np) || (a.D && a.ldd < np) || (a.CT && a.ldct < mp))
+    if (a.ldp < a.K || a.ldq < (q_columns ? np : a.K) || a.ldc < np || (a.D && a.ldd < np) || (a.CT && a.ldct < mp))
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: leading dimension smaller than the padded row length");
     if ((a.ldp | a.ldq) % 8 || (reinterpret_cast<uintptr_t>(a.P) | reinterpret_cast<uintptr_t>(a.Q)) % 16)
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: operands must be 16-byte aligned with leading dimensions multiple of 8");
-    if ((!update && ((a.ldc % 8) || reinterpret_cast<uintptr_t>(a.C) % 16)) || (a.D && ((a.ldd % 8) || reinterpret_cast<uintptr_t>(a.D) % 16)) ||
+    if ((a.ldc % 8) || reinterpret_cast<uintptr_t>(a.C) % 16 || (a.D && ((a.ldd % 8) || reinterpret_cast<uintptr_t>(a.D) % 16)) ||
         (a.CT && ((a.ldct % 8) || reinterpret_cast<uintptr_t>(a.CT) % 16)))
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: C, D and the transposed output must be 16-byte aligned with leading dimensions multiple of 8");
-    if (a.D && (a.K < a.M || a.alpha == 0.0f)) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: a D operand needs K >= M and alpha != 0");
+    if (a.D && (a.K < a.M || g.alpha == 0.0f)) return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: a D operand needs K >= M and alpha != 0");
     if (a.ldp > kMaxGemmLeading || a.ldq > kMaxGemmLeading) return fail(MFSDP_ERR_UNSUPPORTED, "gemm_nt_bf16: leading dimensions beyond 2^22 elements");
-    if (update && (symmetric || (g.update_dtype != MFSDP_F32 && g.update_dtype != MFSDP_BF16) ||
-                   reinterpret_cast<uintptr_t>(a.C) % (g.update_dtype == MFSDP_F32 ? 4 : 2)))
+    if (a.update_param != nullptr && (g.symmetric || (g.update_dtype != MFSDP_F32 && g.update_dtype != MFSDP_BF16) ||
+                                      reinterpret_cast<uintptr_t>(a.update_param) % (g.update_dtype == MFSDP_F32 ? 4 : 2)))
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: parameter update needs a general product and an aligned f32 / bf16 parameter");
-    // residuals lie behind square operands; a general product takes those of P through its D operand only
-    if (((a.flags & (kGemmDiagQ | kGemmDiagC)) && !symmetric) || ((a.flags & kGemmDiagP) && !symmetric && !a.D))
-      return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: diagonal residuals need a symmetric product, or those of P a D operand");
   }
   const GemmTuning tuning = tuning_snapshot();
   // Slabs of 32 (three to five deep) were measured too: each slab row is then half a 128-byte line, the vector
   // cache looks every line up twice, and the products run 15-25 % slower than with slabs of 64 two deep.
-  bool diag = false;
-  for (int i = 0; i < g.n; ++i) diag = diag || (g.problem[i].flags & (kGemmDiagP | kGemmDiagC)) != 0;
-  return diag ? launch_plan<true>(g, plan, scratch, tuning, stream) : launch_plan<false>(g, plan, scratch, tuning, stream);
+  if (plan.variant == kSmallVariant)
+    return g.n <= 2   ? launch_small<2>(g, plan, tuning, stream)
+           : g.n <= 8 ? launch_small<8>(g, plan, tuning, stream)
+                      : launch_small<kMaxGemmGroup>(g, plan, tuning, stream);
+  if (plan.variant == 2)  // 128x128 tile, 4 waves of 64x64, two workgroups per CU
+    return g.n == 1  ? launch<128, 128, 2, 2, 64, 2, 2, 1>(g, plan, scratch, tuning, stream)
+           : g.n <= 8 ? launch<128, 128, 2, 2, 64, 2, 2, 8>(g, plan, scratch, tuning, stream)
+                      : launch<128, 128, 2, 2, 64, 2, 2, kMaxGemmGroup>(g, plan, scratch, tuning, stream);
+  // 256x256 tile, 8 waves of 128x64, one workgroup per CU
+  return g.n == 1  ? launch<256, 256, 2, 4, 64, 2, 1, 1>(g, plan, scratch, tuning, stream)
+         : g.n <= 8 ? launch<256, 256, 2, 4, 64, 2, 1, 8>(g, plan, scratch, tuning, stream)
+                    : launch<256, 256, 2, 4, 64, 2, 1, kMaxGemmGroup>(g, plan, scratch, tuning, stream);
 }
 
 }  // namespace mfsdp
