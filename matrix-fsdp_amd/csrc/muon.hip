@@ -137,11 +137,12 @@ void update_size(const Matrix& w, GemmProblem* p) {
 //   straight into registers, K-contiguous);
 // * where the tiles fill more than a round, so that their stores compete (200 tiles 745 -> 756, 288 1172 -> 1175, 324 1908 -> 1853);
 // * where X and X' are about what the memory-side cache of 256 MB holds (X of 157 MB: gains 2 %; the three matrices of a hidden4096
-//   step, 224 MB, lose 2 %).  This bounds X far below the 2 GiB that kGemmQColumns takes, too.
+//   step, 224 MB, lose 2 %);
+// * where kGemmQColumns takes X padded to whole tiles, which a few rows of 4 Mi elements exceed (kMaxQColumnsElements).
 constexpr int64_t kOneOrientationBytes = 192ll << 20;
 bool stores_transposes(const Group& group) {
   GemmGroup g;
-  int64_t bytes = 0, tiles = 0;
+  int64_t bytes = 0, tiles = 0, padded = 0;
   g.n = group.n;
   for (int i = 0; i < g.n; ++i) {
     const Matrix& w = group.w[i];
@@ -149,8 +150,9 @@ bool stores_transposes(const Group& group) {
     update_size(w, &g.problem[i]);
     bytes += static_cast<int64_t>(w.m) * w.n * 2;
     tiles += static_cast<int64_t>((w.m + 255) / 256) * ((w.n + 255) / 256);
+    padded = std::max(padded, static_cast<int64_t>(w.mp) * w.np);
   }
-  return bytes > kOneOrientationBytes || 4 * tiles < 5 * device_cu_count() || !on_256_tiles(gemm_plan(g, group.scratch));
+  return bytes > kOneOrientationBytes || padded > kMaxQColumnsElements || 4 * tiles < 5 * device_cu_count() || !on_256_tiles(gemm_plan(g, group.scratch));
 }
 
 void choose_transposes(Group* group, int steps) {

@@ -20,8 +20,8 @@ namespace mfsdp {
 //     param <- round(param * update_decay) + update_neg_lr * o        (torch/optim/_muon.py:313-315)
 // on the contiguous row-major parameter (M x N, or N x M with kGemmUpdateTransposed).  General products only.
 //
-// kGemmQColumns: Q is given as K x N row-major (ldq), rows beyond M taken as zero, K spanning M, less than 2 GiB of it; general
-// products on 256 tiles (gemm_plan takes no others for them).  D is then the same matrix.
+// kGemmQColumns: Q is given as K x N row-major (ldq), rows beyond M taken as zero, K spanning M, at most kMaxQColumnsElements of
+// it; general products on 256 tiles (gemm_plan takes no others for them).  D is then the same matrix.
 enum GemmFlags {
   kGemmSkipC = 1,
   kGemmUpdateTransposed = 2,
@@ -43,6 +43,7 @@ struct GemmProblem {
 };
 
 constexpr int kMaxGemmLeading = 1 << 22;  // largest leading dimension of P and Q: a tile's rows are reached by 31-bit byte offsets
+constexpr int64_t kMaxQColumnsElements = (1 << 30) - 1;  // M rounded up to whole tiles times ldq: 31-bit byte offsets again
 constexpr int kMaxGemmGroup = 32;  // problems one launch carries by value in its kernel arguments
 
 // Products of one launch.  symmetric: every P*Q^T is known to be symmetric (M == N); only tiles on or below the diagonal

@@ -1174,7 +1174,7 @@ int gemm_nt_bf16(const GemmGroup& g, const GemmPlan& plan, const GemmScratch& sc
     // tiles reach beyond M and N: rows up to the next multiple of 256 must exist (the caller's word), columns are checked
     const int mp = (a.M + 255) / 256 * 256, np = (a.N + 255) / 256 * 256;
     const bool q_columns = (a.flags & kGemmQColumns) != 0;
-    if (q_columns && (g.symmetric || plan.variant != 1 || a.K < a.M || static_cast<int64_t>(mp) * a.ldq >= 1 << 30))
+    if (q_columns && (g.symmetric || plan.variant != 1 || a.K < a.M || static_cast<int64_t>(mp) * a.ldq > kMaxQColumnsElements))
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: a Q of K rows needs a general product over M on 256 x 256 tiles and less than 2 GiB");
     if (a.ldp < a.K || a.ldq < (q_columns ? np : a.K) || a.ldc < np || (a.D && a.ldd < np) || (a.CT && a.ldct < mp))
       return fail(MFSDP_ERR_INVALID, "gemm_nt_bf16: leading dimension smaller than the padded row length");

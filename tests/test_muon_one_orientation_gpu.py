@@ -37,3 +37,23 @@ def test_groups_without_stored_transposes(variant, split, dtype, tuned):
             assert torch.equal(p, alone), p.shape
         else:
             assert float((p - alone).float().norm() / alone.float().norm()) < 1e-2, p.shape
+
+
+@pytest.mark.parametrize("shape", [(1, 1 << 22), ((1 << 22) - 3, 24)])
+def test_longest_matrices_keep_their_transpose(shape, tuned):
+    """On 256 tiles: X padded to whole tiles is 2 GiB, more than a product takes by columns.  The roundings are torch's and the
+    sums in another order, see above."""
+    tuned(1, 1, 0, 1, 16)
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    grad = torch.randn(shape, generator=gen, device=DEV).bfloat16()
+    param = torch.zeros_like(grad)
+    F.muon_step(param, grad, torch.zeros_like(grad), lr=1.0, weight_decay=0.0, momentum=0.0, nesterov=False)
+    a, b, c = F.NS_COEFFICIENTS
+    x = grad.T if shape[0] > shape[1] else grad
+    x = (x / x.float().norm().bfloat16()).contiguous()
+    for _ in range(5):
+        gram = x @ x.T
+        x = torch.addmm(x, torch.addmm(gram, gram, gram, beta=b, alpha=c), x, beta=a)
+    want = (x.T if shape[0] > shape[1] else x).float()
+    have = param.float() / -F.adjust_lr(1.0, None, shape)
+    assert float((have - want).norm() / want.norm()) < 1e-2
