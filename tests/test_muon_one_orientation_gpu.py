@@ -7,7 +7,10 @@ from matrix_fsdp_amd.optim import functional as F
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-SHAPES = [(1090, 1500), (1500, 1090), (1037, 1283), (1283, 1037), (1025, 1409), (1111, 1111)] * 2  # 30 tiles of 256 or so each
+SHAPES = [(1090, 1500), (1500, 1090), (1037, 1283), (1283, 1037), (1025, 1409), (1111, 1111)] * 4  # 30 tiles of 256 or so each
+# one slab of K, rows shorter than a tile, remainders of tiles and of slabs; rows of X further apart than they are long
+SMALL = [(1, 7), (65, 63), (300, 257), (64, 1153), (1153, 128), (1100, 2040)]
+KW = dict(lr=1.0, weight_decay=0.0, momentum=0.0, nesterov=False)
 
 
 @pytest.fixture
@@ -16,27 +19,56 @@ def tuned():
     _lib.lib().mfsdp_set_muon_tuning(3, 3, 0, 1, 16)
 
 
+def transposes(shapes):
+    """Bytes of all the matrices in the workspace, and of those the two X^T of each."""
+    lib, total, xt = _lib.lib(), 0, 0
+    shared = lib.mfsdp_muon_workspace_bytes(1, 1) - 6 * 256 * 256 * 2
+    for r, c in shapes:
+        bytes_ = lib.mfsdp_muon_workspace_bytes(r, c) - shared
+        side = -(-min(r, c) // 256) * 256
+        total += bytes_
+        xt += (bytes_ - 2 * side * side * 2) // 2  # what A and B leave is X and X^T, two of each
+    return total, xt
+
+
+def step_together(shapes, dtype):
+    """Ragged, wide, tall and square matrices of one group in a workspace of NaN: gradients, parameters, how many bytes of the
+    matrices nothing was stored to."""
+    gen = torch.Generator(device=DEV).manual_seed(1)
+    grads = [torch.randn(s, generator=gen, device=DEV).bfloat16().to(dtype) for s in shapes]
+    params = [torch.zeros(s, device=DEV, dtype=dtype) for s in shapes]
+    total, _ = transposes(shapes)
+    workspace = F.MuonWorkspace(torch.device(DEV))
+    storage = workspace.get_bytes(_lib.lib().mfsdp_muon_workspace_bytes(1, 1) + total)
+    storage.fill_(0xFF)
+    F.muon_step_many([(p, g, torch.zeros_like(p), KW) for p, g in zip(params, grads)], workspace=workspace)
+    return grads, params, 2 * int((storage[:total].view(torch.int16) == -1).sum())  # this NaN comes of no finite input
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("variant,split", [(1, 2), (1, 1), (3, 1)])
 def test_groups_without_stored_transposes(variant, split, dtype, tuned):
-    """Ragged, wide, tall and square matrices in a workspace full of NaN.  Alone each fills less than a round and keeps its
-    transpose.  On 256 tiles with whole K walks both ways sum in the same order: the same bits.  With walks cut, or the
-    library's own choice of tiles, the sums are in another order: 0.003 to 0.005 apart after five iterations in bf16."""
+    """Alone each matrix fills less than a round and keeps its transpose.  On 256 tiles with whole K walks both ways sum in the
+    same order: the same bits.  With walks cut, or the library's own choice of tiles, the sums are in another order: 0.003 to
+    0.005 apart after five iterations in bf16, up to 0.01 of the few elements of the small ones."""
     tuned(variant, variant, 0, split, 16)
-    gen = torch.Generator(device=DEV).manual_seed(1)
-    grads = [torch.randn(s, generator=gen, device=DEV).bfloat16().to(dtype) for s in SHAPES]
-    kw = dict(lr=1.0, weight_decay=0.0, momentum=0.0, nesterov=False)
-    together = [torch.zeros(s, device=DEV, dtype=dtype) for s in SHAPES]
-    workspace = F.MuonWorkspace(torch.device(DEV))
-    workspace.get_bytes(1 << 30).fill_(0xFF)
-    F.muon_step_many([(p, g, torch.zeros_like(p), kw) for p, g in zip(together, grads)], workspace=workspace)
+    shapes = SHAPES + SMALL
+    grads, together, untouched = step_together(shapes, dtype)
+    assert untouched >= transposes(shapes)[1], "X^T was stored"
     for p, g in zip(together, grads):
         alone = torch.zeros_like(p)
-        F.muon_step(alone, g, torch.zeros_like(p), **kw)
+        F.muon_step(alone, g, torch.zeros_like(p), **KW)
         if (variant, split) == (1, 2):
             assert torch.equal(p, alone), p.shape
         else:
             assert float((p - alone).float().norm() / alone.float().norm()) < 1e-2, p.shape
+
+
+def test_smaller_tiles_store_transposes(tuned):
+    """What the test above takes for stored transposes is there when they are."""
+    tuned(2, 2, 0, 1, 16)
+    shapes = SHAPES + SMALL
+    assert step_together(shapes, torch.float32)[2] < transposes(shapes)[1]
 
 
 @pytest.mark.parametrize("shape", [(1, 1 << 22), ((1 << 22) - 3, 24)])
@@ -47,7 +79,7 @@ def test_longest_matrices_keep_their_transpose(shape, tuned):
     gen = torch.Generator(device=DEV).manual_seed(2)
     grad = torch.randn(shape, generator=gen, device=DEV).bfloat16()
     param = torch.zeros_like(grad)
-    F.muon_step(param, grad, torch.zeros_like(grad), lr=1.0, weight_decay=0.0, momentum=0.0, nesterov=False)
+    F.muon_step(param, grad, torch.zeros_like(grad), **KW)
     a, b, c = F.NS_COEFFICIENTS
     x = grad.T if shape[0] > shape[1] else grad
     x = (x / x.float().norm().bfloat16()).contiguous()
