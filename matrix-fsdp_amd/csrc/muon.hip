@@ -130,29 +130,42 @@ void update_size(const Matrix& w, GemmProblem* p) {
 }
 
 // Does the group store X^T beside X?  The update product can take X itself (kGemmQColumns), and the epilogues of the update
-// products and the scale kernel then store one orientation of X instead of two; its walk over X is some percent slower.
-// Whole step with X^T -> without, us: 24 of 1536x1024 1241 -> 1090, a hidden2048 layer 1720 -> 1647, six of 1536x4096 in bf16 1365
-// -> 1227, 3072x9216 1561 -> 1478, 5120x15360 5842 -> 5717.  So:
+// products and the scale kernel then store one orientation of X instead of two; its walk over X is some percent slower, which
+// weighs the more the longer K is, and the stores weigh the less the more rounds of tiles they spread over.
+// Whole step with X^T -> without, us: 24 of 1536x1024 1226 -> 1062, a hidden2048 layer 2057 -> 1887, six of 1536x4096 in bf16 1351
+// -> 1216, 3072x12288 2154 -> 1939, 5120x15360 5931 -> 5862.  It is left out
 // * on 256 tiles (on 128 ones 1024x2048 226 -> 251, 1000x3000 with four smaller 316 -> 331; 64 tiles read their operands
 //   straight into registers, K-contiguous);
-// * where the tiles fill more than a round, so that their stores compete (200 tiles 745 -> 756, 288 1172 -> 1175, 324 1908 -> 1853);
-// * where X and X' are about what the memory-side cache of 256 MB holds (X of 157 MB: gains 2 %; the three matrices of a hidden4096
-//   step, 224 MB, lose 2 %);
-// * where kGemmQColumns takes X padded to whole tiles, which a few rows of 4 Mi elements exceed (kMaxQColumnsElements).
+// * where the tiles fill more than a round, so that their stores compete (200 tiles 779 -> 789, 294 1321 -> 1340; 324 1060 -> 1034, 352 1280 -> 1249);
+// * up to an X of 192 MiB, the largest that was measured to gain (200 MiB in one matrix 7638 -> 7606);
+// * where kGemmQColumns takes X padded to whole tiles, which a few rows of 4 Mi elements exceed (kMaxQColumnsElements);
+// * for one matrix with a short side of up to 5632 (5632x9000 4257 -> 4167, 5632x14000 6067 -> 6081; 5888x8000 4258 -> 4401,
+//   8192x8192 8691 -> 8993, 10240x10240 17734 -> 18516);
+// * for several where X, A and B, what an iteration hands to the next, stay within the memory-side cache of 256 MB beside what else
+//   passes through it: 201e6 bytes 2511 -> 2447 (4096x4096*2), 215e6 2730 -> 2742 (3328x4160*3), 227e6 2586 -> 2538
+//   (3072x3072*4); 253e6 3233 -> 3313 (3700x4000*3), 256e6 3061 -> 3156 (3200x3600*4), 327e6 4626 -> 4709 (4096x5120*3);
+// * beyond that for short sides of up to 1700 (1700x1700*18 2342 -> 2322, 1536x4096*16 3390 -> 3264; 1800x1800*14 2340 -> 2380)
+//   and, where X is at least twice A, of up to 2560 (2560x5120*6 4110 -> 4040, 2304x6912*5 3176 -> 3121; 2816x5632*5 4091 ->
+//   4180, and with X less than twice A 2304x2880*12 4008 -> 4102).
 constexpr int64_t kOneOrientationBytes = 192ll << 20;
 bool stores_transposes(const Group& group) {
   GemmGroup g;
-  int64_t bytes = 0, tiles = 0, padded = 0;
+  int64_t x = 0, a = 0, tiles = 0, padded = 0;  // x, a: bytes of every X and A
+  int side = 0;
   g.n = group.n;
   for (int i = 0; i < g.n; ++i) {
     const Matrix& w = group.w[i];
     g.problem[i] = GemmProblem{};
     update_size(w, &g.problem[i]);
-    bytes += static_cast<int64_t>(w.m) * w.n * 2;
+    x += static_cast<int64_t>(w.m) * w.n * 2;
+    a += static_cast<int64_t>(w.m) * w.m * 2;
     tiles += static_cast<int64_t>((w.m + 255) / 256) * ((w.n + 255) / 256);
     padded = std::max(padded, static_cast<int64_t>(w.mp) * w.np);
+    side = std::max(side, w.m);
   }
-  return bytes > kOneOrientationBytes || padded > kMaxQColumnsElements || 4 * tiles < 5 * device_cu_count() || !on_256_tiles(gemm_plan(g, group.scratch));
+  const bool gains = g.n == 1 ? side <= 5632 : x + 2 * a <= 230'000'000 || side <= 1700 || (side <= 2560 && x >= 2 * a);
+  return !gains || x > kOneOrientationBytes || padded > kMaxQColumnsElements || 4 * tiles < 5 * device_cu_count() ||
+         !on_256_tiles(gemm_plan(g, group.scratch));
 }
 
 void choose_transposes(Group* group, int steps) {

@@ -71,6 +71,19 @@ def test_smaller_tiles_store_transposes(tuned):
     assert step_together(shapes, torch.float32)[2] < transposes(shapes)[1]
 
 
+@pytest.mark.parametrize("shapes,stored", [
+    ([(2500, 2500)] * 3, True), ([(2048, 5000)] * 2, False),  # 300 tiles and 320
+    ([(5632, 5700)], False), ([(5700, 5633)], True), ([(8192, 8192)], True),
+    ([(3072, 3072)] * 4, False), ([(3200, 3600)] * 4, True), ([(3328, 3328)] * 5, True),
+    ([(1700, 1700)] * 20, False), ([(1800, 1800)] * 20, True),
+    ([(2560, 5120)] * 6, False), ([(2304, 2880)] * 12, True), ([(2816, 5632)] * 5, True),
+    ([(1536, 4096)] * 16, False), ([(1536, 4096)] * 17, True),  # 192 MiB of X
+])
+def test_where_the_transpose_is_stored(shapes, stored):
+    """Both sides of every line of the choice."""
+    assert (step_together(shapes, torch.bfloat16)[2] < transposes(shapes)[1]) == stored
+
+
 @pytest.mark.parametrize("shape", [(1, 1 << 22), ((1 << 22) - 3, 24)])
 def test_longest_matrices_keep_their_transpose(shape, tuned):
     """On 256 tiles: X padded to whole tiles is 2 GiB, more than a product takes by columns.  The roundings are torch's and the
