@@ -54,9 +54,6 @@ bool plan_matrix(int64_t rows, int64_t cols, char* base, Matrix* w) {
   w->n = static_cast<int>(std::max(rows, cols));
   w->mp = static_cast<int>(round_up(w->m, kPad));
   w->np = static_cast<int>(round_up(w->n, kPad));
-  // rows of X a multiple of 4 KiB apart slow the Gram products down: those of a hidden4096 step 413 -> 386 us with 512 bytes more.
-  // (The square matrices, padded the same way, are no faster.)
-  if (w->np % 2048 == 0 && w->mp >= 1024 && w->np < kMaxGemmLeading) w->np += kPad;
   const int64_t x_bytes = round_up(static_cast<int64_t>(w->mp) * w->np * 2, kAlign);
   const int64_t a_bytes = round_up(static_cast<int64_t>(w->mp) * w->mp * 2, kAlign);
   int64_t off = 0;
@@ -79,7 +76,7 @@ static_assert(kMuonMaxPartials % 4 == 0 && static_cast<int64_t>(kMaxMuonGroup) *
               "the partial sums borrow the products' scratch");
 
 // Most workspace a group is given beyond what its largest matrix needs anyway: three 12288 x 4096 matrices.
-constexpr int64_t kGroupBytes = 1380ll << 20;
+constexpr int64_t kGroupBytes = 1344ll << 20;
 
 // Does the triangle of 256 x 256 tiles of the matrix's symmetric products occupy three quarters of the CUs?  Such a matrix
 // goes through the stages on its own: others beside it would cost their workspace and gain next to nothing (15360 x 5120

@@ -587,6 +587,17 @@ def test_muon_scratch_of_many_matrices_is_bounded(shapes, like):
         assert need == largest
 
 
+@pytest.mark.parametrize("shape, together", [((2048, 2048), 28), ((12288, 4096), 3), ((1024, 2048), 32), ((2560, 2065), 20), ((300, 16384), 20)])
+def test_muon_workspace_holds_whole_tiles_and_no_more(shape, together):
+    """X and X^T twice, A and B, sides rounded up to 256: as many matrices share a launch as the bound has room for."""
+    lib = _lib.lib()
+    m, n = (-(-side // 256) * 256 for side in sorted(shape))
+    shared = lib.mfsdp_muon_workspace_bytes(1, 1) - 6 * 256 * 256 * 2
+    assert lib.mfsdp_muon_workspace_bytes(*shape) - shared == 4 * m * n * 2 + 2 * m * m * 2
+    sides = [(ctypes.c_int64 * 40)(*[side] * 40) for side in shape]
+    assert lib.mfsdp_muon_many_workspace_bytes(40, *sides) - shared == together * (4 * m * n * 2 + 2 * m * m * 2)
+
+
 def test_muon_executed_flops_of_many_matrices():
     """The count for a list follows the launches of ``mfsdp_muon_step_many``: one matrix, matrices that go alone and a
     workspace for one at a time count as single calls; sixteen small matrices share launches of larger tiles than each

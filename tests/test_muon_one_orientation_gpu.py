@@ -8,7 +8,7 @@ from matrix_fsdp_amd.optim import functional as F
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 SHAPES = [(1090, 1500), (1500, 1090), (1037, 1283), (1283, 1037), (1025, 1409), (1111, 1111)] * 4  # 30 tiles of 256 or so each
-# one slab of K, rows shorter than a tile, remainders of tiles and of slabs; rows of X further apart than they are long
+# one slab of K, rows shorter than a tile, remainders of tiles and of slabs
 SMALL = [(1, 7), (65, 63), (300, 257), (64, 1153), (1153, 128), (1100, 2040)]
 KW = dict(lr=1.0, weight_decay=0.0, momentum=0.0, nesterov=False)
 
