@@ -266,8 +266,9 @@ int mfsdp_muon_step_ex(void* param, const void* grad, void* momentum_buf, int dt
  * mfsdp_muon_many_workspace_bytes is what the library makes best use of (bounded: 1.4 GiB, or what the largest matrix
  * needs), mfsdp_muon_workspace_bytes of the largest job is the least it takes.  Every job is checked before
  * anything is enqueued.  Results depend on the other jobs, and on the workspace, only through the order in which a product
- * sums: which tile a launch takes and how its K walk is cut follow from all matrices of the launch, at any size.  The
- * momentum does not depend on them.  A caller that needs bits independent of the other matrices makes one call per matrix.
+ * sums: which tile a launch takes and how its K walk is cut follow from all matrices of the launch, at any size.  After
+ * five iterations in bf16 that is 0.0005 to 0.006 of an update (relative Frobenius).  The momentum does not depend on
+ * them.  A caller that needs bits independent of the other matrices makes one call per matrix.
  */
 typedef struct mfsdp_muon_job {
   void* param;

@@ -119,6 +119,23 @@ def test_precision_does_not_depend_on_the_other_matrices(kind):
         check(u, p / -F.adjust_lr(0.5, None, p.shape), 5, kind)
 
 
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("shape", [(2048, 6144), (2111, 5001), (300, 520)])
+def test_distance_from_torch_and_from_a_call_alone(kind, shape):
+    """Five iterations: 0.0007 to 0.0065 of the update from torch's, 0.0005 to 0.006 between a call with other matrices and one
+    without, on every spectrum.  The bound is the path's tolerance."""
+    update = spectrum(kind, *shape, 5)
+    others = [spectrum("normal", *shape, 9 + i) for i in range(3)] + [spectrum("normal", 700, 1800, 3)]
+    kw = dict(lr=1.0, weight_decay=0.0, momentum=0.0, nesterov=False)
+    params = [torch.zeros(u.shape, device=DEV) for u in [update] + others]
+    F.muon_step_many([(p, u.float(), torch.zeros_like(p), kw) for p, u in zip(params, [update] + others)])
+    alone = F.newton_schulz(update).double()
+    theirs = torch_iterations(update / update.float().norm().bfloat16().clamp(min=1e-7), 5, torch.bfloat16)
+    together = params[0].double() / -F.adjust_lr(1.0, None, shape)
+    for have, want in ((alone, theirs), (together, theirs), (together, alone)):
+        assert float((have - want).norm() / want.norm()) < 1e-2
+
+
 def test_other_coefficients():
     update = spectrum("normal", 2048, 6144, 7)
     check(update, F.newton_schulz(update, ns_steps=4), 4)
