@@ -129,21 +129,21 @@ void update_size(const Matrix& w, GemmProblem* p) {
 // Does the group store X^T beside X?  The update product can take X itself (kGemmQColumns), and the epilogues of the update
 // products and the scale kernel then store one orientation of X instead of two; its walk over X is some percent slower, which
 // weighs the more the longer K is, and the stores weigh the less the more rounds of tiles they spread over.
-// Whole step with X^T -> without, us: 24 of 1536x1024 1226 -> 1062, a hidden2048 layer 2057 -> 1887, six of 1536x4096 in bf16 1351
-// -> 1216, 3072x12288 2154 -> 1939, 5120x15360 5931 -> 5862.  It is left out
+// Whole step with X^T -> without, us: 24 of 1536x1024 1248 -> 1089, a hidden2048 layer 2048 -> 1841, six of 1536x4096 in bf16 1355
+// -> 1213, 3072x12288 2105 -> 1891, 5120x15360 5863 -> 5740.  It is left out
 // * on 256 tiles (on 128 ones 1024x2048 226 -> 251, 1000x3000 with four smaller 316 -> 331; 64 tiles read their operands
 //   straight into registers, K-contiguous);
-// * where the tiles fill more than a round, so that their stores compete (200 tiles 779 -> 789, 294 1321 -> 1340; 324 1060 -> 1034, 352 1280 -> 1249);
-// * up to an X of 192 MiB, the largest that was measured to gain (200 MiB in one matrix 7638 -> 7606);
+// * where the tiles fill more than a round, so that their stores compete (200 tiles 777 -> 793; 320 1063 -> 1030, 352 1294 -> 1261);
+// * up to an X of 192 MiB, about the largest that was measured to gain (200 MiB in one matrix 7494 -> 7475);
 // * where kGemmQColumns takes X padded to whole tiles, which a few rows of 4 Mi elements exceed (kMaxQColumnsElements);
-// * for one matrix with a short side of up to 5632 (5632x9000 4257 -> 4167, 5632x14000 6067 -> 6081; 5888x8000 4258 -> 4401,
-//   8192x8192 8691 -> 8993, 10240x10240 17734 -> 18516);
+// * for one matrix with a short side of up to 5632 (5632x9000 4305 -> 4222, 5632x14000 6118 -> 6129; 5888x8000 4257 -> 4406,
+//   8192x8192 8509 -> 8795, 10240x10240 17431 -> 18139);
 // * for several where X, A and B, what an iteration hands to the next, stay within the memory-side cache of 256 MB beside what else
-//   passes through it: 201e6 bytes 2511 -> 2447 (4096x4096*2), 215e6 2730 -> 2742 (3328x4160*3), 227e6 2586 -> 2538
-//   (3072x3072*4); 253e6 3233 -> 3313 (3700x4000*3), 256e6 3061 -> 3156 (3200x3600*4), 327e6 4626 -> 4709 (4096x5120*3);
-// * beyond that for short sides of up to 1700 (1700x1700*18 2342 -> 2322, 1536x4096*16 3390 -> 3264; 1800x1800*14 2340 -> 2380)
-//   and, where X is at least twice A, of up to 2560 (2560x5120*6 4110 -> 4040, 2304x6912*5 3176 -> 3121; 2816x5632*5 4091 ->
-//   4180, and with X less than twice A 2304x2880*12 4008 -> 4102).
+//   passes through it: 201e6 bytes 2440 -> 2374 (4096x4096*2), 216e6 2645 -> 2651 (3328x4160*3), 226e6 2531 -> 2461
+//   (3072x3072*4); 253e6 3160 -> 3226 (3700x4000*3), 256e6 3045 -> 3128 (3200x3600*4), 327e6 4496 -> 4562 (4096x5120*3);
+// * beyond that for short sides of up to 1700 (1700x1700*18 2346 -> 2333, 1536x4096*16 3314 -> 3203; 1800x1800*14 2265 -> 2303)
+//   and, where X is at least twice A, of up to 2560 (2560x5120*6 4015 -> 3865, 2304x6912*5 3093 -> 3019; 2816x5632*5 3972 ->
+//   4021, and with X less than twice A 2304x2880*12 3891 -> 3958).
 constexpr int64_t kOneOrientationBytes = 192ll << 20;
 bool stores_transposes(const Group& group) {
   GemmGroup g;
