@@ -77,7 +77,7 @@ def tuned():
 
 
 @pytest.mark.parametrize("kind", KINDS)
-@pytest.mark.parametrize("shape,steps", [((2048, 6144), 5), ((5001, 2111), 5), ((2100, 8190), 6), ((4096, 8192), 8), ((768, 2304), 5)])
+@pytest.mark.parametrize("shape,steps", [((2048, 6144), 5), ((5001, 2111), 5), ((2100, 8190), 6), ((4096, 8192), 8), ((8200, 4100), 5), ((768, 2304), 5)])
 def test_precision_is_that_of_torch(kind, shape, steps):
     update = spectrum(kind, *sorted(shape), 5)
     update = update.T.contiguous() if shape[0] > shape[1] else update
